@@ -305,8 +305,9 @@ struct GemmDesc {
   int m, n, k;
   bool a_ones_row = false;              // A's last row (index m-1) is all ones and is not read from `a`
 };
-// true when launch_gemm would take its 16-byte loaders for this problem (they have no all-ones row)
-bool gemm_takes_fast_loaders(const sn_ctx* ctx, const GemmDesc& g, const float* workspace, int64_t workspace_elems);
+// the split kernels (split_gemm.hpp) behind launch_gemm and the convolutions, for the operands *_ok accepts
+bool split_dense_ok(const GemmDesc& g);
+int launch_split_dense(sn_ctx* ctx, const char* name, const GemmDesc& g, const Epilogue& e, float* ws, int64_t ws_elems, bool bf16);
 int launch_gemm(sn_ctx* ctx, const GemmDesc& g, const Epilogue& ep, float* workspace, int64_t workspace_elems, bool bf16);
 // Gradients of a Dense layer from many features onto at most 16 units, as row streams over X (fp32, contiguous
 // [rows, in_f] / [in_f, out_f] / [rows, out_f] tensors); dense_skinny_shape says whether a shape is in their range.
@@ -402,6 +403,13 @@ struct PoolGrad {
 bool conv_wgrad_is_direct(const sn_ctx* ctx, const ConvGeom& g, const float* ws, int64_t ws_elems, bool with_pool = false);
 int launch_conv_wgrad(sn_ctx* ctx, const ConvGeom& g, const float* x, const float* dy, float* dw, float* ws, int64_t ws_elems,
                       const PoolGrad* pool = nullptr);
+
+bool split_conv_fwd_ok(const ConvGeom& g, const float* x, const float* w);
+int launch_split_conv_fwd(sn_ctx* ctx, const ConvGeom& g, const float* x, const float* w, const Epilogue& e, float* ws, int64_t ws_elems);
+bool split_conv_dgrad_ok(const ConvGeom& g, const float* dy, const float* w);
+int launch_split_conv_dgrad(sn_ctx* ctx, const ConvGeom& g, const float* dy, const float* w, float* dx, float* ws, int64_t ws_elems);
+bool split_conv_wgrad_ok(const ConvGeom& g, const float* x, const float* dy);
+int launch_split_conv_wgrad(sn_ctx* ctx, const ConvGeom& g, const float* x, const float* dy, float* dw, float* ws, int64_t ws_elems);
 
 // the same two products with LDS-direct loads into a three-stage ring (conv_ring_kernels.hip), for the shapes *_ok accepts
 bool conv_ring_fwd_ok(const ConvGeom& g, const float* x, const float* w, const Epilogue& e);

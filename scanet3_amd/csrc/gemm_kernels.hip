@@ -1,24 +1,13 @@
-// MFMA GEMM family for gfx950: one LDS-tiled kernel template whose operand tiles are
-// gathered by small "loader" functors, so the same matrix-core inner loop serves
-//   - Dense forward / dX / dW (strided operands: NN, NT, TN),
-//   - Conv2D forward, input gradient and filter gradient as implicit GEMMs over NHWC,
-//   - the LSTM step (4-gate GEMM over [x_t, h_{t-1}]), its dh/dx and its weight gradients.
-// fp32 path: v_mfma_f32_32x32x2_f32.  bf16 path (Dense, on request): operands are rounded to
-// bf16 while they are staged into LDS and multiplied with v_mfma_f32_32x32x16_bf16, fp32 accumulate.
-//
-// Block = 256 threads = 4 wavefronts in a 2x2 arrangement; block tile BM x BN (64 or 128 each),
-// K step 16; each wavefront owns (BM/2) x (BN/2) as 32x32 MFMA tiles.  Small-output problems
-// are split along K over gridDim.z; partial tiles go to a workspace and a second kernel adds
-// them in split order (deterministic) and applies the epilogue.
-#include "common.hpp"
-
-#include <type_traits>
+// GEMM-shaped products for gfx950 besides the split kernels (split_gemm.hpp), and the dispatch between them.
+//   - gemm_kernel: an LDS-tiled product on v_mfma_f32_32x32x2_f32 whose operand tiles are gathered value by value through
+//     small "loader" functors: whatever the split kernels cannot read (fewer than four values along an operand's
+//     contiguous index, strided input gradients, tensors beyond 2 GiB) and the recurrent products that run one time
+//     step per launch.  bf16 form (Dense, on request): operands are rounded while they are staged.
+//     Block = 256 threads = 4 wavefronts in a 2x2 arrangement; block tile BM x BN (64 or 128 each), K step 16.
+//   - small-output products with a long reduction, first-layer convolutions, Dense layers onto a few units.
+#include "split_launch.hpp"
 
 namespace sn {
-
-typedef float f16v __attribute__((ext_vector_type(16)));
-typedef float f4v __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int BK = 16;
 constexpr int THREADS = 256;
@@ -31,17 +20,9 @@ constexpr int THREADS = 256;
 //   init     position a cursor at (outer, k)
 //   load     value at the cursor (0 outside the matrix or past k_end)
 //   advance  move the cursor dk along k
-// The kernel drives a loader through a second, finer interface that separates what is the same for the
-// whole workgroup in one k tile (struct Tile: the tile's first k and whatever follows from it, kept in
-// scalar registers) from what belongs to the thread (Cursor):
-//   init4(c, outer, k_begin, kk)   kk = the thread's fixed k offset inside every tile
-//   tile_init / tile_advance        uniform state for the tile starting at k0, then k0 += BK
-//   thread_advance                  per-thread part of moving on one tile (nothing for the FAST loaders)
-//   load_t / load4_t                value(s) at (cursor, tile)
-// Loaders written against the cursor interface only get the second one from SN_CURSOR_ONLY_API; the FAST
-// loaders implement it directly with 32-bit offsets, a per-thread validity mask and no branches.
+// The kernel drives a loader through a second interface on top of these (init4, load_t, load4_t, thread_advance), which
+// SN_CURSOR_ONLY_API supplies.
 #define SN_CURSOR_ONLY_API                                                                                         \
-  static constexpr bool FAST = false;                                                                              \
   struct Tile {};                                                                                                  \
   __device__ __forceinline__ void tile_init(Tile&, int) const {}                                                   \
   __device__ __forceinline__ void tile_advance(Tile&) const {}                                                     \
@@ -50,21 +31,6 @@ constexpr int THREADS = 256;
   __device__ __forceinline__ float load_t(const Cursor& c, const Tile&, int k_end) const { return load(c, k_end); } \
   __device__ __forceinline__ bool load4_t(const Cursor& c, const Tile&, int k_end, float (&v)[4]) const { load4(c, k_end, v); return true; }
 
-// 16-byte load without a branch: a lane whose element lies outside the matrix reads the first 16 bytes of
-// the tensor instead (always mapped, 16-byte aligned) and discards them.  Offsets are 32-bit: the host only
-// picks the FAST loaders for tensors below 2 GiB.
-constexpr int64_t FAST_SPAN = (int64_t)1 << 31;
-// Returns `valid` and leaves the select to the caller, who applies it when the values go to LDS one K tile later: a select
-// right here would make the loads' consumer sit directly behind them, and the wait for the data would land in front of
-// the current tile's MFMAs instead of behind them.
-__device__ __forceinline__ bool sel_load4(const float* base, uint32_t byte_off, bool valid, float (&v)[4]) {
-  const f4v r = *(const f4v*)((const char*)base + (valid ? byte_off : 0u));
-  v[0] = r[0];
-  v[1] = r[1];
-  v[2] = r[2];
-  v[3] = r[3];
-  return valid;
-}
 static inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 // ONES: the loader knows one extra outer index that reads as all ones (a separate type, so the plain loader's
@@ -433,297 +399,12 @@ struct LstmWgradA {
   SN_CURSOR_ONLY_API
 };
 
-// ============================================================================ FAST loaders
-// Strided operand with unit stride along its contiguous index: value(outer, k) = p[outer*s_outer + k*s_k].
-template <bool KC>
-struct FlatLoader {
-  static constexpr bool K_CONTIG = KC, FAST = true;
-  const float* p;
-  int s_outer, s_k;  // elements; one of them is 1
-  int outer_n;
-  struct Cursor {
-    uint32_t base;  // byte offset of (outer, kk)
-    int kk;         // < 0: outside the matrix
-  };
-  struct Tile {
-    int k0;
-    uint32_t koff;  // byte offset of k0
-  };
-  __device__ __forceinline__ void init4(Cursor& c, int outer, int, int kk) const {
-    c.kk = outer < outer_n ? kk : -0x40000000;
-    c.base = ((uint32_t)outer * (uint32_t)s_outer + (uint32_t)kk * (uint32_t)s_k) * 4u;
-  }
-  __device__ __forceinline__ void tile_init(Tile& t, int k0) const { t.k0 = k0; t.koff = (uint32_t)k0 * (uint32_t)s_k * 4u; }
-  __device__ __forceinline__ void tile_advance(Tile& t) const { t.k0 += BK; t.koff += (uint32_t)BK * (uint32_t)s_k * 4u; }
-  __device__ __forceinline__ void thread_advance(Cursor&) const {}
-  __device__ __forceinline__ bool load4_t(const Cursor& c, const Tile& t, int k_end, float (&v)[4]) const {
-    return sel_load4(p, c.base + t.koff, c.kk >= 0 && t.k0 + c.kk < k_end, v);
-  }
-  __device__ __forceinline__ float load_t(const Cursor&, const Tile&, int) const { return 0.f; }  // FAST loaders run VEC = 4 only
-  static bool ok(const float* p, int64_t s_outer, int64_t s_k, int outer_n, int K) {
-    if (!aligned16(p) || s_outer < 0 || s_k < 0 || ((int64_t)outer_n * s_outer + (int64_t)K * s_k) * 4 >= FAST_SPAN) return false;
-    return KC ? (s_k == 1 && s_outer % 4 == 0 && K % 4 == 0) : (s_outer == 1 && s_k % 4 == 0 && outer_n % 4 == 0);
-  }
-};
-
-// A operand of a convolution seen as a product: row m is a position (b, iy, ix) of the iteration space
-// (the output for the forward pass, the input for the input gradient), k = (tap r, tap q, channel) with the
-// channel fastest and the channel count a multiple of BK, so that a k tile lies inside one tap:
-//   value = src[b, iy*sy + oy + r*ty, ix*sx + ox + q*tx, channel]   (0 outside the source image)
-// forward: src = x, (sy, sx) = strides, (oy, ox) = -padding, (ty, tx) = (+1, +1);
-// input gradient with unit strides: src = dy, (sy, sx) = (1, 1), (oy, ox) = +padding, (ty, tx) = (-1, -1).
-// Which taps fall inside the image is fixed per row: a 32-bit mask computed once per thread.
-struct TapLoader {
-  static constexpr bool K_CONTIG = true, FAST = true;
-  const float* src;
-  int M, ih, iw;       // iteration space
-  int sy, sx, oy, ox, ty, tx;
-  int H, W, C;         // source image
-  int kh, kw;
-  struct Cursor {
-    uint32_t base;  // byte offset of (b, y0, x0, kk), possibly outside the tensor (then no tap is valid there)
-    uint32_t mask;  // bit r*kw+q: tap inside the image
-    int kk;
-  };
-  struct Tile {
-    int k0, r, q, c0, rq;
-    uint32_t tapoff;  // byte offset of (r*ty, q*tx, c0) relative to (y0, x0, 0)
-  };
-  __device__ __forceinline__ void init4(Cursor& c, int m, int, int kk) const {
-    c.kk = kk;
-    c.mask = 0;
-    c.base = 0;
-    if (m >= M) return;
-    const int ix = m % iw;
-    const int t = m / iw;
-    const int iy = t % ih;
-    const int b = t / ih;
-    const int y0 = iy * sy + oy, x0 = ix * sx + ox;
-    c.base = (uint32_t)(((b * H + y0) * W + x0) * C + kk) * 4u;
-    for (int r = 0; r < kh; ++r)
-      for (int q = 0; q < kw; ++q)
-        if ((unsigned)(y0 + r * ty) < (unsigned)H && (unsigned)(x0 + q * tx) < (unsigned)W) c.mask |= 1u << (r * kw + q);
-  }
-  __device__ __forceinline__ void set_tap(Tile& t) const { t.tapoff = (uint32_t)((t.r * ty * W + t.q * tx) * C + t.c0) * 4u; }
-  __device__ __forceinline__ void tile_init(Tile& t, int k0) const {
-    t.k0 = k0;
-    t.rq = k0 / C;
-    t.c0 = k0 - t.rq * C;
-    t.r = t.rq / kw;
-    t.q = t.rq - t.r * kw;
-    set_tap(t);
-  }
-  __device__ __forceinline__ void tile_advance(Tile& t) const {
-    t.k0 += BK;
-    t.c0 += BK;
-    if (t.c0 >= C) {
-      t.c0 = 0;
-      ++t.rq;
-      if (++t.q == kw) { t.q = 0; ++t.r; }
-    }
-    set_tap(t);
-  }
-  __device__ __forceinline__ void thread_advance(Cursor&) const {}
-  __device__ __forceinline__ bool load4_t(const Cursor& c, const Tile& t, int k_end, float (&v)[4]) const {
-    return sel_load4(src, c.base + t.tapoff, ((c.mask >> (t.rq & 31)) & 1u) != 0 && t.k0 + c.kk < k_end, v);
-  }
-  __device__ __forceinline__ float load_t(const Cursor&, const Tile&, int) const { return 0.f; }
-  static bool ok(const float* src, int n, int H, int W, int C, int kh, int kw) {
-    return C % BK == 0 && kh * kw <= 32 && aligned16(src) && (int64_t)n * H * W * C * 4 < FAST_SPAN;
-  }
-};
-
-// B operand of the input gradient: column n = ci, k = (r, q, co): w[((r*kw+q)*cin + ci)*cout + co], cout % BK == 0
-struct DgradWLoader {
-  static constexpr bool K_CONTIG = true, FAST = true;
-  const float* w;
-  int cin, cout;
-  struct Cursor {
-    uint32_t base;  // byte offset of (tap 0, ci, kk)
-    int kk;         // < 0: outside the matrix
-  };
-  struct Tile {
-    int k0, c0, rq;
-    uint32_t koff;
-  };
-  __device__ __forceinline__ void init4(Cursor& c, int n, int, int kk) const {
-    c.kk = n < cin ? kk : -0x40000000;
-    c.base = (uint32_t)(n * cout + kk) * 4u;
-  }
-  __device__ __forceinline__ void tile_init(Tile& t, int k0) const {
-    t.k0 = k0;
-    t.rq = k0 / cout;
-    t.c0 = k0 - t.rq * cout;
-    t.koff = (uint32_t)(t.rq * cin * cout + t.c0) * 4u;
-  }
-  __device__ __forceinline__ void tile_advance(Tile& t) const {
-    t.k0 += BK;
-    t.c0 += BK;
-    if (t.c0 >= cout) { t.c0 = 0; ++t.rq; }
-    t.koff = (uint32_t)(t.rq * cin * cout + t.c0) * 4u;
-  }
-  __device__ __forceinline__ void thread_advance(Cursor&) const {}
-  __device__ __forceinline__ bool load4_t(const Cursor& c, const Tile& t, int k_end, float (&v)[4]) const {
-    return sel_load4(w, c.base + t.koff, c.kk >= 0 && t.k0 + c.kk < k_end, v);
-  }
-  __device__ __forceinline__ float load_t(const Cursor&, const Tile&, int) const { return 0.f; }
-};
-
-// A operand of the filter gradient: row m = (r, q, ci) with ci fastest (4 consecutive ci per load), k = output
-// pixel (b, oh, ow): x[b, oh*sh - pt + r, ow*sw - pl + q, ci].  Every thread keeps its own pixel and moves it
-// BK pixels per tile, carrying into the next output row / image by additions only.
-struct WgradXLoader {
-  static constexpr bool K_CONTIG = false, FAST = true;
-  const float* x;
-  ConvGeom g;
-  int M;
-  int interior;  // no padding: every tap of every output pixel lies inside the image, no bounds checks
-  struct Cursor {
-    uint32_t off;  // byte offset of the element
-    int ow, oh, iy, ix, kk;  // kk < 0: row outside the matrix
-  };
-  struct Tile {
-    int k0;
-  };
-  __device__ __forceinline__ void init4(Cursor& c, int m, int kb, int kk) const {
-    c.kk = m < M ? kk : -0x40000000;
-    const int ci = m % g.cin;
-    const int rq = m / g.cin;
-    const int q = rq % g.kw, r = rq / g.kw;
-    const int p = kb + kk;
-    c.ow = p % g.wo;
-    const int t = p / g.wo;
-    c.oh = t % g.ho;
-    const int b = t / g.ho;
-    c.iy = c.oh * g.sh - g.pt + r;
-    c.ix = c.ow * g.sw - g.pl + q;
-    c.off = (uint32_t)(((b * g.h + c.iy) * g.w + c.ix) * g.cin + ci) * 4u;
-  }
-  __device__ __forceinline__ void tile_init(Tile& t, int k0) const { t.k0 = k0; }
-  __device__ __forceinline__ void tile_advance(Tile& t) const { t.k0 += BK; }
-  __device__ __forceinline__ void thread_advance(Cursor& c) const {
-    c.ow += BK;
-    c.ix += BK * g.sw;
-    c.off += (uint32_t)(BK * g.sw * g.cin) * 4u;
-    while (c.ow >= g.wo) {  // next output row: back wo pixels, down sh input rows
-      c.ow -= g.wo;
-      c.ix -= g.wo * g.sw;
-      c.off += (uint32_t)((g.sh * g.w - g.wo * g.sw) * g.cin) * 4u;
-      c.iy += g.sh;
-      if (++c.oh == g.ho) {  // next image
-        c.oh = 0;
-        c.iy -= g.ho * g.sh;
-        c.off += (uint32_t)((g.h - g.ho * g.sh) * g.w * g.cin) * 4u;
-      }
-    }
-  }
-  __device__ __forceinline__ bool load4_t(const Cursor& c, const Tile& t, int k_end, float (&v)[4]) const {
-    const bool inside = interior || ((unsigned)c.iy < (unsigned)g.h && (unsigned)c.ix < (unsigned)g.w);
-    return sel_load4(x, c.off, c.kk >= 0 && t.k0 + c.kk < k_end && inside, v);
-  }
-  __device__ __forceinline__ float load_t(const Cursor&, const Tile&, int) const { return 0.f; }
-  static bool ok(const float* x, const ConvGeom& g) {
-    return g.cin % 4 == 0 && aligned16(x) && ((int64_t)g.n + 1) * g.h * g.w * g.cin * 4 < FAST_SPAN;
-  }
-};
-
 // ============================================================================ epilogues
-__device__ __forceinline__ float ep_act(int act, float v, float param) {
-  switch (act) {
-    case SN_ACT_SIGMOID: return 1.0f / (1.0f + expf(-v));
-    case SN_ACT_TANH: return tanhf(v);
-    case SN_ACT_RELU: return fmaxf(param, v);
-    default: return v;
-  }
-}
-
-// The same activation over N values with ONE dispatch on `act`: a switch per value costs a handful of scalar branches
-// each, which in a 16-value accumulator tile is more instruction-fetch stalls than arithmetic.
-template <int N>
-__device__ __forceinline__ void ep_act_block(int act, float (&v)[N], float param) {
-  switch (act) {
-    case SN_ACT_SIGMOID:
-#pragma unroll
-      for (int k = 0; k < N; ++k) v[k] = 1.0f / (1.0f + expf(-v[k]));
-      break;
-    case SN_ACT_TANH:
-#pragma unroll
-      for (int k = 0; k < N; ++k) v[k] = tanhf(v[k]);
-      break;
-    case SN_ACT_RELU:
-#pragma unroll
-      for (int k = 0; k < N; ++k) v[k] = fmaxf(param, v[k]);
-      break;
-    default: break;
-  }
-}
-
-struct StdEpilogue {
-  Epilogue e;
-  __device__ __forceinline__ void store(int m, int n, float acc) const {
-    if (m == e.row_index) {
-      e.row_out[n] = acc;
-      return;
-    }
-    float v = acc;
-    if (e.bias) v = v + e.bias[n];
-    e.out[(int64_t)m * e.ldo + n] = ep_act(e.act, v, e.act_param);
-  }
-};
-
-// A lane's 16 accumulator values of one 32x32 MFMA tile: column n, rows row0 + 8*(v/4) + v%4 (v = 0..15), rows >= M dropped.
-template <class EP>
-__device__ __forceinline__ void store16(const EP& ep, int row0, int n, const f16v& acc, int M) {
-#pragma unroll
-  for (int v = 0; v < 16; ++v) {
-    const int row = row0 + (v >> 2) * 8 + (v & 3);
-    if (row < M) ep.store(row, n, acc[v]);
-  }
-}
-// The plain epilogue reads the column's bias once and dispatches on the activation once for the 16 values: inside an
-// instantiation the activation is a compile-time constant, so the 16 stores carry no scalar branches.
-template <int ACT>
-__device__ __forceinline__ float ep_act_const(float v, float param) {
-  if constexpr (ACT == SN_ACT_SIGMOID) return 1.0f / (1.0f + expf(-v));
-  else if constexpr (ACT == SN_ACT_TANH) return tanhf(v);
-  else if constexpr (ACT == SN_ACT_RELU) return fmaxf(param, v);
-  else return v;
-}
-
-template <int ACT>
-__device__ __forceinline__ void store16_act(const Epilogue& e, int row0, int n, const f16v& acc, int M) {
-  const bool has_bias = e.bias != nullptr;
-  const float b = has_bias ? e.bias[n] : 0.f;
-  float* out = e.out + (int64_t)row0 * e.ldo + n;
-  // One value at a time, each behind its own row check: a straight run of 16 stores lets the compiler compute all 16
-  // addresses and read all 16 accumulators up front, which doubles the kernel's registers and costs the split-K launches
-  // their occupancy (measured: filter gradient 31 -> 37 us).
-#pragma unroll
-  for (int k = 0; k < 16; ++k) {
-    const int dr = (k >> 2) * 8 + (k & 3);
-    if (row0 + dr >= M) continue;
-    if (row0 + dr == e.row_index) {
-      e.row_out[n] = acc[k];
-    } else {
-      const float x = has_bias ? acc[k] + b : acc[k];
-      out[(int64_t)dr * e.ldo] = ep_act_const<ACT>(x, e.act_param);
-    }
-  }
-}
-
-__device__ __forceinline__ void store16(const StdEpilogue& ep, int row0, int n, const f16v& acc, int M) {
-  switch (ep.e.act) {
-    case SN_ACT_SIGMOID: store16_act<SN_ACT_SIGMOID>(ep.e, row0, n, acc, M); break;
-    case SN_ACT_TANH: store16_act<SN_ACT_TANH>(ep.e, row0, n, acc, M); break;
-    case SN_ACT_RELU: store16_act<SN_ACT_RELU>(ep.e, row0, n, acc, M); break;
-    default: store16_act<SN_ACT_IDENTITY>(ep.e, row0, n, acc, M); break;
-  }
-}
-
 struct LstmZEpilogue {  // z[m, n] = acc + b_gate[u]
   float* z;
   const float* b[4];
   int H, G;
+  __device__ __forceinline__ int map_row(int m) const { return m; }
   __device__ __forceinline__ void store(int m, int n, float acc) const {
     const int gate = n / H, u = n - gate * H;
     float v = acc;
@@ -735,6 +416,7 @@ struct LstmZEpilogue {  // z[m, n] = acc + b_gate[u]
 struct LstmWgradEpilogue {  // rows: F kernel rows, H recurrent rows, 1 bias row; columns gate*H + u
   LstmGrads g;
   int F, H;
+  __device__ __forceinline__ int map_row(int m) const { return m; }
   __device__ __forceinline__ void store(int m, int n, float acc) const {
     const int gate = n / H, u = n - gate * H;
     if (m < F) g.wk[gate][(int64_t)m * H + u] = acc;
@@ -746,6 +428,7 @@ struct LstmWgradEpilogue {  // rows: F kernel rows, H recurrent rows, 1 bias row
 struct DxScatterEpilogue {  // dx[m, t, n] of a [rows, T, F] tensor
   float* dx;
   int T, F, t;
+  __device__ __forceinline__ int map_row(int m) const { return m; }
   __device__ __forceinline__ void store(int m, int n, float acc) const { dx[((int64_t)m * T + t) * F + n] = acc; }
 };
 
@@ -923,92 +606,6 @@ __global__ __launch_bounds__(THREADS) void gemm_kernel(int M, int N, int K, int 
     }
 }
 
-// Adds the split-K partial tiles.  Eight lanes share one output: lane g adds splits g, g+8, ... in order, then the
-// eight partial sums are combined pairwise (a fixed tree), so the result does not depend on the launch shape.
-template <class EP>
-__global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restrict__ ws, int splits, int M, int N, EP ep) {
-  const int64_t total = (int64_t)M * N;
-  const int g = threadIdx.x >> 5, j = threadIdx.x & 31;  // 8 groups of 32 consecutive outputs
-  for (int64_t base = (int64_t)blockIdx.x * 32; base < total; base += (int64_t)gridDim.x * 32) {
-    const int64_t i = base + j;
-    float s = 0.f;
-    if (i < total) {
-      int z = g;
-      for (; z + 120 < splits; z += 128) {  // 16 loads in flight, added in split order
-        float a[16];
-#pragma unroll
-        for (int u = 0; u < 16; ++u) a[u] = ws[(int64_t)(z + 8 * u) * total + i];
-#pragma unroll
-        for (int u = 0; u < 16; ++u) s += a[u];
-      }
-      for (; z + 24 < splits; z += 32) {  // 4 loads in flight
-        float a[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) a[u] = ws[(int64_t)(z + 8 * u) * total + i];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) s += a[u];
-      }
-      for (; z < splits; z += 8) s += ws[(int64_t)z * total + i];
-    }
-    __shared__ float part[8][32];
-    part[g][j] = s;
-    __syncthreads();
-    if (g == 0 && i < total) {
-      const float t = ((part[0][j] + part[1][j]) + (part[2][j] + part[3][j])) + ((part[4][j] + part[5][j]) + (part[6][j] + part[7][j]));
-      ep.store((int)(i / N), (int)(i % N), t);
-    }
-    __syncthreads();
-  }
-}
-
-// The same reduction when M*N is a multiple of 4 (every partial tile then starts on a 16-byte boundary): a lane owns 4
-// consecutive outputs and reads them as one 16-byte load per split; every output sees the same additions in the same order.
-template <class EP>
-__global__ __launch_bounds__(256) void splitk_reduce4_kernel(const float* __restrict__ ws, int splits, int M, int N, EP ep) {
-  const int64_t total4 = (int64_t)M * N / 4;
-  const int g = threadIdx.x >> 5, j = threadIdx.x & 31;  // 8 groups of 32 lanes x 4 consecutive outputs
-  for (int64_t base = (int64_t)blockIdx.x * 32; base < total4; base += (int64_t)gridDim.x * 32) {
-    const int64_t i = base + j;
-    f4v s = {0.f, 0.f, 0.f, 0.f};
-    if (i < total4) {
-      const f4v* w4 = reinterpret_cast<const f4v*>(ws) + i;
-      int z = g;
-      for (; z + 56 < splits; z += 64) {  // 8 loads of 16 bytes in flight, added in split order
-        f4v a[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) a[u] = w4[(int64_t)(z + 8 * u) * total4];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) s += a[u];
-      }
-      for (; z < splits; z += 8) s += w4[(int64_t)z * total4];
-    }
-    __shared__ f4v part4[8][32];
-    part4[g][j] = s;
-    __syncthreads();
-    if (g == 0 && i < total4) {
-      const f4v t = ((part4[0][j] + part4[1][j]) + (part4[2][j] + part4[3][j])) + ((part4[4][j] + part4[5][j]) + (part4[6][j] + part4[7][j]));
-      // row and column of the first of the four outputs by one division (32-bit where the index allows: a 64-bit division
-      // is some hundred instructions on this device), the others by stepping
-      const int64_t o0 = i * 4;
-      int m, n;
-      if (o0 < ((int64_t)1 << 31)) {
-        const uint32_t q = (uint32_t)o0 / (uint32_t)N;
-        m = (int)q;
-        n = (int)((uint32_t)o0 - q * (uint32_t)N);
-      } else {
-        m = (int)(o0 / N);
-        n = (int)(o0 % N);
-      }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        ep.store(m, n, t[e]);
-        if (++n == N) { n = 0; ++m; }
-      }
-    }
-    __syncthreads();
-  }
-}
-
 // ============================================================================ small output, long reduction
 // C[M,N] with M*N <= 1024 and K in the thousands (first-layer filter gradients, Dense layers onto a few
 // classes): too little output for MFMA tiles to occupy the chip. Workgroups stride over 64-long slices of K,
@@ -1128,11 +725,12 @@ int64_t gemm_workspace_elems(int m, int n, int k, int cu) {
   // room for the partial sums of the small-output kernel, or for the largest split count launch_tiles may pick
   const int parts = small_parts(m, n, k, cu, -1);
   if (parts) return (int64_t)parts * m * n;
+  const int64_t planned = split_workspace_elems(m, n, k, cu);
   const int64_t tiles = ceil_div(m, 64) * ceil_div(n, 64);
-  if (tiles >= cu || k < SPLIT_MIN_K) return 0;
+  if (tiles >= cu || k < SPLIT_MIN_K) return planned;
   int64_t splits = std::min<int64_t>(ceil_div((int64_t)SPLIT_WG_PER_CU * cu, tiles), std::max<int64_t>(1, k / 32));
   splits = std::min<int64_t>(splits, SPLIT_MAX);
-  return splits * (int64_t)m * n;
+  return std::max(planned, splits * (int64_t)m * n);
 }
 
 template <int BM, int BN, bool BF16, class AL, class BL, class EP>
@@ -1157,41 +755,15 @@ static int launch_tiles(sn_ctx* ctx, const char* name, int M, int N, int K, cons
                                : dim3((unsigned)ceil_div(N, BN), (unsigned)ceil_div(M, BM), 1);
   {
     LaunchScope scope(ctx, name, M, N, K);
-    if constexpr (AL::FAST && BL::FAST) {  // the caller has checked what 16-byte loads need
-      hipLaunchKernelGGL((gemm_kernel<BM, BN, BF16, 4, AL, BL, EP>), grid, dim3(THREADS), 0, ctx->stream, M, N, K, k_per_split, al, bl, ep,
-                         splits > 1 ? ws : nullptr, splits);
-    } else {
       if (al.vec4_ok(K) && bl.vec4_ok(K))
         hipLaunchKernelGGL((gemm_kernel<BM, BN, BF16, 4, AL, BL, EP>), grid, dim3(THREADS), 0, ctx->stream, M, N, K, k_per_split, al, bl, ep,
                            splits > 1 ? ws : nullptr, splits);
       else
         hipLaunchKernelGGL((gemm_kernel<BM, BN, BF16, 1, AL, BL, EP>), grid, dim3(THREADS), 0, ctx->stream, M, N, K, k_per_split, al, bl, ep,
                            splits > 1 ? ws : nullptr, splits);
-    }
-  }
-  if (splits > 1) {
-    const int64_t total = (int64_t)M * N;
-    if constexpr (std::is_same<EP, StdEpilogue>::value) {
-      // a caller that applies the optimizer next takes the sum of the partial tiles into that launch
-      if (ctx->defer && total % 4 == 0 && total >= 4096 && total < ((int64_t)1 << 30) && aligned16(ws) && !ep.e.bias && ep.e.act == SN_ACT_IDENTITY &&
-          ep.e.row_index < 0 && ep.e.ldo == N) {
-        *ctx->defer = DeferredReduce{1, ws, splits, (int)total, ep.e.out};
-        ctx->defer = nullptr;
-        SN_HIP(hipGetLastError());
-        return SN_OK;
-      }
-    }
-    LaunchScope scope(ctx, "splitk_reduce");
-    if (total % 4 == 0 && total >= 4096 && aligned16(ws)) {
-      const int64_t blocks = std::min<int64_t>(ceil_div(total / 4, 32), (int64_t)ctx->compute_units * 16);
-      hipLaunchKernelGGL((splitk_reduce4_kernel<EP>), dim3((unsigned)blocks), dim3(256), 0, ctx->stream, (const float*)ws, splits, M, N, ep);
-    } else {
-      const int64_t blocks = std::min<int64_t>(ceil_div(total, 32), (int64_t)ctx->compute_units * 16);
-      hipLaunchKernelGGL((splitk_reduce_kernel<EP>), dim3((unsigned)blocks), dim3(256), 0, ctx->stream, (const float*)ws, splits, M, N, ep);
-    }
   }
   SN_HIP(hipGetLastError());
-  return SN_OK;
+  return splits > 1 ? launch_split_reduce(ctx, ws, splits, M, N, ep) : SN_OK;
 }
 
 template <bool BF16, class AL, class BL, class EP>
@@ -1199,8 +771,7 @@ static int launch_any(sn_ctx* ctx, const char* name, int M, int N, int K, const 
                       int64_t ws_elems) {
   if (M <= 0 || N <= 0) return SN_OK;
   SN_REQUIRE(K > 0, "%s: empty reduction dimension", name);
-  if constexpr (!(AL::FAST && BL::FAST)) {
-   if (const int parts = ws ? small_parts(M, N, K, ctx->compute_units, ws_elems) : 0) {
+  if (const int parts = ws ? small_parts(M, N, K, ctx->compute_units, ws_elems) : 0) {
     {
       LaunchScope scope(ctx, name, M, N, K);
       hipLaunchKernelGGL((gemm_small_kernel<AL, BL>), dim3((unsigned)parts), dim3(256), (size_t)SMALL_SLICE * (M + N) * sizeof(float),
@@ -1211,7 +782,6 @@ static int launch_any(sn_ctx* ctx, const char* name, int M, int N, int K, const 
                        parts, M, N, ep);
     SN_HIP(hipGetLastError());
     return SN_OK;
-   }
   }
   bool big_m = M > 64, big_n = N > 64;
   // 128-wide tiles only when they still cover every CU at least twice; otherwise more, smaller workgroups
@@ -1223,44 +793,15 @@ static int launch_any(sn_ctx* ctx, const char* name, int M, int N, int K, const 
   return launch_tiles<64, 64, BF16>(ctx, name, M, N, K, al, bl, ep, ws, ws_elems);
 }
 
-static bool fast_pair_ok(const sn_ctx* ctx, const GemmDesc& g, const float* ws, int64_t ws_elems) {
-  if (g.a_ones_row || (ws && small_parts(g.m, g.n, g.k, ctx->compute_units, ws_elems))) return false;
-  const bool akc = g.a_sk == 1, bkc = g.b_sk == 1 && g.b_sn != 1;
-  const bool a_ok = akc ? FlatLoader<true>::ok(g.a, g.a_sm, g.a_sk, g.m, g.k) : FlatLoader<false>::ok(g.a, g.a_sm, g.a_sk, g.m, g.k);
-  const bool b_ok = bkc ? FlatLoader<true>::ok(g.b, g.b_sn, g.b_sk, g.n, g.k) : FlatLoader<false>::ok(g.b, g.b_sn, g.b_sk, g.n, g.k);
-  return a_ok && b_ok;
-}
-
-bool gemm_takes_fast_loaders(const sn_ctx* ctx, const GemmDesc& g, const float* workspace, int64_t workspace_elems) {
-  return fast_pair_ok(ctx, g, workspace, workspace_elems);
-}
-
 template <bool BF16>
 static int launch_gemm_t(sn_ctx* ctx, const GemmDesc& g, const Epilogue& e, float* ws, int64_t ws_elems) {
   StdEpilogue ep{e};
   const char* name = BF16 ? "gemm_bf16" : "gemm_f32";
   const bool akc = g.a_sk == 1, bkc = g.b_sk == 1 && g.b_sn != 1;
-  // FAST loaders whenever both operands allow 16-byte loads, unless the small-output kernel (cursor loaders) takes the problem
-  if (fast_pair_ok(ctx, g, ws, ws_elems)) {
-    if (akc && bkc && FlatLoader<true>::ok(g.a, g.a_sm, g.a_sk, g.m, g.k) && FlatLoader<true>::ok(g.b, g.b_sn, g.b_sk, g.n, g.k)) {
-      FlatLoader<true> al{g.a, (int)g.a_sm, (int)g.a_sk, g.m}, bl{g.b, (int)g.b_sn, (int)g.b_sk, g.n};
-      return launch_any<BF16>(ctx, name, g.m, g.n, g.k, al, bl, ep, ws, ws_elems);
-    }
-    if (akc && !bkc && FlatLoader<true>::ok(g.a, g.a_sm, g.a_sk, g.m, g.k) && FlatLoader<false>::ok(g.b, g.b_sn, g.b_sk, g.n, g.k)) {
-      FlatLoader<true> al{g.a, (int)g.a_sm, (int)g.a_sk, g.m};
-      FlatLoader<false> bl{g.b, (int)g.b_sn, (int)g.b_sk, g.n};
-      return launch_any<BF16>(ctx, name, g.m, g.n, g.k, al, bl, ep, ws, ws_elems);
-    }
-    if (!akc && bkc && FlatLoader<false>::ok(g.a, g.a_sm, g.a_sk, g.m, g.k) && FlatLoader<true>::ok(g.b, g.b_sn, g.b_sk, g.n, g.k)) {
-      FlatLoader<false> al{g.a, (int)g.a_sm, (int)g.a_sk, g.m};
-      FlatLoader<true> bl{g.b, (int)g.b_sn, (int)g.b_sk, g.n};
-      return launch_any<BF16>(ctx, name, g.m, g.n, g.k, al, bl, ep, ws, ws_elems);
-    }
-    if (!akc && !bkc && FlatLoader<false>::ok(g.a, g.a_sm, g.a_sk, g.m, g.k) && FlatLoader<false>::ok(g.b, g.b_sn, g.b_sk, g.n, g.k)) {
-      FlatLoader<false> al{g.a, (int)g.a_sm, (int)g.a_sk, g.m}, bl{g.b, (int)g.b_sn, (int)g.b_sk, g.n};
-      return launch_any<BF16>(ctx, name, g.m, g.n, g.k, al, bl, ep, ws, ws_elems);
-    }
-  }
+  // the small-output kernel takes its shapes first, then the split kernels whatever they can read, and what is left (an
+  // operand with fewer than four values along its contiguous index, tensors beyond 2 GiB) goes through cursor loaders
+  if (!(ws && small_parts(g.m, g.n, g.k, ctx->compute_units, ws_elems)) && split_dense_ok(g))
+    return launch_split_dense(ctx, name, g, e, ws, ws_elems, BF16);
   if (g.a_ones_row) {  // the weight-gradient form: A = X^T (outer index contiguous) plus the ones row, B = dY (row major)
     SN_REQUIRE(!akc && !bkc, "gemm: the all-ones row is built for A^T-major A and row-major B only");
     StridedLoader<false, true> al{g.a, g.a_sm, g.a_sk, g.m - 1, g.m - 1};
@@ -1492,11 +1033,7 @@ int launch_conv_fwd(sn_ctx* ctx, const ConvGeom& g, const float* x, const float*
   }
   if (conv_ring_fwd_ok(g, x, w, e)) return launch_conv_ring_fwd(ctx, g, x, w, e);
   StdEpilogue ep{e};
-  if (TapLoader::ok(x, g.n, g.h, g.w, g.cin, g.kh, g.kw) && FlatLoader<false>::ok(w, 1, g.cout, N, K)) {
-    TapLoader al{x, M, g.ho, g.wo, g.sh, g.sw, -g.pt, -g.pl, 1, 1, g.h, g.w, g.cin, g.kh, g.kw};
-    FlatLoader<false> bl{w, 1, g.cout, N};
-    return launch_any<false>(ctx, "conv2d_forward", M, N, K, al, bl, ep, ws, ws_elems);
-  }
+  if (split_conv_fwd_ok(g, x, w)) return launch_split_conv_fwd(ctx, g, x, w, e, ws, ws_elems);
   ConvFwdA al{x, g, M};
   StridedLoader<false> bl{w, 1, (int64_t)g.cout, N};  // filter [kh,kw,cin,cout] is a row-major [K, cout] matrix
   return launch_any<false>(ctx, "conv2d_forward", M, N, K, al, bl, ep, ws, ws_elems);
@@ -1509,12 +1046,7 @@ int launch_conv_dgrad(sn_ctx* ctx, const ConvGeom& g, const float* dy, const flo
   e.ldo = g.cin;
   if (conv_ring_dgrad_ok(g, dy, w)) return launch_conv_ring_dgrad(ctx, g, dy, w, dx);
   StdEpilogue ep{e};
-  if (g.sh == 1 && g.sw == 1 && TapLoader::ok(dy, g.n, g.ho, g.wo, g.cout, g.kh, g.kw) && aligned16(w) &&
-      (int64_t)K * g.cin * 4 < FAST_SPAN) {
-    TapLoader al{dy, M, g.h, g.w, 1, 1, g.pt, g.pl, -1, -1, g.ho, g.wo, g.cout, g.kh, g.kw};
-    DgradWLoader bl{w, g.cin, g.cout};
-    return launch_any<false>(ctx, "conv2d_input_gradient", M, N, K, al, bl, ep, ws, ws_elems);
-  }
+  if (split_conv_dgrad_ok(g, dy, w)) return launch_split_conv_dgrad(ctx, g, dy, w, dx, ws, ws_elems);
   ConvDgradA al{dy, g, M};
   ConvDgradB bl{w, g};
   return launch_any<false>(ctx, "conv2d_input_gradient", M, N, K, al, bl, ep, ws, ws_elems);
@@ -1761,16 +1293,8 @@ int launch_conv_wgrad(sn_ctx* ctx, const ConvGeom& g, const float* x, const floa
     SN_HIP(hipGetLastError());
     return SN_OK;
   }
-  if (!(ws && small_parts(M, N, K, ctx->compute_units, ws_elems)) && WgradXLoader::ok(x, g) && FlatLoader<false>::ok(dy, 1, g.cout, N, K)) {
-    const int interior = g.pt == 0 && g.pl == 0 && (g.ho - 1) * g.sh + g.kh <= g.h && (g.wo - 1) * g.sw + g.kw <= g.w;
-    WgradXLoader al{x, g, M, interior};
-    FlatLoader<false> bl{dy, 1, g.cout, N};
-    Epilogue e;
-    e.out = dw;
-    e.ldo = g.cout;
-    StdEpilogue ep{e};
-    return launch_any<false>(ctx, "conv2d_filter_gradient", M, N, K, al, bl, ep, ws, ws_elems);
-  }
+  if (!(ws && small_parts(M, N, K, ctx->compute_units, ws_elems)) && split_conv_wgrad_ok(g, x, dy))
+    return launch_split_conv_wgrad(ctx, g, x, dy, dw, ws, ws_elems);
   ConvWgradA al{x, g, M};
   StridedLoader<false> bl{dy, 1, (int64_t)g.cout, N};
   Epilogue e;

@@ -1968,3 +1968,80 @@ def test_nan_input_propagates_and_returns(S, ctx):
         o.close()
     for b in (xb, yb, xrb, yrb):
         b.free()
+
+
+# ----------------------------------------------------------------------------- float32 products taken apart into bf16 parts
+def _affine_bounds(x, y, w1, b1, w2, b2):
+    """The two-layer network's values and gradients in float64, and the same with every operand replaced by its magnitude:
+    what a product's rounding errors are measured against."""
+    def run(x, y, w1, b1, w2, b2, sign):
+        h = x @ w1 + b1
+        p = h @ w2 + b2
+        dp = 2.0 * (p + sign * y) / y.size
+        dh = dp @ w2.T
+        return {"0/weights": x.T @ dh, "1/weights": dh.sum(0), "2/weights": h.T @ dp, "3/weights": dp.sum(0), "out": p}
+    d = [v.astype(np.float64) for v in (x, y, w1, b1, w2, b2)]
+    return run(*d, -1.0), run(*[np.abs(v) for v in d], 1.0)
+
+
+# edges of the 32- to 128-wide tiles and of the 32- and 64-long stages, rows that are no multiple of four values, a reduction
+# long enough for several splits, and a product large enough for 128 x 128 tiles
+@pytest.mark.parametrize("rows,features,hidden,outputs", [(4, 5, 6, 5), (31, 33, 63, 7), (64, 32, 64, 64), (65, 67, 129, 33), (128, 100, 36, 130),
+                                                          (3, 257, 70, 31), (200, 1003, 97, 66), (700, 127, 515, 1026), (513, 2050, 260, 8)])
+def test_split_products_at_tile_edges(S, ctx, rows, features, hidden, outputs):
+    rng = np.random.default_rng(rows * 7 + features)
+    h = Harness(S, ctx, [("dense", hidden, "identity"), ("dense", outputs, "identity")], "mse", (features,), rows)
+    x = rng.standard_normal((rows, features)).astype(f32)
+    y = rng.standard_normal((rows, outputs)).astype(f32)
+    params = {"0/weights": rng.standard_normal((features, hidden)).astype(f32), "1/weights": rng.standard_normal(hidden).astype(f32),
+              "2/weights": rng.standard_normal((hidden, outputs)).astype(f32), "3/weights": rng.standard_normal(outputs).astype(f32)}
+    h.rep.set_params(params)
+    xb, yb = ctx.to_device(x), ctx.to_device(y)
+    want, size = _affine_bounds(x, y, *[params[f"{i}/weights"] for i in range(4)])
+    got = {"out": h.rep.forward(xb)}
+    h.rep.grad(xb, yb)
+    got.update(h.rep.get_grads())
+    # Every sum of K products meets the accumulator in at most 6 K / 16 roundings of 2^-24, the parts of a product that are left
+    # out and the split-K, bias and loss additions are a few more; the reductions of the chain add up.
+    steps = 6.0 / 16.0 * (features + hidden + outputs + rows) + 16.0
+    for name in got:
+        assert np.all(np.abs(got[name] - want[name]) <= steps * 2.0 ** -24 * size[name]), name
+    # ... and the forward product is no further from float64 than the float32 sum in k order is
+    acc = np.zeros((rows, hidden), f32)
+    for k in range(features):
+        acc += x[:, k:k + 1] * params["0/weights"][k]
+    one = Harness(S, ctx, [("dense", hidden, "identity")], "mse", (features,), rows)
+    one.rep.set_params({p: v for (p, _, _), v in zip(one.cm.params, (params["0/weights"], np.zeros(hidden, f32)))})
+    exact = x.astype(np.float64) @ params["0/weights"].astype(np.float64)
+    rms = lambda v: float(np.sqrt(np.mean((v - exact) ** 2)))
+    assert rms(one.rep.forward(xb)) <= 1.05 * rms(acc)
+    for o in (h, one):
+        o.close()
+    xb.free()
+    yb.free()
+
+
+@pytest.mark.parametrize("rows,features,hidden", [(70, 37, 66), (130, 300, 40)])
+def test_split_products_carry_infinities_as_float32_does(S, ctx, rows, features, hidden):
+    rng = np.random.default_rng(5)
+    x = rng.standard_normal((rows, features)).astype(f32)
+    w = rng.standard_normal((features, hidden)).astype(f32)
+    w[3, :] = 1.0                                  # a short significand: its middle and low parts are zero
+    x[2, 3], x[5, 3], x[9, 4] = np.inf, -np.inf, np.nan
+    w[7, 11] = np.inf
+    x[:, 7] = np.where(np.arange(rows) % 2 == 0, 1.5, -2.0)
+    x[1, 7] = 0.0                                  # 0 * Inf
+    h = Harness(S, ctx, [("dense", hidden, "identity")], "mse", (features,), rows)
+    h.rep.set_params({p: v for (p, _, _), v in zip(h.cm.params, (w, np.zeros(hidden, f32)))})
+    xb = ctx.to_device(x)
+    got = h.rep.forward(xb)
+    with np.errstate(all="ignore"):
+        want = np.zeros((rows, hidden), f32)
+        for k in range(features):
+            want += x[:, k:k + 1] * w[k]
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(np.isposinf(got), np.isposinf(want)) and np.array_equal(np.isneginf(got), np.isneginf(want))
+    fine = np.isfinite(want)
+    assert np.isinf(want).any() and rel_err(got[fine], want[fine]) <= TOL_GEMM
+    h.close()
+    xb.free()
