@@ -17,10 +17,10 @@
 // 700 x 770 x 1003 with unaligned rows 59 -> 23 us, 1000 x 1500 x 1000 72 -> 32 us.
 //
 // Infinities: Inf taken apart is Inf + NaN + NaN.  Every thread keeps the largest magnitude it has staged (half an instruction
-// per value; NaNs do not count), and a workgroup that met an Inf multiplies its tile once more with the hi parts alone: a sum
-// that is not finite there is what float32 arithmetic gives (Inf b = +-Inf, Inf 0 = Inf - Inf = NaN) and replaces the stored
-// one.  NaN needs nothing: its parts are NaN.  (A finite value within 0.4 % of the largest float32 rounds to Inf and counts
-// as one.)
+// per value; NaNs do not count), and a workgroup that met an Inf, or a finite value within 0.4 % of the largest float32, which
+// rounds to Inf, multiplies its tile twice more.  First with the largest bf16 value as the hi part of such finite values (mid
+// and lo hold the rest: the sum stays exact); then with the hi parts alone: a sum that is not finite there is what float32
+// arithmetic gives (Inf b = +-Inf, Inf 0 = Inf - Inf = NaN) and replaces the stored one.  NaN needs nothing: its parts are NaN.
 //
 // Workgroup = WVM x WVN x WVK wavefronts; block tile BM x BN, K stage BK.  Global loads go to registers (one stage ahead), are
 // split there and stored to LDS as PLANES bf16 tiles [BK / 32][row][32 k] of 64 bytes per row, from where a fragment (8
@@ -423,10 +423,15 @@ __device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
   return r;
 }
 
-// hi + mid + lo of a pair, PLANES of them
-template <int PLANES>
+constexpr float LARGEST_BF16 = 3.3895313892515355e38f, LARGEST_F32 = 3.4028234663852886e38f;
+__device__ __forceinline__ float below_inf(float a) {
+  return fabsf(a) > LARGEST_BF16 && fabsf(a) <= LARGEST_F32 ? copysignf(LARGEST_BF16, a) : a;
+}
+
+// hi + mid + lo of a pair, PLANES of them; CLAMP: no finite value's hi part is Inf
+template <int PLANES, bool CLAMP>
 __device__ __forceinline__ void split_pair(float a, float b, uint32_t (&p)[PLANES]) {
-  p[0] = pack_bf16(a, b);
+  p[0] = CLAMP ? pack_bf16(below_inf(a), below_inf(b)) : pack_bf16(a, b);
 #pragma unroll
   for (int i = 1; i < PLANES; ++i) {
     a = a - __uint_as_float(p[i - 1] << 16);
@@ -441,7 +446,6 @@ __device__ __forceinline__ float max_magnitude(float m, float a, float b) {
   asm("v_max3_f32 %0, %1, |%2|, |%3|" : "=v"(r) : "v"(m), "v"(a), "v"(b));
   return r;
 }
-constexpr float LARGEST_BF16 = 3.3895313892515355e38f;
 
 // the vector as its code says: elements moved into place, the invalid ones zero
 template <bool SIGNED_SHIFT>
@@ -541,7 +545,7 @@ struct Stager {
     if constexpr (OP::KC) op.advance(k[0], BK);
   }
   // PL planes of the fetched vectors go to LDS.  sum (KC = false only): adds the thread's KB rows to its four column sums
-  template <int PL>
+  template <int PL, bool CLAMP>
   __device__ __forceinline__ void stage(char* lds, bool sum) {
     if (!on) return;
     if (OP::MASKED || tail) {
@@ -556,8 +560,8 @@ struct Stager {
 #pragma unroll
       for (int e = 0; e < E; ++e) {
         uint32_t a[PL], b[PL];
-        split_pair<PL>(v[e][0], v[e][1], a);
-        split_pair<PL>(v[e][2], v[e][3], b);
+        split_pair<PL, CLAMP>(v[e][0], v[e][1], a);
+        split_pair<PL, CLAMP>(v[e][2], v[e][3], b);
 #pragma unroll
         for (int p = 0; p < PL; ++p) *(u2v*)(lds + p * PLANE + at[0] + e * RP * 64) = u2v{a[p], b[p]};
       }
@@ -569,9 +573,9 @@ struct Stager {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         uint32_t a[PL], b[PL];
-        split_pair<PL>(v[0][i], v[1][i], a);
+        split_pair<PL, CLAMP>(v[0][i], v[1][i], a);
         if constexpr (KB == 4) {
-          split_pair<PL>(v[2][i], v[3][i], b);
+          split_pair<PL, CLAMP>(v[2][i], v[3][i], b);
 #pragma unroll
           for (int p = 0; p < PL; ++p) *(u2v*)(lds + p * PLANE + at[i]) = u2v{a[p], b[p]};
         } else {
@@ -650,9 +654,11 @@ __global__ __launch_bounds__(64 * WVM * WVN * WVK) void split_gemm_kernel(SplitG
     fb[h] = SB::place(wn + l32 + 4, k);
   }
 
-  // the tile's sums of the products of PL planes, in acc: complete in every wavefront for the values it keeps
-  auto multiply = [&](auto planes, bool sums) {
-    constexpr int PL = decltype(planes)::value;
+  // the tile's sums of products, in acc: complete in every wavefront for the values it keeps (hi_only, with CLAMP: the hi
+  // parts' products alone)
+  auto multiply = [&](auto clamp, bool sums, bool hi_only) {
+    constexpr int PL = PLANES;
+    constexpr bool CLAMP = decltype(clamp)::value;
     sa.init(al, m0, k_begin);
     sb.init(bl, n0, k_begin);
 #pragma unroll
@@ -666,8 +672,8 @@ __global__ __launch_bounds__(64 * WVM * WVN * WVK) void split_gemm_kernel(SplitG
     sa.fetch(al, k_begin + BK > k_end);
     sb.fetch(bl, k_begin + BK > k_end);
     for (int k0 = k_begin; k0 < k_end; k0 += BK) {
-      sa.template stage<PL>(la, false);
-      sb.template stage<PL>(lb, sums);
+      sa.template stage<PL, CLAMP>(la, false);
+      sb.template stage<PL, CLAMP>(lb, sums);
       __syncthreads();
       if (k0 + BK < k_end) {  // the next stage's global loads fly while this one is multiplied
         const bool tail = k0 + 2 * BK > k_end;
@@ -689,11 +695,13 @@ __global__ __launch_bounds__(64 * WVM * WVN * WVK) void split_gemm_kernel(SplitG
 #pragma unroll
         for (int s = PL - 1; s >= 0; --s)
 #pragma unroll
-          for (int p = 0; p <= s; ++p)
+          for (int p = 0; p <= s; ++p) {
+            if (CLAMP && hi_only && s > 0) continue;
 #pragma unroll
             for (int i = 0; i < TM; ++i)
 #pragma unroll
               for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[i][p], bf[j][s - p], acc[i][j], 0, 0, 0);
+          }
       }
       __syncthreads();
     }
@@ -732,7 +740,7 @@ __global__ __launch_bounds__(64 * WVM * WVN * WVK) void split_gemm_kernel(SplitG
   };
   float* const part = g.ws ? g.ws + (int64_t)bz * g.ws_rows * g.N : nullptr;
 
-  multiply(std::integral_constant<int, PLANES>{}, sum_columns);
+  multiply(std::false_type{}, sum_columns, false);
   bool huge = false;
   if constexpr (PLANES > 1) huge = __syncthreads_or(sa.largest > LARGEST_BF16 || sb.largest > LARGEST_BF16);
   kept([&](int row0, int col, const f16v& a, int first, int last) {
@@ -765,14 +773,14 @@ __global__ __launch_bounds__(64 * WVM * WVN * WVK) void split_gemm_kernel(SplitG
     }
   }
   if constexpr (PLANES > 1) {
-    if (huge) {  // (see the head of the file)
+    for (int hi_only = 0; huge && hi_only < 2; ++hi_only) {  // (see the head of the file)
       __syncthreads();
-      multiply(std::integral_constant<int, 1>{}, false);
+      multiply(std::true_type{}, false, hi_only != 0);
       kept([&](int row0, int col, const f16v& a, int first, int last) {
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
           const int row = row0 + (v >> 2) * 8 + (v & 3);
-          const int to = v >= first && v < last && row < g.M && !(fabsf(a[v]) <= 3.402823466e38f) ? ep.map_row(row) : -1;
+          const int to = v >= first && v < last && row < g.M && (hi_only == 0 || !(fabsf(a[v]) <= LARGEST_F32)) ? ep.map_row(row) : -1;
           if (to < 0) continue;
           if (part) part[(int64_t)to * g.N + col] = a[v];
           else ep.store(to, col, a[v]);

@@ -2022,6 +2022,37 @@ def test_split_products_at_tile_edges(S, ctx, rows, features, hidden, outputs):
 
 
 @pytest.mark.parametrize("rows,features,hidden", [(70, 37, 66), (130, 300, 40)])
+def test_split_products_of_the_largest_finite_values(S, ctx, rows, features, hidden):
+    """A finite value that rounds to Inf as bf16 (a mask of the type's lowest value) is no Inf: its products are finite where
+    float32's are, also beside a real Inf.  Errors as at the tile edges, against float64."""
+    rng = np.random.default_rng(6)
+    x = rng.standard_normal((rows, features)).astype(f32)
+    w = (rng.standard_normal((features, hidden)) * 0.1).astype(f32)
+    big = np.finfo(f32).max
+    x[2, 3], x[5, 4], x[9, 1] = big, -big, f32(3.395e38)
+    w[3], w[4], w[1] = w[3] * 0.5, w[4] * 0.5, w[1] * 0.5
+    w[0, 5] = -big
+    x[:, 0] *= 0.05
+    for with_inf in (False, True):
+        if with_inf:
+            x[7, 2] = np.inf
+        h = Harness(S, ctx, [("dense", hidden, "identity")], "mse", (features,), rows)
+        h.rep.set_params({p: v for (p, _, _), v in zip(h.cm.params, (w, np.zeros(hidden, f32)))})
+        xb = ctx.to_device(x)
+        got = h.rep.forward(xb)
+        with np.errstate(all="ignore"):
+            want = x.astype(np.float64) @ w.astype(np.float64)
+        size = np.abs(x).astype(np.float64) @ np.abs(w).astype(np.float64)
+        fine = np.isfinite(want) & (np.abs(want) < 0.99 * big)
+        assert fine.sum() > 0.9 * fine.size and fine[2].any() and fine[5].any() and fine[9].any() and fine[10, 5]
+        assert np.all(np.abs(got[fine] - want[fine]) <= (6.0 / 16.0 * features + 16.0) * 2.0 ** -24 * size[fine])
+        if with_inf:
+            assert np.isinf(got[7]).all() and np.array_equal(got[7] > 0, w[2] > 0)
+        h.close()
+        xb.free()
+
+
+@pytest.mark.parametrize("rows,features,hidden", [(70, 37, 66), (130, 300, 40)])
 def test_split_products_carry_infinities_as_float32_does(S, ctx, rows, features, hidden):
     rng = np.random.default_rng(5)
     x = rng.standard_normal((rows, features)).astype(f32)
