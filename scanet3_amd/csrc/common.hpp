@@ -452,6 +452,27 @@ int launch_lstm_wgrad(sn_ctx* ctx, const float* x, const float* h_prev_all, cons
 
 int64_t gemm_workspace_elems(int m, int n, int k, int cu);
 
+// ---- products of a recurrent layer over all time steps at once (split_recurrent.hip) ------------------------------
+// inputs: out, slice t (`step` floats apart): [rows, gates * H] = x[:, t, :] Wk + b of every gate; x [rows, T, F].
+// dx[b, t, :] = sum over the gates of dz_t[b] Wk^T, dz being T slices [rows, gates * H] without gaps.
+bool recurrent_products_fit(int rows, int T, int F, int H, int gates);
+int launch_recurrent_inputs(sn_ctx* ctx, const float* x, int rows, int T, int F, int H, const LstmWeights& w, int gates, float* out, int64_t step);
+int launch_recurrent_dx(sn_ctx* ctx, const float* dz, int rows, int T, int F, int H, const LstmWeights& w, int gates, float* dx);
+
+// ---- recurrent layers whose recurrence fits one CU (recurrent_local_kernels.hip) ----------------------------------
+// Every time step in one launch, nothing handed between workgroups.  Buffers as for the one-launch kernels below; h0 / c0
+// null: zeros; h: T slices h_0 .. h_{T-1}; y_seq: [rows, T, H] or null.
+bool recurrent_local_fits(int rows, int T, int F, int H, int gates);
+int launch_lstm_local_fwd(sn_ctx* ctx, const float* x, int T, int F, const float* h0, const float* c0, int rows, int H, const LstmWeights& w,
+                          float* gates, float* c, float* h, int64_t slice, float* y_seq);
+int launch_lstm_local_bwd(sn_ctx* ctx, const float* gates, const float* c, const float* c0, const float* dh_last, const float* dy_seq, int T,
+                          int rows, int H, const LstmWeights& w, float* dz, int64_t slice);
+// r_slices: T + 1, slice 0 the carried state (read if first_valid); w.b[0] has to be null (no bias inside the recurrence)
+int launch_rnn_local_fwd(sn_ctx* ctx, const float* x, int T, int F, bool first_valid, int rows, int H, const LstmWeights& w, float* r_slices,
+                         int64_t slice);
+// dr_slices: T, the last one given; dy_seq (or null) is added to the ones below it
+int launch_rnn_local_bwd(sn_ctx* ctx, float* dr_slices, const float* dy_seq, int T, int rows, int H, const float* wr, int64_t slice);
+
 // ---- fused LSTM steps (lstm_kernels.hip) ------------------------------------------------
 // true when the fused step kernels handle this layer (F % 4 == 0, H % 16 == 0, F + H <= 400, 16-byte aligned tensors)
 bool lstm_step_fused_ok(int F, int H, const float* x, const LstmWeights& w, int gates = 4);

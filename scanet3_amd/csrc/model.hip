@@ -567,6 +567,18 @@ static LstmWeights lstm_weights(sn_replica* r, const Op& op, float* base) {
   return w;
 }
 
+// Whether a recurrent layer runs on the kernels that keep a row's whole recurrence in one workgroup.  Any layer they fit does
+// that the one-launch kernels with a hand-over between workgroups (`handed`) do not take: those need unit counts that are
+// multiples of 16 and take one launch or more per step otherwise (LSTM 9 -> 100 -> 60 units, 130 rows, 50 steps: 3.76 ms a
+// step against 0.46).  Where both fit (500 rows, 64 steps, 32 features; the inputs' product included, us): LSTM forward 16
+// units 68 against 132, 64: 93 / 157, 96: 128 / 160, 128: 190 / 181; backward 16: 55 / 102, 64: 72 / 118, 128: 167 / 137;
+// simple cell, either direction, 64: 43 / 96, 128: 57 / 105.
+constexpr int LSTM_LOCAL_UNITS = 96, RNN_LOCAL_UNITS = 128;
+static bool recurrent_local(const Op& op, int rows, int gates, bool handed) {
+  if (!recurrent_local_fits(rows, op.T, op.F, op.H, gates)) return false;
+  return !handed || op.H <= (gates == 4 ? LSTM_LOCAL_UNITS : RNN_LOCAL_UNITS);
+}
+
 static BatchNormArgs batchnorm_args(sn_replica* r, const Op& op, int i) {
   const int64_t c = align_up(op.out_dims.back(), 64);
   float* b = r->bn_buf[i];
@@ -659,7 +671,13 @@ static int forward(sn_replica* r, const float* x, int rows, bool skip_last = fal
         if (carried)
           SN_HIP(hipMemcpyAsync(r->lstm_h[i], param_ptr(r, r->w, op.state_p[1]), (size_t)rows * op.H * sizeof(float), hipMemcpyDeviceToDevice,
                                 ctx->stream));
-        if (fused && op.T > 1 && lstm_sequence_fwd_ok(ctx, rows, op.F, op.H, in, w)) {  // every step in one launch (it reads the weights as they lie)
+        const bool handed = fused && op.T > 1 && lstm_sequence_fwd_ok(ctx, rows, op.F, op.H, in, w);
+        if (recurrent_local(op, rows, 4, handed)) {
+          SN_TRY(launch_lstm_local_fwd(ctx, in, op.T, op.F, carried ? r->lstm_h[i] : nullptr, carried ? param_ptr(r, r->w, op.state_p[0]) : nullptr,
+                                       rows, op.H, w, r->lstm_gates[i], r->lstm_c[i], r->lstm_h[i] + bh, bh, op.ret_seq ? r->act[i] : nullptr));
+          break;
+        }
+        if (handed) {  // every step in one launch (it reads the weights as they lie)
           SN_TRY(launch_lstm_sequence_fwd(ctx, in, op.T, op.F, carried ? 1 : 0, carried ? param_ptr(r, r->w, op.state_p[0]) : nullptr, rows, op.H,
                                           w, r->lstm_gates[i], r->lstm_c[i], r->lstm_h[i], bh));
           if (op.ret_seq) SN_TRY(launch_sequence_gather(ctx, r->lstm_h[i], bh, 1, r->act[i], rows, op.T, op.H));
@@ -700,8 +718,10 @@ static int forward(sn_replica* r, const float* x, int rows, bool skip_last = fal
         if (carried)
           SN_HIP(hipMemcpyAsync(r->lstm_h[i], param_ptr(r, r->w, op.state_p[0]), (size_t)rows * op.H * sizeof(float), hipMemcpyDeviceToDevice,
                                 ctx->stream));
-        const bool whole = fused && op.T > 1 && rnn_sequence_fwd_ok(ctx, rows, op.F, op.H, in);
-        if (whole)  // every step in one launch (it reads the weights as they lie)
+        const bool handed = fused && op.T > 1 && rnn_sequence_fwd_ok(ctx, rows, op.F, op.H, in);
+        const bool local = recurrent_local(op, rows, 1, handed), whole = local || handed;
+        if (local) SN_TRY(launch_rnn_local_fwd(ctx, in, op.T, op.F, carried, rows, op.H, w, r->lstm_h[i], bh));
+        else if (whole)  // every step in one launch (it reads the weights as they lie)
           SN_TRY(launch_rnn_sequence_fwd(ctx, in, op.T, op.F, carried ? 1 : 0, rows, op.H, w.wk[0], w.wr[0], r->lstm_h[i], bh));
         else if (fused) SN_TRY(launch_lstm_pack(ctx, w, op.F, op.H, r->lstm_pk_fwd[i], nullptr, 1));  // the step kernel's LDS order
         for (int t = whole ? op.T : 0; t < op.T; ++t) {
@@ -948,7 +968,11 @@ static int backward(sn_replica* r, const float* x, int rows, int first = -1, int
         // one launch per step (gate gradients + the product that carries dh back) where the layer's shape allows it
         const bool fused_bwd = fused && lstm_step_bwd_fused_ok(op.H, w);
         // every reverse step in one launch where the whole grid fits the device; the input gradients follow per step
-        const bool whole = fused && op.T > 1 && lstm_sequence_bwd_ok(ctx, rows, op.H, w);
+        const bool handed = fused && op.T > 1 && lstm_sequence_bwd_ok(ctx, rows, op.H, w);
+        // (a launch that carries the weight gradient along is kept: 128 units, 64 rows 177 us against 167 + 21)
+        const bool local = recurrent_local(op, rows, 4, handed) && !(handed && lstm_sequence_bwd_wgrad_workspace(rows, op.T, op.F, op.H) > 0);
+        const bool whole = local || handed;
+        const bool dx_at_once = need_dx && recurrent_products_fit(rows, op.T, op.F, op.H, 4);
         LstmGrads gr;
         for (int gi = 0; gi < 4; ++gi) {
           gr.wk[gi] = param_ptr(r, r->g, op.lstm_p[gi][0]);
@@ -956,12 +980,15 @@ static int backward(sn_replica* r, const float* x, int rows, int first = -1, int
           gr.b[gi] = param_ptr(r, r->g, op.lstm_p[gi][2]);
         }
         int wgrad_parts = 0;  // > 0: the backward launch has left the weight gradient's partial sums in the workspace
-        if (whole) {
+        if (local) {
+          SN_TRY(launch_lstm_local_bwd(ctx, r->lstm_gates[i], r->lstm_c[i], param_ptr(r, r->w, op.state_p[0]), op.ret_seq ? nullptr : dy,
+                                       op.ret_seq ? dy : nullptr, op.T, rows, op.H, w, r->lstm_dz[i], bh));
+        } else if (whole) {
           SN_TRY(launch_lstm_sequence_bwd(ctx, r->lstm_gates[i], r->lstm_c[i], param_ptr(r, r->w, op.state_p[0]), op.ret_seq ? nullptr : dy,
                                           op.ret_seq ? dy : nullptr, op.T, rows, op.H, w, r->lstm_dz[i], bh, in, r->lstm_h[i], op.F, r->ws,
                                           m->workspace_elems, &wgrad_parts));
           if (wgrad_parts > 0) SN_TRY(launch_lstm_wgrad_reduce(ctx, r->ws, wgrad_parts, op.F, op.H, 4, gr));  // before the workspace's next user
-          if (need_dx)
+          if (need_dx && !dx_at_once)
             for (int t = op.T - 1; t >= 0; --t)
               SN_TRY(launch_lstm_dx(ctx, r->lstm_dz[i] + (int64_t)t * bh * 4, rows, op.H, op.F, t, op.T, w, dx, r->ws, m->workspace_elems));
         } else if (fused_bwd && op.T > 1) SN_TRY(launch_lstm_pack_bwd(ctx, w, op.H, r->lstm_pk_dh[i]));
@@ -980,14 +1007,14 @@ static int backward(sn_replica* r, const float* x, int rows, int first = -1, int
             SN_TRY(launch_lstm_step_bwd(ctx, a, t == op.T - 1 ? nullptr : dcbuf[db], dcbuf[db ^ 1], t > 0 ? r->lstm_pk_dh[i] : nullptr,
                                         r->lstm_dh[hb], bh, rows, op.H));
             db ^= 1;
-            if (need_dx) SN_TRY(launch_lstm_dx(ctx, a.dz, rows, op.H, op.F, t, op.T, w, dx, r->ws, m->workspace_elems));
+            if (need_dx && !dx_at_once) SN_TRY(launch_lstm_dx(ctx, a.dz, rows, op.H, op.F, t, op.T, w, dx, r->ws, m->workspace_elems));
             dh = r->lstm_dh[hb];
             dh_parts = lstm_bwd_parts(op.H);
             hb ^= 1;
             continue;
           }
           SN_TRY(launch_lstm_gates_bwd(ctx, a, rows, op.H));
-          if (need_dx) SN_TRY(launch_lstm_dx(ctx, a.dz, rows, op.H, op.F, t, op.T, w, dx, r->ws, m->workspace_elems));
+          if (need_dx && !dx_at_once) SN_TRY(launch_lstm_dx(ctx, a.dz, rows, op.H, op.F, t, op.T, w, dx, r->ws, m->workspace_elems));
           if (t > 0) {
             if (fused) {  // four per-gate partial products; the next gate-gradient kernel adds them
               SN_TRY(launch_lstm_step_dh(ctx, a.dz, rows, op.H, r->lstm_pk_dh[i], r->lstm_dh[hb], bh));
@@ -1000,6 +1027,7 @@ static int backward(sn_replica* r, const float* x, int rows, int first = -1, int
             hb ^= 1;
           }
         }
+        if (dx_at_once) SN_TRY(launch_recurrent_dx(ctx, r->lstm_dz[i], rows, op.T, op.F, op.H, w, 4, dx));
         if (wgrad_parts == 0) SN_TRY(launch_lstm_wgrad(ctx, in, r->lstm_h[i], r->lstm_dz[i], rows, op.T, op.F, op.H, gr, r->ws, m->workspace_elems));
         if (need_dx) cur ^= 1;
         break;
@@ -1032,7 +1060,10 @@ static int backward(sn_replica* r, const float* x, int rows, int first = -1, int
           if (op.b >= 0) SN_TRY(launch_col_sum(ctx, dr, op.H, param_ptr(r, r->g, op.b), rows, op.H, r->ws, m->workspace_elems));
         }
         const bool fused = lstm_step_fused_ok(op.F, op.H, in, w, 1);
-        const bool whole = fused && op.T > 1 && rnn_sequence_bwd_ok(ctx, rows, op.H, w.wr[0]);
+        const bool handed = fused && op.T > 1 && rnn_sequence_bwd_ok(ctx, rows, op.H, w.wr[0]);
+        const bool local = recurrent_local(op, rows, 1, handed) && !(handed && rnn_sequence_bwd_wgrad_workspace(rows, op.T, op.F, op.H) > 0);
+        const bool whole = local || handed;
+        const bool dx_at_once = need_dx && recurrent_products_fit(rows, op.T, op.F, op.H, 1);
         if (fused && op.T > 1 && !whole) SN_TRY(launch_lstm_pack(ctx, w, op.F, op.H, nullptr, r->lstm_pk_dh[i], 1));  // the step kernel's LDS order
         LstmGrads gr{};
         gr.wk[0] = param_ptr(r, r->g, op.lstm_p[0][0]);
@@ -1041,22 +1072,24 @@ static int backward(sn_replica* r, const float* x, int rows, int first = -1, int
         if (whole) {  // every step in one launch (it adds a returned sequence's output gradients itself), then the input gradients
           dr = r->lstm_dz[i] + (int64_t)(op.T - 1) * bh;
           if (op.ret_seq) SN_TRY(launch_step_slice_add(ctx, dr, dy + (int64_t)(op.T - 1) * op.H, (int64_t)op.T * op.H, rows, op.H, false));
-          SN_TRY(launch_rnn_sequence_bwd(ctx, r->lstm_dz[i], op.ret_seq ? dy : nullptr, op.T, rows, op.H, w.wr[0], bh, in, r->lstm_h[i], op.F,
-                                         r->ws, m->workspace_elems, &wgrad_parts));
+          if (local) SN_TRY(launch_rnn_local_bwd(ctx, r->lstm_dz[i], op.ret_seq ? dy : nullptr, op.T, rows, op.H, w.wr[0], bh));
+          else SN_TRY(launch_rnn_sequence_bwd(ctx, r->lstm_dz[i], op.ret_seq ? dy : nullptr, op.T, rows, op.H, w.wr[0], bh, in, r->lstm_h[i], op.F,
+                                              r->ws, m->workspace_elems, &wgrad_parts));
           if (wgrad_parts > 0) SN_TRY(launch_lstm_wgrad_reduce(ctx, r->ws, wgrad_parts, op.F, op.H, 1, gr));  // before the workspace's next user
-          if (need_dx)
+          if (need_dx && !dx_at_once)
             for (int t = op.T - 1; t >= 0; --t)
               SN_TRY(launch_lstm_dx(ctx, r->lstm_dz[i] + (int64_t)t * bh, rows, op.H, op.F, t, op.T, w, dx, r->ws, m->workspace_elems, 1));
         }
         for (int t = whole ? -1 : op.T - 1; t >= 0; --t) {
           dr = r->lstm_dz[i] + (int64_t)t * bh;
           if (op.ret_seq) SN_TRY(launch_step_slice_add(ctx, dr, dy + (int64_t)t * op.H, (int64_t)op.T * op.H, rows, op.H, t < op.T - 1));
-          if (need_dx) SN_TRY(launch_lstm_dx(ctx, dr, rows, op.H, op.F, t, op.T, w, dx, r->ws, m->workspace_elems, 1));
+          if (need_dx && !dx_at_once) SN_TRY(launch_lstm_dx(ctx, dr, rows, op.H, op.F, t, op.T, w, dx, r->ws, m->workspace_elems, 1));
           if (t > 0) {
             if (fused) SN_TRY(launch_lstm_step_dh(ctx, dr, rows, op.H, r->lstm_pk_dh[i], dr - bh, 0, 1));
             else SN_TRY(launch_lstm_dh(ctx, dr, rows, op.H, w, dr - bh, r->ws, m->workspace_elems, 1));
           }
         }
+        if (dx_at_once) SN_TRY(launch_recurrent_dx(ctx, r->lstm_dz[i], rows, op.T, op.F, op.H, w, 1, dx));
         if (wgrad_parts == 0) SN_TRY(launch_lstm_wgrad(ctx, in, r->lstm_h[i], r->lstm_dz[i], rows, op.T, op.F, op.H, gr, r->ws, m->workspace_elems, 1));
         if (need_dx) cur ^= 1;
         break;

@@ -1361,6 +1361,93 @@ def test_simple_rnn_backward_launch_that_carries_the_weight_gradient(S, ctx, mon
     yb.free()
 
 
+@pytest.mark.parametrize("kind,units,features,batch,T", [
+    ("lstm", 1, 1, 1, 2), ("lstm", 3, 3, 5, 1), ("lstm", 16, 2, 4, 3), ("lstm", 17, 5, 33, 4), ("lstm", 32, 7, 18, 3), ("lstm", 33, 1, 130, 3),
+    ("lstm", 63, 9, 7, 5), ("lstm", 64, 66, 31, 3), ("lstm", 65, 4, 70, 2), ("lstm", 96, 10, 9, 4), ("lstm", 100, 9, 130, 3), ("lstm", 128, 3, 37, 3),
+    ("lstm", 30, 4, 2100, 2), ("lstm", 60, 3, 2053, 2),
+    ("simple_rnn", 1, 1, 1, 2), ("simple_rnn", 2, 3, 9, 3), ("simple_rnn", 31, 5, 33, 4), ("simple_rnn", 64, 6, 18, 3), ("simple_rnn", 97, 9, 70, 3),
+    ("simple_rnn", 129, 2, 21, 3), ("simple_rnn", 192, 7, 35, 3), ("simple_rnn", 193, 10, 13, 3), ("simple_rnn", 256, 5, 50, 2),
+    ("simple_rnn", 70, 4, 2065, 2), ("simple_rnn", 150, 3, 2050, 2), ("simple_rnn", 250, 2, 2049, 2)])
+def test_recurrent_layers_whose_recurrence_stays_in_one_workgroup(S, ctx, kind, units, features, batch, T):
+    """Every block count of the kernels (32 values of the recurrence each), the last one full and partial, both row counts of
+    a workgroup (4, and 16 from some 2000 rows on), rows that do not fill the last workgroup, products of fewer than four
+    values; a carried state at the start, the returned sequence feeding a second layer of 3 units (whose input gradient the
+    product over all steps delivers).  Bounds as for the one-launch kernels: float32 sums, or three times the oracle's own
+    distance from float64."""
+    first = {"lstm": (O.LSTM, S.LSTM), "simple_rnn": (O.SimpleRNN, S.SimpleRNN)}[kind]
+    om = O.Model([first[0](units, return_sequence=True, stateful=True), first[0](3), O.Dense(2, O.ACT_IDENTITY)], O.LOSS_MSE)
+    layers = first[1](units, returnSequence=True, stateful=True) >> first[1](3) >> S.Dense(2, S.Identity)
+    cm = S.CompiledModel(ctx, [l.desc() for l in layers.layers], S.MeanSquaredError.kind, (T, features), batch)
+    rep = cm.replica(None)
+    rng = np.random.default_rng(7000 + units + features)
+    params = glorot_params(om, (batch, T, features), rng)
+    for p in params:
+        if O.is_unaggregated_path(p) or params[p].ndim == 1:
+            params[p] = rng.uniform(-0.4, 0.4, params[p].shape).astype(f32)
+    x = rng.standard_normal((batch, T, features)).astype(f32)
+    y = rng.uniform(-1, 1, (batch, 2)).astype(f32)
+    rep.set_params(params)
+    xb, yb = ctx.to_device(x), ctx.to_device(y)
+    assert rel_err(rep.forward(xb), om.forward(x, params)) <= TOL_GEMM
+    if batch > 2:
+        assert rel_err(rep.forward(xb, batch - 2), om.forward(x[:-2], params)) <= TOL_GEMM
+    oloss, ograds = om.grad(x, y, params)
+    ctx.profile_reset()
+    ctx.profile(True)
+    assert abs(rep.grad(xb, yb) - float(oloss)) <= TOL_GEMM * max(1.0, abs(float(oloss)))
+    ctx.sync()
+    ctx.profile(False)
+    local = "lstm_local" if kind == "lstm" else "rnn_local"
+    assert any(l.startswith(local + "_forward") for l in ctx.profile_report()) and any(l.startswith("recurrent_input_gradient") for l in ctx.profile_report())
+    ggrads = rep.get_grads()
+    _, grads64 = om.grad(x.astype(np.float64), y.astype(np.float64), {k: v.astype(np.float64) for k, v in params.items()})
+    for p in ograds:
+        assert rel_err(ggrads[p], ograds[p]) <= max(TOL_GEMM, 3.0 * rel_err(ograds[p], grads64[p])), p
+    for o in (rep, cm):
+        o.close()
+    xb.free()
+    yb.free()
+
+
+@pytest.mark.parametrize("kind", ["lstm", "simple_rnn"])
+@pytest.mark.parametrize("value", [np.inf, -np.inf, 3.4e38, np.nan])
+def test_recurrence_in_one_workgroup_with_values_at_the_end_of_the_range(S, ctx, kind, value):
+    """Inf, NaN and the largest finite values in the recurrent weights and in the inputs come out as float32 arithmetic
+    gives them: finite where that is finite (3.4e38 rounds to Inf as a bf16 value), otherwise not finite.  The first step
+    starts from a carried state (without one its product is left out, and with it the oracle's 0 Inf)."""
+    first = {"lstm": (O.LSTM, S.LSTM), "simple_rnn": (O.SimpleRNN, S.SimpleRNN)}[kind]
+    units, features, batch, T = 20, 3, 6, 3
+    om = O.Model([first[0](units, stateful=True), O.Dense(2, O.ACT_IDENTITY)], O.LOSS_MSE)
+    layers = first[1](units, stateful=True) >> S.Dense(2, S.Identity)
+    cm = S.CompiledModel(ctx, [l.desc() for l in layers.layers], S.MeanSquaredError.kind, (T, features), batch)
+    rep = cm.replica(None)
+    rng = np.random.default_rng(71)
+    base = glorot_params(om, (batch, T, features), rng)
+    for p in base:
+        if O.is_unaggregated_path(p):
+            base[p] = rng.uniform(0.1, 0.4, base[p].shape).astype(f32)
+    wr = next(p for p in base if p.endswith("recurrent_weights"))
+    x = rng.standard_normal((batch, T, features)).astype(f32)
+    for place in ("weights", "inputs"):
+        params, xs = {k: v.copy() for k, v in base.items()}, x.copy()
+        if place == "weights":
+            params[wr][7, 11] = value
+        else:
+            xs[2, 0, 1] = value
+        rep.set_params(params)
+        xb = ctx.to_device(xs)
+        with np.errstate(all="ignore"):
+            want = om.forward(xs, params)
+        got = rep.forward(xb)
+        assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want)), (place, got, want)
+        finite = np.isfinite(want)
+        scale = np.maximum(np.abs(want), 1.0) if kind == "simple_rnn" else 1.0
+        assert np.all(np.abs(got - want)[finite] <= (TOL_GEMM * scale * np.ones_like(want))[finite]), place
+        xb.free()
+    for o in (rep, cm):
+        o.close()
+
+
 @pytest.mark.parametrize("kind", ["lstm", "simple_rnn"])
 def test_lstm_sequence_kernel_gives_up_instead_of_hanging(S, monkeypatch, kind):
     """A workgroup of a one-launch recurrent kernel that waits for its neighbours polls a bounded number of times.  With the
