@@ -404,11 +404,27 @@ bool conv_wgrad_is_direct(const sn_ctx* ctx, const ConvGeom& g, const float* ws,
 int launch_conv_wgrad(sn_ctx* ctx, const ConvGeom& g, const float* x, const float* dy, float* dw, float* ws, int64_t ws_elems,
                       const PoolGrad* pool = nullptr);
 
-bool split_conv_fwd_ok(const ConvGeom& g, const float* x, const float* w);
+// What the split convolutions can read: vectors of four values, clamped to the inside of an image tensor of n * h * w * c
+// values (so it has to hold four of them), and 32-bit byte offsets up to one image behind its end.
+constexpr int64_t SPLIT_SPAN = (int64_t)1 << 31;
+static inline bool split_image_ok(const float* p, int n, int h, int w, int64_t c) {
+  const int64_t image = (int64_t)h * w * c;
+  return p && (reinterpret_cast<uintptr_t>(p) & 3u) == 0 && n * image >= 4 && (n + (int64_t)1) * image * 4 < SPLIT_SPAN;
+}
+static inline bool split_filter_ok(const ConvGeom& g, const float* w) {
+  return split_image_ok(w, 1, g.kh, g.kw, (int64_t)g.cin * g.cout);
+}
+static inline bool split_conv_fwd_ok(const ConvGeom& g, const float* x, const float* w) {
+  return g.cout >= 4 && split_image_ok(x, g.n, g.h, g.w, g.cin) && split_filter_ok(g, w);
+}
+static inline bool split_conv_dgrad_ok(const ConvGeom& g, const float* dy, const float* w) {
+  return g.sh == 1 && g.sw == 1 && split_image_ok(dy, g.n, g.ho, g.wo, g.cout) && split_filter_ok(g, w) && (int64_t)g.kw * g.cout >= 4;
+}
+static inline bool split_conv_wgrad_ok(const ConvGeom& g, const float* x, const float* dy) {
+  return g.cout >= 4 && (int64_t)g.kw * g.cin >= 4 && split_image_ok(x, g.n, g.h, g.w, g.cin) && split_image_ok(dy, g.n, g.ho, g.wo, g.cout);
+}
 int launch_split_conv_fwd(sn_ctx* ctx, const ConvGeom& g, const float* x, const float* w, const Epilogue& e, float* ws, int64_t ws_elems);
-bool split_conv_dgrad_ok(const ConvGeom& g, const float* dy, const float* w);
 int launch_split_conv_dgrad(sn_ctx* ctx, const ConvGeom& g, const float* dy, const float* w, float* dx, float* ws, int64_t ws_elems);
-bool split_conv_wgrad_ok(const ConvGeom& g, const float* x, const float* dy);
 int launch_split_conv_wgrad(sn_ctx* ctx, const ConvGeom& g, const float* x, const float* dy, float* dw, float* ws, int64_t ws_elems);
 
 // the same two products with LDS-direct loads into a three-stage ring (conv_ring_kernels.hip), for the shapes *_ok accepts

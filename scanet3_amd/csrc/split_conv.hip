@@ -7,14 +7,6 @@ namespace sn {
 static bool interior(const ConvGeom& g) {
   return g.pt == 0 && g.pl == 0 && (g.ho - 1) * g.sh + g.kh <= g.h && (g.wo - 1) * g.sw + g.kw <= g.w;
 }
-static bool readable(const void* p, int64_t elems) {
-  return p && (reinterpret_cast<uintptr_t>(p) & 3u) == 0 && elems >= 4 && elems * 4 < SPLIT_SPAN;
-}
-
-bool split_conv_fwd_ok(const ConvGeom& g, const float* x, const float* w) {
-  return g.cout >= 4 && readable(x, ((int64_t)g.n + 1) * g.h * g.w * g.cin) && readable(w, (int64_t)g.kh * g.kw * g.cin * g.cout);
-}
-
 int launch_split_conv_fwd(sn_ctx* ctx, const ConvGeom& g, const float* x, const float* w, const Epilogue& e, float* ws, int64_t ws_elems) {
   const int L = g.kw * g.cin, Lp = (int)align_up(L, 4), M = g.n * g.ho * g.wo, K = g.kh * Lp, N = g.cout;
   const int total = g.n * g.h * g.w * g.cin;
@@ -30,11 +22,6 @@ int launch_split_conv_fwd(sn_ctx* ctx, const ConvGeom& g, const float* x, const 
   };
   if (interior(g) && L == Lp) return run(ConvRunOp<false>{});
   return run(ConvRunOp<true>{});
-}
-
-bool split_conv_dgrad_ok(const ConvGeom& g, const float* dy, const float* w) {
-  return g.sh == 1 && g.sw == 1 && readable(dy, ((int64_t)g.n + 1) * g.ho * g.wo * g.cout) && readable(w, (int64_t)g.kh * g.kw * g.cin * g.cout) &&
-         (int64_t)g.kw * g.cout >= 4;
 }
 
 int launch_split_conv_dgrad(sn_ctx* ctx, const ConvGeom& g, const float* dy, const float* w, float* dx, float* ws, int64_t ws_elems) {
@@ -54,11 +41,6 @@ int launch_split_conv_dgrad(sn_ctx* ctx, const ConvGeom& g, const float* dy, con
   if (g.cout % 4 == 0)
     return launch_split<3>(ctx, "conv2d_input_gradient", M, N, K, M, -1, al, ConvDgradFilterOp<true>{w, g.cin, g.cout, g.kh, g.kw, L, Lp, by_cout}, ep, ws, ws_elems);
   return launch_split<3>(ctx, "conv2d_input_gradient", M, N, K, M, -1, al, ConvDgradFilterOp<false>{w, g.cin, g.cout, g.kh, g.kw, L, Lp, by_cout}, ep, ws, ws_elems);
-}
-
-bool split_conv_wgrad_ok(const ConvGeom& g, const float* x, const float* dy) {
-  return g.cout >= 4 && (int64_t)g.kw * g.cin >= 4 && readable(x, ((int64_t)g.n + 1) * g.h * g.w * g.cin) &&
-         readable(dy, ((int64_t)g.n + 1) * g.ho * g.wo * g.cout);
 }
 
 int launch_split_conv_wgrad(sn_ctx* ctx, const ConvGeom& g, const float* x, const float* dy, float* dw, float* ws, int64_t ws_elems) {

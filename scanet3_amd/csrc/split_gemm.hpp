@@ -42,8 +42,6 @@ typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));  // 16-byte l
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u2v __attribute__((ext_vector_type(2)));
 
-constexpr int64_t SPLIT_SPAN = (int64_t)1 << 31;  // operands are addressed with 32-bit byte offsets
-
 // ============================================================================ operands
 // An operand loader describes A as a function of (outer = row m, k), B of (outer = column n, k) and fetches four values
 // along its contiguous index: k when KC, the outer index otherwise.  Its state is split by what it depends on:

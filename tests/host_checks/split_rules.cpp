@@ -1,0 +1,19 @@
+// Host-side rules of the split products, asked on the command line and answered without a GPU:
+//   conv n h w cin ho wo cout kh kw sh sw pt pl      which convolution products read tensors of exactly these sizes: three 0/1
+#include "../../scanet3_amd/csrc/split_launch.hpp"
+
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+
+int main(int argc, char** argv) {
+  std::vector<int> v;
+  for (int i = 2; i < argc; ++i) v.push_back(std::atoi(argv[i]));
+  alignas(16) static float at[4];
+  if (argc == 15 && !std::strcmp(argv[1], "conv")) {
+    const sn::ConvGeom g{v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7], v[8], v[9], v[10], v[11], v[12]};
+    std::printf("%d %d %d\n", sn::split_conv_fwd_ok(g, at, at), sn::split_conv_dgrad_ok(g, at, at), sn::split_conv_wgrad_ok(g, at, at));
+    return 0;
+  }
+  return 2;
+}

@@ -500,6 +500,16 @@ MODELS = {
                                               ("flatten",), ("dense", 3, "softmax")], "cce", (9, 13, 1), 11, "uniform_onehot"),
     "conv_input_gradient_32_channels_2x3_same": ([("conv", 32, (3, 3), (1, 1), "valid", "relu", False), ("conv", 32, (2, 3), (1, 1), "same", "tanh", False),
                                                   ("flatten",), ("dense", 3, "softmax")], "cce", (8, 9, 1), 13, "uniform_onehot"),
+    # images that hold two or three values in all: too few for a product that loads four at a time
+    "conv_tensor_of_two_values": ([("conv", 5, (1, 1), (1, 1), "valid", "identity", True), ("conv", 2, (3, 3), (1, 1), "same", "tanh", False),
+                                   ("conv", 6, (2, 2), (1, 1), "same", "tanh", False), ("flatten",), ("dense", 2, "identity")], "mse", (1, 1, 2), 1,
+                                  "normal_regression"),
+    "conv_tensor_of_three_values": ([("conv", 5, (3, 3), (1, 1), "same", "identity", True), ("conv", 3, (3, 3), (1, 1), "same", "tanh", False),
+                                     ("conv", 7, (1, 4), (1, 1), "same", "tanh", False), ("flatten",), ("dense", 2, "identity")], "mse", (1, 1, 3), 1,
+                                    "normal_regression"),
+    "conv_three_images_of_one_value": ([("conv", 8, (3, 3), (1, 1), "same", "tanh", False), ("conv", 1, (2, 2), (1, 1), "same", "tanh", True),
+                                        ("conv", 4, (3, 3), (1, 1), "same", "identity", False), ("flatten",), ("dense", 2, "identity")], "mse",
+                                       (1, 1, 1), 3, "normal_regression"),
     # Dense from thousands of features onto a few units: gradients as row streams (2048+ features, at most 16 units); a feature count
     # that leaves a partial block of 64, 7 rows over 4 wavefronts, 16 and 5 units, an L2 penalty on the streamed weights
     "dense_many_features_few_units": ([("dense", 2050, "tanh"), ("dense", 5, "softmax", "l2", 0.01)], "cce", (33,), 7, "normal_onehot"),

@@ -1,0 +1,40 @@
+"""Host-side rules of the split products (csrc/split_launch.hpp, csrc/common.hpp), compiled without device code: what the
+kernels are given to read, and which tile a product takes."""
+import itertools
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+@pytest.fixture(scope="module")
+def ask(tmp_path_factory):
+    binary = str(tmp_path_factory.mktemp("host_checks") / "split_rules")
+    cmd = ["/opt/rocm/bin/hipcc", "-x", "hip", "--offload-arch=gfx950", "--offload-host-only", "-O1", "-std=c++17",
+           os.path.join(ROOT, "tests", "host_checks", "split_rules.cpp"), "-o", binary]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    assert res.returncode == 0, res.stderr
+    return lambda *q: [int(v) for v in subprocess.run([binary, *map(str, q)], capture_output=True, text=True, check=True).stdout.split()]
+
+
+def test_split_convolutions_hold_four_values_of_every_image_they_read(ask):
+    """The masked loaders clamp a vector of four to [0, total - 4]: a tensor of one to three values would be read in front of
+    its start.  One-row batches and 1 x 1 images reach such sizes; one value more and the kernels may take them."""
+    seen = {False: 0, True: 0}
+    for n, side, cin, cout, kw in itertools.product((1, 2, 3, 4), (1, 2), (1, 2, 3, 4), (1, 2, 3, 4, 5), (1, 2, 4)):
+        pad = (kw - 1) // 2
+        forward, input_gradient, filter_gradient = ask("conv", n, side, side, cin, side, side, cout, kw, kw, 1, 1, pad, pad)
+        x, dy, w = n * side * side * cin, n * side * side * cout, kw * kw * cin * cout
+        assert forward == (x >= 4 and w >= 4 and cout >= 4)
+        assert input_gradient == (dy >= 4 and w >= 4 and kw * cout >= 4)
+        assert filter_gradient == (x >= 4 and dy >= 4 and cout >= 4 and kw * cin >= 4)
+        seen[bool(forward)] += 1
+    assert min(seen.values()) > 100
+
+
+def test_split_convolutions_stay_inside_32_bit_offsets(ask):
+    assert ask("conv", 1023, 32, 32, 128, 32, 32, 128, 3, 3, 1, 1, 1, 1) == [1, 1, 1]
+    # (n + 1) images of 2^21 bytes reach 2^31
+    assert ask("conv", 4095, 32, 32, 128, 32, 32, 128, 3, 3, 1, 1, 1, 1) == [0, 0, 0]
