@@ -24,6 +24,11 @@ constexpr int ROWS = 4;  // batch rows of a workgroup
 
 __device__ __forceinline__ float sigmoidf_(float x) { return 1.0f / (1.0f + expf(-x)); }
 
+constexpr float LARGEST_F32 = 3.4028234663852886e38f;
+__device__ __forceinline__ float below_inf(float a) {
+  return fabsf(a) > LARGEST_BF16 && fabsf(a) <= LARGEST_F32 ? copysignf(LARGEST_BF16, a) : a;
+}
+
 __device__ __forceinline__ float hi_of(float a, bool& huge) {
   huge = huge || fabsf(a) > LARGEST_BF16;
   return below_inf(a);

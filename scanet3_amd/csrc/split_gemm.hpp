@@ -16,11 +16,10 @@
 // = 184 TFLOP/s (the float32 matrix peak is 157; the v_mfma_f32_32x32x2_f32 kernel this replaces ran such shapes at 60-80);
 // 700 x 770 x 1003 with unaligned rows 59 -> 23 us, 1000 x 1500 x 1000 72 -> 32 us.
 //
-// Infinities: Inf taken apart is Inf + NaN + NaN.  Every thread keeps the largest magnitude it has staged (half an instruction
-// per value; NaNs do not count), and a workgroup that met an Inf, or a finite value within 0.4 % of the largest float32, which
-// rounds to Inf, multiplies its tile twice more.  First with the largest bf16 value as the hi part of such finite values (mid
-// and lo hold the rest: the sum stays exact); then with the hi parts alone: a sum that is not finite there is what float32
-// arithmetic gives (Inf b = +-Inf, Inf 0 = Inf - Inf = NaN) and replaces the stored one.  NaN needs nothing: its parts are NaN.
+// The end of the range: an Inf taken apart is Inf + NaN + NaN, a finite value within 0.4 % of the largest float32 rounds to
+// Inf as bf16, and where a product overflows its part products may do so with either sign.  Every thread keeps the largest
+// magnitude it has taken apart (half an instruction per value; NaNs do not count: their parts are NaN), and a workgroup whose
+// two largest could make a sum leave the range multiplies its tile once more with v_mfma_f32_32x32x2_f32, on float32 values.
 //
 // Workgroup = WVM x WVN x WVK wavefronts; block tile BM x BN, K stage BK.  Global loads go to registers (one stage ahead), are
 // split there and stored to LDS as PLANES bf16 tiles [BK / 32][row][32 k] of 64 bytes per row, from where a fragment (8
@@ -421,21 +420,25 @@ __device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
   return r;
 }
 
-constexpr float LARGEST_BF16 = 3.3895313892515355e38f, LARGEST_F32 = 3.4028234663852886e38f;
-__device__ __forceinline__ float below_inf(float a) {
-  return fabsf(a) > LARGEST_BF16 && fabsf(a) <= LARGEST_F32 ? copysignf(LARGEST_BF16, a) : a;
-}
-
-// hi + mid + lo of a pair, PLANES of them; CLAMP: no finite value's hi part is Inf
-template <int PLANES, bool CLAMP>
+// hi + mid + lo of a pair, PLANES of them
+template <int PLANES>
 __device__ __forceinline__ void split_pair(float a, float b, uint32_t (&p)[PLANES]) {
-  p[0] = CLAMP ? pack_bf16(below_inf(a), below_inf(b)) : pack_bf16(a, b);
+  p[0] = pack_bf16(a, b);
 #pragma unroll
   for (int i = 1; i < PLANES; ++i) {
     a = a - __uint_as_float(p[i - 1] << 16);
     b = b - __uint_as_float(p[i - 1] & 0xffff0000u);
     p[i] = pack_bf16(a, b);
   }
+}
+
+// Up to these magnitudes of two operands, and k products a sum, no part of a value and no sum of part products leaves float32's
+// range (an Inf taken apart is Inf + NaN + NaN, and part products that overflow do so with either sign).
+constexpr float LARGEST_BF16 = 3.3895313892515355e38f, LARGEST_SUM = 0x1p126f;
+// whatever the other operand and k <= 2^31 are, as long as it holds for both
+constexpr float SURELY_IN_RANGE = 0x1p47f;
+__device__ __forceinline__ bool parts_in_range(float a, float b, int k) {
+  return a <= LARGEST_BF16 && b <= LARGEST_BF16 && a * b * (float)k <= LARGEST_SUM;
 }
 
 // max(m, |a|, |b|), NaNs ignored
@@ -500,33 +503,32 @@ struct Stager {
   uint32_t at[OP::KC ? 1 : 4];  // KC: byte offset of the thread's 8 bytes of its first row; else of its bytes of each row
   bool on;
   bool tail;
-  f4v colsum;
-  float largest;  // magnitude of what this thread has staged
+  f4v colsum = {0.f, 0.f, 0.f, 0.f};
+  float largest = 0.f;  // magnitude of what this thread has taken apart
 
-  __device__ __forceinline__ int kgroup() const { return OP::KC ? (int)threadIdx.x % KG : ((int)threadIdx.x / OW) % KG; }
-  __device__ __forceinline__ int ogroup() const {
-    return OP::KC ? (int)threadIdx.x / KG : (int)threadIdx.x % OW + OW * ((int)threadIdx.x / (OW * KG));
-  }
+  static __device__ __forceinline__ int kgroup(int tid) { return OP::KC ? tid % KG : (tid / OW) % KG; }
+  static __device__ __forceinline__ int ogroup(int tid) { return OP::KC ? tid / KG : tid % OW + OW * (tid / (OW * KG)); }
   static __device__ __forceinline__ uint32_t place(int row, int k) {  // byte offset of element k of a stage
     return (uint32_t)((k >> 5) * SUB) + plane_at(row, (k >> 3) & 3) + (uint32_t)(k & 7) * 2u;
   }
-  __device__ __forceinline__ void init(const OP& op, int outer0, int k_begin) {
-    colsum = f4v{0.f, 0.f, 0.f, 0.f};
-    largest = 0.f;
-    on = ACTIVE == T || (int)threadIdx.x < ACTIVE;
-    const int kg = kgroup(), ov = on ? ogroup() : 0;
+  static __device__ __forceinline__ uint32_t f32_place(int row, int k) { return (uint32_t)((k * ROWS + row) * 4); }  // ... in float32
+  static_assert(BK * ROWS * 4 <= 3 * PLANE, "a stage in float32 fits the three planes");
+  template <bool F32>
+  __device__ __forceinline__ void init(const OP& op, int tid, int outer0, int k_begin) {
+    on = ACTIVE == T || tid < ACTIVE;
+    const int kg = kgroup(tid), ov = on ? ogroup(tid) : 0;
     if constexpr (OP::KC) {
 #pragma unroll
       for (int e = 0; e < E; ++e) op.init_outer(o[e], outer0 + ov + RP * e);
       op.init_k(k[0], k_begin + kg * 4);
-      at[0] = place(ov + 4, kg * 4);  // rows RP apart: the same swizzle
+      at[0] = F32 ? f32_place(ov + 4, kg * 4) : place(ov + 4, kg * 4);  // rows RP apart: the same swizzle
     } else {
       op.init_outer(o[0], outer0 + 4 * ov);
 #pragma unroll
       for (int e = 0; e < E; ++e) op.init_k(k[e], k_begin + kg * KB + e);
       const int local = op.row(outer0 + 4 * ov) - outer0 + 4;  // >= 1
 #pragma unroll
-      for (int i = 0; i < 4; ++i) at[i] = place(local + i, kg * KB);
+      for (int i = 0; i < 4; ++i) at[i] = F32 ? f32_place(local + i, kg * KB) : place(local + i, kg * KB);
     }
   }
   __device__ __forceinline__ void fetch(const OP& op, bool is_tail) {
@@ -543,7 +545,7 @@ struct Stager {
     if constexpr (OP::KC) op.advance(k[0], BK);
   }
   // PL planes of the fetched vectors go to LDS.  sum (KC = false only): adds the thread's KB rows to its four column sums
-  template <int PL, bool CLAMP>
+  template <int PL>
   __device__ __forceinline__ void stage(char* lds, bool sum) {
     if (!on) return;
     if (OP::MASKED || tail) {
@@ -558,8 +560,8 @@ struct Stager {
 #pragma unroll
       for (int e = 0; e < E; ++e) {
         uint32_t a[PL], b[PL];
-        split_pair<PL, CLAMP>(v[e][0], v[e][1], a);
-        split_pair<PL, CLAMP>(v[e][2], v[e][3], b);
+        split_pair<PL>(v[e][0], v[e][1], a);
+        split_pair<PL>(v[e][2], v[e][3], b);
 #pragma unroll
         for (int p = 0; p < PL; ++p) *(u2v*)(lds + p * PLANE + at[0] + e * RP * 64) = u2v{a[p], b[p]};
       }
@@ -571,9 +573,9 @@ struct Stager {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         uint32_t a[PL], b[PL];
-        split_pair<PL, CLAMP>(v[0][i], v[1][i], a);
+        split_pair<PL>(v[0][i], v[1][i], a);
         if constexpr (KB == 4) {
-          split_pair<PL, CLAMP>(v[2][i], v[3][i], b);
+          split_pair<PL>(v[2][i], v[3][i], b);
 #pragma unroll
           for (int p = 0; p < PL; ++p) *(u2v*)(lds + p * PLANE + at[i]) = u2v{a[p], b[p]};
         } else {
@@ -581,6 +583,16 @@ struct Stager {
           for (int p = 0; p < PL; ++p) *(uint32_t*)(lds + p * PLANE + at[i]) = a[p];
         }
       }
+    }
+  }
+  // the fetched vectors go to LDS as they are
+  __device__ __forceinline__ void stage_f32(char* lds) {
+    if (!on) return;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      if (OP::MASKED || tail) apply_code<OP::SIGNED>(v[e], code[e]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) *(float*)(lds + (OP::KC ? at[0] + i * ROWS * 4 + e * RP * 4 : at[i % (OP::KC ? 1 : 4)] + e * ROWS * 4)) = v[e][i];
     }
   }
 };
@@ -652,57 +664,16 @@ __global__ __launch_bounds__(64 * WVM * WVN * WVK) void split_gemm_kernel(SplitG
     fb[h] = SB::place(wn + l32 + 4, k);
   }
 
-  // the tile's sums of products, in acc: complete in every wavefront for the values it keeps (hi_only, with CLAMP: the hi
-  // parts' products alone)
-  auto multiply = [&](auto clamp, bool sums, bool hi_only) {
-    constexpr int PL = PLANES;
-    constexpr bool CLAMP = decltype(clamp)::value;
-    sa.init(al, m0, k_begin);
-    sb.init(bl, n0, k_begin);
+  auto clear = [&]() {
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
       for (int j = 0; j < TN; ++j)
 #pragma unroll
         for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
-    // (Two, three and four stages of loads in flight instead of one were measured: no faster at any size, and the registers
-    // cost a wavefront per SIMD.)
-    sa.fetch(al, k_begin + BK > k_end);
-    sb.fetch(bl, k_begin + BK > k_end);
-    for (int k0 = k_begin; k0 < k_end; k0 += BK) {
-      sa.template stage<PL, CLAMP>(la, false);
-      sb.template stage<PL, CLAMP>(lb, sums);
-      __syncthreads();
-      if (k0 + BK < k_end) {  // the next stage's global loads fly while this one is multiplied
-        const bool tail = k0 + 2 * BK > k_end;
-        sa.fetch(al, tail);
-        sb.fetch(bl, tail);
-      }
-#pragma unroll
-      for (int h = 0; h < PARTS; ++h) {
-        bf16x8 af[TM][PL], bf[TN][PL];
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-          for (int p = 0; p < PL; ++p) af[i][p] = *(const bf16x8*)(la + p * SA::PLANE + fa[h] + i * 2048);
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-          for (int p = 0; p < PL; ++p) bf[j][p] = *(const bf16x8*)(lb + p * SB::PLANE + fb[h] + j * 2048);
-        // small terms first; consecutive MFMAs go to different accumulators
-#pragma unroll
-        for (int s = PL - 1; s >= 0; --s)
-#pragma unroll
-          for (int p = 0; p <= s; ++p) {
-            if (CLAMP && hi_only && s > 0) continue;
-#pragma unroll
-            for (int i = 0; i < TM; ++i)
-#pragma unroll
-              for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[i][p], bf[j][s - p], acc[i][j], 0, 0, 0);
-          }
-      }
-      __syncthreads();
-    }
+  };
+  // adds the wavefronts' shares of the stages' k-values: the sums are complete in every wavefront for the values it keeps
+  auto exchange = [&]() {
     if constexpr (WVK > 1) {
       // value u (of TM x TN x 16) of a lane belongs to wavefront u / KEEP of its tile; the others hand theirs over:
       // [tile of the workgroup][keeper][sender other than the keeper][value of the keeper's share][lane]
@@ -723,6 +694,98 @@ __global__ __launch_bounds__(64 * WVM * WVN * WVK) void split_gemm_kernel(SplitG
       }
     }
   };
+
+  sa.template init<false>(al, threadIdx.x, m0, k_begin);
+  sb.template init<false>(bl, threadIdx.x, n0, k_begin);
+  clear();
+  // (Two, three and four stages of loads in flight instead of one were measured: no faster at any size, and the registers
+  // cost a wavefront per SIMD.)
+  sa.fetch(al, k_begin + BK > k_end);
+  sb.fetch(bl, k_begin + BK > k_end);
+  for (int k0 = k_begin; k0 < k_end; k0 += BK) {
+    sa.template stage<PLANES>(la, false);
+    sb.template stage<PLANES>(lb, sum_columns);
+    __syncthreads();
+    if (k0 + BK < k_end) {  // the next stage's global loads fly while this one is multiplied
+      const bool tail = k0 + 2 * BK > k_end;
+      sa.fetch(al, tail);
+      sb.fetch(bl, tail);
+    }
+#pragma unroll
+    for (int h = 0; h < PARTS; ++h) {
+      bf16x8 af[TM][PLANES], bf[TN][PLANES];
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int p = 0; p < PLANES; ++p) af[i][p] = *(const bf16x8*)(la + p * SA::PLANE + fa[h] + i * 2048);
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int p = 0; p < PLANES; ++p) bf[j][p] = *(const bf16x8*)(lb + p * SB::PLANE + fb[h] + j * 2048);
+      // small terms first; consecutive MFMAs go to different accumulators
+#pragma unroll
+      for (int s = PLANES - 1; s >= 0; --s)
+#pragma unroll
+        for (int p = 0; p <= s; ++p)
+#pragma unroll
+          for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[i][p], bf[j][s - p], acc[i][j], 0, 0, 0);
+    }
+    __syncthreads();
+  }
+  exchange();
+
+  if constexpr (PLANES > 1) {
+    if (__syncthreads_or(sa.largest > SURELY_IN_RANGE || sb.largest > SURELY_IN_RANGE)) {  // (see the head of the file)
+      int* const top = reinterpret_cast<int*>(lds);  // (magnitudes order as their bits do)
+      if (threadIdx.x < 2) top[threadIdx.x] = 0;
+      __syncthreads();
+      atomicMax(top, __float_as_int(sa.largest));
+      atomicMax(top + 1, __float_as_int(sb.largest));
+      __syncthreads();
+      const bool in_range = parts_in_range(__int_as_float(top[0]), __int_as_float(top[1]), k_end - k_begin);
+      __syncthreads();
+      if (!in_range) {
+        // Everything is worked out anew from values the compiler cannot know to be the same: nothing is kept in registers
+        // through the loop above for the sake of this one.
+        int tid = threadIdx.x, from = k_begin;
+        asm volatile("" : "+v"(tid), "+s"(from));
+        sa.template init<true>(al, tid, m0, from);
+        sb.template init<true>(bl, tid, n0, from);
+        clear();
+        sa.fetch(al, from + BK > k_end);
+        sb.fetch(bl, from + BK > k_end);
+        const int khalf = (tid >> 5) & 1, part = ((tid >> 6) % WVK) * (BK / WVK) + khalf;
+        const uint32_t fa32 = SA::f32_place(wm + (tid & 31) + 4, part), fb32 = SB::f32_place(wn + (tid & 31) + 4, part);
+#pragma unroll 1
+        for (int k0 = from; k0 < k_end; k0 += BK) {
+          sa.stage_f32(la);
+          sb.stage_f32(lb);
+          __syncthreads();
+          if (k0 + BK < k_end) {
+            const bool tail = k0 + 2 * BK > k_end;
+            sa.fetch(al, tail);
+            sb.fetch(bl, tail);
+          }
+#pragma unroll 1
+          for (int k = 0; k < BK / WVK; k += 2) {
+            float af[TM], bf[TN];
+#pragma unroll
+            for (int i = 0; i < TM; ++i) af[i] = *(const float*)(la + fa32 + k * (SA::ROWS * 4) + i * 128);
+#pragma unroll
+            for (int j = 0; j < TN; ++j) bf[j] = *(const float*)(lb + fb32 + k * (SB::ROWS * 4) + j * 128);
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+              for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(af[i], bf[j], acc[i][j], 0, 0, 0);
+          }
+          __syncthreads();
+        }
+        exchange();
+      }
+    }
+  }
   // f(row0, col, tile's accumulator, first, last) for every 32x32 tile this wavefront keeps values of: value v of lane l sits at
   // row 8*(v/4) + 4*(l/32) + v%4, column l%32 of its tile
   auto kept = [&](auto f) {
@@ -738,9 +801,6 @@ __global__ __launch_bounds__(64 * WVM * WVN * WVK) void split_gemm_kernel(SplitG
   };
   float* const part = g.ws ? g.ws + (int64_t)bz * g.ws_rows * g.N : nullptr;
 
-  multiply(std::false_type{}, sum_columns, false);
-  bool huge = false;
-  if constexpr (PLANES > 1) huge = __syncthreads_or(sa.largest > LARGEST_BF16 || sb.largest > LARGEST_BF16);
   kept([&](int row0, int col, const f16v& a, int first, int last) {
     if (part) {
 #pragma unroll
@@ -758,7 +818,7 @@ __global__ __launch_bounds__(64 * WVM * WVN * WVK) void split_gemm_kernel(SplitG
     if (sum_columns) {  // a group of four columns was read by KG threads (one per group of k): their sums meet in LDS
       __syncthreads();
       float* cs = reinterpret_cast<float*>(lds);
-      if (sb.on) *(f4v*)(cs + sb.kgroup() * BN + sb.ogroup() * 4) = sb.colsum;
+      if (sb.on) *(f4v*)(cs + SB::kgroup(threadIdx.x) * BN + SB::ogroup(threadIdx.x) * 4) = sb.colsum;
       __syncthreads();
       if ((int)threadIdx.x < BN) {
         const int c = bl.row(n0 + ((int)threadIdx.x & ~3)) + ((int)threadIdx.x & 3);  // (a moved group repeats its neighbour's columns)
@@ -768,22 +828,6 @@ __global__ __launch_bounds__(64 * WVM * WVN * WVK) void split_gemm_kernel(SplitG
         if (part) part[(int64_t)g.colsum_row * g.N + c] = s;
         else ep.store(g.colsum_row, c, s);
       }
-    }
-  }
-  if constexpr (PLANES > 1) {
-    for (int hi_only = 0; huge && hi_only < 2; ++hi_only) {  // (see the head of the file)
-      __syncthreads();
-      multiply(std::true_type{}, false, hi_only != 0);
-      kept([&](int row0, int col, const f16v& a, int first, int last) {
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int row = row0 + (v >> 2) * 8 + (v & 3);
-          const int to = v >= first && v < last && row < g.M && (hi_only == 0 || !(fabsf(a[v]) <= LARGEST_F32)) ? ep.map_row(row) : -1;
-          if (to < 0) continue;
-          if (part) part[(int64_t)to * g.N + col] = a[v];
-          else ep.store(to, col, a[v]);
-        }
-      });
     }
   }
 }

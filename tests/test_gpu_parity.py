@@ -2173,3 +2173,114 @@ def test_split_products_carry_infinities_as_float32_does(S, ctx, rows, features,
     assert np.isinf(want).any() and rel_err(got[fine], want[fine]) <= TOL_GEMM
     h.close()
     xb.free()
+
+
+def _as_float32_would(want):
+    """Float64 results as float32 holds them: what is beyond its largest value is infinite."""
+    with np.errstate(over="ignore"):
+        return np.asarray(want).astype(f32)
+
+
+def _assert_same_range(got, want, rel):
+    assert np.array_equal(np.isnan(got), np.isnan(want)), (got, want)
+    assert np.array_equal(np.where(np.isinf(got), got, 0), np.where(np.isinf(want), want, 0)), (got, want)
+    fine = np.isfinite(want)
+    assert np.all(np.abs(got[fine] - want[fine]) <= rel * np.abs(want[fine])), np.max(np.abs(got[fine] - want[fine]) / np.maximum(np.abs(want[fine]), 1e-45))
+
+
+# Pairs whose float32 product overflows, or nearly does, or is Inf times something.  In most of them no operand rounds to Inf as
+# bf16: the parts of such a product leave the range before the product does, or with the other sign.
+RANGE_PAIRS = [(3e38, 1e38), (-2.9e38, 1.7e38), (1e30, -1e25), (1.8439e19, 1.8439e19), (-1.8446e19, 1.8447e19), (3.39e38, 1.0), (3.4e38, 1.00001),
+               (3.4028e38, -0.99), (np.inf, 1e-39), (-np.inf, 1e-44), (np.inf, -2.0), (1e38, 1e-37)]
+
+
+@pytest.mark.parametrize("pair", RANGE_PAIRS)
+@pytest.mark.parametrize("rows,features,hidden", [(8, 9, 9), (70, 133, 66)])
+def test_split_products_at_the_end_of_the_range(S, ctx, rows, features, hidden, pair):
+    """One output is ONE float32 product of the pair (the other terms of its sum are zeros): it is finite, infinite or not a
+    number as float32 says, and a finite one is right to the two roundings that a sum of part products and a product of
+    float32 values may differ by.  Every other output stays what it is without the pair."""
+    rng = np.random.default_rng(rows)
+    a, b = f32(pair[0]), f32(pair[1])
+    x, w = rng.standard_normal((rows, features)).astype(f32), rng.standard_normal((features, hidden)).astype(f32)
+    r, k, c = rows - 2, features - 1, 3
+    x[r] = 0
+    x[:, k] = 0
+    w[k] = 1.0  # (an Inf times zero is NaN: the pair's row gets the pair's first value everywhere else)
+    x[r, k], w[k, c] = a, b
+    with np.errstate(all="ignore"):
+        want = (x.astype(np.float64) @ w.astype(np.float64)).astype(f32)
+        want[r] = a * w[k]
+    h = Harness(S, ctx, [("dense", hidden, "identity")], "mse", (features,), rows)
+    h.rep.set_params({p: v for (p, _, _), v in zip(h.cm.params, (w, np.zeros(hidden, f32)))})
+    xb = ctx.to_device(x)
+    got = h.rep.forward(xb)
+    _assert_same_range(got[r], want[r], 2.0 ** -22)
+    others = np.arange(rows) != r
+    size = np.abs(x[others]).astype(np.float64) @ np.abs(w).astype(np.float64)
+    assert np.all(np.abs(got[others] - want[others]) <= (features + 16.0) * 2.0 ** -24 * size)
+    h.close()
+    xb.free()
+
+
+@pytest.mark.parametrize("a,b", [(1e30, 3e10), (-1e20, 1e25), (-0.5, 3.4e38), (1e25, 1e-30), (2.0, 3.39e38)])
+@pytest.mark.parametrize("n", [12, 70])
+def test_split_gradients_at_the_end_of_the_range(S, ctx, n, a, b):
+    """The same for the gradients of a Dense layer: dX = dY W^T and dW = X^T dY, whose bias row is not touched by what the
+    product does.  dY = diag(a, 1, 1, ..), seen through two layers without biases: the targets make it, the outputs are 0."""
+    a, b = f32(a), f32(b)
+    d = np.ones(n, f32)
+    d[1] = a
+    targets = np.diag(-d * f32(n * n / 2)).astype(f32)  # dP = 2 (p - y) / n^2
+    other = np.ones(n, f32)
+    other[1] = b
+    zero, eye, spread = np.zeros((n, n), f32), np.eye(n, dtype=f32), np.ones((n, n), f32)
+    spread[1, :] = b
+    for name, params, x in (("0/weights", (zero, np.zeros(n, f32), spread, np.zeros(n, f32)), eye),   # dW1 = X^T (dP W2^T), X = 1: dP W2^T
+                            ("2/weights", (eye, np.zeros(n, f32), zero, np.zeros(n, f32)), spread.T)):  # dW2 = H^T dP, H = X
+        h = Harness(S, ctx, [("dense", n, "identity"), ("dense", n, "identity")], "mse", (n,), n)
+        h.rep.set_params({p: v for (p, _, _), v in zip(h.cm.params, params)})
+        xb, yb = ctx.to_device(np.ascontiguousarray(x)), ctx.to_device(targets)
+        h.rep.grad(xb, yb)
+        got = h.rep.get_grads()
+        with np.errstate(all="ignore"):
+            if name == "0/weights":
+                want = eye.astype(np.float64) @ _as_float32_would(np.diag(d.astype(np.float64)) @ spread.T).astype(np.float64)
+            else:
+                want = _as_float32_would(spread.astype(np.float64) @ np.diag(d.astype(np.float64)))
+        want = want.astype(f32)
+        _assert_same_range(got[name], want, 2.0 ** -21)  # (dP is off by a rounding itself)
+        assert np.all(np.abs(got["3/weights"] - d) <= 2.0 ** -22 * np.abs(d))
+        h.close()
+        xb.free()
+        yb.free()
+
+
+@pytest.mark.parametrize("filters,channels", [(8, 3), (5, 4), (12, 1)])
+@pytest.mark.parametrize("value", [3.4e38, 1e30, np.inf])
+def test_split_convolutions_at_the_end_of_the_range(S, ctx, filters, channels, value):
+    """A pixel of the largest values under a padded convolution: its outputs and the filter gradients it takes part in are what
+    float64 gives, taken to float32's range; nothing else changes."""
+    rng = np.random.default_rng(filters)
+    spec = [("conv", 6, (1, 1), (1, 1), "valid", "identity", False), ("conv", filters, (3, 3), (1, 1), "same", "identity", False), ("flatten",)]
+    shape, batch = (5, 6, channels), 3
+    h = Harness(S, ctx, spec, "mse", shape, batch)
+    x = rng.uniform(0.5, 1.0, (batch,) + shape).astype(f32)
+    params = glorot_params(h.omodel, (batch,) + shape, rng)
+    for p in params:  # positive weights: no Inf - Inf
+        params[p] = np.abs(params[p]) + f32(0.05)
+    first, second = [p for p in params if params[p].ndim == 4]
+    if value == 1e30:
+        params[second][1, 2, 3, 4] = f32(1e10)  # two operands far from the end of the range
+    x[1, 2, 3, 0] = value
+    y = np.zeros((batch, 30 * filters), f32)
+    h.rep.set_params(params)
+    xb, yb = ctx.to_device(x), ctx.to_device(y)
+    p64 = {k: v.astype(np.float64) for k, v in params.items()}
+    want = _as_float32_would(h.omodel.forward(np.where(np.isfinite(x), x, 1e300).astype(np.float64), p64))
+    got = h.rep.forward(xb).reshape(want.shape)
+    _assert_same_range(got, want, 1e-5)
+    assert np.isinf(want).any() or value == 3.4e38
+    h.close()
+    xb.free()
+    yb.free()
