@@ -5,7 +5,8 @@
 //
 // gfx950 multiplies float32 on its matrix cores at 1/16 of the bf16 rate (64 against 1024 flop per clock and SIMD).  So
 // every float32 value is taken apart into three bf16 values on its way into LDS, hi + mid + lo, each the round-to-nearest
-// bf16 of what the ones before left over: 3 x 8 significand bits hold all 24 of a float32, the sum is EXACT.  A product is
+// bf16 of what the ones before left over: 3 x 8 significand bits hold all 24 of a float32, the sum is EXACT from 2^-110 on
+// (below that the lo part runs out of exponents).  A product is
 //   a b = ah bh + (ah bm + am bh) + (ah bl + am bm + al bh) + (am bl + al bm + al bl)
 // and the kernel multiplies the first six of these (bf16 x bf16 is exact in float32, the accumulator is float32); what is
 // left out is below 2^-24 of |a b| (|am| <= 2^-8 |a|, |al| <= 2^-16 |a|, both halves of that on average), less than the
@@ -16,10 +17,14 @@
 // = 184 TFLOP/s (the float32 matrix peak is 157; the v_mfma_f32_32x32x2_f32 kernel this replaces ran such shapes at 60-80);
 // 700 x 770 x 1003 with unaligned rows 59 -> 23 us, 1000 x 1500 x 1000 72 -> 32 us.
 //
-// The end of the range: an Inf taken apart is Inf + NaN + NaN, a finite value within 0.4 % of the largest float32 rounds to
+// The ends of the range.  An Inf taken apart is Inf + NaN + NaN, a finite value within 0.4 % of the largest float32 rounds to
 // Inf as bf16, and where a product overflows its part products may do so with either sign.  Every thread keeps the largest
 // magnitude it has taken apart (half an instruction per value; NaNs do not count: their parts are NaN), and a workgroup whose
 // two largest could make a sum leave the range multiplies its tile once more with v_mfma_f32_32x32x2_f32, on float32 values.
+// A value below 2^-110 loses up to 2^-134 in its lo part (a bf16 denormal; the matrix cores keep those), and a sum of k
+// products up to k 2^-134 (A + B), A and B being the two largest magnitudes: less than a rounding of every sum of at least
+// k 2^-110 (A + B).  Every thread keeps the smallest magnitude that is not zero, too (one and a half instructions per value),
+// and a workgroup that has met one below 2^-110 and holds a smaller sum than that takes the same way.
 //
 // Workgroup = WVM x WVN x WVK wavefronts; block tile BM x BN, K stage BK.  Global loads go to registers (one stage ahead), are
 // split there and stored to LDS as PLANES bf16 tiles [BK / 32][row][32 k] of 64 bytes per row, from where a fragment (8
@@ -437,6 +442,11 @@ __device__ __forceinline__ void split_pair(float a, float b, uint32_t (&p)[PLANE
 constexpr float LARGEST_BF16 = 3.3895313892515355e38f, LARGEST_SUM = 0x1p126f;
 // whatever the other operand and k <= 2^31 are, as long as it holds for both
 constexpr float SURELY_IN_RANGE = 0x1p47f;
+// sums of k products from k (A + B) times this on
+constexpr float LOSSLESS_SUM = 0x1p-110f;
+// |a| below 2^-110, but not zero (by its bits: twice the magnitude, minus one, so that a zero is the largest)
+constexpr uint32_t LEAST_WHOLE = (17u << 24) - 1u;
+__device__ __forceinline__ uint32_t magnitude_key(float a) { return (__float_as_uint(a) << 1) - 1u; }
 __device__ __forceinline__ bool parts_in_range(float a, float b, int k) {
   return a <= LARGEST_BF16 && b <= LARGEST_BF16 && a * b * (float)k <= LARGEST_SUM;
 }
@@ -504,7 +514,8 @@ struct Stager {
   bool on;
   bool tail;
   f4v colsum = {0.f, 0.f, 0.f, 0.f};
-  float largest = 0.f;  // magnitude of what this thread has taken apart
+  float largest = 0.f;           // magnitude of what this thread has taken apart
+  uint32_t least = 0xffffffffu;  // magnitude_key of the same
 
   static __device__ __forceinline__ int kgroup(int tid) { return OP::KC ? tid % KG : (tid / OW) % KG; }
   static __device__ __forceinline__ int ogroup(int tid) { return OP::KC ? tid / KG : tid % OW + OW * (tid / (OW * KG)); }
@@ -554,7 +565,11 @@ struct Stager {
     }
     if constexpr (PL > 1) {
 #pragma unroll
-      for (int e = 0; e < E; ++e) largest = max_magnitude(max_magnitude(largest, v[e][0], v[e][1]), v[e][2], v[e][3]);
+      for (int e = 0; e < E; ++e) {
+        largest = max_magnitude(max_magnitude(largest, v[e][0], v[e][1]), v[e][2], v[e][3]);
+        least = min(min(least, magnitude_key(v[e][0])), magnitude_key(v[e][1]));
+        least = min(min(least, magnitude_key(v[e][2])), magnitude_key(v[e][3]));
+      }
     }
     if constexpr (OP::KC) {
 #pragma unroll
@@ -736,17 +751,44 @@ __global__ __launch_bounds__(64 * WVM * WVN * WVK) void split_gemm_kernel(SplitG
   }
   exchange();
 
-  if constexpr (PLANES > 1) {
-    if (__syncthreads_or(sa.largest > SURELY_IN_RANGE || sb.largest > SURELY_IN_RANGE)) {  // (see the head of the file)
+  // f(row0, col, tile's accumulator, first, last) for every 32x32 tile this wavefront keeps values of: value v of lane l sits at
+  // row 8*(v/4) + 4*(l/32) + v%4, column l%32 of its tile
+  auto kept = [&](auto f) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        const int t16 = (i * TN + j) * 16;
+        const int first = WVK == 1 ? 0 : min(max(wk * KEEP - t16, 0), 16), last = WVK == 1 ? 16 : min(max((wk + 1) * KEEP - t16, 0), 16);
+        const int col = n0 + wn + j * 32 + l32;
+        if (first < last && col < g.N) f(m0 + wm + i * 32 + lhi * 4, col, acc[i][j], first, last);
+      }
+  };
+
+  if constexpr (PLANES > 1) {  // (see the head of the file)
+    const bool lossy = sa.least < LEAST_WHOLE || sb.least < LEAST_WHOLE;
+    if (__syncthreads_or(sa.largest > SURELY_IN_RANGE || sb.largest > SURELY_IN_RANGE || lossy)) {
       int* const top = reinterpret_cast<int*>(lds);  // (magnitudes order as their bits do)
       if (threadIdx.x < 2) top[threadIdx.x] = 0;
       __syncthreads();
       atomicMax(top, __float_as_int(sa.largest));
       atomicMax(top + 1, __float_as_int(sb.largest));
       __syncthreads();
-      const bool in_range = parts_in_range(__int_as_float(top[0]), __int_as_float(top[1]), k_end - k_begin);
-      __syncthreads();
-      if (!in_range) {
+      const float top_a = __int_as_float(top[0]), top_b = __int_as_float(top[1]);
+      bool whole = parts_in_range(top_a, top_b, k_end - k_begin);
+      if (__syncthreads_or(lossy)) {
+        const float limit = (float)(k_end - k_begin) * LOSSLESS_SUM * (top_a + top_b);
+        bool small = false;
+        kept([&](int row0, int, const f16v& a, int first, int last) {
+#pragma unroll
+          for (int v = 0; v < 16; ++v) {
+            const int row = row0 + (v >> 2) * 8 + (v & 3);
+            if (fabsf(a[v]) < limit && v >= first && v < last && row < g.M && ep.map_row(row) >= 0) small = true;
+          }
+        });
+        whole = !__syncthreads_or(small || !whole);
+      }
+      if (!whole) {
         // Everything is worked out anew from values the compiler cannot know to be the same: nothing is kept in registers
         // through the loop above for the sake of this one.
         int tid = threadIdx.x, from = k_begin;
@@ -786,19 +828,6 @@ __global__ __launch_bounds__(64 * WVM * WVN * WVK) void split_gemm_kernel(SplitG
       }
     }
   }
-  // f(row0, col, tile's accumulator, first, last) for every 32x32 tile this wavefront keeps values of: value v of lane l sits at
-  // row 8*(v/4) + 4*(l/32) + v%4, column l%32 of its tile
-  auto kept = [&](auto f) {
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int t16 = (i * TN + j) * 16;
-        const int first = WVK == 1 ? 0 : min(max(wk * KEEP - t16, 0), 16), last = WVK == 1 ? 16 : min(max((wk + 1) * KEEP - t16, 0), 16);
-        const int col = n0 + wn + j * 32 + l32;
-        if (first < last && col < g.N) f(m0 + wm + i * 32 + lhi * 4, col, acc[i][j], first, last);
-      }
-  };
   float* const part = g.ws ? g.ws + (int64_t)bz * g.ws_rows * g.N : nullptr;
 
   kept([&](int row0, int col, const f16v& a, int first, int last) {

@@ -1457,7 +1457,6 @@ def test_recurrence_in_one_workgroup_with_values_at_the_end_of_the_range(S, ctx,
     for o in (rep, cm):
         o.close()
 
-
 @pytest.mark.parametrize("kind", ["lstm", "simple_rnn"])
 def test_lstm_sequence_kernel_gives_up_instead_of_hanging(S, monkeypatch, kind):
     """A workgroup of a one-launch recurrent kernel that waits for its neighbours polls a bounded number of times.  With the
@@ -2284,3 +2283,93 @@ def test_split_convolutions_at_the_end_of_the_range(S, ctx, filters, channels, v
     h.close()
     xb.free()
     yb.free()
+
+
+def _small(rng, shape, exponent):
+    return np.ldexp(rng.standard_normal(shape), exponent).astype(f32)
+
+
+@pytest.mark.parametrize("exponent", [-107, -112, -119, -126, -133, -141])
+@pytest.mark.parametrize("n,k,m", [(5, 4, 6), (70, 133, 66), (200, 700, 40)])
+def test_split_products_of_small_values(S, ctx, exponent, n, k, m):
+    """Values below 2^-110 (float32 denormals among them) are no sums of three bf16 parts.  Their products are as right as any
+    others, with every operand of that size and with one row or column of it beside ordinary ones: all products of a Dense
+    layer against float64, errors as at the tile edges."""
+    rng = np.random.default_rng(n - exponent)
+    up = min(-exponent - 10, 110)
+    # x small: the forward product's A, the weight gradient's A;  targets small: the A of dX and the B of dW
+    for case in ("all of x", "a row of x", "a column of w", "dP"):
+        x, w1, w2 = _small(rng, (n, k), 0), _small(rng, (k, m), 0), _small(rng, (m, 5), 0)
+        y = _small(rng, (n, 5), 0)
+        if case == "all of x":
+            x, w1 = _small(rng, (n, k), exponent), _small(rng, (k, m), up)
+        elif case == "a row of x":
+            x[n - 2] = _small(rng, k, exponent)
+        elif case == "a column of w":
+            w1[:, 3] = _small(rng, k, exponent)
+        else:  # outputs of zero: dP = 2 (p - y) / size is as small as the targets
+            w1, w2, y = np.zeros_like(w1), _small(rng, (m, 5), up), np.ldexp(rng.standard_normal((n, 5)), exponent + 9).astype(f32)
+        zeros = [np.zeros(m, f32), np.zeros(5, f32)]
+        h = Harness(S, ctx, [("dense", m, "identity"), ("dense", 5, "identity")], "mse", (k,), n)
+        h.rep.set_params({"0/weights": w1, "1/weights": zeros[0], "2/weights": w2, "3/weights": zeros[1]})
+        xb, yb = ctx.to_device(x), ctx.to_device(y)
+        want, size = _affine_bounds(x, y, w1, zeros[0], w2, zeros[1])
+        got = {"out": h.rep.forward(xb)}
+        h.rep.grad(xb, yb)
+        got.update(h.rep.get_grads())
+        steps = 6.0 / 16.0 * (n + k + m + 5) + 16.0
+        for name in got:
+            # ... and float32's own smallest step, 2^-149, for each of a chain of values that lie below its normal range, times
+            # what they are multiplied with (dP off by 2^-150 and dH by as much again for every product of the last sum)
+            denormal = 2.0 ** -149 * (k + m + 5) * max(1.0, 16.0 * float(np.abs(w2).max()) * (n * float(np.abs(x).max()) if name in ("0/weights", "1/weights") else 1.0))
+            assert np.all(np.abs(got[name] - want[name]) <= steps * 2.0 ** -24 * size[name] + denormal), (case, name)
+        # the first product alone, row by row, relative to the magnitudes of that row's own products
+        one = Harness(S, ctx, [("dense", m, "identity")], "mse", (k,), n)
+        one.rep.set_params({p: v for (p, _, _), v in zip(one.cm.params, (w1, zeros[0]))})
+        exact, scale = x.astype(np.float64) @ w1.astype(np.float64), np.abs(x).astype(np.float64) @ np.abs(w1).astype(np.float64)
+        assert np.all(np.abs(one.rep.forward(xb) - exact) <= (6.0 / 16.0 * k + 16.0) * 2.0 ** -24 * scale + 2.0 ** -150 * (k + 1)), case
+        for o in (h, one):
+            o.close()
+        xb.free()
+        yb.free()
+
+
+@pytest.mark.parametrize("filters,channels", [(8, 3), (5, 4), (12, 1)])
+@pytest.mark.parametrize("exponent", [-112, -126, -133])
+def test_split_convolutions_of_small_values(S, ctx, filters, channels, exponent):
+    """The same for padded convolutions: forward, filter gradient and input gradient of the second of two, whose input (the
+    first one's output) or output gradient is small."""
+    rng = np.random.default_rng(filters - exponent)
+    spec = [("conv", 6, (1, 1), (1, 1), "valid", "identity", False), ("conv", filters, (3, 3), (1, 1), "same", "identity", False), ("flatten",)]
+    shape, batch = (5, 6, channels), 3
+    h = Harness(S, ctx, spec, "mse", shape, batch)
+    names = [p for p, _, _ in h.cm.params]
+    shapes = {p: s for p, s, _ in h.cm.params}
+    up = min(-exponent - 10, 110)
+    for case in ("input", "output gradient"):
+        x = _small(rng, (batch,) + shape, exponent if case == "input" else 0)
+        w = [_small(rng, shapes[names[0]], 0), _small(rng, shapes[names[1]], up)]
+        y = _small(rng, (batch, 30 * filters), 0 if case == "input" else exponent + 12)
+        if case != "input":
+            w[0] *= 0
+        h.rep.set_params(dict(zip(names, w)))
+        xb, yb = ctx.to_device(x), ctx.to_device(y)
+
+        def run(x, y, w1, w2, sign):
+            a = O.conv2d(x, w1)
+            p = O.conv2d(a, w2, padding=O.PAD_SAME)
+            dp = 2.0 * (p + sign * y.reshape(p.shape)) / y.size
+            da = O.conv2d_grad_input(a.shape, w2, dp, padding=O.PAD_SAME)
+            return {"out": p.reshape(y.shape), names[1]: O.conv2d_grad_filter(a, w2.shape, dp, padding=O.PAD_SAME), names[0]: O.conv2d_grad_filter(x, w1.shape, da)}
+        d = [v.astype(np.float64) for v in (x, y, *w)]
+        want, size = run(*d, -1.0), run(*[np.abs(v) for v in d], 1.0)
+        got = {"out": h.rep.forward(xb)}
+        h.rep.grad(xb, yb)
+        got.update(h.rep.get_grads())
+        steps = 6.0 / 16.0 * (9 * (6 + filters) + channels + 90) + 16.0
+        for name in got:
+            denormal = 2.0 ** -149 * 100 * max(1.0, 16.0 * float(np.abs(w[1]).max()) * (90 * float(np.abs(x).max()) if name == names[0] else 1.0))
+            assert np.all(np.abs(got[name].reshape(want[name].shape) - want[name]) <= steps * 2.0 ** -24 * size[name] + denormal), (case, name)
+        xb.free()
+        yb.free()
+    h.close()
