@@ -24,21 +24,26 @@ constexpr int ROWS = 4;  // batch rows of a workgroup
 
 __device__ __forceinline__ float sigmoidf_(float x) { return 1.0f / (1.0f + expf(-x)); }
 
-constexpr float LARGEST_F32 = 3.4028234663852886e38f;
-__device__ __forceinline__ float below_inf(float a) {
-  return fabsf(a) > LARGEST_BF16 && fabsf(a) <= LARGEST_F32 ? copysignf(LARGEST_BF16, a) : a;
-}
-
-__device__ __forceinline__ float hi_of(float a, bool& huge) {
-  huge = huge || fabsf(a) > LARGEST_BF16;
-  return below_inf(a);
-}
+// The ends of the range (split_gemm.hpp).  Up to LARGEST_USUAL no sum of 256 products nor any part of one overflows, and a nonzero
+// value below 2^-110 is not the sum of three bf16 parts.  A workgroup that has met a value outside (in the weights, or in any
+// state so far) multiplies in float32 from then on.  Its wavefronts have to agree on that at every step: values of the state a
+// step reads raise the flag of that step's parity, which is written next two barriers later.
+constexpr float LARGEST_USUAL = 0x1p47f;
+struct Seen {
+  float largest = 0.f;
+  uint32_t least = LEAST_WHOLE;
+  __device__ __forceinline__ void add(float a) {
+    largest = fmaxf(largest, fabsf(a));
+    least = min(least, magnitude_key(a));
+  }
+  __device__ __forceinline__ bool outside() const { return (int)(largest > LARGEST_USUAL) | (int)(least < LEAST_WHOLE); }
+};
 
 // Column u of [H, H] weights (TRANSPOSED: row u) in operand order: lane (column, g) holds k = 32 kb + 8 g .. + 7 of every kb,
 // in three parts, zeros from H on.  Every load is made, from inside the tensor, and what lies outside is dropped after: loads
 // under a condition come one at a time (128 of them were 90 us before the first step).
 template <int KB, bool TRANSPOSED>
-__device__ __forceinline__ void load_column(bf16x8 (&b)[KB][3], int g, const float* __restrict__ w, int u, int H, bool& huge) {
+__device__ __forceinline__ void load_column(bf16x8 (&b)[KB][3], int g, const float* __restrict__ w, int u, int H, Seen& seen) {
   const uint32_t uc = (uint32_t)min(u, H - 1);
   float all[KB][8];
 #pragma unroll
@@ -57,7 +62,9 @@ __device__ __forceinline__ void load_column(bf16x8 (&b)[KB][3], int g, const flo
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       float l = x[2 * j], r = x[2 * j + 1];
-      const uint32_t hi = pack_bf16(hi_of(l, huge), hi_of(r, huge));
+      seen.add(l);
+      seen.add(r);
+      const uint32_t hi = pack_bf16(l, r);
       l -= __uint_as_float(hi << 16);
       r -= __uint_as_float(hi & 0xffff0000u);
       const uint32_t mid = pack_bf16(l, r);
@@ -79,9 +86,9 @@ template <int KB>
 struct State {
   static constexpr int PITCH = 64 * KB + 16, BYTES = 16 * PITCH;
   // value k of batch row r
-  static __device__ __forceinline__ void put(char* lds, int r, int k, float a, bool& huge) {
+  static __device__ __forceinline__ void put(char* lds, int r, int k, float a) {
     char* at = lds + 4 * r * PITCH + 2 * k;
-    const uint32_t hi = pack_bf16(hi_of(a, huge), 0.f);
+    const uint32_t hi = pack_bf16(a, 0.f);
     a -= __uint_as_float(hi << 16);
     const uint32_t mid = pack_bf16(a, 0.f);
     a -= __uint_as_float(mid << 16);
@@ -117,21 +124,18 @@ __device__ __forceinline__ void multiply_state(const char* at, const bf16x8 (&w)
   }
 }
 
-// An Inf taken apart is Inf + NaN + NaN.  Where one was met (in the weights, or in any state so far), the product of the hi
-// parts alone says what float32 arithmetic gives: where that is not finite it is the result.
-template <int KB, int N>
-__device__ __forceinline__ void multiply_huge(const char* at, const bf16x8 (&w)[N][KB][3], float (&out)[N]) {
-#pragma unroll
-  for (int n = 0; n < N; ++n) {
-    f4v acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int kb = 0; kb < KB; ++kb) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8*)(at + 64 * kb), w[n][kb][0], acc, 0, 0, 0);
-    out[n] = fabsf(acc[0]) <= LARGEST_F32 ? out[n] : acc[0];
-  }
-}
-
 // LDS writes are visible, reads done; stores to memory stay in flight (no other lane reads them in this launch)
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// The same cell in float32: a row of the state x column u (TRANSPOSED: row u) of the weights in memory, k ascending.
+template <bool TRANSPOSED>
+__device__ __forceinline__ float multiply_float32(const float* state, const float* __restrict__ w, int u, int H) {
+  const uint32_t uc = (uint32_t)min(u, H - 1);
+  float s = 0.f;
+#pragma unroll 4
+  for (int k = 0; k < H; ++k) s = fmaf(state[k], w[TRANSPOSED ? uc * (uint32_t)H + (uint32_t)k : (uint32_t)k * (uint32_t)H + uc], s);
+  return s;
+}
 
 // uniform base + a lane's byte offset of 32 bits: one register of address, not two per tensor
 __device__ __forceinline__ const float& at_bytes(const float* base, uint32_t off) { return *(const float*)((const char*)base + off); }
@@ -158,16 +162,17 @@ template <int KB>
 __global__ __launch_bounds__(512) void lstm_local_fwd_kernel(LocalFwdArgs a) {
   typedef State<KB> P;
   __shared__ __attribute__((aligned(16))) char lds[2 * P::BYTES];
-  __shared__ int any_huge;
+  __shared__ float whole[ROWS][32 * KB];  // the state in float32, where it is needed
+  __shared__ int outside[2];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c16 = lane & 15, g = lane >> 4;
   const int u = wave * 16 + c16, r = blockIdx.x * ROWS + g;
   const int H = a.H;
   clear_lds(lds, 2 * P::BYTES);
-  if (threadIdx.x == 0) any_huge = 0;
-  bool huge = false;
+  if (threadIdx.x < 2) outside[threadIdx.x] = 0;
+  Seen seen;
   bf16x8 w[4][KB][3];
 #pragma unroll
-  for (int q = 0; q < 4; ++q) load_column<KB, false>(w[q], g, a.wr[q], u, H, huge);
+  for (int q = 0; q < 4; ++q) load_column<KB, false>(w[q], g, a.wr[q], u, H, seen);
   __syncthreads();
 
   // this lane's cell; lanes without one read cell 0 and write nothing
@@ -177,10 +182,13 @@ __global__ __launch_bounds__(512) void lstm_local_fwd_kernel(LocalFwdArgs a) {
   float c = a.c0 ? at_bytes(a.c0, ci) : 0.f, z[4];
 #pragma unroll
   for (int q = 0; q < 4; ++q) z[q] = at_bytes(a.gates + q * H, zi);
-  if (a.h0 && live) P::put(lds, g, u, at_bytes(a.h0, ci), huge);
-  if (huge) any_huge = 1;
+  float h = a.h0 && live ? at_bytes(a.h0, ci) : 0.f;
+  if (a.h0 && live) P::put(lds, g, u, h);
+  seen.add(h);
+  if (seen.outside()) outside[0] = outside[1] = 1;
   __syncthreads();
   const int at = c16 * P::PITCH + 16 * g;
+  int float32 = 0;
   for (int t = 0; t < a.T; ++t) {
     const char* now = lds + (t & 1) * P::BYTES + at;
     char* next = lds + ((t + 1) & 1) * P::BYTES;
@@ -189,9 +197,15 @@ __global__ __launch_bounds__(512) void lstm_local_fwd_kernel(LocalFwdArgs a) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) zn[q] = at_bytes(zt + q * H, zi);
     if (t > 0 || a.h0) {
-      const int met_huge = any_huge;
+      const int met = outside[t & 1];
       multiply_state<KB, 4>(now, w, s);
-      if (__builtin_amdgcn_readfirstlane(met_huge)) multiply_huge<KB, 4>(now, w, s);
+      float32 |= __builtin_amdgcn_readfirstlane(met);
+      if (float32) {
+        if (live) whole[g][u] = h;
+        lds_barrier();
+#pragma unroll
+        for (int q = 0; q < 4; ++q) s[q] = multiply_float32<false>(whole[g], a.wr[q], u, H);
+      }
     }
     // c = c_prev * f + i * g ; h = o * tanh(c)   (layer/RNN.scala:336-337)
     const float f = sigmoidf_(s[0] + z[0]);
@@ -199,9 +213,10 @@ __global__ __launch_bounds__(512) void lstm_local_fwd_kernel(LocalFwdArgs a) {
     const float gg = tanhf(s[2] + z[2]);
     const float o = sigmoidf_(s[3] + z[3]);
     c = c * f + in * gg;
-    const float h = o * tanhf(c);
+    h = o * tanhf(c);
     if (live) {
-      P::put(next, g, u, h, huge);
+      P::put(next, g, u, h);
+      seen.add(h);
       float* gt = a.gates + (int64_t)t * 4 * a.slice;
       at_bytes(gt, zi) = f;
       at_bytes(gt + H, zi) = in;
@@ -213,6 +228,7 @@ __global__ __launch_bounds__(512) void lstm_local_fwd_kernel(LocalFwdArgs a) {
     }
 #pragma unroll
     for (int q = 0; q < 4; ++q) z[q] = zn[q];
+    if (seen.outside()) outside[(t + 1) & 1] = 1;
     lds_barrier();
   }
 }
@@ -235,16 +251,17 @@ template <int KB>
 __global__ __launch_bounds__(512) void lstm_local_bwd_kernel(LocalBwdArgs a) {
   typedef State<KB> P;
   extern __shared__ __attribute__((aligned(16))) char lds[];
-  __shared__ int any_huge;
+  __shared__ float whole[4][ROWS][32 * KB];  // the state in float32, where it is needed
+  __shared__ int outside[2];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c16 = lane & 15, g = lane >> 4;
   const int u = wave * 16 + c16, r = blockIdx.x * ROWS + g;
   const int H = a.H;
   clear_lds(lds, 2 * 4 * P::BYTES);
-  if (threadIdx.x == 0) any_huge = 0;
-  bool huge = false;
+  if (threadIdx.x < 2) outside[threadIdx.x] = 0;
+  Seen seen;
   bf16x8 w[4][1][KB][3];
 #pragma unroll
-  for (int q = 0; q < 4; ++q) load_column<KB, true>(w[q][0], g, a.wr[q], u, H, huge);
+  for (int q = 0; q < 4; ++q) load_column<KB, true>(w[q][0], g, a.wr[q], u, H, seen);
 
   const bool live = u < H && r < a.rows;
   const uint32_t ci = live ? 4u * (uint32_t)(r * H + u) : 0u, zi = live ? 4u * (uint32_t)(r * 4 * H + u) : 0u;
@@ -258,8 +275,9 @@ __global__ __launch_bounds__(512) void lstm_local_bwd_kernel(LocalBwdArgs a) {
   float c = at_bytes(a.c + (int64_t)(a.T - 1) * a.slice, ci), dc = 0.f, dh = a.dh_last ? at_bytes(a.dh_last, ci) : 0.f, gate[4], cp, dy;
   fetch(a.T - 1, gate, cp, dy);
   __syncthreads();
-  if (huge) any_huge = 1;  // (read after the next barrier)
+  if (seen.outside()) outside[0] = outside[1] = 1;  // (read after the next barrier)
   const int at = c16 * P::PITCH + 16 * g;
+  int float32 = 0;
   for (int t = a.T - 1; t >= 0; --t) {
     char* buf = lds + (t & 1) * 4 * P::BYTES;
     float gn[4], cpn, dyn;
@@ -273,22 +291,30 @@ __global__ __launch_bounds__(512) void lstm_local_bwd_kernel(LocalBwdArgs a) {
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         at_bytes(a.dz + (int64_t)t * 4 * a.slice + q * H, zi) = dz[q];
-        P::put(buf + q * P::BYTES, g, u, dz[q], huge);
+        P::put(buf + q * P::BYTES, g, u, dz[q]);
+        seen.add(dz[q]);
       }
     }
-    if (huge) any_huge = 1;
+    if (seen.outside()) outside[t & 1] = 1;
     if (t == 0) break;
     lds_barrier();
-    const int met_huge = any_huge;
+    const int met = outside[t & 1];
     float s[4][1];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       multiply_state<KB, 1>(buf + q * P::BYTES + at, w[q], s[q]);
       if constexpr (KB > 3) __builtin_amdgcn_sched_barrier(0);  // (four gates' sums and state reads at once are more than the registers hold)
     }
-    if (__builtin_amdgcn_readfirstlane(met_huge))
+    float32 |= __builtin_amdgcn_readfirstlane(met);
+    if (float32) {
+      if (live) {
 #pragma unroll
-      for (int q = 0; q < 4; ++q) multiply_huge<KB, 1>(buf + q * P::BYTES + at, w[q], s[q]);
+        for (int q = 0; q < 4; ++q) whole[q][g][u] = dz[q];
+      }
+      lds_barrier();
+#pragma unroll
+      for (int q = 0; q < 4; ++q) s[q][0] = multiply_float32<true>(whole[q][g], a.wr[q], u, H);
+    }
     dh = (s[0][0] + s[1][0]) + (s[2][0] + s[3][0]);
     c = cp;
     cp = cpn;
@@ -317,21 +343,22 @@ template <int KB, int UBW, bool BACKWARD>
 __global__ __launch_bounds__(512) void rnn_local_kernel(LocalMulArgs a) {
   typedef State<KB> P;
   __shared__ __attribute__((aligned(16))) char lds[2 * P::BYTES];
-  __shared__ int any_huge;
+  __shared__ float whole[ROWS][32 * KB];  // the state in float32, where it is needed
+  __shared__ int outside[2];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c16 = lane & 15, g = lane >> 4;
   const int u0 = wave * 16 * UBW + c16, r = blockIdx.x * ROWS + g;
   const int H = a.H;
   clear_lds(lds, 2 * P::BYTES);
-  if (threadIdx.x == 0) any_huge = 0;
-  bool huge = false;
+  if (threadIdx.x < 2) outside[threadIdx.x] = 0;
+  Seen seen;
   bf16x8 w[UBW][KB][3];
 #pragma unroll
-  for (int b = 0; b < UBW; ++b) load_column<KB, BACKWARD>(w[b], g, a.wr, u0 + 16 * b, H, huge);
+  for (int b = 0; b < UBW; ++b) load_column<KB, BACKWARD>(w[b], g, a.wr, u0 + 16 * b, H, seen);
   __syncthreads();
 
   bool live[UBW];
   uint32_t ai[UBW], oi[UBW];
-  float add[UBW];
+  float add[UBW], state[UBW];
 #pragma unroll
   for (int b = 0; b < UBW; ++b) {
     const int u = u0 + 16 * b;
@@ -339,11 +366,14 @@ __global__ __launch_bounds__(512) void rnn_local_kernel(LocalMulArgs a) {
     ai[b] = live[b] ? 4u * (uint32_t)(r * a.add_ld + u) : 0u;
     oi[b] = live[b] ? 4u * (uint32_t)(r * H + u) : 0u;
     add[b] = a.add ? at_bytes(a.add, ai[b]) : 0.f;
-    if (a.seed && live[b]) P::put(lds, g, u, at_bytes(a.seed, oi[b]), huge);
+    state[b] = a.seed && live[b] ? at_bytes(a.seed, oi[b]) : 0.f;
+    if (a.seed && live[b]) P::put(lds, g, u, state[b]);
+    seen.add(state[b]);
   }
-  if (huge) any_huge = 1;
+  if (seen.outside()) outside[0] = outside[1] = 1;
   __syncthreads();
   const int at = c16 * P::PITCH + 16 * g;
+  int float32 = 0;
   for (int s = 0; s < a.steps; ++s) {
     const char* now = lds + (s & 1) * P::BYTES + at;
     char* next = lds + ((s + 1) & 1) * P::BYTES;
@@ -351,20 +381,30 @@ __global__ __launch_bounds__(512) void rnn_local_kernel(LocalMulArgs a) {
 #pragma unroll
     for (int b = 0; b < UBW; ++b) add_next[b] = a.add ? at_bytes(a.add + (int64_t)min(s + 1, a.steps - 1) * a.add_step, ai[b]) : 0.f;
     if (s > 0 || a.seed) {
-      const int met_huge = any_huge;
+      const int met = outside[s & 1];
       multiply_state<KB, UBW>(now, w, x);
-      if (__builtin_amdgcn_readfirstlane(met_huge)) multiply_huge<KB, UBW>(now, w, x);
+      float32 |= __builtin_amdgcn_readfirstlane(met);
+      if (float32) {
+#pragma unroll
+        for (int b = 0; b < UBW; ++b)
+          if (live[b]) whole[g][u0 + 16 * b] = state[b];
+        lds_barrier();
+#pragma unroll
+        for (int b = 0; b < UBW; ++b) x[b] = multiply_float32<BACKWARD>(whole[g], a.wr, u0 + 16 * b, H);
+      }
     }
 #pragma unroll
     for (int b = 0; b < UBW; ++b) {
       if (a.add) x[b] += add[b];
       if (live[b]) {
-        P::put(next, g, u0 + 16 * b, x[b], huge);
+        P::put(next, g, u0 + 16 * b, x[b]);
+        seen.add(x[b]);
         at_bytes(a.out + (int64_t)s * a.out_step, oi[b]) = x[b];
       }
       add[b] = add_next[b];
+      state[b] = x[b];
     }
-    if (huge) any_huge = 1;
+    if (seen.outside()) outside[(s + 1) & 1] = 1;
     lds_barrier();
   }
 }

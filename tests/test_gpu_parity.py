@@ -1458,6 +1458,105 @@ def test_recurrence_in_one_workgroup_with_values_at_the_end_of_the_range(S, ctx,
         o.close()
 
 @pytest.mark.parametrize("kind", ["lstm", "simple_rnn"])
+@pytest.mark.parametrize("units", [20, 100])
+@pytest.mark.parametrize("exponent", [-107, -114, -122])
+def test_recurrence_in_one_workgroup_with_small_values(S, ctx, kind, units, exponent):
+    """A state, its gradient and recurrent weights below 2^-110 lose nothing: outputs and gradients against float64, relative
+    to their own largest value.  A simple cell carries the small state itself; an LSTM's state is ordinary, its gradients
+    are as small as the last layer's."""
+    features, batch, T = 3, 6, 4
+    first = {"lstm": (O.LSTM, S.LSTM), "simple_rnn": (O.SimpleRNN, S.SimpleRNN)}[kind]
+    activation = {"lstm": {}, "simple_rnn": {"activation": O.ACT_IDENTITY}}[kind]
+    om = O.Model([first[0](units, stateful=True, **activation), O.Dense(2, O.ACT_IDENTITY)], O.LOSS_MSE)
+    layer = S.LSTM(units, stateful=True) if kind == "lstm" else S.SimpleRNN(units, S.Identity, stateful=True)
+    layers = layer >> S.Dense(2, S.Identity)
+    cm = S.CompiledModel(ctx, [l.desc() for l in layers.layers], S.MeanSquaredError.kind, (T, features), batch)
+    rep = cm.replica(None)
+    rng = np.random.default_rng(units - exponent)
+    base = glorot_params(om, (batch, T, features), rng)
+    for p in base:
+        if O.is_unaggregated_path(p):
+            base[p] = rng.uniform(0.1, 0.4, base[p].shape).astype(f32)
+    last = [p for p in base if base[p].shape[-1] == 2]
+    x, y = rng.standard_normal((batch, T, features)).astype(f32), rng.uniform(-1, 1, (batch, 2)).astype(f32)
+    for place in ("state", "gradient", "weights"):
+        params, xs, ys = {k: v.copy() for k, v in base.items()}, x, y
+        if place == "state":
+            if kind == "lstm":
+                continue
+            xs = np.ldexp(x, exponent)
+            for p in params:
+                if O.is_unaggregated_path(p):
+                    params[p] = np.ldexp(params[p], exponent)
+                elif p not in last and params[p].ndim == 1:
+                    params[p] = params[p] * 0
+            for p in last:
+                params[p] = np.ldexp(params[p], -exponent - 10) if params[p].ndim == 2 else params[p] * 0
+        elif place == "gradient":  # dP = 2 (p - y) / 12, and p = 0
+            for p in last:
+                params[p] = params[p] * 0 if params[p].ndim == 1 else np.ldexp(params[p], exponent + 4)
+            ys = np.full_like(y, 12.0)
+        else:
+            for p in params:
+                if p.endswith("recurrent_weights"):
+                    params[p] = np.ldexp(params[p], exponent)
+            if kind == "simple_rnn":  # a step's output is the product alone: what it is off by shows
+                xs = x.copy()
+                xs[:, -1] = 0
+                for p in last:
+                    params[p] = np.ldexp(params[p], -exponent) if params[p].ndim == 2 else params[p] * 0
+                for p in params:
+                    if p not in last and params[p].ndim == 1 and not O.is_unaggregated_path(p):
+                        params[p] = params[p] * 0
+        rep.set_params(params)
+        xb, yb = ctx.to_device(xs.astype(f32)), ctx.to_device(ys)
+        p64 = {k: v.astype(np.float64) for k, v in params.items()}
+        want, (_, grads64) = om.forward(xs.astype(np.float64), p64), om.grad(xs.astype(np.float64), ys.astype(np.float64), p64)
+        # float32's own roundings, of the values of a chain of T steps and of the sums over units and rows
+        rel = 2.0 ** -24 * (T * (units + 16) + batch * T)
+        got = rep.forward(xb)
+        assert np.max(np.abs(got - want)) <= rel * np.max(np.abs(want)) + 2.0 ** -149 * units * max(1.0, 2.0 ** (-exponent - 8)), place
+        rep.grad(xb, yb)
+        grads = rep.get_grads()
+        for p in grads64:
+            top = float(np.max(np.abs(grads64[p])))
+            assert np.max(np.abs(grads[p] - grads64[p])) <= rel * top + 2.0 ** -149 * units * T, (place, p)
+        xb.free()
+        yb.free()
+    for o in (rep, cm):
+        o.close()
+
+
+@pytest.mark.parametrize("units", [5, 40, 200])
+def test_simple_cell_that_overflows_in_one_workgroup(S, ctx, units):
+    """A linear recurrence that outgrows float32 becomes infinite, as the oracle's does: no part of a product turns it into
+    NaN on the way (1e25 times 3e14 has none that is infinite by itself)."""
+    om = O.Model([O.SimpleRNN(units, activation=O.ACT_IDENTITY), O.Dense(2, O.ACT_IDENTITY)], O.LOSS_MSE)
+    layers = S.SimpleRNN(units, S.Identity) >> S.Dense(2, S.Identity)
+    cm = S.CompiledModel(ctx, [l.desc() for l in layers.layers], S.MeanSquaredError.kind, (5, 2), 6)
+    rep = cm.replica(None)
+    rng = np.random.default_rng(units)
+    params = {p: np.abs(v) + f32(0.01) for p, v in glorot_params(om, (6, 5, 2), rng).items()}
+    for p in params:
+        if p.endswith("recurrent_weights"):
+            params[p] = (params[p] * f32(3e14)).astype(f32)
+    x = rng.uniform(0.5, 1.0, (6, 5, 2)).astype(f32)
+    x[3:] *= f32(1e-20)
+    x[5] *= f32(1e-10)
+    rep.set_params(params)
+    xb = ctx.to_device(x)
+    with np.errstate(all="ignore"):
+        want = om.forward(x.astype(np.float64), {k: v.astype(np.float64) for k, v in params.items()}).astype(f32)
+    got = rep.forward(xb)
+    assert np.array_equal(np.isinf(got), np.isinf(want)) and not np.isnan(got).any(), (got, want)
+    fine = np.isfinite(want)
+    assert fine.any() and not fine.all() and np.all(np.abs(got[fine] - want[fine]) <= 2.0 ** -24 * 6 * (units + 16) * want[fine])
+    for o in (rep, cm):
+        o.close()
+    xb.free()
+
+
+@pytest.mark.parametrize("kind", ["lstm", "simple_rnn"])
 def test_lstm_sequence_kernel_gives_up_instead_of_hanging(S, monkeypatch, kind):
     """A workgroup of a one-launch recurrent kernel that waits for its neighbours polls a bounded number of times.  With the
     bound forced to zero (SCANET_SEQUENCE_SPIN_LIMIT, read when a context first launches such a kernel) every workgroup
