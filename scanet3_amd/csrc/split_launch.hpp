@@ -93,25 +93,33 @@ __global__ __launch_bounds__(256) void splitk_reduce4_kernel(const float* __rest
   }
 }
 
+// Whether a caller that applies the optimizer next (ctx->defer) can add the partial results: every sum goes straight to one
+// contiguous tensor, `plain`, in vectors of four, and there are enough of them to be worth a section of that launch.
+template <class EP>
+inline float* split_plain_destination(const EP& ep, int N) {
+  if constexpr (std::is_same<EP, StdEpilogue>::value) {
+    if (!ep.e.bias && ep.e.act == SN_ACT_IDENTITY && ep.e.row_index < 0 && ep.e.ldo == N) return ep.e.out;
+  } else if constexpr (std::is_same<EP, RunRowsEpilogue>::value) {
+    if (ep.ldo == N) return ep.out;
+  }
+  return nullptr;
+}
+inline bool split_defers(const float* plain, const float* ws, int M, int N) {
+  const int64_t total = (int64_t)M * N;
+  return plain && total % 4 == 0 && total >= 4096 && total < ((int64_t)1 << 30) && (reinterpret_cast<uintptr_t>(ws) & 15u) == 0;
+}
 
 // Adds `splits` partial results [split][M][N] and hands every sum to the epilogue, or leaves that to a caller that applies
-// the optimizer next (ctx->defer).
+// the optimizer next.
 template <class EP>
 static int launch_split_reduce(sn_ctx* ctx, const float* ws, int splits, int M, int N, const EP& ep) {
   const int64_t total = (int64_t)M * N;
   const bool aligned = (reinterpret_cast<uintptr_t>(ws) & 15u) == 0;
-  if (ctx->defer && total % 4 == 0 && total >= 4096 && total < ((int64_t)1 << 30) && aligned) {
-    float* plain = nullptr;  // the destination when every sum goes straight to one contiguous tensor
-    if constexpr (std::is_same<EP, StdEpilogue>::value) {
-      if (!ep.e.bias && ep.e.act == SN_ACT_IDENTITY && ep.e.row_index < 0 && ep.e.ldo == N) plain = ep.e.out;
-    } else if constexpr (std::is_same<EP, RunRowsEpilogue>::value) {
-      if (ep.ldo == N) plain = ep.out;
-    }
-    if (plain) {
-      *ctx->defer = DeferredReduce{1, ws, splits, (int)total, plain};
-      ctx->defer = nullptr;
-      return SN_OK;
-    }
+  float* const plain = split_plain_destination(ep, N);
+  if (ctx->defer && split_defers(plain, ws, M, N)) {
+    *ctx->defer = DeferredReduce{1, ws, splits, (int)total, plain};
+    ctx->defer = nullptr;
+    return SN_OK;
   }
   LaunchScope scope(ctx, "splitk_reduce");
   if (total % 4 == 0 && total >= 4096 && aligned) {
@@ -199,7 +207,8 @@ static int launch_split(sn_ctx* ctx, const char* name, int M, int N, int K, int 
   g.M = M; g.N = N; g.K = K;
   g.ws_rows = rows;
   g.colsum_row = colsum_row;
-  const SplitChoice c = split_choose(M, N, K, ctx->compute_units, ws ? ws_elems / ((int64_t)rows * N) : 1, ctx->defer != nullptr, PLANES);
+  const SplitChoice c = split_choose(M, N, K, ctx->compute_units, ws ? ws_elems / ((int64_t)rows * N) : 1,
+                                     ctx->defer && split_defers(split_plain_destination(ep, N), ws, rows, N), PLANES);
   g.ws = c.splits > 1 ? ws : nullptr;
   {
     LaunchScope scope(ctx, name, rows, N, K);

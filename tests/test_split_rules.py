@@ -38,3 +38,13 @@ def test_split_convolutions_stay_inside_32_bit_offsets(ask):
     assert ask("conv", 1023, 32, 32, 128, 32, 32, 128, 3, 3, 1, 1, 1, 1) == [1, 1, 1]
     # (n + 1) images of 2^21 bytes reach 2^31
     assert ask("conv", 4095, 32, 32, 128, 32, 32, 128, 3, 3, 1, 1, 1, 1) == [0, 0, 0]
+
+
+def test_a_sum_that_the_optimizer_cannot_take_is_priced_as_a_launch(ask):
+    """The choice of tile and splits charges 1 us for partial sums that the optimizer's launch adds and 4.5 for a launch of
+    their own: only sums that launch takes are the cheap kind.  The 3 x 3 x 3 x 48 filter of a colour image's first layer has
+    1296 values and is not, whatever its caller asked for."""
+    assert [ask("defers", m, n, 1)[0] for m, n in ((27, 48), (32, 128), (63, 65), (33, 125), (64, 65), (432, 80))] == [0, 1, 0, 0, 1, 1]
+    assert ask("defers", 432, 80, 0) == [0] and ask("defers", 1 << 15, 1 << 15, 1) == [0]
+    cheap, dear = ask("choose", 27, 48, 6000, 3, 1), ask("choose", 27, 48, 6000, 3, 0)
+    assert cheap[3] >= dear[3]
