@@ -17,8 +17,9 @@ int launch_split_conv_fwd(sn_ctx* ctx, const ConvGeom& g, const float* x, const 
     al.H = g.h; al.W = g.w; al.C = g.cin; al.kh = g.kh; al.L = L; al.Lp = Lp; al.total = total;
     al.by_iw = fast_div((uint32_t)g.wo);
     al.by_ih = fast_div((uint32_t)g.ho);
+    al.walk = run_walk(Lp);
     if (L == Lp) return launch_split<3>(ctx, "conv2d_forward", M, N, K, M, -1, al, FlatOp<false>{w, N, N, K}, ep, ws, ws_elems);
-    return launch_split<3>(ctx, "conv2d_forward", M, N, K, M, -1, al, ConvRunFilterOp{w, N, g.kh, L, Lp}, ep, ws, ws_elems);
+    return launch_split<3>(ctx, "conv2d_forward", M, N, K, M, -1, al, ConvRunFilterOp{w, N, g.kh, L, Lp, run_walk(Lp)}, ep, ws, ws_elems);
   };
   if (interior(g) && L == Lp) return run(ConvRunOp<false>{});
   return run(ConvRunOp<true>{});
@@ -37,10 +38,11 @@ int launch_split_conv_dgrad(sn_ctx* ctx, const ConvGeom& g, const float* dy, con
   al.total = g.n * g.ho * g.wo * g.cout;
   al.by_iw = fast_div((uint32_t)g.w);
   al.by_ih = fast_div((uint32_t)g.h);
+  al.walk = run_walk(Lp);
   const FastDiv by_cout = fast_div((uint32_t)g.cout);
   if (g.cout % 4 == 0)
-    return launch_split<3>(ctx, "conv2d_input_gradient", M, N, K, M, -1, al, ConvDgradFilterOp<true>{w, g.cin, g.cout, g.kh, g.kw, L, Lp, by_cout}, ep, ws, ws_elems);
-  return launch_split<3>(ctx, "conv2d_input_gradient", M, N, K, M, -1, al, ConvDgradFilterOp<false>{w, g.cin, g.cout, g.kh, g.kw, L, Lp, by_cout}, ep, ws, ws_elems);
+    return launch_split<3>(ctx, "conv2d_input_gradient", M, N, K, M, -1, al, ConvDgradFilterOp<true>{w, g.cin, g.cout, g.kh, g.kw, L, Lp, by_cout, run_walk(Lp)}, ep, ws, ws_elems);
+  return launch_split<3>(ctx, "conv2d_input_gradient", M, N, K, M, -1, al, ConvDgradFilterOp<false>{w, g.cin, g.cout, g.kh, g.kw, L, Lp, by_cout, run_walk(Lp)}, ep, ws, ws_elems);
 }
 
 int launch_split_conv_wgrad(sn_ctx* ctx, const ConvGeom& g, const float* x, const float* dy, float* dw, float* ws, int64_t ws_elems) {
@@ -50,6 +52,9 @@ int launch_split_conv_wgrad(sn_ctx* ctx, const ConvGeom& g, const float* x, cons
     al.x = x; al.g = g; al.L = L; al.Lp = Lp; al.K = K; al.total = g.n * g.h * g.w * g.cin; al.rows = g.kh * Lp;
     al.by_wo = fast_div((uint32_t)g.wo);
     al.by_ho = fast_div((uint32_t)g.ho);
+    al.step_ow = 32 % g.wo;
+    al.step_oh = 32 / g.wo % g.ho;
+    al.step_b = 32 / g.wo / g.ho;
     if (L == Lp) {
       Epilogue e;
       e.out = dw;

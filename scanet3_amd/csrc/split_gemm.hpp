@@ -60,6 +60,22 @@ typedef uint32_t u2v __attribute__((ext_vector_type(2)));
 struct KIndex {
   int k;
 };
+// Walking a k that is kept as (row r, place j of Lp): what 32 values are in rows and places is worked out on the host (a loop of
+// carries took up to a quarter as many trips as a stage has values: filter gradient of 72 x 48 x 31232, rows of 8 positions, 40 us).
+struct RunWalk {
+  int rows, places;  // 32 = rows * Lp + places
+};
+inline RunWalk run_walk(int Lp) { return RunWalk{32 / Lp, 32 % Lp}; }
+__device__ __forceinline__ void walk_run(int& r, int& j, int dk, int Lp, const RunWalk& w) {
+#pragma unroll
+  for (int i = 0; i < dk / 32; ++i) {
+    r += w.rows;
+    j += w.places;
+    const bool carry = j >= Lp;
+    r += carry ? 1 : 0;
+    j -= carry ? Lp : 0;
+  }
+}
 
 template <bool KC_>
 struct FlatOp {  // value(outer, k) = p[outer * ld + k] (KC) or p[k * ld + outer]
@@ -115,6 +131,7 @@ struct ConvRunOp {
   int H, W, C, kh, L, Lp;
   int total;  // elements of src
   FastDiv by_iw, by_ih;
+  RunWalk walk;
   struct Outer {
     int base, y0;   // element offset of (b, y0, x0, 0), possibly outside the tensor
     int jlo, jhi;   // j inside the image's width
@@ -138,11 +155,7 @@ struct ConvRunOp {
     s.j = k - s.r * Lp;
   }
   __device__ __forceinline__ void advance(KState& s, int dk) const {
-    s.j += dk;
-    while (s.j >= Lp) {
-      s.j -= Lp;
-      ++s.r;
-    }
+    walk_run(s.r, s.j, dk, Lp, walk);
   }
   __device__ __forceinline__ uint32_t load(const Outer& o, const KState& s, bool tail, f4v& v) const {
     int off = o.base + s.r * (ty * W * C) + s.j;
@@ -170,6 +183,7 @@ struct ConvRunFilterOp {
   static constexpr bool KC = false, MASKED = true, SIGNED = false;
   const float* w;
   int N, kh, L, Lp;
+  RunWalk walk;
   struct Outer {
     int off;
   };
@@ -183,11 +197,7 @@ struct ConvRunFilterOp {
     s.j = k - s.r * Lp;
   }
   __device__ __forceinline__ void advance(KState& s, int dk) const {
-    s.j += dk;
-    while (s.j >= Lp) {
-      s.j -= Lp;
-      ++s.r;
-    }
+    walk_run(s.r, s.j, dk, Lp, walk);
   }
   __device__ __forceinline__ uint32_t load(const Outer& o, const KState& s, bool, f4v& v) const {
     const bool in = s.r < kh && s.j < L;
@@ -204,6 +214,7 @@ struct ConvDgradFilterOp {
   const float* w;
   int cin, cout, kh, kw, L, Lp;
   FastDiv by_cout;
+  RunWalk walk;
   struct Outer {
     int off;
   };
@@ -217,11 +228,7 @@ struct ConvDgradFilterOp {
     s.j = k - s.r * Lp;
   }
   __device__ __forceinline__ void advance(KState& s, int dk) const {
-    s.j += dk;
-    while (s.j >= Lp) {
-      s.j -= Lp;
-      ++s.r;
-    }
+    walk_run(s.r, s.j, dk, Lp, walk);
   }
   __device__ __forceinline__ int place(int r, int j) const {
     const int qq = (int)div_by((uint32_t)j, by_cout);
@@ -254,6 +261,7 @@ struct ConvWgradRunOp {
   ConvGeom g;
   int L, Lp, K, total, rows;  // rows = kh * Lp
   FastDiv by_wo, by_ho;
+  int step_ow, step_oh, step_b;  // 32 = (step_b * ho + step_oh) * wo + step_ow
   struct Outer {
     int off, r, j;
   };
@@ -276,13 +284,15 @@ struct ConvWgradRunOp {
   }
   __device__ __forceinline__ void advance(KState& s, int dk) const {
     s.k += dk;
-    s.ow += dk;
-    while (s.ow >= g.wo) {
-      s.ow -= g.wo;
-      if (++s.oh == g.ho) {
-        s.oh = 0;
-        ++s.b;
-      }
+#pragma unroll
+    for (int i = 0; i < dk / 32; ++i) {
+      s.ow += step_ow;
+      const bool next_row = s.ow >= g.wo;
+      s.ow -= next_row ? g.wo : 0;
+      s.oh += step_oh + (next_row ? 1 : 0);
+      const bool next_image = s.oh >= g.ho;  // (step_oh < ho: at most one)
+      s.oh -= next_image ? g.ho : 0;
+      s.b += step_b + (next_image ? 1 : 0);
     }
   }
   __device__ __forceinline__ uint32_t load(const Outer& o, const KState& s, bool tail, f4v& v) const {
@@ -634,7 +644,7 @@ struct SplitShape {
   static constexpr int SUM_BYTES = BL::KC ? 0 : SB::KG * BN * 4;                       // column sums of B
   static constexpr int LDS = STAGE_BYTES > SWAP_BYTES ? (STAGE_BYTES > SUM_BYTES ? STAGE_BYTES : SUM_BYTES)
                                                       : (SWAP_BYTES > SUM_BYTES ? SWAP_BYTES : SUM_BYTES);
-  static_assert(TM >= 1 && TN >= 1 && BK % (16 * WVK) == 0 && VALUES % WVK == 0 && KEEP % 4 == 0, "tile does not suit the wavefronts");
+  static_assert(BK % 32 == 0 && TM >= 1 && TN >= 1 && BK % (16 * WVK) == 0 && VALUES % WVK == 0 && KEEP % 4 == 0, "tile does not suit the wavefronts");
   static_assert(LDS <= 160 * 1024, "more LDS than a CU has");
 };
 

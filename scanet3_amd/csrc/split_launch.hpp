@@ -158,10 +158,10 @@ inline SplitChoice split_choose(int M, int N, int K, int cu, int64_t max_parts, 
     const SplitTile& c = SPLIT_TILE[t];
     const int64_t tiles = ceil_div(M, c.bm) * ceil_div(N, c.bn);
     const int stages = (int)ceil_div(K, c.bk);
-    for (int s : counts) {
-      if (s > max_parts && s > 1) break;
-      const int per = (int)ceil_div(stages, s);
-      if (s > 1 && (per * c.bk < 64 || ceil_div(stages, per) != s)) continue;
+    for (int wanted : counts) {
+      if (wanted > max_parts && wanted > 1) break;
+      const int per = (int)ceil_div(stages, wanted), s = (int)ceil_div(stages, per);  // (the same s gives the same `per` again)
+      if (s > 1 && per * c.bk < 64) continue;
       const float wgs = (float)ceil_div(tiles * s, cu);
       float us = 3.0f + (float)(per * c.bk / 32) * std::max(c.lone[p], wgs * c.full[p]);
       if (s > 1) us += (deferred ? 1.0f : 4.5f) + 8.0e-6f * (float)s * (float)M * (float)N / 3.5f;
