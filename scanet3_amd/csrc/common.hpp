@@ -423,6 +423,13 @@ static inline bool split_conv_dgrad_ok(const ConvGeom& g, const float* dy, const
 static inline bool split_conv_wgrad_ok(const ConvGeom& g, const float* x, const float* dy) {
   return g.cout >= 4 && (int64_t)g.kw * g.cin >= 4 && split_image_ok(x, g.n, g.h, g.w, g.cin) && split_image_ok(dy, g.n, g.ho, g.wo, g.cout);
 }
+// Many positions, few output columns and a short reduction over whole vectors of channels: a split product's workgroup pays
+// for finding its positions and for half-empty column and K tiles more than the float32 instruction costs the value-by-value
+// kernel.  Forward of 378450 positions x 8 / 16 / 32 filters x 72: 41 / 42 / 43 us against 79 / 80 / 81; input gradient x 8 x
+// 144 53 / 101, x 14 x 216 80 / 120; at 92510 positions 17 / 25; at 25230 12 / 11.  With 10 channels (no whole vectors) 91 / 84.
+static inline bool conv_prefers_float32_tiles(int64_t positions, int columns, int64_t k, int channels) {
+  return channels % 4 == 0 && columns <= 32 && k <= 216 && positions >= 40000;
+}
 int launch_split_conv_fwd(sn_ctx* ctx, const ConvGeom& g, const float* x, const float* w, const Epilogue& e, float* ws, int64_t ws_elems);
 int launch_split_conv_dgrad(sn_ctx* ctx, const ConvGeom& g, const float* dy, const float* w, float* dx, float* ws, int64_t ws_elems);
 int launch_split_conv_wgrad(sn_ctx* ctx, const ConvGeom& g, const float* x, const float* dy, float* dw, float* ws, int64_t ws_elems);

@@ -1033,7 +1033,7 @@ int launch_conv_fwd(sn_ctx* ctx, const ConvGeom& g, const float* x, const float*
   }
   if (conv_ring_fwd_ok(g, x, w, e)) return launch_conv_ring_fwd(ctx, g, x, w, e);
   StdEpilogue ep{e};
-  if (split_conv_fwd_ok(g, x, w)) return launch_split_conv_fwd(ctx, g, x, w, e, ws, ws_elems);
+  if (!conv_prefers_float32_tiles(M, N, K, g.cin) && split_conv_fwd_ok(g, x, w)) return launch_split_conv_fwd(ctx, g, x, w, e, ws, ws_elems);
   ConvFwdA al{x, g, M};
   StridedLoader<false> bl{w, 1, (int64_t)g.cout, N};  // filter [kh,kw,cin,cout] is a row-major [K, cout] matrix
   return launch_any<false>(ctx, "conv2d_forward", M, N, K, al, bl, ep, ws, ws_elems);
@@ -1046,7 +1046,7 @@ int launch_conv_dgrad(sn_ctx* ctx, const ConvGeom& g, const float* dy, const flo
   e.ldo = g.cin;
   if (conv_ring_dgrad_ok(g, dy, w)) return launch_conv_ring_dgrad(ctx, g, dy, w, dx);
   StdEpilogue ep{e};
-  if (split_conv_dgrad_ok(g, dy, w)) return launch_split_conv_dgrad(ctx, g, dy, w, dx, ws, ws_elems);
+  if (!(g.sh == 1 && g.sw == 1 && conv_prefers_float32_tiles(M, N, K, g.cout)) && split_conv_dgrad_ok(g, dy, w)) return launch_split_conv_dgrad(ctx, g, dy, w, dx, ws, ws_elems);
   ConvDgradA al{dy, g, M};
   ConvDgradB bl{w, g};
   return launch_any<false>(ctx, "conv2d_input_gradient", M, N, K, al, bl, ep, ws, ws_elems);

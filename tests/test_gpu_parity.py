@@ -1379,9 +1379,8 @@ def test_simple_rnn_backward_launch_that_carries_the_weight_gradient(S, ctx, mon
     ("simple_rnn", 129, 2, 21, 3), ("simple_rnn", 192, 7, 35, 3), ("simple_rnn", 193, 10, 13, 3), ("simple_rnn", 256, 5, 50, 2),
     ("simple_rnn", 70, 4, 2065, 2), ("simple_rnn", 150, 3, 2050, 2), ("simple_rnn", 250, 2, 2049, 2)])
 def test_recurrent_layers_whose_recurrence_stays_in_one_workgroup(S, ctx, kind, units, features, batch, T):
-    """Every block count of the kernels (32 values of the recurrence each), the last one full and partial, both row counts of
-    a workgroup (4, and 16 from some 2000 rows on), rows that do not fill the last workgroup, products of fewer than four
-    values; a carried state at the start, the returned sequence feeding a second layer of 3 units (whose input gradient the
+    """Every block count of the kernels (32 values of the recurrence each), the last one full and partial, rows that do
+    not fill the last workgroup of four, more workgroups than the chip has CUs, products of fewer than four values; a carried state at the start, the returned sequence feeding a second layer of 3 units (whose input gradient the
     product over all steps delivers).  Bounds as for the one-launch kernels: float32 sums, or three times the oracle's own
     distance from float64."""
     first = {"lstm": (O.LSTM, S.LSTM), "simple_rnn": (O.SimpleRNN, S.SimpleRNN)}[kind]
@@ -2179,8 +2178,8 @@ def _affine_bounds(x, y, w1, b1, w2, b2):
     return run(*d, -1.0), run(*[np.abs(v) for v in d], 1.0)
 
 
-# edges of the 32- to 128-wide tiles and of the 32- and 64-long stages, rows that are no multiple of four values, a reduction
-# long enough for several splits, and a product large enough for 128 x 128 tiles
+# edges of the 32- to 64-wide tiles and of the 32- and 64-long stages, rows that are no multiple of four values, a reduction
+# long enough for several splits (every tile shape has its product below)
 @pytest.mark.parametrize("rows,features,hidden,outputs", [(4, 5, 6, 5), (31, 33, 63, 7), (64, 32, 64, 64), (65, 67, 129, 33), (128, 100, 36, 130),
                                                           (3, 257, 70, 31), (200, 1003, 97, 66), (700, 127, 515, 1026), (513, 2050, 260, 8)])
 def test_split_products_at_tile_edges(S, ctx, rows, features, hidden, outputs):
@@ -2472,3 +2471,58 @@ def test_split_convolutions_of_small_values(S, ctx, filters, channels, exponent)
         xb.free()
         yb.free()
     h.close()
+
+
+@pytest.mark.parametrize("channels,filters", [(8, 16), (8, 32), (10, 16), (24, 8)])
+@pytest.mark.parametrize("batch", [99, 100])
+def test_convolutions_of_many_positions_and_few_columns(S, ctx, channels, filters, batch):
+    """Both sides of the line between the split products and the float32 tiles (40000 positions, whole vectors of channels),
+    rows of 20 positions that a stage of 32 or 64 does not divide: forward, input and filter gradient against float64."""
+    rng = np.random.default_rng(channels + filters)
+    spec = [("conv", channels, (1, 1), (1, 1), "valid", "identity", False), ("conv", filters, (3, 3), (1, 1), "same", "identity", False), ("flatten",)]
+    h = Harness(S, ctx, spec, "mse", (20, 20, 1), batch)
+    names = [p for p, _, _ in h.cm.params]
+    shapes = {p: s for p, s, _ in h.cm.params}
+    x, w = rng.standard_normal((batch, 20, 20, 1)).astype(f32), [rng.standard_normal(shapes[n]).astype(f32) for n in names]
+    y = rng.standard_normal((batch, 400 * filters)).astype(f32)
+    h.rep.set_params(dict(zip(names, w)))
+    xb, yb = ctx.to_device(x), ctx.to_device(y)
+
+    def run(x, y, w1, w2, sign):
+        a = O.conv2d(x, w1)
+        p = O.conv2d(a, w2, padding=O.PAD_SAME)
+        dp = 2.0 * (p + sign * y.reshape(p.shape)) / y.size
+        da = O.conv2d_grad_input(a.shape, w2, dp, padding=O.PAD_SAME)
+        return {"out": p.reshape(y.shape), names[1]: O.conv2d_grad_filter(a, w2.shape, dp, padding=O.PAD_SAME), names[0]: O.conv2d_grad_filter(x, w1.shape, da)}
+    d = [v.astype(np.float64) for v in (x, y, *w)]
+    want, size = run(*d, -1.0), run(*[np.abs(v) for v in d], 1.0)
+    got = {"out": h.rep.forward(xb)}
+    h.rep.grad(xb, yb)
+    got.update(h.rep.get_grads())
+    # float32 sums of K products round at most K times; the positions' sums are split over at least 32 workgroups
+    steps = 9 * (channels + filters) + 400 * batch / 32 + 64
+    for name in got:
+        assert np.all(np.abs(got[name].reshape(want[name].shape) - want[name]) <= steps * 2.0 ** -24 * size[name]), name
+    h.close()
+    xb.free()
+    yb.free()
+
+
+# A product for each tile of the split kernels (host_checks' `choose` says which one it takes)
+TILE_SHAPES = {(128, 128, 32): (1000, 4096, 70), (128, 64, 32): (50000, 64, 30), (64, 64, 32): (1030, 2050, 37), (64, 64, 64): (515, 1026, 127),
+               (64, 32, 64): (33, 600, 70), (32, 64, 64): (30, 1000, 1000)}
+
+
+@pytest.mark.parametrize("tile", sorted(TILE_SHAPES))
+def test_every_split_tile(S, ctx, tile):
+    rows, hidden, features = TILE_SHAPES[tile]
+    rng = np.random.default_rng(sum(tile))
+    x, w, b = rng.standard_normal((rows, features)).astype(f32), rng.standard_normal((features, hidden)).astype(f32), rng.standard_normal(hidden).astype(f32)
+    h = Harness(S, ctx, [("dense", hidden, "identity")], "mse", (features,), rows)
+    h.rep.set_params({p: v for (p, _, _), v in zip(h.cm.params, (w, b))})
+    xb = ctx.to_device(x)
+    want = x.astype(np.float64) @ w.astype(np.float64) + b
+    size = np.abs(x).astype(np.float64) @ np.abs(w).astype(np.float64) + np.abs(b)
+    assert np.all(np.abs(h.rep.forward(xb) - want) <= (6.0 / 16.0 * features + 16.0) * 2.0 ** -24 * size)
+    h.close()
+    xb.free()

@@ -48,3 +48,29 @@ def test_a_sum_that_the_optimizer_cannot_take_is_priced_as_a_launch(ask):
     assert ask("defers", 432, 80, 0) == [0] and ask("defers", 1 << 15, 1 << 15, 1) == [0]
     cheap, dear = ask("choose", 27, 48, 6000, 3, 1), ask("choose", 27, 48, 6000, 3, 0)
     assert cheap[3] >= dear[3]
+
+
+def test_many_positions_with_few_columns_stay_off_the_split_kernels(ask):
+    for m, n, k, c, want in ((378450, 16, 72, 8, 1), (40000, 32, 216, 24, 1), (39999, 16, 72, 8, 0), (378450, 33, 72, 8, 0), (378450, 16, 90, 10, 0),
+                             (378450, 8, 288, 32, 0)):
+        assert ask("float32", m, n, k, c) == [want]
+
+
+def test_the_split_count_is_one_the_stages_reach(ask):
+    """Partial results are written by ceil(stages / per workgroup) splits and read by as many: the chosen count is that one,
+    and a long reduction onto one or two tiles fills the chip whatever its number of stages is."""
+    for m, n, k in ((72, 48, 31232), (72, 8, 32076), (432, 8, 8232), (288, 8, 118800), (30, 30, 65537), (700, 770, 1003), (5, 2000, 333)):
+        for deferred in (0, 1):
+            bm, bn, bk, splits = ask("choose", m, n, k, 3, deferred)
+            stages = -(-k // bk)
+            assert -(-stages // -(-stages // splits)) == splits
+            if k > 8000:
+                assert splits * -(-m // bm) * -(-n // bn) >= 200
+
+
+def test_every_tile_has_a_product_in_the_parity_tests(ask):
+    source = open(os.path.join(ROOT, "tests", "test_gpu_parity.py")).read()
+    shapes = eval(source[source.index("TILE_SHAPES = ") + 14:source.index("}", source.index("TILE_SHAPES = ")) + 1])
+    assert len(shapes) == 6
+    for tile, (rows, hidden, features) in shapes.items():
+        assert tuple(ask("choose", rows, hidden, features, 3, 0)[:3]) == tile
