@@ -1,8 +1,8 @@
 // GEMM-shaped products for gfx950 besides the split kernels (split_gemm.hpp), and the dispatch between them.
 //   - gemm_kernel: an LDS-tiled product on v_mfma_f32_32x32x2_f32 whose operand tiles are gathered value by value through
 //     small "loader" functors: whatever the split kernels cannot read (fewer than four values along an operand's
-//     contiguous index, strided input gradients, tensors beyond 2 GiB) and the recurrent products that run one time
-//     step per launch.  bf16 form (Dense, on request): operands are rounded while they are staged.
+//     contiguous index, strided input gradients, tensors beyond 2 GiB), convolutions of many positions onto few columns
+//     (conv_prefers_float32_tiles), and the recurrent products that run one time step per launch.  bf16 form (Dense, on request): operands are rounded while they are staged.
 //     Block = 256 threads = 4 wavefronts in a 2x2 arrangement; block tile BM x BN (64 or 128 each), K step 16.
 //   - small-output products with a long reduction, first-layer convolutions, Dense layers onto a few units.
 #include "split_launch.hpp"

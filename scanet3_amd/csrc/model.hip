@@ -569,10 +569,12 @@ static LstmWeights lstm_weights(sn_replica* r, const Op& op, float* base) {
 
 // Whether a recurrent layer runs on the kernels that keep a row's whole recurrence in one workgroup.  Any layer they fit does
 // that the one-launch kernels with a hand-over between workgroups (`handed`) do not take: those need unit counts that are
-// multiples of 16 and take one launch or more per step otherwise (LSTM 9 -> 100 -> 60 units, 130 rows, 50 steps: 3.76 ms a
-// step against 0.46).  Where both fit (500 rows, 64 steps, 32 features; the inputs' product included, us): LSTM forward 16
+// multiples of 16 and take one launch or more per step otherwise (LSTM 9 -> 100 -> 60 units, 130 rows, 50 steps: 3.80 ms a
+// step against 0.43).  Where both fit (500 rows, 64 steps, 32 features; the inputs' product included, us): LSTM forward 16
 // units 68 against 132, 64: 93 / 157, 96: 128 / 160, 128: 190 / 181; backward 16: 55 / 102, 64: 72 / 118, 128: 167 / 137;
-// simple cell, either direction, 64: 43 / 96, 128: 57 / 105.
+// simple cell, either direction, 64: 43 / 96, 128: 57 / 105.  Whole training steps of 32 time steps at 1024, 2048 and 4096 rows:
+// LSTM 16 units 90 / 103 / 137 against 145 / 153 / 181, 64: 155 / 217 / 401 against 185 / 243 / 388, 96: 212 / 380 / 717 against
+// 370 / 501 / 1131; simple cell 128: 123 / 176 / 323 against 151 / 230 / 407.
 constexpr int LSTM_LOCAL_UNITS = 96, RNN_LOCAL_UNITS = 128;
 static bool recurrent_local(const Op& op, int rows, int gates, bool handed) {
   if (!recurrent_local_fits(rows, op.T, op.F, op.H, gates)) return false;

@@ -1,5 +1,5 @@
-// The tiled matrix-core product behind every float32 Dense, Conv2D and recurrent GEMM (and, with one plane, the bf16 Dense
-// products whose shapes gemm_bf16.hip does not take).
+// The tiled matrix-core product behind most float32 Dense, Conv2D and recurrent input products (gemm_kernels.hip says what runs
+// elsewhere) and, with one plane, the bf16 Dense products whose shapes gemm_bf16.hip does not take.
 //
 //   C[M, N] = A[M, K] * B[K, N], float32 in, float32 accumulate, float32 out
 //
