@@ -8,7 +8,10 @@
 //
 // All of it is memory bound: every pass reads the activation once with 8 row-loads in flight per
 // lane; the per-channel reductions are cut into row slices so the grid covers the chip, and the
-// slices are added in slice order by one thread per channel (deterministic, no atomics).
+// slices are added in slice order by one thread per channel (deterministic, no atomics).  So what a pass
+// can be spared is what counts: mean and variance come out of one read, and where a 2 x 2 max pooling
+// follows, the normalised tensor and its gradient are never in memory (the pooling's windows are normalised as
+// they are compared, and their gradients are looked up where they are needed).
 #include "common.hpp"
 
 namespace sn {
@@ -67,111 +70,299 @@ __global__ __launch_bounds__(256) void bn_reduce_kernel(const float* __restrict_
   }
 }
 
-// Few channels (C/4 divides 256): the tensor is read as one stream of float4; a thread's float4 index moves in steps
-// of 256, so it stays on the same four channels and every wavefront load covers 1 KiB of consecutive memory.
-// A block owns `per4` consecutive float4 (a multiple of 256); threads with equal t % (C/4) meet in LDS.
-template <int MODE>
-__global__ __launch_bounds__(256) void bn_reduce_v4_kernel(const bn_f4* __restrict__ x, const bn_f4* __restrict__ dy,
-                                                            const float* __restrict__ mean, float* __restrict__ part0,
-                                                            float* __restrict__ part1, int64_t n4, int cols, int64_t per4) {
+// Whole vectors of channels (C % 4 == 0, C <= 1024): the tensor is read as one stream of float4.  The `active` threads of a block
+// are the largest multiple of C/4 up to 256 and a thread's float4 index moves in steps of them, so it stays on the same four
+// channels and a wavefront's load covers 1 KiB of consecutive memory.  A block owns `per4` consecutive float4 (a multiple of
+// `active`); threads with equal t % (C/4) meet in LDS.
+
+// Joins the values in LDS of the threads t, t + cg, t + 2 cg, ... of a block pairwise: f(to, from) folds one into the other, thread
+// t < cg ends with the whole.  (One thread adding 32 in a row waits for LDS 32 times: 2 us of such a launch.)
+template <class F>
+__device__ __forceinline__ void over_channel_peers(int t, int cg, int active, F f) {
+  const int peers = active / cg, j = t / cg;
+  int half = 1;
+  while (2 * half < peers) half *= 2;
+  for (; half > 0; half >>= 1) {
+    __syncthreads();
+    if (t < active && j < half && j + half < peers) f(t, t + half * cg);
+  }
+  __syncthreads();
+}
+
+// part0 = sum dy, part1 = sum dy * (x - mean)
+__global__ __launch_bounds__(256) void bn_grad_sums_v4_kernel(const bn_f4* __restrict__ x, const bn_f4* __restrict__ dy,
+                                                               const float* __restrict__ mean, float* __restrict__ part0,
+                                                               float* __restrict__ part1, int64_t n4, int cols, int active, int64_t per4) {
   __shared__ bn_f4 smem[2][256];
   const int t = threadIdx.x, cg = cols / 4, g = t % cg;
   const int64_t begin = (int64_t)blockIdx.x * per4;
   const int64_t end = begin + per4 < n4 ? begin + per4 : n4;
-  bn_f4 m = {0.f, 0.f, 0.f, 0.f};
-  if (MODE != BN_SUM) m = *(const bn_f4*)(mean + 4 * g);
+  const bn_f4 m = *(const bn_f4*)(mean + 4 * g);
   bn_f4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
-  int64_t i = begin + t;
-  for (; i + 7 * 256 < end; i += 8 * 256) {
+  int64_t i = t < active ? begin + t : end;
+  for (; i + 7 * active < end; i += 8 * active) {
     bn_f4 a[8], b[8];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) a[u] = __builtin_nontemporal_load(x + i + u * 256);
-    if (MODE == BN_GRAD) {
+    for (int u = 0; u < 8; ++u) a[u] = __builtin_nontemporal_load(x + i + u * active);
 #pragma unroll
-      for (int u = 0; u < 8; ++u) b[u] = __builtin_nontemporal_load(dy + i + u * 256);
-    }
+    for (int u = 0; u < 8; ++u) b[u] = __builtin_nontemporal_load(dy + i + u * active);
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      if (MODE == BN_SUM) s0 = s0 + a[u];
-      if (MODE == BN_SQDIFF) { const bn_f4 d = a[u] - m; s0 = s0 + d * d; }
-      if (MODE == BN_GRAD) { s0 = s0 + b[u]; s1 = s1 + b[u] * (a[u] - m); }
-    }
+    for (int u = 0; u < 8; ++u) { s0 = s0 + b[u]; s1 = s1 + b[u] * (a[u] - m); }
   }
-  for (; i < end; i += 256) {
-    const bn_f4 a = x[i];
-    if (MODE == BN_SUM) s0 = s0 + a;
-    if (MODE == BN_SQDIFF) { const bn_f4 d = a - m; s0 = s0 + d * d; }
-    if (MODE == BN_GRAD) { const bn_f4 b = dy[i]; s0 = s0 + b; s1 = s1 + b * (a - m); }
+  for (; i < end; i += active) {
+    const bn_f4 a = x[i], b = dy[i];
+    s0 = s0 + b;
+    s1 = s1 + b * (a - m);
   }
   smem[0][t] = s0;
-  if (MODE == BN_GRAD) smem[1][t] = s1;
-  __syncthreads();
+  smem[1][t] = s1;
+  over_channel_peers(t, cg, active, [&](int to, int from) {
+    smem[0][to] = smem[0][to] + smem[0][from];
+    smem[1][to] = smem[1][to] + smem[1][from];
+  });
   if (t < cg) {
-    bn_f4 r0 = smem[0][t], r1 = smem[1][t];
-    for (int j = t + cg; j < 256; j += cg) {
-      r0 = r0 + smem[0][j];
-      if (MODE == BN_GRAD) r1 = r1 + smem[1][j];
-    }
-    *(bn_f4*)(part0 + (int64_t)blockIdx.x * cols + 4 * t) = r0;
-    if (MODE == BN_GRAD) *(bn_f4*)(part1 + (int64_t)blockIdx.x * cols + 4 * t) = r1;
+    *(bn_f4*)(part0 + (int64_t)blockIdx.x * cols + 4 * t) = smem[0][t];
+    *(bn_f4*)(part1 + (int64_t)blockIdx.x * cols + 4 * t) = smem[1][t];
   }
 }
 
-// Sum of one channel's slices by 16 threads: a block is 16 channels x 16 slice lanes; lane j adds slices j, j+16, ...
-// (8 loads in flight), the 16 lane sums are added in lane order.  Every thread of the block must call it; the total is
-// returned to all of them.  (One thread per channel would walk up to 1024 slices one memory latency after another.)
-__device__ __forceinline__ float slices_total(const float* __restrict__ part, int slices, int cols, int c, float (*smem)[16]) {
-  const int cl = threadIdx.x & 15, sl = threadIdx.x >> 4;
-  float s = 0.f;
-  if (c < cols) {
-    int i = sl;
-    for (; i + 7 * 16 < slices; i += 8 * 16) {
-      float a[8];
+// The same sums where dy is the gradient of a 2 x 2 max pooling right above: it is zero but at the windows' recorded first
+// maxima, so the sums run over the pooling's output (n4 = its float4).  A window whose recorded place lies in the padding
+// (nothing inside it was above -inf) has no element to hand its gradient to.
+// [1000 x 26 x 26 x 32] with stride 2: 19 us for 113 MB; the pooling's backward pass and the sums over its 86 MB result took 29 + 29.
+struct PoolWindows {
+  int h, w, ho, wo, sh, sw, pt, pl;
+  FastDiv by_cg, by_wo, by_ho;
+};
+__global__ __launch_bounds__(256) void bn_pool_grad_sums_kernel(const float* __restrict__ x, const bn_f4* __restrict__ dy,
+                                                                 const uint32_t* __restrict__ arg, const float* __restrict__ mean,
+                                                                 float* __restrict__ part0, float* __restrict__ part1, uint32_t n4, int cols,
+                                                                 int active, uint32_t per4, PoolWindows p) {
+  __shared__ bn_f4 smem[2][256];
+  const int t = threadIdx.x, cg = cols / 4, g = t % cg;
+  const uint32_t begin = blockIdx.x * per4, end = begin + per4 < n4 ? begin + per4 : n4;
+  const bn_f4 m = *(const bn_f4*)(mean + 4 * g);
+  bn_f4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
+  constexpr int U = 2;  // windows in flight
+  for (uint32_t i0 = t < active ? begin + t : end; i0 < end; i0 += U * active) {
+    bn_f4 gv[U], xv[U][4];
+    uint32_t av[U];
+    bool in[U][4];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) a[u] = part[(int64_t)(i + 16 * u) * cols + c];
+    for (int u = 0; u < U; ++u) {
+      const bool on = i0 + u * active < end;
+      const uint32_t i = on ? i0 + u * active : i0;
+      const uint32_t win = div_by(i, p.by_cg), row = div_by(win, p.by_wo), b = div_by(row, p.by_ho);
+      const int ix0 = (int)(win - row * (uint32_t)p.wo) * p.sw - p.pl, iy0 = (int)(row - b * (uint32_t)p.ho) * p.sh - p.pt;
+      gv[u] = dy[i];
+      av[u] = arg[i];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) s += a[u];
+      for (int k = 0; k < 4; ++k) {
+        const int iy = iy0 + (k >> 1), ix = ix0 + (k & 1);
+        in[u][k] = on && (unsigned)iy < (unsigned)p.h && (unsigned)ix < (unsigned)p.w;
+        xv[u][k] = *(const bn_f4*)(x + (in[u][k] ? ((b * p.h + iy) * p.w + ix) * cols + 4 * g : 0u));
+      }
     }
-    for (; i < slices; i += 16) s += part[(int64_t)i * cols + c];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const uint32_t at = (av[u] >> (8 * e)) & 255u;
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          if (in[u][k] && at == (uint32_t)k) { s0[e] += gv[u][e]; s1[e] += gv[u][e] * (xv[u][k][e] - m[e]); }
+      }
   }
+  smem[0][t] = s0;
+  smem[1][t] = s1;
+  over_channel_peers(t, cg, active, [&](int to, int from) {
+    smem[0][to] = smem[0][to] + smem[0][from];
+    smem[1][to] = smem[1][to] + smem[1][from];
+  });
+  if (t < cg) {
+    *(bn_f4*)(part0 + (int64_t)blockIdx.x * cols + 4 * t) = smem[0][t];
+    *(bn_f4*)(part1 + (int64_t)blockIdx.x * cols + 4 * t) = smem[1][t];
+  }
+}
+
+// Mean and sum of squared deviations of a block's rows in one read: a thread takes eight values of a channel at a time, forms their own
+// mean and deviations in registers and joins them to what it has by the pairwise update of Chan, Golub and LeVeque (1983)
+//   mean += d w, M2 += M2_8 + d^2 n w   with d = mean_8 - mean, w = 8 / (n + 8);
+// no large squares are subtracted anywhere, so the variance is as good as the two-read form's.
+// [676000 x 32]: 17 us, where a read for the mean, its finishing launch and a read for the variance took 15 + 5 + 15.
+__global__ __launch_bounds__(256) void bn_stats_v4_kernel(const bn_f4* __restrict__ x, float* __restrict__ part_mean, float* __restrict__ part_m2,
+                                                           int64_t n4, int cols, int active, int64_t per4) {
+  __shared__ bn_f4 smem[2][256];
+  __shared__ float count[256];
+  const int t = threadIdx.x, cg = cols / 4;
+  const int64_t begin = (int64_t)blockIdx.x * per4;
+  const int64_t end = begin + per4 < n4 ? begin + per4 : n4;
+  const bn_f4 zero = {0.f, 0.f, 0.f, 0.f};
+  bn_f4 mean = zero, m2 = zero;
+  float n = 0.f;
+  auto join = [&](const bn_f4& m, const bn_f4& q, float k) {  // k values of mean m and squared deviations q
+    const float w = k / (n + k);
+    if (n > 0.f) {
+      const bn_f4 d = m - mean;
+      mean = mean + d * w;
+      m2 = m2 + (q + d * d * (n * w));
+    } else {
+      mean = m;
+      m2 = q;
+    }
+    n += k;
+  };
+  int64_t i = t < active ? begin + t : end;
+  for (; i + 7 * active < end; i += 8 * active) {
+    bn_f4 a[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) a[u] = __builtin_nontemporal_load(x + i + u * active);
+    const bn_f4 m = (((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]))) * 0.125f;
+    bn_f4 q = zero;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) { const bn_f4 d = a[u] - m; q = q + d * d; }
+    join(m, q, 8.0f);
+  }
+  if (i < end) {  // what is left of the block, one to seven values, requested together as well
+    const int left = (int)((end - i + active - 1) / active);
+    bn_f4 a[7];
+#pragma unroll
+    for (int u = 0; u < 7; ++u) a[u] = __builtin_nontemporal_load(x + i + (u < left ? u * active : 0));
+    bn_f4 m = zero, q = zero;
+#pragma unroll
+    for (int u = 0; u < 7; ++u) m = u < left ? m + a[u] : m;
+    m = m / (float)left;
+#pragma unroll
+    for (int u = 0; u < 7; ++u) { const bn_f4 d = a[u] - m; q = u < left ? q + d * d : q; }
+    join(m, q, (float)left);
+  }
+  smem[0][t] = mean;
+  smem[1][t] = m2;
+  count[t] = n;
+  over_channel_peers(t, cg, active, [&](int to, int from) {
+    const float na = count[to], nb = count[from];
+    if (nb == 0.f) return;
+    if (na == 0.f) {
+      smem[0][to] = smem[0][from];
+      smem[1][to] = smem[1][from];
+    } else {
+      const float w = nb / (na + nb);
+      const bn_f4 d = smem[0][from] - smem[0][to];
+      smem[0][to] = smem[0][to] + d * w;
+      smem[1][to] = smem[1][to] + (smem[1][from] + d * d * (na * w));
+    }
+    count[to] = na + nb;
+  });
+  if (t < cg) {
+    *(bn_f4*)(part_mean + (int64_t)blockIdx.x * cols + 4 * t) = smem[0][t];
+    *(bn_f4*)(part_m2 + (int64_t)blockIdx.x * cols + 4 * t) = smem[1][t];
+  }
+}
+
+// Sums over one channel's slices by 64 threads: a block is 4 channels x 64 slice lanes; lane j takes slices j, j+64, ..., 16 of them
+// requested together (nearly always all there are), the lanes' sums meet in a fixed tree.  Every thread of the block must
+// call these.  (One thread per channel would walk up to 1024 slices one memory latency after another; 16 threads a channel
+// took 8.1 us for 1024 slices of two sums, 64 with all their loads at once take 4.7.)
+constexpr int FINISH_CHANNELS = 4, FINISH_LOADS = 16;
+// f(slice, place in the slices' arrays, whether there is such a slice): places that do not exist repeat the last slice
+template <class F>
+__device__ __forceinline__ void for_slices(int first, int slices, int cols, int c, F f) {
+#pragma unroll
+  for (int u = 0; u < FINISH_LOADS; ++u) {
+    const int i = first + 64 * u, at = min(i, slices - 1);
+    f(u, (int64_t)at * cols + min(c, cols - 1), i < slices);
+  }
+}
+__device__ __forceinline__ float over_slice_lanes(float s, float (*smem)[FINISH_CHANNELS]) {
+#pragma unroll
+  for (int d = 4; d < 64; d <<= 1) s += __shfl_xor(s, d);
   __syncthreads();  // a previous call's readers are done with smem
-  smem[sl][cl] = s;
+  if ((threadIdx.x & 63) < 4) smem[threadIdx.x >> 6][threadIdx.x & 3] = s;
   __syncthreads();
-  float total = smem[0][cl];
-#pragma unroll
-  for (int j = 1; j < 16; ++j) total += smem[j][cl];
-  return total;
+  const int cl = threadIdx.x & 3;
+  return (smem[0][cl] + smem[1][cl]) + (smem[2][cl] + smem[3][cl]);
+}
+__device__ __forceinline__ float slices_total(const float* __restrict__ part, int slices, int cols, int c, float (*smem)[FINISH_CHANNELS]) {
+  float s = 0.f;
+  for (int i = threadIdx.x >> 2; i < slices; i += 64 * FINISH_LOADS) {
+    float a[FINISH_LOADS];
+    for_slices(i, slices, cols, c, [&](int u, int64_t at, bool) { a[u] = part[at]; });
+    for_slices(i, slices, cols, c, [&](int u, int64_t, bool in) { s += in ? a[u] : 0.f; });
+  }
+  return over_slice_lanes(s, smem);
 }
 
-// Finishing kernels: block = 16 channels x 16 slice lanes, grid = ceil(C/16).
+// Finishing kernels: grid = ceil(C / FINISH_CHANNELS).
 __global__ __launch_bounds__(256) void bn_mean_kernel(const float* __restrict__ part, int slices, int cols, float n, float* __restrict__ mean) {
-  __shared__ float smem[16][16];
-  const int c = blockIdx.x * 16 + (threadIdx.x & 15);
+  __shared__ float smem[4][FINISH_CHANNELS];
+  const int c = blockIdx.x * FINISH_CHANNELS + (threadIdx.x & (FINISH_CHANNELS - 1));
   const float total = slices_total(part, slices, cols, c, smem);
-  if (threadIdx.x < 16 && c < cols) mean[c] = total / n;
+  if (threadIdx.x < FINISH_CHANNELS && c < cols) mean[c] = total / n;
 }
 
-// var from the slices (training) or from the moving variance (part == null), then r = 1/sqrt(var+eps), inv = r*gamma
-__global__ __launch_bounds__(256) void bn_scale_kernel(const float* __restrict__ part, int slices, int cols, float n, float eps,
-                                                        const float* __restrict__ gamma, const float* __restrict__ moving_mean,
-                                                        const float* __restrict__ moving_var, float* __restrict__ mean,
-                                                        float* __restrict__ var, float* __restrict__ r, float* __restrict__ inv) {
-  __shared__ float smem[16][16];
-  const int c = blockIdx.x * 16 + (threadIdx.x & 15);
+// What follows from a channel's statistics: r = 1/sqrt(var+eps), inv = r*gamma and, under the fused wiring, the statistics the
+// reference hands to the gradient op: "mean" = the unbiased variance, "variance" = the mean.
+struct BnScale {
+  const float* gamma;
+  float* mean;
+  float* var;
+  float* r;
+  float* inv;
+  float eps, unbias;
+  float* g_mean;  // null: not the fused wiring
+  float* g_r;
+  float* g_inv;
+};
+__device__ __forceinline__ void bn_finish_channel(const BnScale& a, int c, float mean, float var) {
+  a.mean[c] = mean;
+  a.var[c] = var;
+  const float rr = 1.0f / sqrtf(var + a.eps);
+  a.r[c] = rr;
+  a.inv[c] = rr * a.gamma[c];
+  if (a.g_mean) {
+    a.g_mean[c] = var * a.unbias;
+    const float gr = 1.0f / sqrtf(mean + a.eps);   // NaN for a channel whose mean is below -epsilon, as in the reference
+    a.g_r[c] = gr;
+    a.g_inv[c] = gr * a.gamma[c];
+  }
+}
+BnScale bn_scale_of(const BatchNormArgs& a, int64_t rows, bool wiring) {
+  return BnScale{a.gamma, a.mean, a.var, a.r, a.inv, a.epsilon, (float)rows / (float)(rows > 1 ? rows - 1 : 1), wiring ? a.g_mean : nullptr, a.g_r, a.g_inv};
+}
+
+// var from the slices' squared deviations (training; the mean is known) or both from the moving statistics (part == null)
+__global__ __launch_bounds__(256) void bn_scale_kernel(const float* __restrict__ part, int slices, int cols, float n,
+                                                        const float* __restrict__ moving_mean, const float* __restrict__ moving_var, BnScale a) {
+  __shared__ float smem[4][FINISH_CHANNELS];
+  const int c = blockIdx.x * FINISH_CHANNELS + (threadIdx.x & (FINISH_CHANNELS - 1));
   float total = 0.f;
   if (part) total = slices_total(part, slices, cols, c, smem);  // uniform over the block
-  if (threadIdx.x >= 16 || c >= cols) return;
-  float v;
-  if (part) {
-    v = total / n;
-  } else {
-    v = moving_var[c];
-    mean[c] = moving_mean[c];
+  if (threadIdx.x >= FINISH_CHANNELS || c >= cols) return;
+  if (part) bn_finish_channel(a, c, a.mean[c], total / n);
+  else bn_finish_channel(a, c, moving_mean[c], moving_var[c]);
+}
+
+// Joins bn_stats_v4_kernel's slices of `whole` rows each (the last one: `last`)
+__global__ __launch_bounds__(256) void bn_moments_kernel(const float* __restrict__ part_mean, const float* __restrict__ part_m2, int slices, int cols,
+                                                          float whole, float last, float n, BnScale a) {
+  __shared__ float smem[4][FINISH_CHANNELS];
+  const int c = blockIdx.x * FINISH_CHANNELS + (threadIdx.x & (FINISH_CHANNELS - 1));
+  float pm[FINISH_LOADS], pq[FINISH_LOADS], s = 0.f, q = 0.f;
+  const int first = threadIdx.x >> 2;
+  for (int i = first; i < slices; i += 64 * FINISH_LOADS) {
+    for_slices(i, slices, cols, c, [&](int u, int64_t at, bool) { pm[u] = part_mean[at]; pq[u] = part_m2[at]; });
+    for_slices(i, slices, cols, c, [&](int u, int64_t, bool in) { s += in ? pm[u] * (i + 64 * u + 1 < slices ? whole : last) : 0.f; });
   }
-  var[c] = v;
-  const float rr = 1.0f / sqrtf(v + eps);
-  r[c] = rr;
-  inv[c] = rr * gamma[c];
+  const float mean = over_slice_lanes(s, smem) / n;
+  for (int i = first; i < slices; i += 64 * FINISH_LOADS) {
+    if (slices > 64 * FINISH_LOADS) for_slices(i, slices, cols, c, [&](int u, int64_t at, bool) { pm[u] = part_mean[at]; pq[u] = part_m2[at]; });
+    for_slices(i, slices, cols, c, [&](int u, int64_t, bool in) {
+      const float d = pm[u] - mean;
+      q += in ? pq[u] + d * d * (i + 64 * u + 1 < slices ? whole : last) : 0.f;
+    });
+  }
+  const float m2 = over_slice_lanes(q, smem);
+  if (threadIdx.x < FINISH_CHANNELS && c < cols) bn_finish_channel(a, c, mean, m2 / n);
 }
 
 template <bool V4>
@@ -201,28 +392,53 @@ __global__ __launch_bounds__(256) void bn_apply_kernel(const float* __restrict__
   }
 }
 
-// The statistics the reference's wiring hands to the fused gradient op: "mean" = the unbiased variance, "variance" = the mean.
-__global__ __launch_bounds__(256) void bn_fused_wiring_kernel(const float* __restrict__ mean, const float* __restrict__ var,
-                                                               const float* __restrict__ gamma, float unbias, float eps,
-                                                               float* __restrict__ g_mean, float* __restrict__ g_r,
-                                                               float* __restrict__ g_inv, int cols) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= cols) return;
-  g_mean[c] = var[c] * unbias;
-  const float rr = 1.0f / sqrtf(mean[c] + eps);   // NaN for a channel whose mean is below -epsilon, as in the reference
-  g_r[c] = rr;
-  g_inv[c] = rr * gamma[c];
+// Normalisation and a 2 x 2 max pooling of the result in one pass: a thread normalises the four cells of a window (four channels)
+// as bn_apply_kernel does and compares them as pool2x2_fwd_kernel (elementwise_kernels.hip) does; what lies between is not stored.
+// [1000 x 26 x 26 x 32], stride 2: 24 us; the two passes took 28.7 + 23.6.
+__global__ __launch_bounds__(256) void bn_pool2x2_fwd_kernel(const float* __restrict__ x, const float* __restrict__ mean,
+                                                              const float* __restrict__ inv, const float* __restrict__ beta, float* __restrict__ y,
+                                                              uint8_t* __restrict__ arg, uint32_t total, int cols, int centred, PoolWindows p) {
+  const uint32_t cg = (uint32_t)cols / 4, stride = gridDim.x * blockDim.x;
+  const uint32_t block = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);  // every XCD takes a contiguous run (the grid is a multiple of 8)
+  for (uint32_t i = block * blockDim.x + threadIdx.x; i < total; i += stride) {
+    const uint32_t win = div_by(i, p.by_cg), ch = (i - win * cg) * 4;
+    const uint32_t row = div_by(win, p.by_wo), b = div_by(row, p.by_ho);
+    const int ix0 = (int)(win - row * (uint32_t)p.wo) * p.sw - p.pl, iy0 = (int)(row - b * (uint32_t)p.ho) * p.sh - p.pt;
+    const bn_f4 mv = *(const bn_f4*)(mean + ch), iv = *(const bn_f4*)(inv + ch), bv = *(const bn_f4*)(beta + ch);
+    bn_f4 xv[4];
+    bool in[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int iy = iy0 + (k >> 1), ix = ix0 + (k & 1);
+      in[k] = (unsigned)iy < (unsigned)p.h && (unsigned)ix < (unsigned)p.w;
+      xv[k] = *(const bn_f4*)(x + (in[k] ? ((b * p.h + iy) * p.w + ix) * cols + ch : 0u));
+    }
+    bn_f4 best = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+    uint32_t at = 0u;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      uint32_t place = 0u;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const float v = centred ? (xv[k][e] - mv[e]) * iv[e] + bv[e] : (xv[k][e] * iv[e] - mv[e] * iv[e]) + bv[e];
+        if (in[k] && v > best[e]) { best[e] = v; place = (uint32_t)k; }
+      }
+      at |= place << (8 * e);
+    }
+    *(bn_f4*)(y + i * 4) = best;
+    *(uint32_t*)(arg + i * 4) = at;
+  }
 }
 
 // d beta = S1, d gamma = S2 * r; k1 = S1/n, k2 = r*r*S2/n for the input gradient
 __global__ __launch_bounds__(256) void bn_grad_finish_kernel(const float* __restrict__ part0, const float* __restrict__ part1, int slices,
                                                               int cols, float n, const float* __restrict__ r, float* __restrict__ dbeta,
                                                               float* __restrict__ dgamma, float* __restrict__ k1, float* __restrict__ k2) {
-  __shared__ float smem[16][16];
-  const int c = blockIdx.x * 16 + (threadIdx.x & 15);
+  __shared__ float smem[4][FINISH_CHANNELS];
+  const int c = blockIdx.x * FINISH_CHANNELS + (threadIdx.x & (FINISH_CHANNELS - 1));
   const float s1 = slices_total(part0, slices, cols, c, smem);
   const float s2 = slices_total(part1, slices, cols, c, smem);
-  if (threadIdx.x >= 16 || c >= cols) return;
+  if (threadIdx.x >= FINISH_CHANNELS || c >= cols) return;
   const float rr = r[c];
   dbeta[c] = s1;
   dgamma[c] = s2 * rr;
@@ -294,40 +510,41 @@ int slices_for(const sn_ctx* ctx, int64_t rows, int cols) {
   return s < 1 ? 1 : (int)s;
 }
 
-// the float4-stream reduction: C/4 divides 256 and enough data for more than one block
-bool stream_form(int64_t rows, int cols) { return cols % 4 == 0 && cols <= 1024 && 256 % (cols / 4) == 0 && rows * cols >= 4 * 8 * 256; }
-int stream_slices(const sn_ctx* ctx, int64_t n4) {
-  int64_t s = ceil_div(n4, (int64_t)8 * 256);  // at least one full trip of 8 loads per thread
-  const int64_t cap = (int64_t)ctx->compute_units * 4;
-  if (s > cap) s = cap;
-  return s < 1 ? 1 : (int)s;
+// the float4-stream reductions: whole vectors of channels and enough data for more than one block
+bool stream_form(int64_t rows, int cols) { return cols % 4 == 0 && cols <= 1024 && rows * cols >= 4 * 8 * 256; }
+struct Stream {
+  int active, slices;
+  int64_t n4, per4;
+};
+Stream stream_of(const sn_ctx* ctx, int64_t rows, int cols) {
+  Stream st;
+  const int cg = cols / 4;
+  st.active = 256 / cg * cg;
+  st.n4 = rows * cols / 4;
+  int64_t s = ceil_div(st.n4, (int64_t)8 * 256);  // at least one full trip of 8 loads per thread
+  s = std::min<int64_t>(s, (int64_t)ctx->compute_units * 4);
+  if (256 % cg != 0) s = std::min<int64_t>(s, slices_for(ctx, rows, cols));  // (the workspace such a layer has always asked for)
+  s = std::max<int64_t>(s, 1);
+  st.per4 = ceil_div(ceil_div(st.n4, s), (int64_t)st.active) * st.active;
+  st.slices = (int)ceil_div(st.n4, st.per4);  // every slice has rows
+  return st;
 }
-
-// One reduction pass in whichever form fits; returns the number of slices written to part0 (and part1).
-template <int MODE>
-int reduce_pass(sn_ctx* ctx, const float* x, const float* dy, const float* mean, float* part0, int64_t part1_offset, int64_t rows,
-                int cols, int* slices_out) {
-  const bool aligned = ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(dy) | reinterpret_cast<uintptr_t>(part0)) & 15u) == 0;
-  if (stream_form(rows, cols) && aligned && part1_offset % 4 == 0) {
-    const int64_t n4 = rows * cols / 4;
-    const int s = stream_slices(ctx, n4);
-    const int64_t per4 = align_up(ceil_div(n4, (int64_t)s), 256);
-    hipLaunchKernelGGL((bn_reduce_v4_kernel<MODE>), dim3((unsigned)s), dim3(256), 0, ctx->stream, (const bn_f4*)x, (const bn_f4*)dy, mean,
-                       part0, part0 + part1_offset, n4, cols, per4);
-    *slices_out = s;
-  } else {
-    const int s = slices_for(ctx, rows, cols);
-    hipLaunchKernelGGL((bn_reduce_kernel<MODE>), dim3((unsigned)ceil_div((int64_t)cols, (int64_t)64), (unsigned)s), dim3(256), 0,
-                       ctx->stream, x, dy, mean, part0, part0 + part1_offset, rows, cols, ceil_div(rows, (int64_t)s));
-    *slices_out = s;
-  }
-  SN_HIP(hipGetLastError());
-  return SN_OK;
-}
-
 int max_slices(const sn_ctx* ctx, int64_t rows, int cols) {
   int s = slices_for(ctx, rows, cols);
-  if (stream_form(rows, cols)) s = std::max(s, stream_slices(ctx, rows * cols / 4));
+  if (stream_form(rows, cols)) s = std::max(s, stream_of(ctx, rows, cols).slices);
+  return s;
+}
+bool stream_ok(int64_t rows, int cols, const void* x, const void* dy, const void* part0, int64_t part1_offset) {
+  return stream_form(rows, cols) && part1_offset % 4 == 0 &&
+         ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(dy) | reinterpret_cast<uintptr_t>(part0)) & 15u) == 0;
+}
+
+// One row-walking reduction pass; returns the number of slices written to part0 (and part1).
+template <int MODE>
+int reduce_rows(sn_ctx* ctx, const float* x, const float* dy, const float* mean, float* part0, float* part1, int64_t rows, int cols) {
+  const int s = slices_for(ctx, rows, cols);
+  hipLaunchKernelGGL((bn_reduce_kernel<MODE>), dim3((unsigned)ceil_div((int64_t)cols, (int64_t)64), (unsigned)s), dim3(256), 0, ctx->stream, x, dy,
+                     mean, part0, part1, rows, cols, ceil_div(rows, (int64_t)s));
   return s;
 }
 
@@ -342,37 +559,47 @@ bool vec4_ok(int cols, std::initializer_list<const void*> ptrs) {
 
 int64_t batchnorm_workspace_elems(const sn_ctx* ctx, int64_t rows, int cols) { return (int64_t)2 * max_slices(ctx, rows, cols) * cols; }
 
+// mean, var and what follows from them (BnScale)
+static int batchnorm_statistics(sn_ctx* ctx, const float* x, int64_t rows, int cols, const BatchNormArgs& a, bool training, float* ws,
+                                int64_t ws_elems) {
+  SN_REQUIRE(rows * cols <= (int64_t)INT32_MAX * 4, "batch norm over %lld elements exceeds one launch", (long long)(rows * cols));
+  const int cb = (int)ceil_div((int64_t)cols, (int64_t)FINISH_CHANNELS);
+  if (!training) {
+    LaunchScope scope(ctx, "batchnorm_frozen_scale");
+    hipLaunchKernelGGL(bn_scale_kernel, dim3(cb), dim3(256), 0, ctx->stream, (const float*)nullptr, 0, cols, 1.0f, a.moving_mean, a.moving_var,
+                       bn_scale_of(a, rows, false));
+    SN_HIP(hipGetLastError());
+    return SN_OK;
+  }
+  const int64_t half = (int64_t)max_slices(ctx, rows, cols) * cols;
+  const BnScale scale = bn_scale_of(a, rows, a.fused_wiring);
+  SN_REQUIRE(half <= ws_elems, "batch norm needs %lld workspace elements, %lld given", (long long)half, (long long)ws_elems);
+  if (2 * half <= ws_elems && stream_ok(rows, cols, x, nullptr, ws, half)) {
+    const Stream st = stream_of(ctx, rows, cols);
+    LaunchScope scope(ctx, "batchnorm_mean_and_variance");
+    hipLaunchKernelGGL(bn_stats_v4_kernel, dim3((unsigned)st.slices), dim3(256), 0, ctx->stream, (const bn_f4*)x, ws, ws + half, st.n4, cols, st.active,
+                       st.per4);
+    hipLaunchKernelGGL(bn_moments_kernel, dim3(cb), dim3(256), 0, ctx->stream, (const float*)ws, (const float*)(ws + half), st.slices, cols,
+                       (float)(st.per4 / (cols / 4)), (float)((st.n4 - (st.slices - 1) * st.per4) / (cols / 4)), (float)rows, scale);
+  } else {
+    {
+      LaunchScope scope(ctx, "batchnorm_mean");
+      const int s = reduce_rows<BN_SUM>(ctx, x, nullptr, nullptr, ws, nullptr, rows, cols);
+      hipLaunchKernelGGL(bn_mean_kernel, dim3(cb), dim3(256), 0, ctx->stream, (const float*)ws, s, cols, (float)rows, a.mean);
+    }
+    LaunchScope scope(ctx, "batchnorm_variance");
+    const int s = reduce_rows<BN_SQDIFF>(ctx, x, nullptr, a.mean, ws, nullptr, rows, cols);
+    hipLaunchKernelGGL(bn_scale_kernel, dim3(cb), dim3(256), 0, ctx->stream, (const float*)ws, s, cols, (float)rows, (const float*)nullptr,
+                       (const float*)nullptr, scale);
+  }
+  SN_HIP(hipGetLastError());
+  return SN_OK;
+}
+
 int launch_batchnorm_fwd(sn_ctx* ctx, const float* x, float* y, int64_t rows, int cols, const BatchNormArgs& a, bool training, float* ws,
                          int64_t ws_elems) {
   if (rows <= 0 || cols <= 0) return SN_OK;
-  SN_REQUIRE(rows * cols <= (int64_t)INT32_MAX * 4, "batch norm over %lld elements exceeds one launch", (long long)(rows * cols));
-  const int cb = (int)ceil_div((int64_t)cols, (int64_t)16);  // finishing kernels: 16 channels per block
-  if (training) {
-    const int64_t need = (int64_t)max_slices(ctx, rows, cols) * cols;
-    SN_REQUIRE(need <= ws_elems, "batch norm needs %lld workspace elements, %lld given", (long long)need, (long long)ws_elems);
-    int s = 0;
-    {
-      LaunchScope scope(ctx, "batchnorm_mean");
-      SN_TRY(reduce_pass<BN_SUM>(ctx, x, nullptr, nullptr, ws, 0, rows, cols, &s));
-      hipLaunchKernelGGL(bn_mean_kernel, dim3(cb), dim3(256), 0, ctx->stream, (const float*)ws, s, cols, (float)rows, a.mean);
-    }
-    {
-      LaunchScope scope(ctx, "batchnorm_variance");
-      SN_TRY(reduce_pass<BN_SQDIFF>(ctx, x, nullptr, a.mean, ws, 0, rows, cols, &s));
-      hipLaunchKernelGGL(bn_scale_kernel, dim3(cb), dim3(256), 0, ctx->stream, (const float*)ws, s, cols, (float)rows, a.epsilon, a.gamma,
-                         (const float*)nullptr, (const float*)nullptr, a.mean, a.var, a.r, a.inv);
-    }
-    if (a.fused_wiring) {
-      LaunchScope scope(ctx, "batchnorm_fused_wiring");
-      const float unbias = (float)rows / (float)(rows > 1 ? rows - 1 : 1);
-      hipLaunchKernelGGL(bn_fused_wiring_kernel, dim3((unsigned)ceil_div((int64_t)cols, (int64_t)256)), dim3(256), 0, ctx->stream,
-                         (const float*)a.mean, (const float*)a.var, a.gamma, unbias, a.epsilon, a.g_mean, a.g_r, a.g_inv, cols);
-    }
-  } else {
-    LaunchScope scope(ctx, "batchnorm_frozen_scale");
-    hipLaunchKernelGGL(bn_scale_kernel, dim3(cb), dim3(256), 0, ctx->stream, (const float*)nullptr, 0, cols, 1.0f, a.epsilon, a.gamma,
-                       a.moving_mean, a.moving_var, a.mean, a.var, a.r, a.inv);
-  }
+  SN_TRY(batchnorm_statistics(ctx, x, rows, cols, a, training, ws, ws_elems));
   const int64_t n = rows * cols;
   LaunchScope scope(ctx, "batchnorm_apply");
   if (vec4_ok(cols, {x, y, a.mean, a.inv, a.beta}))
@@ -385,22 +612,73 @@ int launch_batchnorm_fwd(sn_ctx* ctx, const float* x, float* y, int64_t rows, in
   return SN_OK;
 }
 
+static PoolWindows pool_windows(const PoolGeom& g) {
+  return PoolWindows{g.h, g.w, g.ho, g.wo, g.sh, g.sw, g.pt, g.pl, fast_div((uint32_t)(g.c / 4)), fast_div((uint32_t)g.wo), fast_div((uint32_t)g.ho)};
+}
+
+// 2 x 2 maxima of whole vectors of channels with 32-bit element indices: what the pooling's own kernel for such windows takes
+bool batchnorm_pool_ok(const PoolGeom& g, const BatchNormArgs& a, const float* x, const float* y, const uint8_t* arg) {
+  return g.kh == 2 && g.kw == 2 && g.n > 0 && g.c <= 1024 && (int64_t)g.n * g.h * g.w * g.c < (1ll << 31) && (int64_t)g.n * g.ho * g.wo * g.c < (1ll << 31) &&
+         (int64_t)g.n * g.ho * g.wo * g.c > 0 && vec4_ok(g.c, {x, y, a.mean, a.inv, a.g_mean, a.g_inv, a.k1, a.k2, a.beta}) &&
+         (reinterpret_cast<uintptr_t>(arg) & 15u) == 0;
+}
+
+int launch_batchnorm_pool_fwd(sn_ctx* ctx, const float* x, float* y, uint8_t* arg, const PoolGeom& g, const BatchNormArgs& a, bool training, float* ws,
+                              int64_t ws_elems) {
+  SN_TRY(batchnorm_statistics(ctx, x, (int64_t)g.n * g.h * g.w, g.c, a, training, ws, ws_elems));
+  const int64_t total = (int64_t)g.n * g.ho * g.wo * g.c / 4;
+  LaunchScope scope(ctx, "batchnorm_apply_and_maxpool");
+  hipLaunchKernelGGL(bn_pool2x2_fwd_kernel, dim3((grid_for(ctx, total, 256) + 7u) & ~7u), dim3(256), 0, ctx->stream, x, (const float*)a.mean,
+                     (const float*)a.inv, a.beta, y, arg, (uint32_t)total, g.c, a.fused_wiring ? 1 : 0, pool_windows(g));
+  SN_HIP(hipGetLastError());
+  return SN_OK;
+}
+
+// d beta, d gamma, k1, k2 from the slices of the two gradient sums
+static void grad_finish(sn_ctx* ctx, const float* part0, const float* part1, int slices, int64_t rows, int cols, const BatchNormArgs& a, float* dbeta,
+                        float* dgamma) {
+  hipLaunchKernelGGL(bn_grad_finish_kernel, dim3((unsigned)ceil_div((int64_t)cols, (int64_t)FINISH_CHANNELS)), dim3(256), 0, ctx->stream, part0, part1, slices, cols,
+                     (float)rows, a.fused_wiring ? (const float*)a.g_r : (const float*)a.r, dbeta, dgamma, a.k1, a.k2);
+}
+
+int launch_batchnorm_pool_bwd(sn_ctx* ctx, const float* x, const float* dy, const uint8_t* arg, const PoolGeom& g, const BatchNormArgs& a, float* dbeta,
+                              float* dgamma, float* ws, int64_t ws_elems) {
+  const int64_t rows = (int64_t)g.n * g.h * g.w;
+  const int64_t half = (int64_t)max_slices(ctx, rows, g.c) * g.c;
+  SN_REQUIRE(2 * half <= ws_elems, "batch norm gradient needs %lld workspace elements, %lld given", (long long)(2 * half), (long long)ws_elems);
+  const int cg = g.c / 4, active = 256 / cg * cg;
+  const int64_t n4 = (int64_t)g.n * g.ho * g.wo * cg;
+  const int64_t wanted = std::min<int64_t>(ceil_div(n4, (int64_t)4 * active), max_slices(ctx, rows, g.c));
+  const int64_t per4 = ceil_div(ceil_div(n4, wanted), (int64_t)active) * active;
+  const int slices = (int)ceil_div(n4, per4);
+  LaunchScope scope(ctx, "batchnorm_gradient_sums_from_maxpool");
+  hipLaunchKernelGGL(bn_pool_grad_sums_kernel, dim3((unsigned)slices), dim3(256), 0, ctx->stream, x, (const bn_f4*)dy, (const uint32_t*)arg,
+                     a.fused_wiring ? (const float*)a.g_mean : (const float*)a.mean, ws, ws + half, (uint32_t)n4, g.c, active, (uint32_t)per4, pool_windows(g));
+  grad_finish(ctx, ws, ws + half, slices, rows, g.c, a, dbeta, dgamma);
+  SN_HIP(hipGetLastError());
+  return SN_OK;
+}
+
 int launch_batchnorm_bwd(sn_ctx* ctx, const float* x, const float* dy, float* dx, int64_t rows, int cols, const BatchNormArgs& a,
                          float* dbeta, float* dgamma, float* ws, int64_t ws_elems, int below_act, float below_act_param) {
   if (rows <= 0 || cols <= 0) return SN_OK;
   const int64_t half = (int64_t)max_slices(ctx, rows, cols) * cols;
   SN_REQUIRE(2 * half <= ws_elems, "batch norm gradient needs %lld workspace elements, %lld given", (long long)(2 * half), (long long)ws_elems);
-  const int cb = (int)ceil_div((int64_t)cols, (int64_t)16);  // finishing kernels: 16 channels per block
   float* part1 = ws + half;
   const float* mean = a.fused_wiring ? a.g_mean : a.mean;
-  const float* r = a.fused_wiring ? a.g_r : a.r;
   const float* inv = a.fused_wiring ? a.g_inv : a.inv;
   {
     LaunchScope scope(ctx, "batchnorm_gradient_sums");
     int s = 0;
-    SN_TRY(reduce_pass<BN_GRAD>(ctx, x, dy, mean, ws, half, rows, cols, &s));
-    hipLaunchKernelGGL(bn_grad_finish_kernel, dim3(cb), dim3(256), 0, ctx->stream, (const float*)ws, (const float*)part1, s, cols,
-                       (float)rows, r, dbeta, dgamma, a.k1, a.k2);
+    if (stream_ok(rows, cols, x, dy, ws, half)) {
+      const Stream st = stream_of(ctx, rows, cols);
+      s = st.slices;
+      hipLaunchKernelGGL(bn_grad_sums_v4_kernel, dim3((unsigned)s), dim3(256), 0, ctx->stream, (const bn_f4*)x, (const bn_f4*)dy, mean, ws, part1, st.n4,
+                         cols, st.active, st.per4);
+    } else {
+      s = reduce_rows<BN_GRAD>(ctx, x, dy, mean, ws, part1, rows, cols);
+    }
+    grad_finish(ctx, ws, part1, s, rows, cols, a, dbeta, dgamma);
   }
   if (dx) {
     const int64_t n = rows * cols;

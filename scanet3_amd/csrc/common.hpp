@@ -283,6 +283,17 @@ int launch_batchnorm_fwd(sn_ctx* ctx, const float* x, float* y, int64_t rows, in
 int launch_batchnorm_bwd(sn_ctx* ctx, const float* x, const float* dy, float* dx, int64_t rows, int cols, const BatchNormArgs& a,
                          float* dbeta, float* dgamma, float* ws, int64_t ws_elems, int below_act = SN_ACT_IDENTITY,
                          float below_act_param = 0.f);
+// Batch normalisation with a 2 x 2 max pooling of its output right above (batchnorm_pool_ok): the normalised tensor [n, h, w, c] is
+// not stored, y and arg are the pooling's output and recorded places.  Backward: the gradients of beta and gamma from the
+// pooling's output gradient dy; the input gradient is left to the reader of PoolGrad, which forms it from a.k1 and a.k2.
+struct PoolGeom {
+  int n, h, w, c, ho, wo, kh, kw, sh, sw, pt, pl;
+};
+bool batchnorm_pool_ok(const PoolGeom& g, const BatchNormArgs& a, const float* x, const float* y, const uint8_t* arg);
+int launch_batchnorm_pool_fwd(sn_ctx* ctx, const float* x, float* y, uint8_t* arg, const PoolGeom& g, const BatchNormArgs& a, bool training, float* ws,
+                              int64_t ws_elems);
+int launch_batchnorm_pool_bwd(sn_ctx* ctx, const float* x, const float* dy, const uint8_t* arg, const PoolGeom& g, const BatchNormArgs& a, float* dbeta,
+                              float* dgamma, float* ws, int64_t ws_elems);
 // moving = momentum*moving + (1-momentum)*batch
 int launch_batchnorm_moving(sn_ctx* ctx, const BatchNormArgs& a, float* moving_mean, float* moving_var, int cols);
 
@@ -399,6 +410,12 @@ struct PoolGrad {
   const float* y = nullptr;
   int ho = 0, wo = 0, sh = 1, sw = 1, pt = 0, pl = 0, act = 0;
   float act_param = 0.f;
+  // with a batch normalisation between convolution and pooling (bn_inv not null): the pooling's gradient g of a value y goes
+  // through it as bn_inv * ((g - bn_k1) - (y - bn_mean) * bn_k2) (launch_batchnorm_pool_bwd has left k1 and k2), one of each per filter
+  const float* bn_mean = nullptr;
+  const float* bn_inv = nullptr;
+  const float* bn_k1 = nullptr;
+  const float* bn_k2 = nullptr;
 };
 bool conv_wgrad_is_direct(const sn_ctx* ctx, const ConvGeom& g, const float* ws, int64_t ws_elems, bool with_pool = false);
 int launch_conv_wgrad(sn_ctx* ctx, const ConvGeom& g, const float* x, const float* dy, float* dw, float* ws, int64_t ws_elems,

@@ -1063,7 +1063,8 @@ int launch_conv_dgrad(sn_ctx* ctx, const ConvGeom& g, const float* dy, const flo
 // kernel computes dy[position, filter] itself from the pooling's output gradient, the recorded first-maximum offsets and
 // the convolution's saved output (for its activation gradient), exactly as pool2x2_bwd_kernel does: an element lies in at
 // most 2 x 2 windows, whose contributions are added in (oh, ow) order, then act'(y) multiplies.  One launch and one pass
-// over the tensor less for a first layer, whose input gradient nobody needs.
+// over the tensor less for a first layer, whose input gradient nobody needs.  With a batch normalisation in between (pg.bn_inv) its
+// input gradient is formed on the way as well: two launches and five passes over the tensor less.
 __device__ __forceinline__ float pool_grad_act_bwd(int act, float y, float dy, float param) {  // elementwise_kernels.hip: act_bwd
   switch (act) {
     case SN_ACT_SIGMOID: return (y * (1.0f - y)) * dy;
@@ -1157,6 +1158,10 @@ __global__ __launch_bounds__(256) void conv_wgrad_direct_kernel(ConvGeom g, cons
           if (((a4[k] >> 16) & 255u) == want[k]) sum[2] += gk[k][2];
           if ((a4[k] >> 24) == want[k]) sum[3] += gk[k][3];
         }
+        if (pg.bn_inv) {  // (batchnorm_kernels.hip: bn_dx_kernel)
+          const f4v iv = *(const f4v*)(pg.bn_inv + ch), mv = *(const f4v*)(pg.bn_mean + ch), k1 = *(const f4v*)(pg.bn_k1 + ch), k2 = *(const f4v*)(pg.bn_k2 + ch);
+          sum = iv * ((sum - k1) - (yv - mv) * k2);
+        }
 #pragma unroll
         for (int q = 0; q < 4; ++q) dcv[p * g.cout + ch + q] = pool_grad_act_bwd(pg.act, yv[q], sum[q], pg.act_param);
       }
@@ -1199,51 +1204,65 @@ __global__ __launch_bounds__(256) void conv_wgrad_direct_kernel(ConvGeom g, cons
   }
 }
 
-// true when launch_conv_wgrad takes the direct kernel for this layer (which can also stand in for a max pooling's backward
-// pass above it: launch_conv_wgrad's `pool` argument)
-bool conv_wgrad_is_direct(const sn_ctx* ctx, const ConvGeom& g, const float* ws, int64_t ws_elems, bool with_pool) {
+// How the direct kernel cuts a layer into bands of output rows, or nothing if the layer is outside its range.  A band is as tall as
+// it takes to give every workgroup one; where it also holds the band's output gradient in LDS (with_pool) it is as
+// tall as fits, cut evenly, and a workgroup walks several.
+struct DirectWgradPlan {
+  int rows_per_band = 0, bands = 0, lw = 0, parts = 0;
+  int64_t staged = 0, lds_floats = 0;
+};
+static bool direct_wgrad_plan(const sn_ctx* ctx, const ConvGeom& g, const float* ws, int64_t ws_elems, bool with_pool, DirectWgradPlan* p) {
   const int M = g.kh * g.kw * g.cin, N = g.cout;
   const int64_t K = (int64_t)g.n * g.ho * g.wo;
   if (!ws || g.cin > 4 || M > WGRAD_DIRECT_MAX_TAPS || N > 64 || K < SMALL_MIN_K) return false;
   const int64_t room = std::min<int64_t>((int64_t)4 * ctx->compute_units, ws_elems / ((int64_t)M * N));
   if (room < 32) return false;
-  const int lw = (g.wo - 1) * g.sw + g.kw;
-  const int rows_per_band = (int)std::min<int64_t>(g.ho, std::max<int64_t>(1, ceil_div((int64_t)g.n * g.ho, room)));
-  const int bands = (int)ceil_div((int64_t)g.ho, (int64_t)rows_per_band);
-  const int64_t staged = (int64_t)((rows_per_band - 1) * g.sh + g.kh) * lw * g.cin;
-  const int64_t lds_floats = std::max<int64_t>(staged + (int64_t)rows_per_band * g.wo * (with_pool ? 1 + N : 1), (int64_t)256 * M);
-  return lds_floats * 4 <= 48 * 1024 && (int64_t)g.n * bands < (int64_t)1 << 30 && (!with_pool || (N % 4 == 0 && (int64_t)g.n * g.ho * g.wo * N < ((int64_t)1 << 32)));  // (32-bit element offsets there)
+  p->lw = (g.wo - 1) * g.sw + g.kw;
+  const int64_t room_lds = 12 * 1024;  // floats: 48 KiB
+  auto place = [&](int64_t rows) {
+    p->rows_per_band = (int)rows;
+    p->bands = (int)ceil_div((int64_t)g.ho, rows);
+    p->staged = ((rows - 1) * g.sh + g.kh) * p->lw * g.cin;
+    p->lds_floats = std::max<int64_t>(p->staged + rows * g.wo * (with_pool ? 1 + N : 1), (int64_t)256 * M);
+    return p->lds_floats <= room_lds;
+  };
+  const int64_t tall = std::min<int64_t>(g.ho, std::max<int64_t>(1, ceil_div((int64_t)g.n * g.ho, room)));
+  bool fits = place(tall);
+  for (int64_t cuts = 2; with_pool && !fits && p->rows_per_band > 1; ++cuts) fits = place(ceil_div(tall, cuts));
+  const int64_t items = (int64_t)g.n * p->bands;
+  if (!fits || items >= (int64_t)1 << 30) return false;
+  if (with_pool && (N % 4 != 0 || K * N >= ((int64_t)1 << 32))) return false;  // (32-bit element offsets there)
+  p->parts = (int)std::min<int64_t>(items, room);
+  return true;
+}
+
+// true when launch_conv_wgrad takes the direct kernel for this layer (which can also stand in for a max pooling's backward
+// pass above it: launch_conv_wgrad's `pool` argument)
+bool conv_wgrad_is_direct(const sn_ctx* ctx, const ConvGeom& g, const float* ws, int64_t ws_elems, bool with_pool) {
+  DirectWgradPlan p;
+  return direct_wgrad_plan(ctx, g, ws, ws_elems, with_pool, &p);
 }
 
 static bool conv_wgrad_direct(sn_ctx* ctx, const ConvGeom& g, const float* x, const float* dy, float* dw, float* ws, int64_t ws_elems, int* rc,
                               const PoolGrad* pool) {
-  const int M = g.kh * g.kw * g.cin, N = g.cout;
-  const int64_t K = (int64_t)g.n * g.ho * g.wo;
-  if (!ws || g.cin > 4 || M > WGRAD_DIRECT_MAX_TAPS || N > 64 || K < SMALL_MIN_K) return false;
-  const int64_t room = std::min<int64_t>((int64_t)4 * ctx->compute_units, ws_elems / ((int64_t)M * N));
-  if (room < 32) return false;
+  DirectWgradPlan p;
+  if (!direct_wgrad_plan(ctx, g, ws, ws_elems, pool != nullptr, &p)) return false;
+  const int M = g.kh * g.kw * g.cin, N = g.cout, parts = p.parts;
+  const int64_t K = (int64_t)g.n * g.ho * g.wo, items = (int64_t)g.n * p.bands;
   int cshift = 0;
   while ((1 << cshift) < N) ++cshift;
-  const int lw = (g.wo - 1) * g.sw + g.kw;
-  int rows_per_band = (int)std::min<int64_t>(g.ho, std::max<int64_t>(1, ceil_div((int64_t)g.n * g.ho, room)));
-  const int bands = (int)ceil_div((int64_t)g.ho, (int64_t)rows_per_band);
-  const int64_t items = (int64_t)g.n * bands;
-  const int64_t staged = (int64_t)((rows_per_band - 1) * g.sh + g.kh) * lw * g.cin;
-  const int64_t lds_floats = std::max<int64_t>(staged + (int64_t)rows_per_band * g.wo * (pool ? 1 + N : 1), (int64_t)256 * M);
-  if (lds_floats * 4 > 48 * 1024 || items >= (int64_t)1 << 30) return false;
-  const int parts = (int)std::min<int64_t>(items, room);
   {
     LaunchScope scope(ctx, pool ? "maxpool_backward_and_conv2d_filter_gradient_direct" : "conv2d_filter_gradient_direct", M, N, (int)K);
     const PoolGrad pg = pool ? *pool : PoolGrad{};
-    const DirectConvPlan plan = direct_conv_plan(g, lw);
+    const DirectConvPlan plan = direct_conv_plan(g, p.lw);
 #define SN_WGRAD_DIRECT(MT)                                                                                                             \
   do {                                                                                                                                  \
     if (pool)                                                                                                                           \
-      hipLaunchKernelGGL((conv_wgrad_direct_kernel<MT, true>), dim3((unsigned)parts), dim3(256), (size_t)lds_floats * sizeof(float),    \
-                         ctx->stream, g, x, dy, ws, rows_per_band, bands, (int)items, lw, cshift, (int)staged, pg, plan);               \
+      hipLaunchKernelGGL((conv_wgrad_direct_kernel<MT, true>), dim3((unsigned)parts), dim3(256), (size_t)p.lds_floats * sizeof(float),  \
+                         ctx->stream, g, x, dy, ws, p.rows_per_band, p.bands, (int)items, p.lw, cshift, (int)p.staged, pg, plan);       \
     else                                                                                                                                \
-      hipLaunchKernelGGL((conv_wgrad_direct_kernel<MT, false>), dim3((unsigned)parts), dim3(256), (size_t)lds_floats * sizeof(float),   \
-                         ctx->stream, g, x, dy, ws, rows_per_band, bands, (int)items, lw, cshift, (int)staged, pg, plan);               \
+      hipLaunchKernelGGL((conv_wgrad_direct_kernel<MT, false>), dim3((unsigned)parts), dim3(256), (size_t)p.lds_floats * sizeof(float), \
+                         ctx->stream, g, x, dy, ws, p.rows_per_band, p.bands, (int)items, p.lw, cshift, (int)p.staged, pg, plan);       \
   } while (0)
     if (M <= 9) SN_WGRAD_DIRECT(9);
     else if (M <= 18) SN_WGRAD_DIRECT(18);

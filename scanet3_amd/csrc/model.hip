@@ -589,6 +589,18 @@ static BatchNormArgs batchnorm_args(sn_replica* r, const Op& op, int i) {
                        op.bn_fused, b + 6 * c, b + 7 * c, b + 8 * c};
 }
 
+static PoolGeom pool_geom(const Op& op, int rows) {
+  return PoolGeom{rows, (int)op.in_dims[0], (int)op.in_dims[1], (int)op.in_dims[2], (int)op.out_dims[0], (int)op.out_dims[1], op.kh, op.kw, op.sh, op.sw,
+                  op.pt, op.pl};
+}
+// A batch normalisation whose output only a 2 x 2 max pooling right above it reads: one pass does both
+static bool batchnorm_pool_path(const sn_replica* r, size_t i, const float* x, int rows) {
+  const sn_model* m = r->model;
+  if (i + 1 >= m->ops.size() || m->ops[i].kind != OP_BATCHNORM || m->ops[i + 1].kind != OP_POOL || m->ops[i + 1].pool_avg) return false;
+  return batchnorm_pool_ok(pool_geom(m->ops[i + 1], rows), batchnorm_args(const_cast<sn_replica*>(r), m->ops[i], (int)i), op_output(const_cast<sn_replica*>(r), (int)i - 1, x, rows),
+                           r->act[i + 1], r->arg[i + 1]);
+}
+
 // skip_last: leave out the last op (the training pass fuses a Softmax output into the loss kernel)
 // training: the model as the optimizer compiles it; false = frozen, as a trained model predicts (models/Model.scala:126-127).
 //           Only batch normalisation tells the two apart.
@@ -651,6 +663,7 @@ static int forward(sn_replica* r, const float* x, int rows, bool skip_last = fal
         break;
       }
       case OP_POOL:
+        if (i > 0 && batchnorm_pool_path(r, i - 1, x, rows)) break;  // done with the batch normalisation below
         SN_TRY(launch_pool_fwd(ctx, op.pool_avg, in, r->act[i], r->arg[i], rows, (int)op.in_dims[0], (int)op.in_dims[1], (int)op.in_dims[2],
                                   (int)op.out_dims[0], (int)op.out_dims[1], op.kh, op.kw, op.sh, op.sw, op.pt, op.pl));
         break;
@@ -705,6 +718,11 @@ static int forward(sn_replica* r, const float* x, int rows, bool skip_last = fal
       }
       case OP_BATCHNORM: {
         const int c = (int)op.out_dims.back();
+        if (batchnorm_pool_path(r, i, x, rows)) {
+          SN_TRY(launch_batchnorm_pool_fwd(ctx, in, r->act[i + 1], r->arg[i + 1], pool_geom(m->ops[i + 1], rows), batchnorm_args(r, op, (int)i), training,
+                                           r->ws, m->workspace_elems));
+          break;
+        }
         SN_TRY(launch_batchnorm_fwd(ctx, in, r->act[i], (int64_t)rows * (op.out_elems / c), c, batchnorm_args(r, op, (int)i), training, r->ws,
                                     m->workspace_elems));
         break;
@@ -924,17 +942,21 @@ static int backward(sn_replica* r, const float* x, int rows, int first = -1, int
           const bool fuse = below.kind == OP_CONV && below.act != SN_ACT_IDENTITY;
           // The first layer's convolution needs its output gradient for the filter gradient only (and has no bias to sum it
           // for): where that product runs as the direct kernel, the kernel forms the gradient itself from what this pooling
-          // would have read, and the pooling's backward launch and the tensor it writes are not needed.
-          if (i == 1 && below.kind == OP_CONV && below.b < 0 && !op.pool_avg && op.kh == 2 && op.kw == 2 && rows > 0) {
-            const ConvGeom cg{rows, (int)below.in_dims[0], (int)below.in_dims[1], (int)below.in_dims[2], (int)below.out_dims[0],
-                              (int)below.out_dims[1], (int)below.out_dims[2], below.kh, below.kw, below.sh, below.sw, below.pt, below.pl};
+          // would have read, and the pooling's backward launch and the tensor it writes are not needed.  The same holds with a
+          // batch normalisation in between, whose own gradients then come from the pooling's windows.
+          const bool over_bn = i == 2 && below.kind == OP_BATCHNORM && m->ops[0].kind == OP_CONV && batchnorm_pool_path(r, 1, x, rows);
+          const Op& conv = over_bn ? m->ops[0] : below;
+          if ((i == 1 || over_bn) && conv.kind == OP_CONV && conv.b < 0 && !op.pool_avg && op.kh == 2 && op.kw == 2 && rows > 0) {
+            const ConvGeom cg{rows, (int)conv.in_dims[0], (int)conv.in_dims[1], (int)conv.in_dims[2], (int)conv.out_dims[0],
+                              (int)conv.out_dims[1], (int)conv.out_dims[2], conv.kh, conv.kw, conv.sh, conv.sw, conv.pt, conv.pl};
             const bool deferred = r->defer_now && r->ws_defer[0] && r->n_deferred < MAX_DEFERRED;
-            const bool aligned = ((reinterpret_cast<uintptr_t>(dy) | reinterpret_cast<uintptr_t>(r->arg[i]) | reinterpret_cast<uintptr_t>(r->act[i - 1])) & 15u) == 0;
+            const bool aligned = ((reinterpret_cast<uintptr_t>(dy) | reinterpret_cast<uintptr_t>(r->arg[i]) | reinterpret_cast<uintptr_t>(r->act[0])) & 15u) == 0;
             if (aligned && conv_wgrad_is_direct(ctx, cg, deferred ? r->ws_defer[0] : r->ws, m->workspace_elems, true)) {
-              pool_grad.dy = dy; pool_grad.arg = r->arg[i]; pool_grad.y = r->act[i - 1];
+              pool_grad = PoolGrad{};
+              pool_grad.dy = dy; pool_grad.arg = r->arg[i]; pool_grad.y = r->act[0];
               pool_grad.ho = (int)op.out_dims[0]; pool_grad.wo = (int)op.out_dims[1];
               pool_grad.sh = op.sh; pool_grad.sw = op.sw; pool_grad.pt = op.pt; pool_grad.pl = op.pl;
-              pool_grad.act = below.act; pool_grad.act_param = below.act_param;
+              pool_grad.act = conv.act; pool_grad.act_param = conv.act_param;
               pool_pending = true;
               break;
             }
@@ -1036,6 +1058,16 @@ static int backward(sn_replica* r, const float* x, int rows, int first = -1, int
       }
       case OP_BATCHNORM: {
         const int c = (int)op.out_dims.back();
+        if (pool_pending) {  // the pooling above left its backward pass, and with it this layer's input gradient, to the filter gradient
+          const BatchNormArgs a = batchnorm_args(r, op, i);
+          SN_TRY(launch_batchnorm_pool_bwd(ctx, in, dy, pool_grad.arg, pool_geom(m->ops[i + 1], rows), a, param_ptr(r, r->g, op.bn_p[0]),
+                                           param_ptr(r, r->g, op.bn_p[1]), r->ws, m->workspace_elems));
+          pool_grad.bn_mean = a.fused_wiring ? a.g_mean : a.mean;
+          pool_grad.bn_inv = a.fused_wiring ? a.g_inv : a.inv;
+          pool_grad.bn_k1 = a.k1;
+          pool_grad.bn_k2 = a.k2;
+          break;
+        }
         // a convolution right below: its activation gradient rides along in the input-gradient pass (x is its output)
         const bool fuse = need_dx && m->ops[i - 1].kind == OP_CONV && m->ops[i - 1].act != SN_ACT_IDENTITY;
         SN_TRY(launch_batchnorm_bwd(ctx, in, dy, need_dx ? dx : nullptr, (int64_t)rows * (op.out_elems / c), c, batchnorm_args(r, op, i),

@@ -520,6 +520,18 @@ MODELS = {
     # BatchNorm reductions: 200 channels take the row-walking form with four column blocks, 256 the float4 stream form
     "batchnorm_200_channels": ([("dense", 200, "tanh"), ("batchnorm", 0.9, 1e-3), ("dense", 5, "softmax")], "cce", (31,), 300, "normal_onehot"),
     "batchnorm_256_channels": ([("dense", 256, "relu"), ("batchnorm", 0.9, 1e-3), ("dense", 5, "softmax")], "cce", (31,), 300, "normal_onehot"),
+    "batchnorm_50_channels": ([("dense", 50, "tanh"), ("batchnorm", 0.9, 1e-3), ("dense", 5, "softmax")], "cce", (31,), 300, "normal_onehot"),
+    # a 2 x 2 max pooling right above a BatchNorm: overlapping windows that reach into the padding, 12 channels (252 of a block's 256
+    # threads); 48 channels with another stride per direction under the plain form; windows that leave a row and a column of the image
+    # out, behind a second layer (whose convolution wants its input gradient, so the layers' backward passes stay apart)
+    "batchnorm_pool_first_layer_same_s1": ([("conv", 12, (3, 3), (1, 1), "same", "tanh", False), ("batchnorm", 0.9, 1e-3), ("pool", (2, 2), (1, 1), "same"),
+                                            ("flatten",), ("dense", 3, "softmax")], "cce", (15, 14, 2), 40, "uniform_onehot"),
+    "batchnorm_pool_48_channels_stride_2_1": ([("conv", 48, (3, 3), (1, 1), "same", "relu", False), ("batchnorm", 0.99, 1e-3, "fused"),
+                                               ("pool", (2, 2), (2, 1), "valid"), ("flatten",), ("dense", 3, "softmax")], "cce", (9, 10, 3), 30,
+                                              "uniform_onehot"),
+    "batchnorm_pool_second_layer": ([("conv", 4, (2, 2), (1, 1), "valid", "relu", False), ("conv", 8, (2, 2), (1, 1), "valid", "relu", False),
+                                     ("batchnorm", 0.9, 1e-3), ("pool", (2, 2), (2, 2), "valid"), ("flatten",), ("dense", 3, "softmax")], "cce",
+                                    (11, 9, 1), 50, "uniform_onehot"),
     "dense_identity_mse": ([("dense", 6, "identity")], "mse", (4,), 8, "normal_regression"),
     # Dense >> Dense(Softmax) + CategoricalCrossentropy small enough for the two-launch training pass: a reduction length
     # that is no multiple of 16, rows that are no multiple of 16, all 64 hidden units / 16 classes, penalties on top
@@ -591,6 +603,9 @@ KERNEL_OF_MODEL = {
     "conv_input_gradient_32_channels_2x3_same": "conv2d_input_gradient[",
     "conv_pool_first_layer_same_s1": "maxpool_backward_and_conv2d_filter_gradient_direct",
     "conv_first_layer_uneven": "conv2d_filter_gradient_direct",
+    "batchnorm_pool_first_layer_same_s1": "batchnorm_gradient_sums_from_maxpool",
+    "batchnorm_pool_48_channels_stride_2_1": "batchnorm_gradient_sums_from_maxpool",
+    "batchnorm_pool_second_layer": "batchnorm_apply_and_maxpool",
     "dense_many_features_few_units": "dense_weight_and_input_gradient_rows",
     "dense_many_features_16_units": "dense_weight_and_input_gradient_rows",
     "dense_odd_feature_count_9_units": "small_output_reduce_softmax_crossentropy_fused",
