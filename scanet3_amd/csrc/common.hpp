@@ -401,7 +401,7 @@ int64_t conv_wgrad_taps_workspace(const sn_ctx* ctx, const ConvGeom& g);  // flo
 int launch_conv_wgrad_taps(sn_ctx* ctx, const ConvGeom& g, const float* x, const float* dy, float* ws, int64_t ws_elems, int* parts);
 int launch_conv_fwd(sn_ctx* ctx, const ConvGeom& g, const float* x, const float* w, const Epilogue& ep, float* ws, int64_t ws_elems);
 int launch_conv_dgrad(sn_ctx* ctx, const ConvGeom& g, const float* dy, const float* w, float* dx, float* ws, int64_t ws_elems);
-// A 2 x 2 max pooling right above a first-layer convolution, for launch_conv_wgrad's direct kernel: the pooling's output
+// A 2 x 2 max pooling right above a first-layer convolution, for launch_conv_wgrad's first-layer kernel: the pooling's output
 // gradient dy [n, ho, wo, cout], its recorded first-maximum offsets (one byte per output value) and the convolution's saved
 // output y with its activation; the kernel then forms the convolution's output gradient itself (no launch_pool_bwd).
 struct PoolGrad {
@@ -417,7 +417,11 @@ struct PoolGrad {
   const float* bn_k1 = nullptr;
   const float* bn_k2 = nullptr;
 };
-bool conv_wgrad_is_direct(const sn_ctx* ctx, const ConvGeom& g, const float* ws, int64_t ws_elems, bool with_pool = false);
+bool conv_wgrad_is_direct(const sn_ctx* ctx, const ConvGeom& g, const float* ws, int64_t ws_elems);
+// First-layer filter gradient (conv_first_kernels.hip): up to 4 input channels, 48 taps, 64 filters.  The number of partial filters
+// [part][kh * kw * cin][cout] it would leave in ws (0: not its shape), and the launch.
+int conv_first_wgrad_parts(const sn_ctx* ctx, const ConvGeom& g, const float* ws, int64_t ws_elems, int* rows_per_wave = nullptr);
+int launch_conv_first_wgrad(sn_ctx* ctx, const ConvGeom& g, const float* x, const float* dy, float* ws, int64_t ws_elems, const PoolGrad* pool, int* parts);
 int launch_conv_wgrad(sn_ctx* ctx, const ConvGeom& g, const float* x, const float* dy, float* dw, float* ws, int64_t ws_elems,
                       const PoolGrad* pool = nullptr);
 

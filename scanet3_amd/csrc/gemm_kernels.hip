@@ -910,27 +910,25 @@ __device__ __forceinline__ void fwd_rows_pixels(const float* lds, const int* ori
   for (int u = 0; u < U; ++u) *(f4v*)(outb + (int64_t)(p0 + u * slots) * e.ldo) = f4v{v[u * 4], v[u * 4 + 1], v[u * 4 + 2], v[u * 4 + 3]};
 }
 
-// What a launch of the two direct first-layer kernels below fixes and the device would otherwise divide out per thread
+// What a launch of the direct first-layer kernel below fixes and the device would otherwise divide out per thread
 // (the device has no integer divider): the LDS offset of tap m = (r, q, ci) from a position's top-left input element
 // (taps >= kh*kw*cin repeat tap 0), and the divisors of the index arithmetic.
-constexpr int WGRAD_DIRECT_MAX_TAPS = 36;
+constexpr int DIRECT_ROWS_MAX_TAPS = 18;
 struct DirectConvPlan {
-  int off[WGRAD_DIRECT_MAX_TAPS];
-  FastDiv by_cv, by_wo, by_row_elems, by_cin, by_cout;
+  int off[DIRECT_ROWS_MAX_TAPS];
+  FastDiv by_wo, by_row_elems, by_cin;
 };
 static DirectConvPlan direct_conv_plan(const ConvGeom& g, int lw) {
   DirectConvPlan plan;
   const int M = g.kh * g.kw * g.cin, row_elems = lw * g.cin;
-  for (int m = 0; m < WGRAD_DIRECT_MAX_TAPS; ++m) {
+  for (int m = 0; m < DIRECT_ROWS_MAX_TAPS; ++m) {
     const int mm = m < M ? m : 0;
     const int ci = mm % g.cin, rq = mm / g.cin;
     plan.off[m] = (rq / g.kw) * row_elems + (rq % g.kw) * g.cin + ci;
   }
-  plan.by_cv = fast_div((uint32_t)std::max(1, g.cout / 4));
   plan.by_wo = fast_div((uint32_t)g.wo);
   plan.by_row_elems = fast_div((uint32_t)row_elems);
   plan.by_cin = fast_div((uint32_t)g.cin);
-  plan.by_cout = fast_div((uint32_t)g.cout);
   return plan;
 }
 
@@ -1052,245 +1050,32 @@ int launch_conv_dgrad(sn_ctx* ctx, const ConvGeom& g, const float* dy, const flo
   return launch_any<false>(ctx, "conv2d_input_gradient", M, N, K, al, bl, ep, ws, ws_elems);
 }
 
-// Filter gradient of a first-layer convolution (a few input channels, at most 64 filters): M = kh*kw*cin is a few
-// dozen rows, N = cout a few dozen columns and K = every output position of the batch, so the work is reading dy
-// once.  Direct form: a workgroup takes a band of output rows of one image, keeps the input rows under it in LDS
-// (zero-padded, so taps need no bounds checks), a group of `1 << cshift` >= cout lanes owns one output position at a
-// time, each lane one filter, and keeps all M sums of that filter in registers.  The lanes' sums meet in LDS and
-// leave as one partial [M][cout] per workgroup; gemm_small_reduce_kernel adds the partials in a fixed order.
-
-// POOL: the convolution's output gradient is not in memory yet.  A 2 x 2 max pooling sits right above the layer and the
-// kernel computes dy[position, filter] itself from the pooling's output gradient, the recorded first-maximum offsets and
-// the convolution's saved output (for its activation gradient), exactly as pool2x2_bwd_kernel does: an element lies in at
-// most 2 x 2 windows, whose contributions are added in (oh, ow) order, then act'(y) multiplies.  One launch and one pass
-// over the tensor less for a first layer, whose input gradient nobody needs.  With a batch normalisation in between (pg.bn_inv) its
-// input gradient is formed on the way as well: two launches and five passes over the tensor less.
-__device__ __forceinline__ float pool_grad_act_bwd(int act, float y, float dy, float param) {  // elementwise_kernels.hip: act_bwd
-  switch (act) {
-    case SN_ACT_SIGMOID: return (y * (1.0f - y)) * dy;
-    case SN_ACT_TANH: return (1.0f - y * y) * dy;
-    case SN_ACT_RELU: return (param < y ? 1.0f : 0.0f) * dy;
-    default: return dy;
-  }
-}
-
-template <int MT, bool POOL>  // MT: upper bound of kh*kw*cin
-__global__ __launch_bounds__(256) void conv_wgrad_direct_kernel(ConvGeom g, const float* __restrict__ x, const float* __restrict__ dy,
-                                                                 float* __restrict__ partial, int rows_per_band, int bands_per_image,
-                                                                 int items, int lw, int cshift, int staged_full, PoolGrad pg, DirectConvPlan plan) {
-  extern __shared__ float wg_lds[];
-  const int tid = threadIdx.x;
-  const int M = g.kh * g.kw * g.cin;
-  const int row_elems = lw * g.cin;
-  int off[MT];
-#pragma unroll
-  for (int m = 0; m < MT; ++m) off[m] = plan.off[m];
-  const FastDiv by_cv = plan.by_cv, by_wo = plan.by_wo;
-  float acc[MT];
-#pragma unroll
-  for (int m = 0; m < MT; ++m) acc[m] = 0.f;
-  const int lanes = 1 << cshift;
-  const int c = tid & (lanes - 1);
-  const int slot = tid >> cshift, slots = 256 >> cshift;
-  const bool live = c < g.cout;
-  const int cc = live ? c : 0;
-  for (int item = blockIdx.x; item < items; item += gridDim.x) {
-    const int b = item / bands_per_image, band = item % bands_per_image;
-    const int oh0 = band * rows_per_band;
-    const int oh1 = oh0 + rows_per_band < g.ho ? oh0 + rows_per_band : g.ho;
-    const int iy0 = oh0 * g.sh - g.pt;
-    const int staged = ((oh1 - oh0 - 1) * g.sh + g.kh) * row_elems;
-    const int P = (oh1 - oh0) * g.wo;
-    const float* dyb = dy + ((int64_t)b * g.ho + oh0) * g.wo * g.cout;
-    constexpr int U = 16;  // positions per lane whose dy loads are in flight together
-    int* origin = reinterpret_cast<int*>(wg_lds + staged_full);  // per position of the band: LDS offset of its top-left input element
-    float* dcv = wg_lds + staged_full + rows_per_band * g.wo;    // POOL: the band's output gradient [P][cout]
-    __syncthreads();  // the previous item's readers are done with the staged rows
-    for (int e = tid; e < staged; e += 256) {
-      const int row = (int)div_by((uint32_t)e, plan.by_row_elems), rem = e - row * row_elems;
-      const int px = (int)div_by((uint32_t)rem, plan.by_cin);
-      const int iy = iy0 + row, ix = px - g.pl, ci = rem - px * g.cin;
-      wg_lds[e] = ((unsigned)iy < (unsigned)g.h && (unsigned)ix < (unsigned)g.w) ? x[(((int64_t)b * g.h + iy) * g.w + ix) * g.cin + ci] : 0.f;
-    }
-    for (int p = tid; p < P; p += 256) {  // once per position, not per lane
-      const int prow = (int)div_by((uint32_t)p, by_wo);
-      origin[p] = prow * g.sh * row_elems + (p - prow * g.wo) * g.sw * g.cin;
-    }
-    if constexpr (POOL) {
-      // the band's output gradient [P][cout], four filters per thread: position (iy, ix) of the convolution's output = of the
-      // pooling's input lies in the windows oh_lo + {0, 1} x ow_lo + {0, 1} (those that exist)
-      // (index arithmetic is what this phase costs: divisions by the launch's constants are multiplications, those by the
-      // pooling's stride shifts for strides 1 and 2, element offsets 32-bit)
-      const int cv = g.cout >> 2;
-      auto by_stride = [](int v, int st) { return st == 1 ? v : (st == 2 ? v >> 1 : v / st); };  // v >= 0
-      const uint32_t img_y = (uint32_t)b * g.ho, img_p = (uint32_t)b * pg.ho;
-      for (int e = tid; e < P * cv; e += 256) {
-        const int p = (int)div_by((uint32_t)e, by_cv), ch = (e - p * cv) * 4;
-        const int prow = (int)div_by((uint32_t)p, by_wo);
-        const int iy = oh0 + prow, ix = p - prow * g.wo;
-        int oh_lo = iy + pg.pt - 1;
-        oh_lo = oh_lo <= 0 ? 0 : by_stride(oh_lo + pg.sh - 1, pg.sh);
-        int oh_hi = by_stride(iy + pg.pt, pg.sh);
-        if (oh_hi > pg.ho - 1) oh_hi = pg.ho - 1;
-        int ow_lo = ix + pg.pl - 1;
-        ow_lo = ow_lo <= 0 ? 0 : by_stride(ow_lo + pg.sw - 1, pg.sw);
-        int ow_hi = by_stride(ix + pg.pl, pg.sw);
-        if (ow_hi > pg.wo - 1) ow_hi = pg.wo - 1;
-        const f4v yv = *(const f4v*)(pg.y + (((img_y + iy) * g.wo + ix) * g.cout + ch));
-        uint32_t a4[4], want[4];
-        f4v gk[4];
-        bool on[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {  // windows that do not exist re-read the first element and are ignored
-          const int oh = oh_lo + (k >> 1), ow = ow_lo + (k & 1);
-          on[k] = oh <= oh_hi && ow <= ow_hi;
-          const uint32_t o = on[k] ? ((img_p + oh) * pg.wo + ow) * g.cout + ch : (uint32_t)ch;
-          want[k] = (uint32_t)((iy - (oh * pg.sh - pg.pt)) * 2 + (ix - (ow * pg.sw - pg.pl)));
-          a4[k] = *(const uint32_t*)(pg.arg + o);
-          gk[k] = *(const f4v*)(pg.dy + o);
-        }
-        f4v sum = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          if (!on[k]) continue;
-          if ((a4[k] & 255u) == want[k]) sum[0] += gk[k][0];
-          if (((a4[k] >> 8) & 255u) == want[k]) sum[1] += gk[k][1];
-          if (((a4[k] >> 16) & 255u) == want[k]) sum[2] += gk[k][2];
-          if ((a4[k] >> 24) == want[k]) sum[3] += gk[k][3];
-        }
-        if (pg.bn_inv) {  // (batchnorm_kernels.hip: bn_dx_kernel)
-          const f4v iv = *(const f4v*)(pg.bn_inv + ch), mv = *(const f4v*)(pg.bn_mean + ch), k1 = *(const f4v*)(pg.bn_k1 + ch), k2 = *(const f4v*)(pg.bn_k2 + ch);
-          sum = iv * ((sum - k1) - (yv - mv) * k2);
-        }
-#pragma unroll
-        for (int q = 0; q < 4; ++q) dcv[p * g.cout + ch + q] = pool_grad_act_bwd(pg.act, yv[q], sum[q], pg.act_param);
-      }
-    }
-    __syncthreads();
-    for (int p0 = slot; p0 < P; p0 += slots * U) {
-      float d[U];
-      int base[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int p = p0 + u * slots;
-        const bool in = p < P;
-        const int pp = in ? p : 0;
-        float v;
-        if constexpr (POOL) v = dcv[pp * g.cout + cc];  // formed below, once per band
-        else v = dyb[(int64_t)pp * g.cout + cc];  // always a valid address: no branch around the load
-        d[u] = (in && live) ? v : 0.f;
-        base[u] = origin[pp];
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-#pragma unroll
-        for (int m = 0; m < MT; ++m)  // rows m >= M repeat tap 0 and are dropped at the end: no branch between the LDS reads
-          acc[m] = __builtin_fmaf(wg_lds[base[u] + off[m]], d[u], acc[m]);
-      }
-    }
-  }
-  __syncthreads();
-  // [slot][m][lane] -> one sum per (m, filter), slots added in order
-#pragma unroll
-  for (int m = 0; m < MT; ++m)
-    if (m < M) wg_lds[(slot * M + m) * lanes + c] = acc[m];
-  __syncthreads();
-  const int outs = M * g.cout;
-  for (int o = tid; o < outs; o += 256) {
-    const int m = (int)div_by((uint32_t)o, plan.by_cout), co = o - m * g.cout;
-    float t = 0.f;
-    for (int sl = 0; sl < slots; ++sl) t += wg_lds[(sl * M + m) * lanes + co];
-    partial[(int64_t)blockIdx.x * outs + o] = t;
-  }
-}
-
-// How the direct kernel cuts a layer into bands of output rows, or nothing if the layer is outside its range.  A band is as tall as
-// it takes to give every workgroup one; where it also holds the band's output gradient in LDS (with_pool) it is as
-// tall as fits, cut evenly, and a workgroup walks several.
-struct DirectWgradPlan {
-  int rows_per_band = 0, bands = 0, lw = 0, parts = 0;
-  int64_t staged = 0, lds_floats = 0;
-};
-static bool direct_wgrad_plan(const sn_ctx* ctx, const ConvGeom& g, const float* ws, int64_t ws_elems, bool with_pool, DirectWgradPlan* p) {
-  const int M = g.kh * g.kw * g.cin, N = g.cout;
-  const int64_t K = (int64_t)g.n * g.ho * g.wo;
-  if (!ws || g.cin > 4 || M > WGRAD_DIRECT_MAX_TAPS || N > 64 || K < SMALL_MIN_K) return false;
-  const int64_t room = std::min<int64_t>((int64_t)4 * ctx->compute_units, ws_elems / ((int64_t)M * N));
-  if (room < 32) return false;
-  p->lw = (g.wo - 1) * g.sw + g.kw;
-  const int64_t room_lds = 12 * 1024;  // floats: 48 KiB
-  auto place = [&](int64_t rows) {
-    p->rows_per_band = (int)rows;
-    p->bands = (int)ceil_div((int64_t)g.ho, rows);
-    p->staged = ((rows - 1) * g.sh + g.kh) * p->lw * g.cin;
-    p->lds_floats = std::max<int64_t>(p->staged + rows * g.wo * (with_pool ? 1 + N : 1), (int64_t)256 * M);
-    return p->lds_floats <= room_lds;
-  };
-  const int64_t tall = std::min<int64_t>(g.ho, std::max<int64_t>(1, ceil_div((int64_t)g.n * g.ho, room)));
-  bool fits = place(tall);
-  for (int64_t cuts = 2; with_pool && !fits && p->rows_per_band > 1; ++cuts) fits = place(ceil_div(tall, cuts));
-  const int64_t items = (int64_t)g.n * p->bands;
-  if (!fits || items >= (int64_t)1 << 30) return false;
-  if (with_pool && (N % 4 != 0 || K * N >= ((int64_t)1 << 32))) return false;  // (32-bit element offsets there)
-  p->parts = (int)std::min<int64_t>(items, room);
-  return true;
-}
-
-// true when launch_conv_wgrad takes the direct kernel for this layer (which can also stand in for a max pooling's backward
-// pass above it: launch_conv_wgrad's `pool` argument)
-bool conv_wgrad_is_direct(const sn_ctx* ctx, const ConvGeom& g, const float* ws, int64_t ws_elems, bool with_pool) {
-  DirectWgradPlan p;
-  return direct_wgrad_plan(ctx, g, ws, ws_elems, with_pool, &p);
-}
-
-static bool conv_wgrad_direct(sn_ctx* ctx, const ConvGeom& g, const float* x, const float* dy, float* dw, float* ws, int64_t ws_elems, int* rc,
-                              const PoolGrad* pool) {
-  DirectWgradPlan p;
-  if (!direct_wgrad_plan(ctx, g, ws, ws_elems, pool != nullptr, &p)) return false;
-  const int M = g.kh * g.kw * g.cin, N = g.cout, parts = p.parts;
-  const int64_t K = (int64_t)g.n * g.ho * g.wo, items = (int64_t)g.n * p.bands;
-  int cshift = 0;
-  while ((1 << cshift) < N) ++cshift;
-  {
-    LaunchScope scope(ctx, pool ? "maxpool_backward_and_conv2d_filter_gradient_direct" : "conv2d_filter_gradient_direct", M, N, (int)K);
-    const PoolGrad pg = pool ? *pool : PoolGrad{};
-    const DirectConvPlan plan = direct_conv_plan(g, p.lw);
-#define SN_WGRAD_DIRECT(MT)                                                                                                             \
-  do {                                                                                                                                  \
-    if (pool)                                                                                                                           \
-      hipLaunchKernelGGL((conv_wgrad_direct_kernel<MT, true>), dim3((unsigned)parts), dim3(256), (size_t)p.lds_floats * sizeof(float),  \
-                         ctx->stream, g, x, dy, ws, p.rows_per_band, p.bands, (int)items, p.lw, cshift, (int)p.staged, pg, plan);       \
-    else                                                                                                                                \
-      hipLaunchKernelGGL((conv_wgrad_direct_kernel<MT, false>), dim3((unsigned)parts), dim3(256), (size_t)p.lds_floats * sizeof(float), \
-                         ctx->stream, g, x, dy, ws, p.rows_per_band, p.bands, (int)items, p.lw, cshift, (int)p.staged, pg, plan);       \
-  } while (0)
-    if (M <= 9) SN_WGRAD_DIRECT(9);
-    else if (M <= 18) SN_WGRAD_DIRECT(18);
-    else SN_WGRAD_DIRECT(36);
-#undef SN_WGRAD_DIRECT
-  }
-  if (ctx->defer && (M * N) % 4 == 0) {  // the caller's optimizer launch adds the partials
-    *ctx->defer = DeferredReduce{2, ws, parts, M * N, dw};
-    ctx->defer = nullptr;
-    *rc = hipGetLastError() == hipSuccess ? SN_OK : fail(SN_E_HIP, "conv2d_filter_gradient_direct: launch failed");
-    return true;
-  }
-  Epilogue e;
-  e.out = dw;
-  e.ldo = g.cout;
-  StdEpilogue ep{e};
-  LaunchScope scope(ctx, "small_output_reduce");
-  hipLaunchKernelGGL((gemm_small_reduce_kernel<StdEpilogue>), dim3((unsigned)ceil_div(M * N, 4)), dim3(256), 0, ctx->stream, (const float*)ws,
-                     parts, M, N, ep);
-  *rc = hipGetLastError() == hipSuccess ? SN_OK : fail(SN_E_HIP, "conv2d_filter_gradient_direct: launch failed");
-  return true;
+// true when launch_conv_wgrad takes the first-layer kernel (conv_first_kernels.hip), which can also stand in for a max
+// pooling's backward pass above it: launch_conv_wgrad's `pool` argument
+bool conv_wgrad_is_direct(const sn_ctx* ctx, const ConvGeom& g, const float* ws, int64_t ws_elems) {
+  return conv_first_wgrad_parts(ctx, g, ws, ws_elems) > 0;
 }
 
 int launch_conv_wgrad(sn_ctx* ctx, const ConvGeom& g, const float* x, const float* dy, float* dw, float* ws, int64_t ws_elems,
                       const PoolGrad* pool) {
   const int M = g.kh * g.kw * g.cin, N = g.cout, K = g.n * g.ho * g.wo;
-  int rc = SN_OK;
-  if (conv_wgrad_direct(ctx, g, x, dy, dw, ws, ws_elems, &rc, pool)) return rc;
+  if (conv_wgrad_is_direct(ctx, g, ws, ws_elems)) {
+    int parts = 0;
+    SN_TRY(launch_conv_first_wgrad(ctx, g, x, dy, ws, ws_elems, pool, &parts));
+    if (ctx->defer && (M * N) % 4 == 0) {  // the caller's optimizer launch adds the partials
+      *ctx->defer = DeferredReduce{2, ws, parts, M * N, dw};
+      ctx->defer = nullptr;
+      return SN_OK;
+    }
+    Epilogue e;
+    e.out = dw;
+    e.ldo = g.cout;
+    LaunchScope scope(ctx, "small_output_reduce");
+    hipLaunchKernelGGL((gemm_small_reduce_kernel<StdEpilogue>), dim3((unsigned)ceil_div(M * N, 4)), dim3(256), 0, ctx->stream, (const float*)ws,
+                       parts, M, N, StdEpilogue{e});
+    SN_HIP(hipGetLastError());
+    return SN_OK;
+  }
   SN_REQUIRE(pool == nullptr, "conv2d_filter_gradient: only the direct kernel takes a pooling's gradient (ask conv_wgrad_is_direct first)");
   if (ws && aligned16(ws) && conv_wgrad_taps_shape(ctx, g, x, dy) && conv_wgrad_taps_workspace(ctx, g) <= ws_elems) {
     // a tile per filter tap: a few dozen partial filters instead of the 64 x 64 tiling's hundreds

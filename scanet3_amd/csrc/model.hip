@@ -950,8 +950,7 @@ static int backward(sn_replica* r, const float* x, int rows, int first = -1, int
             const ConvGeom cg{rows, (int)conv.in_dims[0], (int)conv.in_dims[1], (int)conv.in_dims[2], (int)conv.out_dims[0],
                               (int)conv.out_dims[1], (int)conv.out_dims[2], conv.kh, conv.kw, conv.sh, conv.sw, conv.pt, conv.pl};
             const bool deferred = r->defer_now && r->ws_defer[0] && r->n_deferred < MAX_DEFERRED;
-            const bool aligned = ((reinterpret_cast<uintptr_t>(dy) | reinterpret_cast<uintptr_t>(r->arg[i]) | reinterpret_cast<uintptr_t>(r->act[0])) & 15u) == 0;
-            if (aligned && conv_wgrad_is_direct(ctx, cg, deferred ? r->ws_defer[0] : r->ws, m->workspace_elems, true)) {
+            if (conv_wgrad_is_direct(ctx, cg, deferred ? r->ws_defer[0] : r->ws, m->workspace_elems)) {
               pool_grad = PoolGrad{};
               pool_grad.dy = dy; pool_grad.arg = r->arg[i]; pool_grad.y = r->act[0];
               pool_grad.ho = (int)op.out_dims[0]; pool_grad.wo = (int)op.out_dims[1];

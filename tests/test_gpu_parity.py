@@ -469,6 +469,14 @@ MODELS = {
                                             ("dense", 3, "softmax")], "cce", (21, 19, 2), 40, "uniform_onehot"),
     "conv_first_layer_four_filters": ([("conv", 4, (2, 2), (1, 1), "valid", "relu", False), ("flatten",), ("dense", 3, "softmax")],
                                       "cce", (30, 30, 3), 8, "uniform_onehot"),
+    # first-layer filter gradient on 16 x 16 matrix tiles: 48 taps and a filter past the second tile under a stride, no pooling; filters that
+    # fill a tile and a half, 24 of them under non-overlapping and 60 under unevenly strided windows that reach into the padding
+    "conv_first_layer_33_filters_48_taps": ([("conv", 33, (4, 4), (2, 1), "same", "tanh", False), ("flatten",), ("dense", 3, "softmax")], "cce",
+                                            (18, 17, 3), 20, "uniform_onehot"),
+    "conv_pool_first_layer_24_filters_s2": ([("conv", 24, (3, 3), (1, 1), "valid", "relu", False), ("pool", (2, 2), (2, 2), "valid"), ("flatten",),
+                                             ("dense", 3, "softmax")], "cce", (14, 13, 1), 30, "uniform_onehot"),
+    "conv_pool_first_layer_60_filters_s_1_2": ([("conv", 60, (2, 2), (1, 1), "same", "sigmoid", False), ("pool", (2, 2), (1, 2), "same"), ("flatten",),
+                                                ("dense", 3, "softmax")], "cce", (11, 10, 2), 40, "uniform_onehot"),
     # second-layer filter gradient in its row form (32 or 64 input channels): an odd row length (one padding position per row), Same
     # padding on all four sides, a stride in each direction, a bias; and 64 input channels under a 5 x 3 kernel onto 32 filters
     "conv_rows_same_stride_bias": ([("conv", 32, (3, 3), (1, 1), "valid", "relu", False), ("conv", 64, (3, 3), (2, 1), "same", "tanh", True),
@@ -603,6 +611,9 @@ KERNEL_OF_MODEL = {
     "conv_input_gradient_32_channels_2x3_same": "conv2d_input_gradient[",
     "conv_pool_first_layer_same_s1": "maxpool_backward_and_conv2d_filter_gradient_direct",
     "conv_first_layer_uneven": "conv2d_filter_gradient_direct",
+    "conv_first_layer_33_filters_48_taps": "conv2d_filter_gradient_direct",
+    "conv_pool_first_layer_24_filters_s2": "maxpool_backward_and_conv2d_filter_gradient_direct",
+    "conv_pool_first_layer_60_filters_s_1_2": "maxpool_backward_and_conv2d_filter_gradient_direct",
     "batchnorm_pool_first_layer_same_s1": "batchnorm_gradient_sums_from_maxpool",
     "batchnorm_pool_48_channels_stride_2_1": "batchnorm_gradient_sums_from_maxpool",
     "batchnorm_pool_second_layer": "batchnorm_apply_and_maxpool",
