@@ -559,9 +559,20 @@ bool vec4_ok(int cols, std::initializer_list<const void*> ptrs) {
 
 int64_t batchnorm_workspace_elems(const sn_ctx* ctx, int64_t rows, int cols) { return (int64_t)2 * max_slices(ctx, rows, cols) * cols; }
 
+ConvStats batchnorm_conv_stats(const sn_ctx* ctx, int64_t rows, int cols, float* ws, int64_t ws_elems) {
+  ConvStats st;
+  const int64_t slices = max_slices(ctx, rows, cols), half = slices * cols;
+  if (ws && 2 * half <= ws_elems) {
+    st.part_mean = ws;
+    st.part_m2 = ws + half;
+    st.max_slices = (int)slices;
+  }
+  return st;
+}
+
 // mean, var and what follows from them (BnScale)
 static int batchnorm_statistics(sn_ctx* ctx, const float* x, int64_t rows, int cols, const BatchNormArgs& a, bool training, float* ws,
-                                int64_t ws_elems) {
+                                int64_t ws_elems, const ConvStats* stats) {
   SN_REQUIRE(rows * cols <= (int64_t)INT32_MAX * 4, "batch norm over %lld elements exceeds one launch", (long long)(rows * cols));
   const int cb = (int)ceil_div((int64_t)cols, (int64_t)FINISH_CHANNELS);
   if (!training) {
@@ -574,7 +585,11 @@ static int batchnorm_statistics(sn_ctx* ctx, const float* x, int64_t rows, int c
   const int64_t half = (int64_t)max_slices(ctx, rows, cols) * cols;
   const BnScale scale = bn_scale_of(a, rows, a.fused_wiring);
   SN_REQUIRE(half <= ws_elems, "batch norm needs %lld workspace elements, %lld given", (long long)half, (long long)ws_elems);
-  if (2 * half <= ws_elems && stream_ok(rows, cols, x, nullptr, ws, half)) {
+  if (stats && stats->slices > 0) {
+    LaunchScope scope(ctx, "batchnorm_mean_and_variance");
+    hipLaunchKernelGGL(bn_moments_kernel, dim3(cb), dim3(256), 0, ctx->stream, (const float*)stats->part_mean, (const float*)stats->part_m2, stats->slices,
+                       cols, stats->whole, stats->last, (float)rows, scale);
+  } else if (2 * half <= ws_elems && stream_ok(rows, cols, x, nullptr, ws, half)) {
     const Stream st = stream_of(ctx, rows, cols);
     LaunchScope scope(ctx, "batchnorm_mean_and_variance");
     hipLaunchKernelGGL(bn_stats_v4_kernel, dim3((unsigned)st.slices), dim3(256), 0, ctx->stream, (const bn_f4*)x, ws, ws + half, st.n4, cols, st.active,
@@ -597,9 +612,9 @@ static int batchnorm_statistics(sn_ctx* ctx, const float* x, int64_t rows, int c
 }
 
 int launch_batchnorm_fwd(sn_ctx* ctx, const float* x, float* y, int64_t rows, int cols, const BatchNormArgs& a, bool training, float* ws,
-                         int64_t ws_elems) {
+                         int64_t ws_elems, const ConvStats* stats) {
   if (rows <= 0 || cols <= 0) return SN_OK;
-  SN_TRY(batchnorm_statistics(ctx, x, rows, cols, a, training, ws, ws_elems));
+  SN_TRY(batchnorm_statistics(ctx, x, rows, cols, a, training, ws, ws_elems, stats));
   const int64_t n = rows * cols;
   LaunchScope scope(ctx, "batchnorm_apply");
   if (vec4_ok(cols, {x, y, a.mean, a.inv, a.beta}))
@@ -624,8 +639,8 @@ bool batchnorm_pool_ok(const PoolGeom& g, const BatchNormArgs& a, const float* x
 }
 
 int launch_batchnorm_pool_fwd(sn_ctx* ctx, const float* x, float* y, uint8_t* arg, const PoolGeom& g, const BatchNormArgs& a, bool training, float* ws,
-                              int64_t ws_elems) {
-  SN_TRY(batchnorm_statistics(ctx, x, (int64_t)g.n * g.h * g.w, g.c, a, training, ws, ws_elems));
+                              int64_t ws_elems, const ConvStats* stats) {
+  SN_TRY(batchnorm_statistics(ctx, x, (int64_t)g.n * g.h * g.w, g.c, a, training, ws, ws_elems, stats));
   const int64_t total = (int64_t)g.n * g.ho * g.wo * g.c / 4;
   LaunchScope scope(ctx, "batchnorm_apply_and_maxpool");
   hipLaunchKernelGGL(bn_pool2x2_fwd_kernel, dim3((grid_for(ctx, total, 256) + 7u) & ~7u), dim3(256), 0, ctx->stream, x, (const float*)a.mean,

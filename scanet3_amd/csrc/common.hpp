@@ -276,8 +276,11 @@ struct BatchNormArgs {
 // workspace (elements) the reductions need for a [rows, cols] activation
 int64_t batchnorm_workspace_elems(const sn_ctx* ctx, int64_t rows, int cols);
 // y = (x*inv - mean*inv) + beta; training: batch statistics, else the moving ones
+// stats (training only, may be null or hold no slices): partial statistics of x that its producer has left in ws
+struct ConvStats;
+ConvStats batchnorm_conv_stats(const sn_ctx* ctx, int64_t rows, int cols, float* ws, int64_t ws_elems);  // ... and where it may leave them
 int launch_batchnorm_fwd(sn_ctx* ctx, const float* x, float* y, int64_t rows, int cols, const BatchNormArgs& a, bool training, float* ws,
-                         int64_t ws_elems);
+                         int64_t ws_elems, const ConvStats* stats = nullptr);
 // gradients of beta, gamma and (dx != null) the input, through the batch statistics; with below_act the input
 // gradient also passes through the activation that produced x (x is that activation's output)
 int launch_batchnorm_bwd(sn_ctx* ctx, const float* x, const float* dy, float* dx, int64_t rows, int cols, const BatchNormArgs& a,
@@ -291,7 +294,7 @@ struct PoolGeom {
 };
 bool batchnorm_pool_ok(const PoolGeom& g, const BatchNormArgs& a, const float* x, const float* y, const uint8_t* arg);
 int launch_batchnorm_pool_fwd(sn_ctx* ctx, const float* x, float* y, uint8_t* arg, const PoolGeom& g, const BatchNormArgs& a, bool training, float* ws,
-                              int64_t ws_elems);
+                              int64_t ws_elems, const ConvStats* stats = nullptr);
 int launch_batchnorm_pool_bwd(sn_ctx* ctx, const float* x, const float* dy, const uint8_t* arg, const PoolGeom& g, const BatchNormArgs& a, float* dbeta,
                               float* dgamma, float* ws, int64_t ws_elems);
 // moving = momentum*moving + (1-momentum)*batch
@@ -399,7 +402,20 @@ struct ConvGeom {
 bool conv_wgrad_taps_shape(const sn_ctx* ctx, const ConvGeom& g, const float* x, const float* dy);
 int64_t conv_wgrad_taps_workspace(const sn_ctx* ctx, const ConvGeom& g);  // floats of workspace
 int launch_conv_wgrad_taps(sn_ctx* ctx, const ConvGeom& g, const float* x, const float* dy, float* ws, int64_t ws_elems, int* parts);
-int launch_conv_fwd(sn_ctx* ctx, const ConvGeom& g, const float* x, const float* w, const Epilogue& ep, float* ws, int64_t ws_elems);
+// Partial statistics of a convolution's output for the batch normalisation above it (batchnorm_conv_stats): where the kernel that
+// runs can, it leaves mean and squared deviations of `slices` runs of output positions (`whole` each, the last one `last`).
+struct ConvStats {
+  float* part_mean = nullptr;  // [slice][cout], room for max_slices
+  float* part_m2 = nullptr;
+  int max_slices = 0;
+  int slices = 0;              // 0: the kernel that ran does not form them
+  float whole = 0.f, last = 0.f;
+};
+int launch_conv_fwd(sn_ctx* ctx, const ConvGeom& g, const float* x, const float* w, const Epilogue& ep, float* ws, int64_t ws_elems,
+                    ConvStats* stats = nullptr);
+// First layers (conv_first_kernels.hip): up to 4 input channels and 64 taps, whole vectors of filters
+bool conv_first_fwd_ok(const ConvGeom& g, const Epilogue& e);
+int launch_conv_first_fwd(sn_ctx* ctx, const ConvGeom& g, const float* x, const float* w, const Epilogue& e, ConvStats* stats);
 int launch_conv_dgrad(sn_ctx* ctx, const ConvGeom& g, const float* dy, const float* w, float* dx, float* ws, int64_t ws_elems);
 // A 2 x 2 max pooling right above a first-layer convolution, for launch_conv_wgrad's first-layer kernel: the pooling's output
 // gradient dy [n, ho, wo, cout], its recorded first-maximum offsets (one byte per output value) and the convolution's saved

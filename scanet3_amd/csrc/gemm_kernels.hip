@@ -830,205 +830,10 @@ int launch_gemm(sn_ctx* ctx, const GemmDesc& g, const Epilogue& ep, float* works
 }
 
 // ---------------------------------------------------------------------------- Conv2D
-// First-layer convolutions (1 to 4 input channels): K = kh*kw*cin is a few dozen, far too short for MFMA tiles
-// to pay for their set-up, and the layer is bound by writing its output.  Direct form: the filter sits in LDS,
-// 8 neighbouring lanes share one output pixel and own 4 output channels each (so a pixel's channels leave as
-// one contiguous run), every lane gathers the pixel's K inputs itself (they stay in L1).
-constexpr int DIRECT_MAX_K = 64;
-__global__ __launch_bounds__(256) void conv_direct_fwd_kernel(ConvGeom g, const float* __restrict__ x, const float* __restrict__ w,
-                                                               Epilogue e, int pixels) {
-  extern __shared__ __attribute__((aligned(16))) float wl[];  // [K][cout]
-  const int K = g.kh * g.kw * g.cin;
-  for (int i = threadIdx.x; i < K * g.cout; i += 256) wl[i] = w[i];
-  __syncthreads();
-  const int quads = g.cout / 4;  // channel quads per pixel
-  const int64_t total = (int64_t)pixels * quads;
-  for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < total; t += (int64_t)gridDim.x * 256) {
-    const int cq = (int)(t % quads);
-    const int p = (int)(t / quads);
-    const int ow = p % g.wo;
-    const int t2 = p / g.wo;
-    const int oh = t2 % g.ho;
-    const int b = t2 / g.ho;
-    const int iy0 = oh * g.sh - g.pt, ix0 = ow * g.sw - g.pl;
-    const float* img = x + (int64_t)b * g.h * g.w * g.cin;
-    f4v acc = {0.f, 0.f, 0.f, 0.f};
-    int k = 0;
-    for (int r = 0; r < g.kh; ++r) {
-      const int iy = iy0 + r;
-      for (int q = 0; q < g.kw; ++q) {
-        const int ix = ix0 + q;
-        const bool in = (unsigned)iy < (unsigned)g.h && (unsigned)ix < (unsigned)g.w;
-        for (int ci = 0; ci < g.cin; ++ci, ++k) {
-          const float xv = in ? img[(iy * g.w + ix) * g.cin + ci] : 0.f;
-          const f4v wv = *(const f4v*)(wl + k * g.cout + cq * 4);
-#pragma unroll
-          for (int i = 0; i < 4; ++i) acc[i] = __builtin_fmaf(xv, wv[i], acc[i]);  // fused like the matrix cores; k in (r, q, ci) order
-        }
-      }
-    }
-    const int col = cq * 4;
-    f4v out;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      float v = acc[i];
-      if (e.bias) v = v + e.bias[col + i];
-      out[i] = ep_act(e.act, v, e.act_param);
-    }
-    *(f4v*)(e.out + (int64_t)p * e.ldo + col) = out;
-  }
-}
-
-// U pixels of one lane (p0, p0 + slots, ...; all inside the band): taps outermost, so a tap's weights are used U times.
-template <int MT, int U>
-__device__ __forceinline__ void fwd_rows_pixels(const float* lds, const int* origin, const int (&off)[MT], const f4v (&wr)[MT], const f4v& bias,
-                                                const Epilogue& e, float* outb, int p0, int slots) {
-  f4v acc[U];
-  int base[U];
-#pragma unroll
-  for (int u = 0; u < U; ++u) {
-    base[u] = origin[p0 + u * slots];
-    acc[u] = f4v{0.f, 0.f, 0.f, 0.f};
-  }
-#pragma unroll
-  for (int m = 0; m < MT; ++m) {
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const float xv = lds[base[u] + off[m]];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) acc[u][i] = __builtin_fmaf(xv, wr[m][i], acc[u][i]);
-    }
-  }
-  float v[U * 4];
-#pragma unroll
-  for (int u = 0; u < U; ++u) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) v[u * 4 + i] = acc[u][i] + bias[i];
-  }
-  ep_act_block<U * 4>(e.act, v, e.act_param);  // one dispatch on the activation for all of the lane's pixels
-#pragma unroll
-  for (int u = 0; u < U; ++u) *(f4v*)(outb + (int64_t)(p0 + u * slots) * e.ldo) = f4v{v[u * 4], v[u * 4 + 1], v[u * 4 + 2], v[u * 4 + 3]};
-}
-
-// What a launch of the direct first-layer kernel below fixes and the device would otherwise divide out per thread
-// (the device has no integer divider): the LDS offset of tap m = (r, q, ci) from a position's top-left input element
-// (taps >= kh*kw*cin repeat tap 0), and the divisors of the index arithmetic.
-constexpr int DIRECT_ROWS_MAX_TAPS = 18;
-struct DirectConvPlan {
-  int off[DIRECT_ROWS_MAX_TAPS];
-  FastDiv by_wo, by_row_elems, by_cin;
-};
-static DirectConvPlan direct_conv_plan(const ConvGeom& g, int lw) {
-  DirectConvPlan plan;
-  const int M = g.kh * g.kw * g.cin, row_elems = lw * g.cin;
-  for (int m = 0; m < DIRECT_ROWS_MAX_TAPS; ++m) {
-    const int mm = m < M ? m : 0;
-    const int ci = mm % g.cin, rq = mm / g.cin;
-    plan.off[m] = (rq / g.kw) * row_elems + (rq % g.kw) * g.cin + ci;
-  }
-  plan.by_wo = fast_div((uint32_t)g.wo);
-  plan.by_row_elems = fast_div((uint32_t)row_elems);
-  plan.by_cin = fast_div((uint32_t)g.cin);
-  return plan;
-}
-
-// The same layer when the filter count is 4 << j (j = 0..6) and there are at most 18 taps: a workgroup takes a band of
-// output rows of one image and keeps the input rows under it in LDS, zero-padded; a lane owns 4 filters, holds their
-// weights for every tap in registers and walks pixels, so a pixel costs its taps' LDS reads (shared by the lanes of the
-// pixel) and 4 FMAs per tap; the pixel's channels leave as one contiguous run.  Same (r, q, ci) accumulation order.
-// Rows m >= taps of the register arrays carry zero weights (they re-read tap 0), so the tap loop has no branch.
-template <int MT>
-__global__ __launch_bounds__(256) void conv_direct_fwd_rows_kernel(ConvGeom g, const float* __restrict__ x, const float* __restrict__ w,
-                                                                    Epilogue e, int rows_per_band, int bands_per_image, int items, int lw,
-                                                                    int qshift, int staged_full, DirectConvPlan plan) {
-  extern __shared__ float fw_lds[];
-  const int tid = threadIdx.x;
-  const int M = g.kh * g.kw * g.cin;
-  const int row_elems = lw * g.cin;
-  const int quads = 1 << qshift;
-  const int col = (tid & (quads - 1)) * 4;
-  const int slot = tid >> qshift, slots = 256 >> qshift;
-  f4v wr[MT];
-  int off[MT];
-#pragma unroll
-  for (int m = 0; m < MT; ++m) {
-    off[m] = plan.off[m];
-    const f4v zero = {0.f, 0.f, 0.f, 0.f};
-    wr[m] = m < M ? *(const f4v*)(w + (int64_t)m * g.cout + col) : zero;
-  }
-  f4v bias = {0.f, 0.f, 0.f, 0.f};
-  if (e.bias) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) bias[i] = e.bias[col + i];
-  }
-  int* origin = reinterpret_cast<int*>(fw_lds + staged_full);
-  constexpr int U = 4;  // pixels per lane in flight
-  for (int item = blockIdx.x; item < items; item += gridDim.x) {
-    const int b = item / bands_per_image, band = item % bands_per_image;
-    const int oh0 = band * rows_per_band;
-    const int oh1 = oh0 + rows_per_band < g.ho ? oh0 + rows_per_band : g.ho;
-    const int iy0 = oh0 * g.sh - g.pt;
-    const int staged = ((oh1 - oh0 - 1) * g.sh + g.kh) * row_elems;
-    const int P = (oh1 - oh0) * g.wo;
-    __syncthreads();  // the previous item's readers are done with the staged rows
-    for (int el = tid; el < staged; el += 256) {
-      const int row = (int)div_by((uint32_t)el, plan.by_row_elems), rem = el - row * row_elems;
-      const int px = (int)div_by((uint32_t)rem, plan.by_cin);
-      const int iy = iy0 + row, ix = px - g.pl, ci = rem - px * g.cin;
-      fw_lds[el] = ((unsigned)iy < (unsigned)g.h && (unsigned)ix < (unsigned)g.w) ? x[(((int64_t)b * g.h + iy) * g.w + ix) * g.cin + ci] : 0.f;
-    }
-    for (int p = tid; p < P; p += 256) {
-      const int prow = (int)div_by((uint32_t)p, plan.by_wo);
-      origin[p] = prow * g.sh * row_elems + (p - prow * g.wo) * g.sw * g.cin;
-    }
-    __syncthreads();
-    float* outb = e.out + (((int64_t)b * g.ho + oh0) * g.wo) * e.ldo + col;
-    int p0 = slot;
-    for (; p0 + (U - 1) * slots < P; p0 += slots * U) fwd_rows_pixels<MT, U>(fw_lds, origin, off, wr, bias, e, outb, p0, slots);
-    for (; p0 < P; p0 += slots) fwd_rows_pixels<MT, 1>(fw_lds, origin, off, wr, bias, e, outb, p0, slots);
-  }
-}
-
-static bool conv_fwd_rows(sn_ctx* ctx, const ConvGeom& g, const float* x, const float* w, const Epilogue& e, int* rc) {
-  const int N = g.cout, K = g.kh * g.kw * g.cin;
-  const int64_t pixels = (int64_t)g.n * g.ho * g.wo;
-  if (g.cin > 4 || K > 18 || N % 4 != 0 || N > 256 || ((N / 4) & (N / 4 - 1)) != 0 || pixels < 2048) return false;
-  if (e.ldo % 4 != 0 || !aligned16(e.out) || !aligned16(w)) return false;
-  int qshift = 0;
-  while ((4 << qshift) < N) ++qshift;
-  const int lw = (g.wo - 1) * g.sw + g.kw;
-  // a band holds at least ~4 pixels per lane, so staging its input rows is a small part of the work
-  const int rows_per_band = (int)std::min<int64_t>(g.ho, std::max<int64_t>(1, ceil_div((int64_t)1024, (int64_t)(N / 4) * g.wo)));
-  const int bands = (int)ceil_div((int64_t)g.ho, (int64_t)rows_per_band);
-  const int64_t items = (int64_t)g.n * bands;
-  const int64_t staged = (int64_t)((rows_per_band - 1) * g.sh + g.kh) * lw * g.cin;
-  const int64_t lds_floats = staged + (int64_t)rows_per_band * g.wo;
-  if (lds_floats * 4 > 48 * 1024 || items >= (int64_t)1 << 30) return false;
-  const unsigned blocks = (unsigned)std::min<int64_t>(items, (int64_t)ctx->compute_units * 8);
-  const DirectConvPlan plan = direct_conv_plan(g, lw);
-  LaunchScope scope(ctx, "conv2d_forward_direct", (int)pixels, N, K);
-#define SN_FWD_ROWS(MT)                                                                                                                  \
-  hipLaunchKernelGGL((conv_direct_fwd_rows_kernel<MT>), dim3(blocks), dim3(256), (size_t)lds_floats * sizeof(float), ctx->stream, g, x, w, e, \
-                     rows_per_band, bands, (int)items, lw, qshift, (int)staged, plan)
-  if (K <= 9) SN_FWD_ROWS(9);
-  else SN_FWD_ROWS(18);
-#undef SN_FWD_ROWS
-  *rc = hipGetLastError() == hipSuccess ? SN_OK : fail(SN_E_HIP, "conv2d_forward_direct: launch failed");
-  return true;
-}
-
-int launch_conv_fwd(sn_ctx* ctx, const ConvGeom& g, const float* x, const float* w, const Epilogue& e, float* ws, int64_t ws_elems) {
+int launch_conv_fwd(sn_ctx* ctx, const ConvGeom& g, const float* x, const float* w, const Epilogue& e, float* ws, int64_t ws_elems,
+                    ConvStats* stats) {
   const int M = g.n * g.ho * g.wo, N = g.cout, K = g.kh * g.kw * g.cin;
-  int rows_rc = SN_OK;
-  if (conv_fwd_rows(ctx, g, x, w, e, &rows_rc)) return rows_rc;
-  if (g.cin <= 4 && K <= DIRECT_MAX_K && N % 4 == 0 && (size_t)K * N * sizeof(float) <= 48 * 1024 && e.ldo % 4 == 0 && aligned16(e.out) && M > 0) {
-    const int64_t total = (int64_t)M * (N / 4);
-    const unsigned blocks = (unsigned)std::min<int64_t>(ceil_div(total, 256), (int64_t)ctx->compute_units * 32);
-    LaunchScope scope(ctx, "conv2d_forward_direct", M, N, K);
-    hipLaunchKernelGGL(conv_direct_fwd_kernel, dim3(blocks), dim3(256), (size_t)K * N * sizeof(float), ctx->stream, g, x, w, e, M);
-    SN_HIP(hipGetLastError());
-    return SN_OK;
-  }
+  if (conv_first_fwd_ok(g, e)) return launch_conv_first_fwd(ctx, g, x, w, e, stats);
   if (conv_ring_fwd_ok(g, x, w, e)) return launch_conv_ring_fwd(ctx, g, x, w, e);
   StdEpilogue ep{e};
   if (!conv_prefers_float32_tiles(M, N, K, g.cin) && split_conv_fwd_ok(g, x, w)) return launch_split_conv_fwd(ctx, g, x, w, e, ws, ws_elems);

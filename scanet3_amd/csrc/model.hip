@@ -615,6 +615,7 @@ static int forward(sn_replica* r, const float* x, int rows, bool skip_last = fal
                                 (int)m->ops[i].out_elems, r->bf_w[i], nullptr, 0, 0.f, nullptr));
     r->bf_weights_stale = false;
   }
+  ConvStats conv_stats;  // what the convolution right below a batch normalisation has left in the workspace
   std::vector<char> bf_ready(m->ops.size() + 1, 0);  // op i's bf16 input copies were written by op i-1's epilogue
   for (size_t i = 0; i + (skip_last ? 1 : 0) < m->ops.size(); ++i) {
     const Op& op = m->ops[i];
@@ -659,7 +660,10 @@ static int forward(sn_replica* r, const float* x, int rows, bool skip_last = fal
                    (int)op.out_dims[2], op.kh, op.kw, op.sh, op.sw, op.pt, op.pl};
         Epilogue ep;
         ep.out = r->act[i]; ep.ldo = g.cout; ep.bias = param_ptr(r, r->w, op.b); ep.act = op.act; ep.act_param = op.act_param;
-        SN_TRY(launch_conv_fwd(ctx, g, in, param_ptr(r, r->w, op.w), ep, r->ws, m->workspace_elems));
+        conv_stats = ConvStats{};
+        if (training && i + 1 < m->ops.size() && m->ops[i + 1].kind == OP_BATCHNORM)  // its statistics, if this product can form them
+          conv_stats = batchnorm_conv_stats(ctx, (int64_t)rows * g.ho * g.wo, g.cout, r->ws, m->workspace_elems);
+        SN_TRY(launch_conv_fwd(ctx, g, in, param_ptr(r, r->w, op.w), ep, r->ws, m->workspace_elems, &conv_stats));
         break;
       }
       case OP_POOL:
@@ -718,13 +722,14 @@ static int forward(sn_replica* r, const float* x, int rows, bool skip_last = fal
       }
       case OP_BATCHNORM: {
         const int c = (int)op.out_dims.back();
+        const ConvStats* const stats = training && i > 0 && m->ops[i - 1].kind == OP_CONV ? &conv_stats : nullptr;
         if (batchnorm_pool_path(r, i, x, rows)) {
           SN_TRY(launch_batchnorm_pool_fwd(ctx, in, r->act[i + 1], r->arg[i + 1], pool_geom(m->ops[i + 1], rows), batchnorm_args(r, op, (int)i), training,
-                                           r->ws, m->workspace_elems));
+                                           r->ws, m->workspace_elems, stats));
           break;
         }
         SN_TRY(launch_batchnorm_fwd(ctx, in, r->act[i], (int64_t)rows * (op.out_elems / c), c, batchnorm_args(r, op, (int)i), training, r->ws,
-                                    m->workspace_elems));
+                                    m->workspace_elems, stats));
         break;
       }
       case OP_SRNN: {

@@ -477,6 +477,11 @@ MODELS = {
                                              ("dense", 3, "softmax")], "cce", (14, 13, 1), 30, "uniform_onehot"),
     "conv_pool_first_layer_60_filters_s_1_2": ([("conv", 60, (2, 2), (1, 1), "same", "sigmoid", False), ("pool", (2, 2), (1, 2), "same"), ("flatten",),
                                                 ("dense", 3, "softmax")], "cce", (11, 10, 2), 40, "uniform_onehot"),
+    # first-layer forward: 64 taps, filters past one launch column of 64, a bias; the same with the statistics of a BatchNorm formed on the way
+    "conv_first_layer_100_filters_64_taps": ([("conv", 100, (4, 4), (1, 2), "same", "sigmoid", True), ("flatten",), ("dense", 3, "softmax")], "cce",
+                                             (9, 11, 4), 6, "uniform_onehot"),
+    "batchnorm_over_first_layer_100_filters": ([("conv", 100, (3, 2), (1, 1), "valid", "tanh", False), ("batchnorm", 0.9, 1e-3), ("flatten",),
+                                                ("dense", 3, "softmax")], "cce", (9, 8, 3), 21, "uniform_onehot"),
     # second-layer filter gradient in its row form (32 or 64 input channels): an odd row length (one padding position per row), Same
     # padding on all four sides, a stride in each direction, a bias; and 64 input channels under a 5 x 3 kernel onto 32 filters
     "conv_rows_same_stride_bias": ([("conv", 32, (3, 3), (1, 1), "valid", "relu", False), ("conv", 64, (3, 3), (2, 1), "same", "tanh", True),
