@@ -696,51 +696,110 @@ __global__ __launch_bounds__(256) void pool_fwd_kernel(const float* __restrict__
     const I o = i * V;
     if constexpr (V == 4) {
       *(float4*)(y + o) = make_float4(best[0], best[1], best[2], best[3]);
-      if constexpr (!AVG) *(uint32_t*)(arg + o) = (uint32_t)at[0] | ((uint32_t)at[1] << 8) | ((uint32_t)at[2] << 16) | ((uint32_t)at[3] << 24);
+      if (!AVG && arg) *(uint32_t*)(arg + o) = (uint32_t)at[0] | ((uint32_t)at[1] << 8) | ((uint32_t)at[2] << 16) | ((uint32_t)at[3] << 24);
     } else {
       y[o] = best[0];
-      if constexpr (!AVG) arg[o] = (uint8_t)at[0];
+      if (!AVG && arg) arg[o] = (uint8_t)at[0];
     }
   }
 }
 
 
-// The same forward pass for 2x2 max windows, 4 channels per thread, 32-bit indices: the four window cells are requested
-// together (cells outside the input re-read the tensor's first element and never win), then compared in window order.
+// The same forward pass for 2x2 max windows, 32-bit indices, V channels and R output rows of one column per thread, all of whose
+// input cells are requested together (cells outside the input re-read the tensor's first element and never win).  Bound by
+// the requests in flight: one window per thread and trip kept 3 TB/s.  SHARE (row stride 1): neighbouring windows have a row of
+// cells in common, which is read and compared once.  The two cells of a row are compared first, then the two rows, and only a
+// larger value replaces an earlier one: the first maximum in window order, as one by one.
+// ARG = false: nothing will ask which cell won (a prediction).
+// [1000 x 26 x 26 x 32] and [1000 x 23 x 23 x 64], stride 1, predicted: 29.6 and 46.6 us
+// (5.6 TB/s), by single windows with their cells recorded 141 together.
+template <int V>
+struct PoolCells {
+  float v[V];
+  uint32_t at;  // V bytes: the winning cell of each
+};
+template <int V, int R, bool SHARE, bool ARG>
 __global__ __launch_bounds__(256) void pool2x2_fwd_kernel(const float* __restrict__ x, float* __restrict__ y, uint8_t* __restrict__ arg,
-                                                           int n, int h, int w, int c, int ho, int wo, int sh, int sw, int pt, int pl,
-                                                           FastDiv by_cv, FastDiv by_wo, FastDiv by_ho) {
-  const uint32_t cv = (uint32_t)(c / 4);
-  const uint32_t total = (uint32_t)n * ho * wo * cv;
-  const uint32_t stride = (uint32_t)gridDim.x * blockDim.x;
-  for (uint32_t i = (uint32_t)xcd_contiguous_block() * blockDim.x + threadIdx.x; i < total; i += stride) {
-    uint32_t t = div_by(i, by_cv);
-    const uint32_t ch = (i - t * cv) * 4;
-    uint32_t t2 = div_by(t, by_wo);
-    const int ow = (int)(t - t2 * (uint32_t)wo);
-    const uint32_t b = div_by(t2, by_ho);
-    const int oh = (int)(t2 - b * (uint32_t)ho);
-    float4 val[4];
-    bool in[4];
+                                                           uint32_t items, int h, int w, int c, int ho, int wo, int sh, int sw, int pt, int pl,
+                                                           FastDiv by_cv, FastDiv by_wo, FastDiv by_strips) {
+  constexpr int ROWS = SHARE ? R + 1 : 2 * R;
+  const uint32_t i = (uint32_t)xcd_contiguous_block() * blockDim.x + threadIdx.x;
+  if (i >= items) return;
+  const uint32_t t = div_by(i, by_cv), ch = (i - t * by_cv.d) * V;
+  const uint32_t t2 = div_by(t, by_wo), b = div_by(t2, by_strips);
+  const int ow = (int)(t - t2 * (uint32_t)wo), oh0 = (int)(t2 - b * by_strips.d) * R;
+  const int ix0 = ow * sw - pl, iy0 = oh0 * sh - pt;
+  float cell[ROWS][2][V];
+  bool in[ROWS][2];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int iy = oh * sh - pt + (k >> 1), ix = ow * sw - pl + (k & 1);
-      in[k] = (unsigned)iy < (unsigned)h && (unsigned)ix < (unsigned)w;
-      val[k] = *(const float4*)(x + (in[k] ? ((b * h + iy) * w + ix) * c + ch : 0u));
+  for (int k = 0; k < ROWS; ++k) {
+    const int iy = SHARE ? iy0 + k : iy0 + (k >> 1) * sh + (k & 1);
+    const bool row = (unsigned)iy < (unsigned)h;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      in[k][q] = row && (unsigned)(ix0 + q) < (unsigned)w;
+      const float* const src = x + (in[k][q] ? ((b * h + iy) * w + ix0 + q) * c + ch : 0u);
+      if constexpr (V == 4) {
+        const float4 f = *(const float4*)src;
+        cell[k][q][0] = f.x; cell[k][q][1] = f.y; cell[k][q][2] = f.z; cell[k][q][3] = f.w;
+      } else {
+        cell[k][q][0] = *src;
+      }
     }
-    float best[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
-    uint32_t at[4] = {0u, 0u, 0u, 0u};
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const float v[4] = {val[k].x, val[k].y, val[k].z, val[k].w};
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (in[k] && v[e] > best[e]) { best[e] = v[e]; at[e] = (uint32_t)k; }
-    }
-    const uint32_t o = i * 4;
-    *(float4*)(y + o) = make_float4(best[0], best[1], best[2], best[3]);
-    *(uint32_t*)(arg + o) = at[0] | (at[1] << 8) | (at[2] << 16) | (at[3] << 24);
   }
+  auto row_of = [&](int k) {
+    PoolCells<V> r;
+    r.at = 0u;
+#pragma unroll
+    for (int e = 0; e < V; ++e) {
+      r.v[e] = -INFINITY;
+      if (in[k][0] && cell[k][0][e] > r.v[e]) r.v[e] = cell[k][0][e];
+      const bool second = in[k][1] && cell[k][1][e] > r.v[e];
+      if (second) r.v[e] = cell[k][1][e];
+      if constexpr (ARG) r.at |= second ? 1u << (8 * e) : 0u;
+    }
+    return r;
+  };
+  PoolCells<V> upper;
+  if constexpr (SHARE) upper = row_of(0);
+#pragma unroll
+  for (int k = 0; k < R; ++k) {
+    if constexpr (!SHARE) upper = row_of(2 * k);
+    const PoolCells<V> lower = row_of(SHARE ? k + 1 : 2 * k + 1);
+    float best[V];
+    uint32_t at = 0u;
+#pragma unroll
+    for (int e = 0; e < V; ++e) {
+      const bool down = lower.v[e] > upper.v[e];
+      best[e] = down ? lower.v[e] : upper.v[e];
+      if constexpr (ARG) at |= down ? (lower.at & (255u << (8 * e))) | (2u << (8 * e)) : upper.at & (255u << (8 * e));
+    }
+    if (oh0 + k < ho) {
+      const uint32_t o = ((b * ho + oh0 + k) * wo + ow) * c + ch;
+      if constexpr (V == 4) *(float4*)(y + o) = make_float4(best[0], best[1], best[2], best[3]);
+      else y[o] = best[0];
+      if constexpr (ARG) {
+        if constexpr (V == 4) *(uint32_t*)(arg + o) = at;
+        else arg[o] = (uint8_t)at;
+      }
+    }
+    if constexpr (SHARE) upper = lower;
+  }
+}
+
+template <int V, int R, bool SHARE>
+static void launch_pool2x2_fwd(sn_ctx* ctx, const float* x, float* y, uint8_t* arg, int n, int h, int w, int c, int ho, int wo, int sh, int sw,
+                               int pt, int pl) {
+  const int strips = (int)ceil_div(ho, R);
+  const uint32_t items = (uint32_t)n * (uint32_t)strips * (uint32_t)wo * (uint32_t)(c / V);  // (at most outputs / V)
+  const dim3 grid((unsigned)((ceil_div(items, 256) + 7) & ~(int64_t)7));
+  const FastDiv by_cv = fast_div((uint32_t)(c / V)), by_wo = fast_div((uint32_t)wo), by_strips = fast_div((uint32_t)strips);
+  if (arg)
+    hipLaunchKernelGGL((pool2x2_fwd_kernel<V, R, SHARE, true>), grid, dim3(256), 0, ctx->stream, x, y, arg, items, h, w, c, ho, wo, sh, sw, pt, pl, by_cv,
+                       by_wo, by_strips);
+  else
+    hipLaunchKernelGGL((pool2x2_fwd_kernel<V, R, SHARE, false>), grid, dim3(256), 0, ctx->stream, x, y, arg, items, h, w, c, ho, wo, sh, sw, pt, pl, by_cv,
+                       by_wo, by_strips);
 }
 
 static bool pool_vec4(const void* a, const void* b, const void* m, int c) {
@@ -760,9 +819,19 @@ int launch_pool_fwd(sn_ctx* ctx, bool avg, const float* x, float* y, uint8_t* ar
     if (avg) hipLaunchKernelGGL((pool_fwd_kernel<V, I, true>), grid, dim3(256), 0, ctx->stream, x, y, arg, n, h, w, c, ho, wo, kh, kw, sh, sw, pt, pl); \
     else hipLaunchKernelGGL((pool_fwd_kernel<V, I, false>), grid, dim3(256), 0, ctx->stream, x, y, arg, n, h, w, c, ho, wo, kh, kw, sh, sw, pt, pl);    \
   } while (0)
-  if (v4 && small && !avg && kh == 2 && kw == 2)
-    hipLaunchKernelGGL(pool2x2_fwd_kernel, grid, dim3(256), 0, ctx->stream, x, y, arg, n, h, w, c, ho, wo, sh, sw, pt, pl, fast_div((uint32_t)(c / 4)),
-                       fast_div((uint32_t)wo), fast_div((uint32_t)ho));
+  if (small && !avg && kh == 2 && kw == 2) {
+    // strips of rows once a window per thread gives every CU more than its 2048 threads (125 x 16 x 16 x 48: 5.8 us by windows, 6.4 by strips)
+    const bool strips = total / (v4 ? 4 : 1) > (int64_t)ctx->compute_units * 2048;
+#define SN_POOL2X2_FWD(V)                                                                                                   \
+  do {                                                                                                                      \
+    if (!strips) launch_pool2x2_fwd<V, 1, false>(ctx, x, y, arg, n, h, w, c, ho, wo, sh, sw, pt, pl);                          \
+    else if (sh == 1) launch_pool2x2_fwd<V, 4, true>(ctx, x, y, arg, n, h, w, c, ho, wo, sh, sw, pt, pl);                    \
+    else launch_pool2x2_fwd<V, 2, false>(ctx, x, y, arg, n, h, w, c, ho, wo, sh, sw, pt, pl);                                  \
+  } while (0)
+    if (v4) SN_POOL2X2_FWD(4);
+    else SN_POOL2X2_FWD(1);
+#undef SN_POOL2X2_FWD
+  }
   else if (v4 && small) SN_POOL_FWD(4, uint32_t);
   else if (v4) SN_POOL_FWD(4, uint64_t);
   else if (small) SN_POOL_FWD(1, uint32_t);
@@ -850,21 +919,23 @@ __global__ __launch_bounds__(256) void pool_bwd_kernel(const float* __restrict__
   }
 }
 
-// The same backward pass for 2x2 max windows, 4 channels per thread, 32-bit indices: an input element lies in at most 2 x 2
+// The same backward pass for 2x2 max windows, V channels per thread, 32-bit indices: an input element lies in at most 2 x 2
 // windows (oh_hi - a, ow_hi - d for a, d in {0, 1}); their argmax words and gradients are requested together (windows that do
 // not exist re-read the first element and are ignored) and added in the order of the general kernel (oh, then ow, ascending).
-template <int S>  // both strides when they are equal and 1 or 2 (divisions by a constant), 0: read sh, sw
+template <int V>
+using pool_vec = float __attribute__((ext_vector_type(V)));
+template <int V, int S>  // S: both strides when they are equal and 1 or 2 (divisions by a constant), 0: read sh, sw
 __global__ __launch_bounds__(256) void pool2x2_bwd_kernel(const float* __restrict__ dy, const uint8_t* __restrict__ arg,
                                                            float* __restrict__ dx, int n, int h, int w, int c, int ho, int wo, int sh_,
                                                            int sw_, int pt, int pl, const float* __restrict__ y_in, int act, float act_param,
                                                            FastDiv by_cv, FastDiv by_w, FastDiv by_h) {
   const int sh = S ? S : sh_, sw = S ? S : sw_;
-  const uint32_t cv = (uint32_t)(c / 4);
+  const uint32_t cv = (uint32_t)(c / V);
   const uint32_t total = (uint32_t)n * h * w * cv;
   const uint32_t stride = (uint32_t)gridDim.x * blockDim.x;
   for (uint32_t i = (uint32_t)xcd_contiguous_block() * blockDim.x + threadIdx.x; i < total; i += stride) {
     uint32_t t = div_by(i, by_cv);
-    const uint32_t ch = (i - t * cv) * 4;
+    const uint32_t ch = (i - t * cv) * V;
     uint32_t t2 = div_by(t, by_w);
     const int ix = (int)(t - t2 * (uint32_t)w);
     const uint32_t b = div_by(t2, by_h);
@@ -877,10 +948,10 @@ __global__ __launch_bounds__(256) void pool2x2_bwd_kernel(const float* __restric
     ow_lo = ow_lo <= 0 ? 0 : (ow_lo + sw - 1) / sw;
     int ow_hi = (ix + pl) / sw;
     if (ow_hi > wo - 1) ow_hi = wo - 1;
-    float4 yv = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (y_in) yv = *(const float4*)(y_in + i * 4);
+    pool_vec<V> yv = {};
+    if (y_in) yv = *(const pool_vec<V>*)(y_in + i * V);
     uint32_t a4[4], want[4];
-    float4 g[4];
+    pool_vec<V> g[4];
     bool on[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
@@ -888,26 +959,35 @@ __global__ __launch_bounds__(256) void pool2x2_bwd_kernel(const float* __restric
       on[k] = oh <= oh_hi && ow <= ow_hi;
       const uint32_t o = on[k] ? ((b * ho + oh) * wo + ow) * c + ch : 0u;
       want[k] = (uint32_t)((iy - (oh * sh - pt)) * 2 + (ix - (ow * sw - pl)));
-      a4[k] = *(const uint32_t*)(arg + o);
-      g[k] = *(const float4*)(dy + o);
+      a4[k] = V == 4 ? *(const uint32_t*)(arg + o) : (uint32_t)arg[o];
+      g[k] = *(const pool_vec<V>*)(dy + o);
     }
-    float s[4] = {0.f, 0.f, 0.f, 0.f};
+    pool_vec<V> s = {};
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      if (!on[k]) continue;
-      if ((a4[k] & 255u) == want[k]) s[0] += g[k].x;
-      if (((a4[k] >> 8) & 255u) == want[k]) s[1] += g[k].y;
-      if (((a4[k] >> 16) & 255u) == want[k]) s[2] += g[k].z;
-      if ((a4[k] >> 24) == want[k]) s[3] += g[k].w;
+#pragma unroll
+      for (int e = 0; e < V; ++e)
+        if (on[k] && ((a4[k] >> (8 * e)) & 255u) == want[k]) s[e] += g[k][e];
     }
     if (y_in) {
-      s[0] = act_bwd(act, yv.x, s[0], act_param);
-      s[1] = act_bwd(act, yv.y, s[1], act_param);
-      s[2] = act_bwd(act, yv.z, s[2], act_param);
-      s[3] = act_bwd(act, yv.w, s[3], act_param);
+#pragma unroll
+      for (int e = 0; e < V; ++e) s[e] = act_bwd(act, yv[e], s[e], act_param);
     }
-    *(float4*)(dx + i * 4) = make_float4(s[0], s[1], s[2], s[3]);
+    *(pool_vec<V>*)(dx + i * V) = s;
   }
+}
+
+template <int V>
+static void launch_pool2x2_bwd(sn_ctx* ctx, const dim3& grid, const float* dy, const uint8_t* arg, float* dx, int n, int h, int w, int c, int ho, int wo,
+                               int sh, int sw, int pt, int pl, const float* y_in, int act, float act_param) {
+  const FastDiv by_cv = fast_div((uint32_t)(c / V)), by_w = fast_div((uint32_t)w), by_h = fast_div((uint32_t)h);
+#define SN_POOL2X2_BWD(S)                                                                                                                  \
+  hipLaunchKernelGGL((pool2x2_bwd_kernel<V, S>), grid, dim3(256), 0, ctx->stream, dy, arg, dx, n, h, w, c, ho, wo, sh, sw, pt, pl, y_in, act, \
+                     act_param, by_cv, by_w, by_h)
+  if (sh == 1 && sw == 1) SN_POOL2X2_BWD(1);
+  else if (sh == 2 && sw == 2) SN_POOL2X2_BWD(2);
+  else SN_POOL2X2_BWD(0);
+#undef SN_POOL2X2_BWD
 }
 
 int launch_pool_bwd(sn_ctx* ctx, bool avg, const float* dy, const uint8_t* arg, float* dx, int n, int h, int w, int c, int ho, int wo,
@@ -927,15 +1007,9 @@ int launch_pool_bwd(sn_ctx* ctx, bool avg, const float* dy, const uint8_t* arg, 
       hipLaunchKernelGGL((pool_bwd_kernel<V, I, false>), grid, dim3(256), 0, ctx->stream, dy, arg, dx, n, h, w, c, ho, wo, kh, kw, sh, sw, \
                          pt, pl, y_in, act, act_param);                                                                       \
   } while (0)
-  if (v4 && small && !avg && kh == 2 && kw == 2)
-  {
-    const FastDiv by_cv = fast_div((uint32_t)(c / 4)), by_w = fast_div((uint32_t)w), by_h = fast_div((uint32_t)h);
-    if (sh == 1 && sw == 1)
-      hipLaunchKernelGGL(pool2x2_bwd_kernel<1>, grid, dim3(256), 0, ctx->stream, dy, arg, dx, n, h, w, c, ho, wo, sh, sw, pt, pl, y_in, act, act_param, by_cv, by_w, by_h);
-    else if (sh == 2 && sw == 2)
-      hipLaunchKernelGGL(pool2x2_bwd_kernel<2>, grid, dim3(256), 0, ctx->stream, dy, arg, dx, n, h, w, c, ho, wo, sh, sw, pt, pl, y_in, act, act_param, by_cv, by_w, by_h);
-    else
-      hipLaunchKernelGGL(pool2x2_bwd_kernel<0>, grid, dim3(256), 0, ctx->stream, dy, arg, dx, n, h, w, c, ho, wo, sh, sw, pt, pl, y_in, act, act_param, by_cv, by_w, by_h);
+  if (small && !avg && kh == 2 && kw == 2) {
+    if (v4) launch_pool2x2_bwd<4>(ctx, grid, dy, arg, dx, n, h, w, c, ho, wo, sh, sw, pt, pl, y_in, act, act_param);
+    else launch_pool2x2_bwd<1>(ctx, grid, dy, arg, dx, n, h, w, c, ho, wo, sh, sw, pt, pl, y_in, act, act_param);
   }
   else if (v4 && small) SN_POOL_BWD(4, uint32_t);
   else if (v4) SN_POOL_BWD(4, uint64_t);

@@ -668,7 +668,7 @@ static int forward(sn_replica* r, const float* x, int rows, bool skip_last = fal
       }
       case OP_POOL:
         if (i > 0 && batchnorm_pool_path(r, i - 1, x, rows)) break;  // done with the batch normalisation below
-        SN_TRY(launch_pool_fwd(ctx, op.pool_avg, in, r->act[i], r->arg[i], rows, (int)op.in_dims[0], (int)op.in_dims[1], (int)op.in_dims[2],
+        SN_TRY(launch_pool_fwd(ctx, op.pool_avg, in, r->act[i], training ? r->arg[i] : nullptr, rows, (int)op.in_dims[0], (int)op.in_dims[1], (int)op.in_dims[2],
                                   (int)op.out_dims[0], (int)op.out_dims[1], op.kh, op.kw, op.sh, op.sw, op.pt, op.pl));
         break;
       case OP_FLATTEN:

@@ -255,6 +255,37 @@ def test_golden_conv_and_pool(S, ctx, golden, key, strides, pad):
     h.close()
 
 
+@pytest.mark.parametrize("many", [False, True])
+@pytest.mark.parametrize("channels", [3, 8])
+@pytest.mark.parametrize("height,strides,pad", [(2, (1, 1), "valid"), (5, (1, 1), "valid"), (6, (1, 1), "same"), (9, (1, 2), "same"), (7, (2, 1), "valid"),
+                                                (3, (2, 2), "same"), (11, (3, 3), "same")])
+def test_max_pool_strips(S, ctx, height, strides, pad, channels, many):
+    """A thread pools one window, or four rows (row stride 1) or two of a large tensor: row counts around those, whole vectors of
+    channels and single ones, values with ties and infinities.  Training passes also record the cells, predictions do not: both
+    are the oracle's values.  The recorded cells show in the weight gradient of a 1x1 convolution below: sums of integers."""
+    rng = np.random.default_rng(height)
+    pads = O.PAD_SAME if pad == "same" else O.PAD_VALID
+    per_image = O.max_pool(np.zeros((1, height, 10, channels), f32), (2, 2), strides, pads).size
+    batch = 2100 * 256 * (4 if channels % 4 == 0 else 1) // per_image if many else 3
+    x = rng.integers(-3, 3, (batch, height, 10, channels)).astype(f32)
+    h = Harness(S, ctx, [("conv", channels, (1, 1), (1, 1), "valid", "identity", False), ("pool", (2, 2), strides, pad)], "mse", x.shape[1:], batch)
+    h.rep.set_params({"0/weights": np.eye(channels, dtype=f32).reshape(1, 1, channels, channels)})
+    exp = O.max_pool(x, (2, 2), strides, pads)
+    xb, yb = ctx.to_device(x), ctx.to_device(exp - f32(exp.size / 2.0))  # d loss / d out = 1
+    np.testing.assert_array_equal(h.rep.forward(xb).reshape(exp.shape), exp)
+    np.testing.assert_array_equal(h.rep.forward(xb, training=True).reshape(exp.shape), exp)
+    h.rep.grad(xb, yb)
+    dpool = O.max_pool_grad(x, np.ones_like(exp), (2, 2), strides, pads).reshape(-1, channels)
+    want = x.reshape(-1, channels).astype(np.float64).T @ dpool.astype(np.float64)
+    # d loss / d out is one within a rounding or two, and below 2^22 terms of magnitude 3 add in float32
+    np.testing.assert_allclose(h.rep.get_grads()["0/weights"].reshape(channels, channels), want, rtol=1e-5, atol=1e-5 * np.abs(dpool).sum())
+    h.close()
+    h = Harness(S, ctx, [("pool", (2, 2), strides, pad)], "mse", x.shape[1:], batch)
+    x[rng.random(x.shape) < 0.1] = -np.inf
+    np.testing.assert_array_equal(h.rep.forward(ctx.to_device(x)).reshape(exp.shape), O.max_pool(x, (2, 2), strides, pads))
+    h.close()
+
+
 def test_golden_conv_explicit_padding(S, ctx, golden):
     """math/nn/KernelsSpec.scala (explicit paddings (1, 0), (1, 0), stride 2) through the layer."""
     g = golden["conv2d"]
@@ -545,6 +576,13 @@ MODELS = {
     "batchnorm_pool_second_layer": ([("conv", 4, (2, 2), (1, 1), "valid", "relu", False), ("conv", 8, (2, 2), (1, 1), "valid", "relu", False),
                                      ("batchnorm", 0.9, 1e-3), ("pool", (2, 2), (2, 2), "valid"), ("flatten",), ("dense", 3, "softmax")], "cce",
                                     (11, 9, 1), 50, "uniform_onehot"),
+    # 2 x 2 max poolings of channel counts that are no multiple of four, behind a second layer (a first one pools in its own gradient)
+    "pool_5_channels_same_s1": ([("conv", 4, (2, 2), (1, 1), "valid", "relu", False), ("conv", 5, (2, 2), (1, 1), "valid", "tanh", False),
+                                 ("pool", (2, 2), (1, 1), "same"), ("flatten",), ("dense", 3, "softmax")], "cce", (9, 8, 1), 20, "uniform_onehot"),
+    "pool_7_channels_s2": ([("conv", 4, (2, 2), (1, 1), "valid", "relu", False), ("conv", 7, (2, 2), (1, 1), "valid", "tanh", False),
+                            ("pool", (2, 2), (2, 2), "same"), ("flatten",), ("dense", 3, "softmax")], "cce", (11, 9, 1), 20, "uniform_onehot"),
+    "pool_6_channels_s_3_1": ([("conv", 4, (2, 2), (1, 1), "valid", "relu", False), ("conv", 6, (2, 2), (1, 1), "valid", "sigmoid", False),
+                               ("pool", (2, 2), (3, 1), "valid"), ("flatten",), ("dense", 3, "softmax")], "cce", (12, 9, 1), 20, "uniform_onehot"),
     "dense_identity_mse": ([("dense", 6, "identity")], "mse", (4,), 8, "normal_regression"),
     # Dense >> Dense(Softmax) + CategoricalCrossentropy small enough for the two-launch training pass: a reduction length
     # that is no multiple of 16, rows that are no multiple of 16, all 64 hidden units / 16 classes, penalties on top
