@@ -258,6 +258,8 @@ SN_API int sn_forward(sn_replica* rep, const float* x_dev, int32_t rows, float* 
  * BatchNorm normalises with the statistics of these `rows`.  The next state it would return is not applied;
  * only sn_step and the epoch calls move layer state. */
 SN_API int sn_forward_training(sn_replica* rep, const float* x_dev, int32_t rows, float* out_dev);
+/* sn_forward (training = 0) or sn_forward_training into host memory: waits for the pass, and out_host holds its output. */
+SN_API int sn_forward_host(sn_replica* rep, const float* x_dev, int32_t rows, float* out_host, int32_t training);
 /* sn_forward for callers that cannot allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  It has no counterpart in the reference.  What is tested is that the call leaves
  * the device's free memory unchanged; recording it into a graph is not.  Same result as sn_forward, but every

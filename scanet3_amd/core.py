@@ -274,12 +274,9 @@ class Replica:
     def forward(self, x, rows: Optional[int] = None, training: bool = False) -> np.ndarray:
         """training=False: the frozen model (`TrainedModel.result`); True: `model.resultStateful`'s output."""
         rows = self.model.batch if rows is None else rows
-        out = DeviceBuffer(self.ctx, rows * self.model.out_elems, (rows,) + self.model.output_shape)
-        try:
-            check((lib.sn_forward_training if training else lib.sn_forward)(self.handle, self._ptr(x), rows, out.ptr))
-            return out.numpy()
-        finally:
-            out.free()
+        out = np.empty((max(rows, 0),) + self.model.output_shape, np.float32)
+        check(lib.sn_forward_host(self.handle, self._ptr(x), rows, out.ctypes.data_as(C.c_void_p), int(training)))
+        return out
 
     def forward_static(self, x, out: "DeviceBuffer", rows: Optional[int] = None) -> None:
         """`sn_forward_static`: the frozen forward pass into the caller's buffer, with no device allocation in the call."""
