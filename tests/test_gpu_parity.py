@@ -589,6 +589,10 @@ MODELS = {
     "mlp2_odd_sizes_tanh": ([("dense", 37, "tanh"), ("dense", 16, "softmax")], "cce", (36,), 33, "normal_onehot"),
     "mlp2_64_hidden_relu": ([("dense", 64, "relu"), ("dense", 3, "softmax")], "cce", (1024,), 100, "normal_onehot"),
     "mlp2_identity_one_class": ([("dense", 5, "identity"), ("dense", 1, "softmax")], "cce", (8,), 16, "normal_onehot"),
+    # 65 row blocks of 16 (more than eight a wavefront), a last one of 6 rows, 13 features a wavefront rounded up to 16; 33 row blocks,
+    # 36 features a wavefront of which the last has 8, 17 hidden units
+    "mlp2_1030_rows": ([("dense", 33, "sigmoid"), ("dense", 16, "softmax")], "cce", (100,), 1030, "normal_onehot"),
+    "mlp2_515_rows": ([("dense", 17, "tanh"), ("dense", 2, "softmax")], "cce", (260,), 515, "normal_onehot"),
     "mlp2_regularized": ([("dense", 20, "sigmoid", "l2", 0.05), ("dense", 4, "softmax", "l1", 0.01)], "cce", (8,), 17, "uniform_onehot"),
 }
 
@@ -664,6 +668,8 @@ KERNEL_OF_MODEL = {
     "dense_many_features_16_units": "dense_weight_and_input_gradient_rows",
     "dense_odd_feature_count_9_units": "small_output_reduce_softmax_crossentropy_fused",
     "mlp_cfg1": "mlp2_",
+    "mlp2_1030_rows": "mlp2_",
+    "mlp2_515_rows": "mlp2_",
 }
 
 
