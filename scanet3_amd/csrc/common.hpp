@@ -324,6 +324,17 @@ struct GemmDesc {
 bool split_dense_ok(const GemmDesc& g);
 int launch_split_dense(sn_ctx* ctx, const char* name, const GemmDesc& g, const Epilogue& e, float* ws, int64_t ws_elems, bool bf16);
 int launch_gemm(sn_ctx* ctx, const GemmDesc& g, const Epilogue& ep, float* workspace, int64_t workspace_elems, bool bf16);
+// An input gradient product whose result passes through the gradient of the activation below (y: that activation's output) on
+// the way out; for the products that gemm_act_grad_ok accepts, the form dX = dY . W^T on the split kernels.
+struct ActGrad {
+  float* out;
+  const float* y;
+  int64_t ldo;
+  int act;
+  float act_param;
+};
+bool gemm_act_grad_ok(const sn_ctx* ctx, const GemmDesc& g, const float* workspace, int64_t workspace_elems);
+int launch_split_dense_act_grad(sn_ctx* ctx, const GemmDesc& g, const ActGrad& a, float* ws, int64_t ws_elems, bool bf16);
 // Gradients of a Dense layer from many features onto at most 16 units, as row streams over X (fp32, contiguous
 // [rows, in_f] / [in_f, out_f] / [rows, out_f] tensors); dense_skinny_shape says whether a shape is in their range.
 bool dense_skinny_shape(int rows, int in_f, int out_f);

@@ -829,6 +829,11 @@ int launch_gemm(sn_ctx* ctx, const GemmDesc& g, const Epilogue& ep, float* works
   return bf16 ? launch_gemm_t<true>(ctx, g, ep, workspace, workspace_elems) : launch_gemm_t<false>(ctx, g, ep, workspace, workspace_elems);
 }
 
+// what launch_gemm_t gives to the split kernels, in the operand form of an input gradient
+bool gemm_act_grad_ok(const sn_ctx* ctx, const GemmDesc& g, const float* ws, int64_t ws_elems) {
+  return g.a_sk == 1 && g.b_sk == 1 && g.b_sn != 1 && !g.a_ones_row && !(ws && small_parts(g.m, g.n, g.k, ctx->compute_units, ws_elems)) && split_dense_ok(g);
+}
+
 // ---------------------------------------------------------------------------- Conv2D
 int launch_conv_fwd(sn_ctx* ctx, const ConvGeom& g, const float* x, const float* w, const Epilogue& e, float* ws, int64_t ws_elems,
                     ConvStats* stats) {

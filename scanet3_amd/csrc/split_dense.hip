@@ -36,4 +36,13 @@ int launch_split_dense(sn_ctx* ctx, const char* name, const GemmDesc& g, const E
   return bf16 ? launch_planes<1>(ctx, name, g, e, ws, ws_elems) : launch_planes<3>(ctx, name, g, e, ws, ws_elems);
 }
 
+// dX = dY . W^T through the gradient of the layer below's activation
+int launch_split_dense_act_grad(sn_ctx* ctx, const GemmDesc& g, const ActGrad& a, float* ws, int64_t ws_elems, bool bf16) {
+  SN_REQUIRE(split_dense_ok(g) && g.a_sk == 1 && g.b_sk == 1 && g.b_sn != 1 && !g.a_ones_row, "input gradient outside the split kernels' range");
+  FlatOp<true> al{g.a, (int)g.a_sm, g.m, g.k}, bl{g.b, (int)g.b_sn, g.n, g.k};
+  const ActGradEpilogue ep{a.out, a.y, a.ldo, a.act, a.act_param};
+  return bf16 ? launch_split<1>(ctx, "gemm_bf16_and_activation_gradient", g.m, g.n, g.k, g.m, -1, al, bl, ep, ws, ws_elems)
+              : launch_split<3>(ctx, "gemm_f32_and_activation_gradient", g.m, g.n, g.k, g.m, -1, al, bl, ep, ws, ws_elems);
+}
+
 }  // namespace sn

@@ -363,6 +363,28 @@ struct StdEpilogue {
   }
 };
 
+// An input gradient dX on its way through the activation of the layer below, whose output y [rows, ldo] lies beside it: the
+// arithmetic of act_bwd_kernel on the finished sum.
+struct ActGradEpilogue {
+  float* out;
+  const float* y;
+  int64_t ldo;
+  int act;
+  float act_param;
+  __device__ __forceinline__ int map_row(int m) const { return m; }
+  __device__ __forceinline__ void store(int m, int n, float acc) const {
+    const int64_t at = (int64_t)m * ldo + n;
+    float g = acc;
+    switch (act) {
+      case SN_ACT_SIGMOID: { const float s = y[at]; g = (s * (1.0f - s)) * acc; break; }
+      case SN_ACT_TANH: { const float s = y[at]; g = (1.0f - s * s) * acc; break; }
+      case SN_ACT_RELU: g = (act_param < y[at] ? 1.0f : 0.0f) * acc; break;
+      default: break;
+    }
+    out[at] = g;
+  }
+};
+
 // the filter gradient's rows m' = r * Lp + j: row r * L + j of the tensor, nothing for the padding
 struct RunRowsEpilogue {
   float* out;
@@ -424,6 +446,27 @@ __device__ __forceinline__ void store16(const StdEpilogue& ep, int row0, int n, 
     case SN_ACT_TANH: store16_act<SN_ACT_TANH>(ep.e, row0, n, acc, M, first, last); break;
     case SN_ACT_RELU: store16_act<SN_ACT_RELU>(ep.e, row0, n, acc, M, first, last); break;
     default: store16_act<SN_ACT_IDENTITY>(ep.e, row0, n, acc, M, first, last); break;
+  }
+}
+
+// All of a lane's values of y are requested before the first is used, and the activation is looked at once.
+__device__ __forceinline__ void store16(const ActGradEpilogue& ep, int row0, int n, const f16v& acc, int M, int first = 0, int last = 16) {
+  float y[16];
+#pragma unroll
+  for (int v = 0; v < 16; ++v)
+    if (v >= first && v < last) y[v] = ep.y[(int64_t)min(row0 + (v >> 2) * 8 + (v & 3), M - 1) * ep.ldo + n];
+  auto store = [&](auto grad) {
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const int row = row0 + (v >> 2) * 8 + (v & 3);
+      if (row < M && v >= first && v < last) ep.out[(int64_t)row * ep.ldo + n] = grad(y[v], acc[v]);
+    }
+  };
+  switch (ep.act) {
+    case SN_ACT_SIGMOID: store([](float s, float a) { return (s * (1.0f - s)) * a; }); break;
+    case SN_ACT_TANH: store([](float s, float a) { return (1.0f - s * s) * a; }); break;
+    case SN_ACT_RELU: store([&](float s, float a) { return (ep.act_param < s ? 1.0f : 0.0f) * a; }); break;
+    default: store([](float, float a) { return a; }); break;
   }
 }
 

@@ -583,6 +583,12 @@ MODELS = {
                             ("pool", (2, 2), (2, 2), "same"), ("flatten",), ("dense", 3, "softmax")], "cce", (11, 9, 1), 20, "uniform_onehot"),
     "pool_6_channels_s_3_1": ([("conv", 4, (2, 2), (1, 1), "valid", "relu", False), ("conv", 6, (2, 2), (1, 1), "valid", "sigmoid", False),
                                ("pool", (2, 2), (3, 1), "valid"), ("flatten",), ("dense", 3, "softmax")], "cce", (12, 9, 1), 20, "uniform_onehot"),
+    # input gradients that leave through the gradient of the activation below: one row and one column past the tiles, two rows only, and a
+    # sum divided over workgroups (the launch that adds the parts applies it)
+    "dense_act_grad_tile_edges": ([("dense", 65, "tanh"), ("dense", 97, "sigmoid"), ("dense", 36, "relu"), ("dense", 20, "softmax")], "cce", (21,), 129,
+                                  "normal_onehot"),
+    "dense_act_grad_two_rows": ([("dense", 200, "sigmoid"), ("dense", 70, "tanh"), ("dense", 20, "softmax")], "cce", (35,), 2, "normal_onehot"),
+    "dense_act_grad_splits": ([("dense", 45, "tanh"), ("dense", 1203, "sigmoid"), ("dense", 30, "softmax")], "cce", (50,), 100, "normal_onehot"),
     "dense_identity_mse": ([("dense", 6, "identity")], "mse", (4,), 8, "normal_regression"),
     # Dense >> Dense(Softmax) + CategoricalCrossentropy small enough for the two-launch training pass: a reduction length
     # that is no multiple of 16, rows that are no multiple of 16, all 64 hidden units / 16 classes, penalties on top
@@ -667,6 +673,9 @@ KERNEL_OF_MODEL = {
     "dense_many_features_few_units": "dense_weight_and_input_gradient_rows",
     "dense_many_features_16_units": "dense_weight_and_input_gradient_rows",
     "dense_odd_feature_count_9_units": "small_output_reduce_softmax_crossentropy_fused",
+    "dense_act_grad_tile_edges": "gemm_f32_and_activation_gradient",
+    "dense_act_grad_two_rows": "gemm_f32_and_activation_gradient",
+    "dense_act_grad_splits": "gemm_f32_and_activation_gradient",
     "mlp_cfg1": "mlp2_",
     "mlp2_1030_rows": "mlp2_",
     "mlp2_515_rows": "mlp2_",
