@@ -12,6 +12,7 @@
 // can be spared is what counts: mean and variance come out of one read, and where a 2 x 2 max pooling
 // follows, the normalised tensor and its gradient are never in memory (the pooling's windows are normalised as
 // they are compared, and their gradients are looked up where they are needed).
+#include "batchnorm_rules.hpp"
 #include "common.hpp"
 
 namespace sn {
@@ -501,48 +502,15 @@ unsigned grid_for(const sn_ctx* ctx, int64_t n, int per_block) {
   return blocks < 1 ? 1u : (unsigned)blocks;
 }
 
-int slices_for(const sn_ctx* ctx, int64_t rows, int cols) {
-  const int64_t col_blocks = ceil_div((int64_t)cols, (int64_t)64);
-  int64_t s = ceil_div((int64_t)ctx->compute_units * 4, col_blocks);
-  const int64_t by_rows = ceil_div(rows, (int64_t)64);  // at least 64 rows (16 per wave) in a slice
-  if (s > by_rows) s = by_rows;
-  if (s > 1024) s = 1024;
-  return s < 1 ? 1 : (int)s;
-}
-
-// the float4-stream reductions: whole vectors of channels and enough data for more than one block
-bool stream_form(int64_t rows, int cols) { return cols % 4 == 0 && cols <= 1024 && rows * cols >= 4 * 8 * 256; }
-struct Stream {
-  int active, slices;
-  int64_t n4, per4;
-};
-Stream stream_of(const sn_ctx* ctx, int64_t rows, int cols) {
-  Stream st;
-  const int cg = cols / 4;
-  st.active = 256 / cg * cg;
-  st.n4 = rows * cols / 4;
-  int64_t s = ceil_div(st.n4, (int64_t)8 * 256);  // at least one full trip of 8 loads per thread
-  s = std::min<int64_t>(s, (int64_t)ctx->compute_units * 4);
-  if (256 % cg != 0) s = std::min<int64_t>(s, slices_for(ctx, rows, cols));  // (the workspace such a layer has always asked for)
-  s = std::max<int64_t>(s, 1);
-  st.per4 = ceil_div(ceil_div(st.n4, s), (int64_t)st.active) * st.active;
-  st.slices = (int)ceil_div(st.n4, st.per4);  // every slice has rows
-  return st;
-}
-int max_slices(const sn_ctx* ctx, int64_t rows, int cols) {
-  int s = slices_for(ctx, rows, cols);
-  if (stream_form(rows, cols)) s = std::max(s, stream_of(ctx, rows, cols).slices);
-  return s;
-}
 bool stream_ok(int64_t rows, int cols, const void* x, const void* dy, const void* part0, int64_t part1_offset) {
-  return stream_form(rows, cols) && part1_offset % 4 == 0 &&
+  return bn_stream_form(rows, cols) && part1_offset % 4 == 0 &&
          ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(dy) | reinterpret_cast<uintptr_t>(part0)) & 15u) == 0;
 }
 
 // One row-walking reduction pass; returns the number of slices written to part0 (and part1).
 template <int MODE>
 int reduce_rows(sn_ctx* ctx, const float* x, const float* dy, const float* mean, float* part0, float* part1, int64_t rows, int cols) {
-  const int s = slices_for(ctx, rows, cols);
+  const int s = bn_row_slices(ctx->compute_units, rows, cols);
   hipLaunchKernelGGL((bn_reduce_kernel<MODE>), dim3((unsigned)ceil_div((int64_t)cols, (int64_t)64), (unsigned)s), dim3(256), 0, ctx->stream, x, dy,
                      mean, part0, part1, rows, cols, ceil_div(rows, (int64_t)s));
   return s;
@@ -557,11 +525,11 @@ bool vec4_ok(int cols, std::initializer_list<const void*> ptrs) {
 
 }  // namespace
 
-int64_t batchnorm_workspace_elems(const sn_ctx* ctx, int64_t rows, int cols) { return (int64_t)2 * max_slices(ctx, rows, cols) * cols; }
+int64_t batchnorm_workspace_elems(const sn_ctx* ctx, int64_t rows, int cols) { return (int64_t)2 * bn_max_slices(ctx->compute_units, rows, cols) * cols; }
 
 ConvStats batchnorm_conv_stats(const sn_ctx* ctx, int64_t rows, int cols, float* ws, int64_t ws_elems) {
   ConvStats st;
-  const int64_t slices = max_slices(ctx, rows, cols), half = slices * cols;
+  const int64_t slices = bn_max_slices(ctx->compute_units, rows, cols), half = slices * cols;
   if (ws && 2 * half <= ws_elems) {
     st.part_mean = ws;
     st.part_m2 = ws + half;
@@ -582,7 +550,7 @@ static int batchnorm_statistics(sn_ctx* ctx, const float* x, int64_t rows, int c
     SN_HIP(hipGetLastError());
     return SN_OK;
   }
-  const int64_t half = (int64_t)max_slices(ctx, rows, cols) * cols;
+  const int64_t half = (int64_t)bn_max_slices(ctx->compute_units, rows, cols) * cols;
   const BnScale scale = bn_scale_of(a, rows, a.fused_wiring);
   SN_REQUIRE(half <= ws_elems, "batch norm needs %lld workspace elements, %lld given", (long long)half, (long long)ws_elems);
   if (stats && stats->slices > 0) {
@@ -590,7 +558,7 @@ static int batchnorm_statistics(sn_ctx* ctx, const float* x, int64_t rows, int c
     hipLaunchKernelGGL(bn_moments_kernel, dim3(cb), dim3(256), 0, ctx->stream, (const float*)stats->part_mean, (const float*)stats->part_m2, stats->slices,
                        cols, stats->whole, stats->last, (float)rows, scale);
   } else if (2 * half <= ws_elems && stream_ok(rows, cols, x, nullptr, ws, half)) {
-    const Stream st = stream_of(ctx, rows, cols);
+    const BnStream st = bn_stream_of(ctx->compute_units, rows, cols);
     LaunchScope scope(ctx, "batchnorm_mean_and_variance");
     hipLaunchKernelGGL(bn_stats_v4_kernel, dim3((unsigned)st.slices), dim3(256), 0, ctx->stream, (const bn_f4*)x, ws, ws + half, st.n4, cols, st.active,
                        st.per4);
@@ -659,11 +627,11 @@ static void grad_finish(sn_ctx* ctx, const float* part0, const float* part1, int
 int launch_batchnorm_pool_bwd(sn_ctx* ctx, const float* x, const float* dy, const uint8_t* arg, const PoolGeom& g, const BatchNormArgs& a, float* dbeta,
                               float* dgamma, float* ws, int64_t ws_elems) {
   const int64_t rows = (int64_t)g.n * g.h * g.w;
-  const int64_t half = (int64_t)max_slices(ctx, rows, g.c) * g.c;
+  const int64_t half = (int64_t)bn_max_slices(ctx->compute_units, rows, g.c) * g.c;
   SN_REQUIRE(2 * half <= ws_elems, "batch norm gradient needs %lld workspace elements, %lld given", (long long)(2 * half), (long long)ws_elems);
   const int cg = g.c / 4, active = 256 / cg * cg;
   const int64_t n4 = (int64_t)g.n * g.ho * g.wo * cg;
-  const int64_t wanted = std::min<int64_t>(ceil_div(n4, (int64_t)4 * active), max_slices(ctx, rows, g.c));
+  const int64_t wanted = std::min<int64_t>(ceil_div(n4, (int64_t)4 * active), bn_max_slices(ctx->compute_units, rows, g.c));
   const int64_t per4 = ceil_div(ceil_div(n4, wanted), (int64_t)active) * active;
   const int slices = (int)ceil_div(n4, per4);
   LaunchScope scope(ctx, "batchnorm_gradient_sums_from_maxpool");
@@ -677,7 +645,7 @@ int launch_batchnorm_pool_bwd(sn_ctx* ctx, const float* x, const float* dy, cons
 int launch_batchnorm_bwd(sn_ctx* ctx, const float* x, const float* dy, float* dx, int64_t rows, int cols, const BatchNormArgs& a,
                          float* dbeta, float* dgamma, float* ws, int64_t ws_elems, int below_act, float below_act_param) {
   if (rows <= 0 || cols <= 0) return SN_OK;
-  const int64_t half = (int64_t)max_slices(ctx, rows, cols) * cols;
+  const int64_t half = (int64_t)bn_max_slices(ctx->compute_units, rows, cols) * cols;
   SN_REQUIRE(2 * half <= ws_elems, "batch norm gradient needs %lld workspace elements, %lld given", (long long)(2 * half), (long long)ws_elems);
   float* part1 = ws + half;
   const float* mean = a.fused_wiring ? a.g_mean : a.mean;
@@ -686,7 +654,7 @@ int launch_batchnorm_bwd(sn_ctx* ctx, const float* x, const float* dy, float* dx
     LaunchScope scope(ctx, "batchnorm_gradient_sums");
     int s = 0;
     if (stream_ok(rows, cols, x, dy, ws, half)) {
-      const Stream st = stream_of(ctx, rows, cols);
+      const BnStream st = bn_stream_of(ctx->compute_units, rows, cols);
       s = st.slices;
       hipLaunchKernelGGL(bn_grad_sums_v4_kernel, dim3((unsigned)s), dim3(256), 0, ctx->stream, (const bn_f4*)x, (const bn_f4*)dy, mean, ws, part1, st.n4,
                          cols, st.active, st.per4);

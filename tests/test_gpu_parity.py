@@ -701,6 +701,24 @@ def test_parity_models_reach_the_kernels_they_are_named_for(S, ctx, name):
     h.close()
 
 
+def test_batchnorm_pass_of_fewer_rows_than_the_batch(S, ctx):
+    """A pass over 8192 rows of 1024 channels is cut into more slices than one over the model's 8275: it is taken all the same,
+    and is the oracle's."""
+    rng = np.random.default_rng(8275)
+    h = Harness(S, ctx, [("batchnorm", 0.9, 1e-3), ("dense", 10, "softmax")], "cce", (1024,), 8275)
+    params = glorot_params(h.omodel, (8275, 1024), rng)
+    x, y = make_data("normal_onehot", rng, 8192, (1024,), 10)
+    h.rep.set_params(params)
+    oloss, ograds = h.omodel.grad(x, y, params)
+    gloss = h.rep.grad(ctx.to_device(x), ctx.to_device(y), rows=8192)
+    assert abs(gloss - float(oloss)) <= TOL_GEMM * max(1.0, abs(float(oloss)))
+    ggrads = h.rep.get_grads()
+    grads64 = h.omodel.grad(x.astype(np.float64), y.astype(np.float64), {p: v.astype(np.float64) for p, v in params.items()})[1]
+    for p in ograds:
+        assert rel_err(ggrads[p], grads64[p]) <= max(TOL_GEMM, 3.0 * rel_err(ograds[p], grads64[p])), p
+    h.close()
+
+
 @pytest.mark.parametrize("name", ["mlp_tanh_relu", "lenet_small", "dense_many_features_few_units", "dense_odd_feature_count_9_units"])
 def test_stable_softmax_flag_changes_nothing_at_moderate_logits(S, ctx, name):
     """SN_FLAG_STABLE_SOFTMAX subtracts the row maximum before exp: mathematically the same softmax, so loss and gradients
