@@ -14,6 +14,7 @@
 // they are compared, and their gradients are looked up where they are needed).
 #include "batchnorm_rules.hpp"
 #include "common.hpp"
+#include "moments.hpp"
 
 namespace sn {
 namespace {
@@ -187,9 +188,8 @@ __global__ __launch_bounds__(256) void bn_pool_grad_sums_kernel(const float* __r
 }
 
 // Mean and sum of squared deviations of a block's rows in one read: a thread takes eight values of a channel at a time, forms their own
-// mean and deviations in registers and joins them to what it has by the pairwise update of Chan, Golub and LeVeque (1983)
-//   mean += d w, M2 += M2_8 + d^2 n w   with d = mean_8 - mean, w = 8 / (n + 8);
-// no large squares are subtracted anywhere, so the variance is as good as the two-read form's.
+// mean and deviations in registers and joins them to what it has (join_moments): no large squares are subtracted anywhere, so the
+// variance is as good as the two-read form's.
 // [676000 x 32]: 17 us, where a read for the mean, its finishing launch and a read for the variance took 15 + 5 + 15.
 __global__ __launch_bounds__(256) void bn_stats_v4_kernel(const bn_f4* __restrict__ x, float* __restrict__ part_mean, float* __restrict__ part_m2,
                                                            int64_t n4, int cols, int active, int64_t per4) {
@@ -202,15 +202,7 @@ __global__ __launch_bounds__(256) void bn_stats_v4_kernel(const bn_f4* __restric
   bn_f4 mean = zero, m2 = zero;
   float n = 0.f;
   auto join = [&](const bn_f4& m, const bn_f4& q, float k) {  // k values of mean m and squared deviations q
-    const float w = k / (n + k);
-    if (n > 0.f) {
-      const bn_f4 d = m - mean;
-      mean = mean + d * w;
-      m2 = m2 + (q + d * d * (n * w));
-    } else {
-      mean = m;
-      m2 = q;
-    }
+    join_moments<4, false>(n, mean, m2, k, m, q);
     n += k;
   };
   int64_t i = t < active ? begin + t : end;
@@ -237,21 +229,22 @@ __global__ __launch_bounds__(256) void bn_stats_v4_kernel(const bn_f4* __restric
     for (int u = 0; u < 7; ++u) { const bn_f4 d = a[u] - m; q = u < left ? q + d * d : q; }
     join(m, q, (float)left);
   }
+  if (n > 0.f && !(__builtin_isfinite(mean[0]) && __builtin_isfinite(mean[1]) && __builtin_isfinite(mean[2]) && __builtin_isfinite(mean[3]))) {
+    // an infinity, or values too far apart for their difference: the sum over the number (0.5 us less than looking at every join)
+    bn_f4 s = zero;
+    for (i = begin + t; i < end; i += active) s = s + x[i];
+    mean = s / n;
+  }
   smem[0][t] = mean;
   smem[1][t] = m2;
   count[t] = n;
   over_channel_peers(t, cg, active, [&](int to, int from) {
     const float na = count[to], nb = count[from];
-    if (nb == 0.f) return;
-    if (na == 0.f) {
-      smem[0][to] = smem[0][from];
-      smem[1][to] = smem[1][from];
-    } else {
-      const float w = nb / (na + nb);
-      const bn_f4 d = smem[0][from] - smem[0][to];
-      smem[0][to] = smem[0][to] + d * w;
-      smem[1][to] = smem[1][to] + (smem[1][from] + d * d * (na * w));
-    }
+    const bn_f4 mb = smem[0][from], qb = smem[1][from];
+    bn_f4 ma = smem[0][to], qa = smem[1][to];
+    join_moments<4>(na, ma, qa, nb, mb, qb);
+    smem[0][to] = ma;
+    smem[1][to] = qa;
     count[to] = na + nb;
   });
   if (t < cg) {

@@ -18,6 +18,7 @@
 // 9 x 32 over 1000 x 26 x 26 under a batch normalisation and a pooling 88 -> 36.5 us (it reads 114 MB); 9 x 32 over 100 x 26 x 26
 // under a pooling of stride 1, 11.6 -> 9.7 us.
 #include "common.hpp"
+#include "moments.hpp"
 
 #include <algorithm>
 
@@ -328,19 +329,6 @@ __device__ __forceinline__ void first_act(int act, float (&v)[N], float param) {
   }
 }
 
-// (na, ma, qa) joined with (nb, mb, qb): counts, means, squared deviations
-__device__ __forceinline__ void join_moments(float na, float& ma, float& qa, float nb, float mb, float qb) {
-  if (nb == 0.f) return;
-  if (na == 0.f) {
-    ma = mb;
-    qa = qb;
-    return;
-  }
-  const float w = nb / (na + nb), d = mb - ma;
-  ma = ma + d * w;
-  qa = qa + (qb + d * d * (na * w));
-}
-
 // KS steps of four taps, NT tiles of 16 filters (blockIdx.y: which 16 NT of them); VEC: a lane's NT filters are neighbours and leave as one
 // vector, otherwise they are 16 apart
 template <int KS, int NT, bool VEC, bool STATS>
@@ -433,24 +421,24 @@ __global__ __launch_bounds__(256) void conv_first_fwd_kernel(FirstForward k) {
     }
     if constexpr (STATS) {
       if (p0 + 16 <= p_end) {
-        const float w = 4.0f / (n + 4.0f), nw = n * w;
+        float m[NT], q[NT];
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
-          const float m = ((v[t] + v[NT + t]) + (v[2 * NT + t] + v[3 * NT + t])) * 0.25f;
-          float q = 0.f;
+          m[t] = ((v[t] + v[NT + t]) + (v[2 * NT + t] + v[3 * NT + t])) * 0.25f;
+          q[t] = 0.f;
 #pragma unroll
-          for (int i = 0; i < 4; ++i) { const float d = v[i * NT + t] - m; q = q + d * d; }
-          const float d = m - mean[t];
-          mean[t] = n > 0.f ? mean[t] + d * w : m;
-          m2[t] = n > 0.f ? m2[t] + (q + d * d * nw) : q;
+          for (int i = 0; i < 4; ++i) { const float d = v[i * NT + t] - m[t]; q[t] = q[t] + d * d; }
         }
+        join_moments<NT>(n, mean, m2, 4.0f, m, q);
         n += 4.0f;
       } else {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           if (i >= mine) continue;
+          float m[NT], q[NT];
 #pragma unroll
-          for (int t = 0; t < NT; ++t) join_moments(n, mean[t], m2[t], 1.0f, v[i * NT + t], 0.f);
+          for (int t = 0; t < NT; ++t) { m[t] = v[i * NT + t]; q[t] = 0.f; }
+          join_moments<NT>(n, mean, m2, 1.0f, m, q);
           n += 1.0f;
         }
       }
@@ -462,11 +450,10 @@ __global__ __launch_bounds__(256) void conv_first_fwd_kernel(FirstForward k) {
 #pragma unroll
     for (int d = 16; d < 64; d <<= 1) {  // (both lanes of a pair join, in opposite order: the lowest ones' sums are kept)
       const float nb = __shfl_xor(n, d);
+      float mb[NT], qb[NT];
 #pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        const float mb = __shfl_xor(mean[t], d), qb = __shfl_xor(m2[t], d);
-        join_moments(n, mean[t], m2[t], nb, mb, qb);
-      }
+      for (int t = 0; t < NT; ++t) { mb[t] = __shfl_xor(mean[t], d); qb[t] = __shfl_xor(m2[t], d); }
+      join_moments<NT>(n, mean, m2, nb, mb, qb);
       n += nb;
     }
     if (lq == 0) {
@@ -480,14 +467,15 @@ __global__ __launch_bounds__(256) void conv_first_fwd_kernel(FirstForward k) {
     __syncthreads();
     const int c = threadIdx.x;
     if (c < 16 * NT && co0 + c < g.cout) {
-      float na = counts[0], ma = moments[0][0][c], qa = moments[0][1][c];
+      float na = counts[0], ma[1] = {moments[0][0][c]}, qa[1] = {moments[0][1][c]};
 #pragma unroll
       for (int w = 1; w < 4; ++w) {
-        join_moments(na, ma, qa, counts[w], moments[w][0][c], moments[w][1][c]);
+        const float mb[1] = {moments[w][0][c]}, qb[1] = {moments[w][1][c]};
+        join_moments<1>(na, ma, qa, counts[w], mb, qb);
         na += counts[w];
       }
-      k.part_mean[(int64_t)block * g.cout + co0 + c] = ma;
-      k.part_m2[(int64_t)block * g.cout + co0 + c] = qa;
+      k.part_mean[(int64_t)block * g.cout + co0 + c] = ma[0];
+      k.part_m2[(int64_t)block * g.cout + co0 + c] = qa[0];
     }
   }
 }

@@ -701,6 +701,42 @@ def test_parity_models_reach_the_kernels_they_are_named_for(S, ctx, name):
     h.close()
 
 
+@pytest.mark.parametrize("form", ["one_read", "two_reads", "by_the_convolution"])
+def test_batchnorm_mean_of_infinities(S, ctx, form):
+    """A channel's mean is its sum over its rows: infinite where an infinity is among them, NaN where both are.  Whole vectors of
+    channels (one read), other channel counts (two reads), and statistics that the first convolution forms."""
+    rng = np.random.default_rng(5)
+    channels, momentum = (5 if form == "two_reads" else 12), f32(0.9)
+    if form == "by_the_convolution":  # 1 x 1 filters of one and minus one: every channel is the image or its negative
+        spec, shape, batch = [("conv", channels, (1, 1), (1, 1), "valid", "identity", False), ("batchnorm", 0.9, 1e-3), ("flatten",), ("dense", 3, "softmax")], (40, 40, 1), 3
+        weights = np.where(np.arange(channels) % 2 == 0, 1.0, -1.0).astype(f32)
+        x = rng.standard_normal((batch,) + shape).astype(f32)
+    else:
+        spec, shape, batch = [("batchnorm", 0.9, 1e-3), ("dense", 3, "softmax")], (channels,), 1203
+        x = rng.standard_normal((batch,) + shape).astype(f32)
+    y = one_hot(rng, batch, 3)
+    for first, second in ((np.inf, None), (-np.inf, None), (np.inf, np.inf), (np.inf, -np.inf), (None, None)):
+        h = Harness(S, ctx, spec, "cce", shape, batch, S.SGD(0.01))
+        h.rep.set_params(glorot_params(h.omodel, (batch,) + shape, rng))
+        v = x.copy()
+        for value, at in ((first, 0.2), (second, 0.7)):  # in one channel, two rows (pixels) far apart
+            if value is not None:
+                v.reshape(-1, v.shape[-1])[int(at * v.size / v.shape[-1]), 0] = value
+        flat = v.reshape(-1, v.shape[-1])
+        seen = flat * weights if form == "by_the_convolution" else flat
+        layer = 1 if form == "by_the_convolution" else 0
+        if layer:
+            h.rep.set_params({"0/weights": weights.reshape(1, 1, 1, channels)})
+        before = h.rep.get_params()[f"{layer}/moving_mean"].reshape(-1).astype(np.float64)
+        h.rep.step(ctx.to_device(v), ctx.to_device(y), 1)
+        got = h.rep.get_params()[f"{layer}/moving_mean"].reshape(-1)
+        with np.errstate(invalid="ignore"):
+            want = momentum * before + (1.0 - 0.9) * seen.astype(np.float64).mean(axis=0)
+        np.testing.assert_allclose(got, want, rtol=1e-5, atol=1e-6)  # (infinities and NaNs in the same places)
+        assert np.isfinite(want[1 if not layer else 0]) == (first is None or not layer)
+        h.close()
+
+
 def test_batchnorm_pass_of_fewer_rows_than_the_batch(S, ctx):
     """A pass over 8192 rows of 1024 channels is cut into more slices than one over the model's 8275: it is taken all the same,
     and is the oracle's."""
