@@ -448,7 +448,7 @@ struct PoolGrad {
 bool conv_wgrad_is_direct(const sn_ctx* ctx, const ConvGeom& g, const float* ws, int64_t ws_elems);
 // First-layer filter gradient (conv_first_kernels.hip): up to 4 input channels, 48 taps, 64 filters.  The number of partial filters
 // [part][kh * kw * cin][cout] it would leave in ws (0: not its shape), and the launch.
-int conv_first_wgrad_parts(const sn_ctx* ctx, const ConvGeom& g, const float* ws, int64_t ws_elems, int* rows_per_wave = nullptr);
+int conv_first_wgrad_parts(const sn_ctx* ctx, const ConvGeom& g, const float* ws, int64_t ws_elems);
 int launch_conv_first_wgrad(sn_ctx* ctx, const ConvGeom& g, const float* x, const float* dy, float* ws, int64_t ws_elems, const PoolGrad* pool, int* parts);
 int launch_conv_wgrad(sn_ctx* ctx, const ConvGeom& g, const float* x, const float* dy, float* dw, float* ws, int64_t ws_elems,
                       const PoolGrad* pool = nullptr);

@@ -18,6 +18,7 @@
 // 9 x 32 over 1000 x 26 x 26 under a batch normalisation and a pooling 88 -> 36.5 us (it reads 114 MB); 9 x 32 over 100 x 26 x 26
 // under a pooling of stride 1, 11.6 -> 9.7 us.
 #include "common.hpp"
+#include "conv_first_rules.hpp"
 #include "moments.hpp"
 
 #include <algorithm>
@@ -32,8 +33,9 @@ struct FirstWgrad {
   const float* x;
   const float* dy;      // [n, ho, wo, cout], POOL: not read
   float* partial;       // [block][M][cout]
-  int M, rows, rows_per_wave;  // taps; n * ho
-  FastDiv by_ho, by_cin, by_kw, by_cout;
+  int M, items;  // taps; n * ho rows in segments
+  FirstWgradCut cut;
+  FastDiv by_segments, by_ho, by_cin, by_kw, by_cout;
   PoolGrad pool;
 };
 
@@ -106,13 +108,15 @@ __global__ __launch_bounds__(256) void conv_first_wgrad_kernel(FirstWgrad k) {
 #pragma unroll
     for (int t = 0; t < NT; ++t) acc[i][t] = f4v{0.f, 0.f, 0.f, 0.f};
 
-  // every XCD (workgroup id modulo 8) takes a contiguous run of rows
+  // every XCD (workgroup id modulo 8) takes a contiguous run of rows, or of their segments
   const int per_xcd = ((int)gridDim.x + 7) >> 3, extra = (int)gridDim.x - (per_xcd - 1) * 8;  // `extra` XCDs have per_xcd workgroups, the others one less
   const int xcd = (int)blockIdx.x & 7;
   const int block = xcd * (per_xcd - 1) + min(xcd, extra) + ((int)blockIdx.x >> 3);
-  const int row0 = (block * 4 + wave) * k.rows_per_wave, row1 = min(k.rows, row0 + k.rows_per_wave);
+  const int item0 = (block * 4 + wave) * k.cut.items_per_wave, item1 = min(k.items, item0 + k.cut.items_per_wave);
   const PoolGrad& pg = k.pool;
-  for (int row = row0; row < row1; ++row) {
+  for (int item = item0; item < item1; ++item) {
+    const int row = (int)div_by((uint32_t)item, k.by_segments);
+    const int ow_begin = (item - row * k.cut.segments) * k.cut.segment_length, ow_end = min(g.wo, ow_begin + k.cut.segment_length);
     const int b = (int)div_by((uint32_t)row, k.by_ho), oh = row - b * g.ho;
     const float* const xb = k.x + (int64_t)b * g.h * g.w * g.cin;
     const int iy = oh * g.sh, x_row = iy * g.w * g.cin;
@@ -133,7 +137,7 @@ __global__ __launch_bounds__(256) void conv_first_wgrad_kernel(FirstWgrad k) {
       pd_row = pg.dy + first;
       pa_row = pg.arg + first;
     }
-    for (int ow0 = 0; ow0 < g.wo; ow0 += 4 * G) {
+    for (int ow0 = ow_begin; ow0 < ow_end; ow0 += 4 * G) {
       float a[G][MT], y[G][NT], pd[G][WIN][NT];
       uint32_t pa[G][WIN][NV], want[G][WIN];
 #pragma unroll
@@ -177,7 +181,7 @@ __global__ __launch_bounds__(256) void conv_first_wgrad_kernel(FirstWgrad k) {
       }
 #pragma unroll
       for (int u = 0; u < G; ++u) {
-        if (ow0 + 4 * u >= g.wo) break;
+        if (ow0 + 4 * u >= ow_end) break;
         float d[NT];
         if constexpr (POOL) {
           const bool on = ow0 + 4 * u + lp < g.wo;
@@ -249,28 +253,29 @@ int launch_taps(sn_ctx* ctx, const FirstWgrad& k, int blocks, bool pool, bool ve
 }  // namespace
 
 constexpr int FIRST_MAX_TAPS = 48, FIRST_MAX_FILTERS = 64, FIRST_MIN_POSITIONS = 2048;
-int conv_first_wgrad_parts(const sn_ctx* ctx, const ConvGeom& g, const float* ws, int64_t ws_elems, int* rows_per_wave) {
+static FirstWgradCut first_wgrad_cut(const sn_ctx* ctx, const ConvGeom& g, const float* ws, int64_t ws_elems) {
   const int M = g.kh * g.kw * g.cin, N = g.cout;
   const int64_t rows = (int64_t)g.n * g.ho;
-  if (!ws || g.cin > 4 || M > FIRST_MAX_TAPS || N > FIRST_MAX_FILTERS || rows * g.wo < FIRST_MIN_POSITIONS) return 0;
-  if (rows >= (1ll << 30) || (int64_t)g.h * g.w * g.cin >= (1ll << 30) || (int64_t)(g.wo + 1) * 2 * N >= (1ll << 30)) return 0;  // 32-bit offsets inside an image and two rows
+  if (!ws || g.cin > 4 || M > FIRST_MAX_TAPS || N > FIRST_MAX_FILTERS || rows * g.wo < FIRST_MIN_POSITIONS) return {};
+  if (rows >= (1ll << 30) || (int64_t)g.h * g.w * g.cin >= (1ll << 30) || (int64_t)(g.wo + 1) * 2 * N >= (1ll << 30)) return {};  // 32-bit offsets inside an image and two rows
   const int64_t room = std::min<int64_t>((int64_t)4 * ctx->compute_units, ws_elems / ((int64_t)M * N));
-  if (room < 32) return 0;
-  const int per = (int)ceil_div(rows, 4 * room);  // as many wavefronts as there are rows, up to four on a SIMD
-  if (rows_per_wave) *rows_per_wave = per;
-  return (int)ceil_div(rows, (int64_t)4 * per);
+  if (room < 32) return {};
+  return conv_first_wgrad_cut(rows, g.wo, room);  // as many wavefronts as there are rows or segments, up to four on a SIMD
 }
+int conv_first_wgrad_parts(const sn_ctx* ctx, const ConvGeom& g, const float* ws, int64_t ws_elems) { return first_wgrad_cut(ctx, g, ws, ws_elems).parts; }
 
 int launch_conv_first_wgrad(sn_ctx* ctx, const ConvGeom& g, const float* x, const float* dy, float* ws, int64_t ws_elems, const PoolGrad* pool, int* parts) {
   FirstWgrad k{};
-  *parts = conv_first_wgrad_parts(ctx, g, ws, ws_elems, &k.rows_per_wave);
+  k.cut = first_wgrad_cut(ctx, g, ws, ws_elems);
+  *parts = k.cut.parts;
   SN_REQUIRE(*parts > 0, "conv2d_filter_gradient_first: shape outside the kernel's range");
   k.g = g;
   k.x = x;
   k.dy = dy;
   k.partial = ws;
   k.M = g.kh * g.kw * g.cin;
-  k.rows = g.n * g.ho;
+  k.items = g.n * g.ho * k.cut.segments;
+  k.by_segments = fast_div((uint32_t)k.cut.segments);
   k.by_ho = fast_div((uint32_t)g.ho);
   k.by_cin = fast_div((uint32_t)g.cin);
   k.by_kw = fast_div((uint32_t)g.kw);

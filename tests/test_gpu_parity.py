@@ -508,6 +508,14 @@ MODELS = {
                                              ("dense", 3, "softmax")], "cce", (14, 13, 1), 30, "uniform_onehot"),
     "conv_pool_first_layer_60_filters_s_1_2": ([("conv", 60, (2, 2), (1, 1), "same", "sigmoid", False), ("pool", (2, 2), (1, 2), "same"), ("flatten",),
                                                 ("dense", 3, "softmax")], "cce", (11, 10, 2), 40, "uniform_onehot"),
+    # first-layer filter gradient of a few long rows, cut into segments: 69 of 16 positions a row, the last of 4; 13 of two trips, the last with one
+    # trip and a part of one; under a pooling whose windows reach across the segments
+    "conv_first_layer_one_long_row": ([("conv", 20, (1, 9), (1, 1), "valid", "relu", False), ("flatten",), ("dense", 3, "softmax")], "cce", (1, 1100, 2), 5,
+                                      "uniform_onehot"),
+    "conv_first_layer_segments_of_32": ([("conv", 16, (1, 3), (1, 1), "valid", "tanh", False), ("flatten",), ("dense", 3, "softmax")], "cce", (20, 400, 1),
+                                        10, "uniform_onehot"),
+    "conv_pool_first_layer_long_rows": ([("conv", 32, (2, 3), (1, 1), "same", "relu", False), ("pool", (2, 2), (1, 1), "same"), ("flatten",),
+                                         ("dense", 3, "softmax")], "cce", (3, 701, 1), 2, "uniform_onehot"),
     # first-layer forward: 64 taps, filters past one launch column of 64, a bias; the same with the statistics of a BatchNorm formed on the way
     "conv_first_layer_100_filters_64_taps": ([("conv", 100, (4, 4), (1, 2), "same", "sigmoid", True), ("flatten",), ("dense", 3, "softmax")], "cce",
                                              (9, 11, 4), 6, "uniform_onehot"),
@@ -667,6 +675,9 @@ KERNEL_OF_MODEL = {
     "conv_first_layer_33_filters_48_taps": "conv2d_filter_gradient_direct",
     "conv_pool_first_layer_24_filters_s2": "maxpool_backward_and_conv2d_filter_gradient_direct",
     "conv_pool_first_layer_60_filters_s_1_2": "maxpool_backward_and_conv2d_filter_gradient_direct",
+    "conv_first_layer_one_long_row": "conv2d_filter_gradient_direct",
+    "conv_first_layer_segments_of_32": "conv2d_filter_gradient_direct",
+    "conv_pool_first_layer_long_rows": "maxpool_backward_and_conv2d_filter_gradient_direct",
     "batchnorm_pool_first_layer_same_s1": "batchnorm_gradient_sums_from_maxpool",
     "batchnorm_pool_48_channels_stride_2_1": "batchnorm_gradient_sums_from_maxpool",
     "batchnorm_pool_second_layer": "batchnorm_apply_and_maxpool",
