@@ -425,8 +425,7 @@ struct ConvStats {
 };
 int launch_conv_fwd(sn_ctx* ctx, const ConvGeom& g, const float* x, const float* w, const Epilogue& ep, float* ws, int64_t ws_elems,
                     ConvStats* stats = nullptr);
-// First layers (conv_first_kernels.hip): up to 4 input channels and 64 taps, whole vectors of filters
-bool conv_first_fwd_ok(const ConvGeom& g, const Epilogue& e);
+// First layers (conv_first_kernels.hip; conv_first_rules.hpp: which)
 int launch_conv_first_fwd(sn_ctx* ctx, const ConvGeom& g, const float* x, const float* w, const Epilogue& e, ConvStats* stats);
 int launch_conv_dgrad(sn_ctx* ctx, const ConvGeom& g, const float* dy, const float* w, float* dx, float* ws, int64_t ws_elems);
 // A 2 x 2 max pooling right above a first-layer convolution, for launch_conv_wgrad's first-layer kernel: the pooling's output

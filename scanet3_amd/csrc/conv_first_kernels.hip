@@ -505,13 +505,6 @@ void launch_first_fwd_steps(sn_ctx* ctx, const FirstForward& k, int blocks, bool
 
 }  // namespace
 
-// up to 64 taps; whole vectors of filters (other first layers stay with the tiled kernels)
-bool conv_first_fwd_ok(const ConvGeom& g, const Epilogue& e) {
-  const int64_t positions = (int64_t)g.n * g.ho * g.wo;
-  return g.cin <= 4 && g.kh * g.kw * g.cin <= 64 && g.cout % 4 == 0 && e.ldo % 4 == 0 && (reinterpret_cast<uintptr_t>(e.out) & 15u) == 0 &&
-         positions > 0 && positions < (1ll << 30) && (int64_t)g.h * g.w * g.cin < (1ll << 30) && g.h < (1 << 20) && g.cout <= 4096;
-}
-
 int launch_conv_first_fwd(sn_ctx* ctx, const ConvGeom& g, const float* x, const float* w, const Epilogue& e, ConvStats* stats) {
   SN_REQUIRE(conv_first_fwd_ok(g, e), "conv2d_forward_first: shape outside the kernel's range");
   FirstForward k{};

@@ -1,4 +1,4 @@
-// How the first-layer filter gradient is divided over wavefronts (host only).
+// Which first layers conv_first_kernels.hip takes, and how it divides them over wavefronts (host only).
 #pragma once
 #include "common.hpp"
 
@@ -6,7 +6,18 @@
 
 namespace sn {
 
-// `rows` rows of `wo` output positions for at most `room` workgroups of four wavefronts.  A wavefront takes items_per_wave rows in
+// Forward: up to 64 taps, whole vectors of filters.  A wavefront keeps 64 filters' weights and gathers its positions' inputs anew for
+// every 64 filters, one value a lane, so many taps onto many filters are the tiled kernels': 64 taps x 256 filters over 10000 positions
+// 16.3 us there and 28.9 here, 36 x 344 26.2 and 33.4, 48 x 512 30.0 and 54.9.  Up to 28 taps it is the other way round at any
+// number of filters (27 x 512 over 10816: 32.2 and 27.7, 9 x 1400 95.0 and 42.7).
+inline bool conv_first_fwd_ok(const ConvGeom& g, const Epilogue& e) {
+  const int64_t positions = (int64_t)g.n * g.ho * g.wo, taps = (int64_t)g.kh * g.kw * g.cin;
+  return g.cin <= 4 && taps <= 64 && (taps <= 28 || taps * g.cout <= 12288) && g.cout % 4 == 0 && e.ldo % 4 == 0 &&
+         (reinterpret_cast<uintptr_t>(e.out) & 15u) == 0 && positions > 0 && positions < (1ll << 30) &&
+         (int64_t)g.h * g.w * g.cin < (1ll << 30) && g.h < (1 << 20) && g.cout <= 4096;
+}
+
+// Filter gradient: `rows` rows of `wo` output positions for at most `room` workgroups of four wavefronts.  A wavefront takes items_per_wave rows in
 // turn; where there are not half as many rows as wavefronts (signals: images of one or a few long rows), rows are cut into
 // segments of whole trips of 16 positions, until there is one for every wavefront.  9 taps x 32 filters with whole rows and
 // with segments: 8 rows of 4088 positions 344 and 6.3 us, 64 of 2040 182 and 8.5, 128 of 504 48 and 7.6, 224 of 20 6.7 and 6.3.

@@ -5,6 +5,7 @@
 //     (conv_prefers_float32_tiles), and the recurrent products that run one time step per launch.  bf16 form (Dense, on request): operands are rounded while they are staged.
 //     Block = 256 threads = 4 wavefronts in a 2x2 arrangement; block tile BM x BN (64 or 128 each), K step 16.
 //   - small-output products with a long reduction, first-layer convolutions, Dense layers onto a few units.
+#include "conv_first_rules.hpp"
 #include "split_launch.hpp"
 
 namespace sn {

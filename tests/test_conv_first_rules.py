@@ -1,4 +1,4 @@
-"""How the first-layer filter gradient is divided over wavefronts (csrc/conv_first_rules.hpp), compiled without device code."""
+"""Which first layers have kernels of their own and how these divide them (csrc/conv_first_rules.hpp), compiled without device code."""
 import itertools
 import os
 import subprocess
@@ -36,3 +36,9 @@ def test_few_long_rows_are_spread_over_the_chip(ask, rows, wo):
 def test_many_rows_stay_whole(ask):
     assert ask("cut", 2600, 26, 1024) == [1, 32, 1, 650]
     assert ask("cut", 26000, 26, 1024)[:3] == [1, 32, 7]
+
+
+def test_many_taps_onto_many_filters_stay_with_the_tiled_kernels(ask):
+    for kh, kw, cin, cout, want in ((4, 4, 4, 192, 1), (4, 4, 4, 196, 0), (4, 4, 4, 256, 0), (4, 4, 3, 512, 0), (3, 3, 4, 344, 0), (5, 5, 2, 256, 0), (8, 8, 1, 512, 0),
+                                    (4, 4, 2, 512, 0), (3, 3, 3, 512, 1), (3, 3, 1, 1400, 1), (7, 4, 1, 700, 1), (3, 3, 3, 50, 0), (9, 8, 1, 32, 0), (3, 3, 5, 32, 0)):
+        assert ask("forward", kh, kw, cin, cout) == [want], (kh, kw, cin, cout)
