@@ -493,7 +493,7 @@ void launch_first_fwd_tiles(sn_ctx* ctx, const FirstForward& k, int blocks, bool
 }
 template <int KS>
 void launch_first_fwd_steps(sn_ctx* ctx, const FirstForward& k, int blocks, bool stats) {
-  const int nt = (int)std::min<int64_t>(ceil_div(k.g.cout, 16), 4);
+  const int nt = conv_first_fwd_tiles(k.taps, k.g.cout, stats);
   const bool vec = k.g.cout % nt == 0 && k.e.ldo % nt == 0 && (reinterpret_cast<uintptr_t>(k.e.out) & 15u) == 0;
   switch (nt) {
     case 1: return launch_first_fwd_tiles<KS, 1, false>(ctx, k, blocks, stats);

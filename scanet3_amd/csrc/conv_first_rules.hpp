@@ -17,6 +17,16 @@ inline bool conv_first_fwd_ok(const ConvGeom& g, const Epilogue& e) {
          (int64_t)g.h * g.w * g.cin < (1ll << 30) && g.h < (1 << 20) && g.cout <= 4096;
 }
 
+// Tiles of 16 filters a wavefront multiplies its positions' inputs with: up to four.  Where the inputs are cheap to gather again and
+// nothing of a second tile is left over, two and twice the wavefronts: the weights are there sooner and fewer registers leave more
+// wavefronts in flight (9 taps x 64 filters, 67600 positions 16.5 -> 15.7 us, 18 x 64 19.3 -> 17.9, 18 x 128 28.0 -> 21.5; but 27 x 64
+// over 225000 29.4 -> 30.9, 32 x 64 over 210000 36 -> 40, 56 filters at 9 taps over 225000 20.9 -> 21.0, and a training step whose
+// first layer of 64 filters also forms a batch normalisation's statistics, over 500 images of 28 x 28, 159 -> 165).
+inline int conv_first_fwd_tiles(int taps, int cout, bool statistics) {
+  const int tiles = (int)ceil_div((int64_t)cout, (int64_t)16);
+  return !statistics && taps <= 20 && cout > 32 && cout % 32 == 0 ? 2 : std::min(tiles, 4);
+}
+
 // Filter gradient: `rows` rows of `wo` output positions for at most `room` workgroups of four wavefronts.  A wavefront takes items_per_wave rows in
 // turn; where there are not half as many rows as wavefronts (signals: images of one or a few long rows), rows are cut into
 // segments of whole trips of 16 positions, until there is one for every wavefront.  9 taps x 32 filters with whole rows and

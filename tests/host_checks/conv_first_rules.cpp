@@ -1,5 +1,6 @@
 // Which first layers have kernels of their own and how these divide them, asked on the command line and answered without a GPU:
 //   forward kh kw cin cout  whether that product of 24 x 24 images runs there (0/1)
+//   tiles taps cout stats  tiles of 16 filters a wavefront of the forward product takes
 //   cut rows wo room        segments, their length, items per wavefront, workgroups
 #include "../../scanet3_amd/csrc/conv_first_rules.hpp"
 
@@ -15,6 +16,10 @@ int main(int argc, char** argv) {
     e.out = at;
     e.ldo = cout;
     std::printf("%d\n", sn::conv_first_fwd_ok(sn::ConvGeom{64, 24, 24, cin, 25 - kh, 25 - kw, cout, kh, kw, 1, 1, 0, 0}, e));
+    return 0;
+  }
+  if (argc == 5 && !std::strcmp(argv[1], "tiles")) {
+    std::printf("%d\n", sn::conv_first_fwd_tiles(std::atoi(argv[2]), std::atoi(argv[3]), std::atoi(argv[4]) != 0));
     return 0;
   }
   if (argc != 5 || std::strcmp(argv[1], "cut")) return 2;

@@ -42,3 +42,9 @@ def test_many_taps_onto_many_filters_stay_with_the_tiled_kernels(ask):
     for kh, kw, cin, cout, want in ((4, 4, 4, 192, 1), (4, 4, 4, 196, 0), (4, 4, 4, 256, 0), (4, 4, 3, 512, 0), (3, 3, 4, 344, 0), (5, 5, 2, 256, 0), (8, 8, 1, 512, 0),
                                     (4, 4, 2, 512, 0), (3, 3, 3, 512, 1), (3, 3, 1, 1400, 1), (7, 4, 1, 700, 1), (3, 3, 3, 50, 0), (9, 8, 1, 32, 0), (3, 3, 5, 32, 0)):
         assert ask("forward", kh, kw, cin, cout) == [want], (kh, kw, cin, cout)
+
+
+def test_two_tiles_of_filters_where_a_wavefront_can_gather_again(ask):
+    for taps, cout, want in ((9, 64, 2), (18, 128, 2), (4, 96, 2), (20, 256, 2), (9, 16, 1), (9, 32, 2), (9, 48, 3), (9, 56, 4), (9, 80, 4), (27, 64, 4), (32, 128, 4)):
+        assert ask("tiles", taps, cout, 0) == [want], (taps, cout)
+    assert ask("tiles", 9, 64, 1) == [4]

@@ -521,6 +521,11 @@ MODELS = {
                                              (9, 11, 4), 6, "uniform_onehot"),
     "batchnorm_over_first_layer_100_filters": ([("conv", 100, (3, 2), (1, 1), "valid", "tanh", False), ("batchnorm", 0.9, 1e-3), ("flatten",),
                                                 ("dense", 3, "softmax")], "cce", (9, 8, 3), 21, "uniform_onehot"),
+    # first-layer forward with two tiles of filters a wavefront, three launch columns; 64 filters with a BatchNorm's statistics (four)
+    "conv_first_layer_96_filters_18_taps": ([("conv", 96, (3, 3), (1, 1), "same", "relu", True), ("flatten",), ("dense", 3, "softmax")], "cce",
+                                            (11, 7, 2), 9, "uniform_onehot"),
+    "batchnorm_over_first_layer_64_filters": ([("conv", 64, (3, 3), (1, 1), "valid", "tanh", False), ("batchnorm", 0.9, 1e-3), ("flatten",),
+                                               ("dense", 3, "softmax")], "cce", (13, 8, 1), 25, "uniform_onehot"),
     # second-layer filter gradient in its row form (32 or 64 input channels): an odd row length (one padding position per row), Same
     # padding on all four sides, a stride in each direction, a bias; and 64 input channels under a 5 x 3 kernel onto 32 filters
     "conv_rows_same_stride_bias": ([("conv", 32, (3, 3), (1, 1), "valid", "relu", False), ("conv", 64, (3, 3), (2, 1), "same", "tanh", True),
