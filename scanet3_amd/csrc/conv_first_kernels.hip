@@ -334,10 +334,11 @@ __device__ __forceinline__ void first_act(int act, float (&v)[N], float param) {
   }
 }
 
-// KS steps of four taps, NT tiles of 16 filters (blockIdx.y: which 16 NT of them); VEC: a lane's NT filters are neighbours and leave as one
-// vector, otherwise they are 16 apart
-template <int KS, int NT, bool VEC, bool STATS>
+// KS steps of four taps, NT tiles of 16 filters (blockIdx.y: which 16 NT of them).  With two or four tiles a lane's NT filters are neighbours
+// and leave as one vector (conv_first_fwd_ok: whole vectors of filters, 16-byte aligned), with three they are 16 apart.
+template <int KS, int NT, bool STATS>
 __global__ __launch_bounds__(256) void conv_first_fwd_kernel(FirstForward k) {
+  constexpr bool VEC = NT == 2 || NT == 4;
   __shared__ float moments[STATS ? 4 : 1][2][STATS ? 16 * NT : 1];
   __shared__ float counts[4];
   const ConvGeom& g = k.g;
@@ -412,7 +413,7 @@ __global__ __launch_bounds__(256) void conv_first_fwd_kernel(FirstForward k) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       if (i >= mine) continue;
-      if constexpr (VEC && NT > 1) {
+      if constexpr (VEC) {
         typedef float vec __attribute__((ext_vector_type(NT)));
         vec o;
 #pragma unroll
@@ -485,21 +486,19 @@ __global__ __launch_bounds__(256) void conv_first_fwd_kernel(FirstForward k) {
   }
 }
 
-template <int KS, int NT, bool VEC>
+template <int KS, int NT>
 void launch_first_fwd_tiles(sn_ctx* ctx, const FirstForward& k, int blocks, bool stats) {
   const dim3 grid((unsigned)blocks, (unsigned)ceil_div(k.g.cout, 16 * NT));
-  if (stats) hipLaunchKernelGGL((conv_first_fwd_kernel<KS, NT, VEC, true>), grid, dim3(256), 0, ctx->stream, k);
-  else hipLaunchKernelGGL((conv_first_fwd_kernel<KS, NT, VEC, false>), grid, dim3(256), 0, ctx->stream, k);
+  if (stats) hipLaunchKernelGGL((conv_first_fwd_kernel<KS, NT, true>), grid, dim3(256), 0, ctx->stream, k);
+  else hipLaunchKernelGGL((conv_first_fwd_kernel<KS, NT, false>), grid, dim3(256), 0, ctx->stream, k);
 }
 template <int KS>
 void launch_first_fwd_steps(sn_ctx* ctx, const FirstForward& k, int blocks, bool stats) {
-  const int nt = conv_first_fwd_tiles(k.taps, k.g.cout, stats);
-  const bool vec = k.g.cout % nt == 0 && k.e.ldo % nt == 0 && (reinterpret_cast<uintptr_t>(k.e.out) & 15u) == 0;
-  switch (nt) {
-    case 1: return launch_first_fwd_tiles<KS, 1, false>(ctx, k, blocks, stats);
-    case 2: return vec ? launch_first_fwd_tiles<KS, 2, true>(ctx, k, blocks, stats) : launch_first_fwd_tiles<KS, 2, false>(ctx, k, blocks, stats);
-    case 3: return launch_first_fwd_tiles<KS, 3, false>(ctx, k, blocks, stats);
-    default: return vec ? launch_first_fwd_tiles<KS, 4, true>(ctx, k, blocks, stats) : launch_first_fwd_tiles<KS, 4, false>(ctx, k, blocks, stats);
+  switch (conv_first_fwd_tiles(k.taps, k.g.cout, stats)) {
+    case 1: return launch_first_fwd_tiles<KS, 1>(ctx, k, blocks, stats);
+    case 2: return launch_first_fwd_tiles<KS, 2>(ctx, k, blocks, stats);
+    case 3: return launch_first_fwd_tiles<KS, 3>(ctx, k, blocks, stats);
+    default: return launch_first_fwd_tiles<KS, 4>(ctx, k, blocks, stats);
   }
 }
 
