@@ -230,12 +230,13 @@ int launch_step_slice_add(sn_ctx* ctx, float* dst, const float* src, int64_t src
 int launch_lstm_gates_bwd(sn_ctx* ctx, const LstmGateBwdArgs& a, int rows, int hidden);
 
 // ---- Dense(H, act) >> Dense(C, Softmax) + CategoricalCrossentropy in two launches (mlp2_kernels.hip): forward, loss terms
-// and every gradient.  scratch_a: what mlp2_fused_ok asks for; parts: mlp2_parts_elems floats; row_loss: `rows` floats.
-bool mlp2_fused_ok(int rows_max, int K, int H, int C, int64_t scratch_a_elems, int64_t scratch_b_elems);
-int64_t mlp2_parts_elems(int rows_max, int H, int C);
+// and every gradient.  scratch: mlp2_scratch_elems floats; row_loss: `rows` floats.
+bool mlp2_fused_ok(int rows_max, int K, int H, int C);
+bool mlp2_input_ok(const float* x);  // (a batch elsewhere takes the general kernels)
+int64_t mlp2_scratch_elems(int rows_max, int H, int C);
 int launch_mlp2_grad(sn_ctx* ctx, const float* x, const float* y, const float* w1, const float* b1, const float* w2, const float* b2, int rows,
-                     int K, int H, int C, int act1, float act1_param, bool stable, float* h, float* z2, float* p, float* scratch_a,
-                     float* parts, float* row_loss, float* loss_dev, float* g_w1, float* g_b1, float* g_w2, float* g_b2,
+                     int K, int H, int C, int act1, float act1_param, bool stable, float* h, float* z2, float* p, float* scratch,
+                     float* row_loss, float* loss_dev, float* g_w1, float* g_b1, float* g_w2, float* g_b2,
                      const struct Mlp2Update* update = nullptr);
 // The optimizer update riding in the second launch: every thread that finishes a gradient value applies it to its
 // parameter on the spot (same arithmetic as the streaming optimizer kernels), so a training step is two launches.  w, g

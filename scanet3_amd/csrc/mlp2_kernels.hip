@@ -338,22 +338,23 @@ void launch_rows(sn_ctx* ctx, const Mlp2Args& a, int blocks, int n) {
 
 }  // namespace
 
-// Shapes the fused pass takes: K a multiple of 4 up to 1024, H <= 64, C <= 16, up to 1792 rows, and activations of a size that
-// the pass was measured at.
-bool mlp2_fused_ok(int rows_max, int K, int H, int C, int64_t scratch_a_elems, int64_t scratch_b_elems) {
-  const int64_t nblk = ceil_div(rows_max, MR);
-  return K % 4 == 0 && K >= 4 && K <= 1024 && H >= 1 && H <= MH && C >= 1 && C <= MC && rows_max <= MAX_ROWS &&
-         scratch_a_elems >= nblk * 4 * 64 * 4 && scratch_b_elems >= nblk * ((int64_t)H * C + H + C);
+// Shapes the fused pass takes: K a multiple of 4 up to 1024, H <= 64, C <= 16, up to 1792 rows; x in whole vectors.
+// A training step here and by the general kernels: 8 -> 5 -> 1 at 16 rows 7.6 and 28.6 us, 36 -> 37 -> 16 at 33 rows 9.5 and 32.5,
+// 32 -> 32 -> 10 at 1000 rows 11.0 and 41.8, 68 -> 64 -> 16 at 1000 rows 12.1 and 40.1.
+bool mlp2_fused_ok(int rows_max, int K, int H, int C) {
+  return K % 4 == 0 && K >= 4 && K <= 1024 && H >= 1 && H <= MH && C >= 1 && C <= MC && rows_max <= MAX_ROWS;
 }
-int64_t mlp2_parts_elems(int rows_max, int H, int C) { return ceil_div(rows_max, MR) * (MR / RB) * ((int64_t)H * C + H + C); }
+bool mlp2_input_ok(const float* x) { return aligned16(x); }
+static int64_t fragment_elems(int rows) { return ceil_div(rows, MR) * 4 * 64 * 4; }
+int64_t mlp2_scratch_elems(int rows_max, int H, int C) { return fragment_elems(rows_max) + ceil_div(rows_max, MR) * (MR / RB) * ((int64_t)H * C + H + C); }
 
 int launch_mlp2_grad(sn_ctx* ctx, const float* x, const float* y, const float* w1, const float* b1, const float* w2, const float* b2, int rows,
-                     int K, int H, int C, int act1, float act1_param, bool stable, float* h, float* z2, float* p, float* scratch_a,
-                     float* parts, float* row_loss, float* loss_dev, float* g_w1, float* g_b1, float* g_w2, float* g_b2,
+                     int K, int H, int C, int act1, float act1_param, bool stable, float* h, float* z2, float* p, float* scratch,
+                     float* row_loss, float* loss_dev, float* g_w1, float* g_b1, float* g_w2, float* g_b2,
                      const Mlp2Update* update) {
   SN_REQUIRE(rows > 0, "loss over an empty batch");
-  SN_REQUIRE(aligned16(x) && aligned16(scratch_a), "mlp2: x and the scratch buffer must be 16-byte aligned");
-  Mlp2Args a{x, y, w1, b1, w2, b2, h, z2, p, scratch_a, row_loss, parts, g_w1, g_b1, g_w2, g_b2,
+  SN_REQUIRE(mlp2_input_ok(x) && aligned16(scratch), "mlp2: x and the scratch buffer must be 16-byte aligned");
+  Mlp2Args a{x, y, w1, b1, w2, b2, h, z2, p, scratch, row_loss, scratch + fragment_elems(rows), g_w1, g_b1, g_w2, g_b2,
              rows, K, H, C, act1, stable ? 1 : 0, act1_param, -(1.0f / (float)rows), update ? *update : Mlp2Update{}};
   const int nblk = (int)ceil_div(rows, MR), nslab = (int)ceil_div(K, 16);
   {

@@ -88,7 +88,7 @@ struct sn_replica {
   std::vector<uint8_t*> arg;    // per op: max-pool argmax
   float* grad_buf[2] = {nullptr, nullptr};
   float* ws = nullptr;
-  float* mlp2_parts = nullptr;  // partial sums of the two-launch training pass (mlp2_kernels.hip)
+  float* mlp2_scratch = nullptr;  // fragments and partial sums of the two-launch training pass (mlp2_kernels.hip)
   float* loss_dev = nullptr;
   float* loss_partials = nullptr;
   unsigned long long* count_dev = nullptr;
@@ -465,7 +465,7 @@ static int alloc_replica(sn_replica* r) {
     SN_TRY(dev_alloc(r, &r->s[s], m->flat_elems));
     SN_TRY(launch_fill(r->ctx, r->s[s], r->opt.init_acc, m->flat_elems));
   }
-  if (mlp2_path(m)) SN_TRY(dev_alloc(r, &r->mlp2_parts, mlp2_parts_elems((int)B, (int)m->ops[0].out_elems, (int)m->ops[1].out_elems)));
+  if (mlp2_path(m)) SN_TRY(dev_alloc(r, &r->mlp2_scratch, mlp2_scratch_elems((int)B, (int)m->ops[0].out_elems, (int)m->ops[1].out_elems)));
   const size_t n_ops = m->ops.size();
   r->act.assign(n_ops, nullptr);
   r->arg.assign(n_ops, nullptr);
@@ -1174,8 +1174,7 @@ static bool mlp2_path(const sn_model* m) {
   const Op& d1 = m->ops[0];
   const Op& d2 = m->ops[1];
   if (d1.kind != OP_DENSE || d2.kind != OP_DENSE || d2.act != SN_ACT_IDENTITY || m->ops[2].kind != OP_SOFTMAX) return false;
-  const int64_t scratch = (int64_t)m->batch * m->max_act_elems;
-  return mlp2_fused_ok(m->batch, (int)d1.in_elems, (int)d1.out_elems, (int)d2.out_elems, scratch, scratch);
+  return mlp2_fused_ok(m->batch, (int)d1.in_elems, (int)d1.out_elems, (int)d2.out_elems);
 }
 
 // for_update: the optimizer update of the same step follows (update()), which may then take over reductions this pass
@@ -1243,7 +1242,7 @@ static int grad_pass(sn_replica* r, const float* x, const float* y, int rows, bo
 static int grad_pass_body(sn_replica* r, const float* x, const float* y, int rows, bool want_loss) {
   sn_model* m = r->model;
   const int last = (int)m->ops.size() - 1;
-  if (mlp2_path(m)) {
+  if (mlp2_path(m) && mlp2_input_ok(x)) {
     const Op& d1 = m->ops[0];
     const Op& d2 = m->ops[1];
     // A training step of a model without penalties: the second launch applies the optimizer to every gradient value it
@@ -1262,7 +1261,7 @@ static int grad_pass_body(sn_replica* r, const float* x, const float* y, int row
     }
     SN_TRY(launch_mlp2_grad(r->ctx, x, y, param_ptr(r, r->w, d1.w), param_ptr(r, r->w, d1.b), param_ptr(r, r->w, d2.w), param_ptr(r, r->w, d2.b), rows,
                             (int)d1.in_elems, (int)d1.out_elems, (int)d2.out_elems, d1.act, d1.act_param,
-                            (m->flags & SN_FLAG_STABLE_SOFTMAX) != 0, r->act[0], r->act[1], r->act[2], r->grad_buf[0], r->mlp2_parts,
+                            (m->flags & SN_FLAG_STABLE_SOFTMAX) != 0, r->act[0], r->act[1], r->act[2], r->mlp2_scratch,
                             r->loss_partials, want_loss ? r->loss_dev : nullptr, param_ptr(r, r->g, d1.w), param_ptr(r, r->g, d1.b),
                             param_ptr(r, r->g, d2.w), param_ptr(r, r->g, d2.b), upd));
     if (want_loss) SN_TRY(add_penalties(r, true));

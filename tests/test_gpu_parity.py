@@ -693,6 +693,10 @@ KERNEL_OF_MODEL = {
     "dense_act_grad_two_rows": "gemm_f32_and_activation_gradient",
     "dense_act_grad_splits": "gemm_f32_and_activation_gradient",
     "mlp_cfg1": "mlp2_",
+    "mlp2_odd_sizes_tanh": "mlp2_",
+    "mlp2_64_hidden_relu": "mlp2_",
+    "mlp2_identity_one_class": "mlp2_",
+    "mlp2_regularized": "mlp2_",
     "mlp2_1030_rows": "mlp2_",
     "mlp2_515_rows": "mlp2_",
 }
@@ -768,6 +772,31 @@ def test_batchnorm_pass_of_fewer_rows_than_the_batch(S, ctx):
     grads64 = h.omodel.grad(x.astype(np.float64), y.astype(np.float64), {p: v.astype(np.float64) for p, v in params.items()})[1]
     for p in ograds:
         assert rel_err(ggrads[p], grads64[p]) <= max(TOL_GEMM, 3.0 * rel_err(ograds[p], grads64[p])), p
+    h.close()
+
+
+def test_two_layer_pass_of_a_batch_off_the_vectors(S, ctx):
+    """The two-launch pass reads whole vectors: a batch 4 bytes off a 16-byte boundary takes the general kernels, to the same gradients."""
+    spec, loss, in_shape, batch, kind = MODELS["mlp2_515_rows"]
+    rng = np.random.default_rng(99)
+    h = Harness(S, ctx, spec, loss, in_shape, batch, S.Adam(0.01))
+    params = glorot_params(h.omodel, (batch,) + in_shape, rng)
+    x, y = make_data(kind, rng, batch, in_shape, 2)
+    h.rep.set_params(params)
+    xb, yb, off = ctx.to_device(x), ctx.to_device(y), ctx.to_device(np.concatenate([[0], x.reshape(-1)]).astype(f32)).offset(1)
+    loss_at = h.rep.grad(xb, yb)
+    want = h.rep.get_grads()
+    assert abs(h.rep.grad(off, yb) - loss_at) <= TOL_GEMM * max(1.0, abs(loss_at))
+    for p, g in h.rep.get_grads().items():
+        assert rel_err(g, want[p]) <= TOL_GEMM, p
+    h.rep.step(xb, yb, 1)
+    want = h.rep.get_params()
+    h.rep.set_params(params)
+    for s in range(2):
+        h.rep.set_opt_state(s, {p: np.zeros_like(v) for p, v in params.items()})
+    h.rep.step(off, yb, 1)
+    for p, v in h.rep.get_params().items():
+        assert np.abs(v - params[p]).max() > 0 and rel_err(v, want[p]) <= TOL_FINAL_WEIGHTS, p
     h.close()
 
 
