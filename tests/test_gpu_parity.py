@@ -2011,6 +2011,42 @@ def test_bf16_dense_path_matches_bf16_rounded_oracle(S, ctx, dims, batch):
     yb.free()
 
 
+@pytest.mark.parametrize("dims,batch,rows,label", [
+    ((100, 150, 60, 10), 72, 72, True),      # no width a multiple of eight: both hidden layers' gradients leave the products through the activations
+    ((64, 128, 10), 64, 64, False),          # a ragged layer over one whose own kernels take its activation's gradient
+    ((256, 256, 256, 10), 256, 256, False),  # ... over two whose outputs are whole tiles
+    ((64, 128, 96, 16), 72, 67, True),       # whole widths, rows that are no multiple of eight
+    ((30, 64, 128, 21), 40, 33, True),
+])
+@pytest.mark.parametrize("acts", [("relu", "tanh"), ("sigmoid", "relu")])
+def test_bf16_ragged_layers_match_bf16_rounded_oracle(S, ctx, dims, batch, rows, label, acts):
+    """Input gradients of bf16 products that leave through the gradient of the activation below, and the layers where they must not."""
+    from scanet3_amd import _lib as L
+    spec = [("dense", d, acts[i % 2]) for i, d in enumerate(dims[1:-1])] + [("dense", dims[-1], "softmax")]
+    rng = np.random.default_rng(20251125 + 5)
+    h = Harness(S, ctx, spec, "cce", (dims[0],), batch, flags=L.FLAG_GEMM_BF16)
+    om = O.Model(h.omodel.layers, O.LOSS_CCE, bf16_dense=True)
+    params = glorot_params(om, (batch, dims[0]), rng)
+    for p in params:
+        if params[p].ndim == 1:
+            params[p] = rng.uniform(-0.1, 0.1, params[p].shape).astype(f32)
+    x, y = rng.standard_normal((rows, dims[0])).astype(f32), one_hot(rng, rows, dims[-1])
+    h.rep.set_params(params)
+    xb, yb = ctx.to_device(x), ctx.to_device(y)
+    oloss, ograds = om.grad(x, y, params)
+    ctx.profile_reset()
+    ctx.profile(True)
+    gloss = h.rep.grad(xb, yb, rows=rows)
+    ctx.sync()
+    ctx.profile(False)
+    assert any(l.startswith("gemm_bf16_and_activation_gradient") for l in ctx.profile_report()) == label, list(ctx.profile_report())
+    assert abs(gloss - float(oloss)) <= TOL_BF16 * max(1.0, abs(float(oloss)))
+    ggrads = h.rep.get_grads()
+    for p in ograds:
+        assert norm_err(ggrads[p], ograds[p]) <= TOL_BF16, p
+    h.close()
+
+
 @pytest.mark.parametrize("alg", ["adam", "amsgrad", "sgd_momentum"])
 def test_bf16_layerwise_updates_equal_one_update_of_the_flat_buffer(S, ctx, alg):
     """A training step of a model of bf16 Dense layers updates each layer as soon as its gradients are complete, on a second
