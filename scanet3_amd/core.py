@@ -275,7 +275,7 @@ class Replica:
         """training=False: the frozen model (`TrainedModel.result`); True: `model.resultStateful`'s output."""
         rows = self.model.batch if rows is None else rows
         out = np.empty((max(rows, 0),) + self.model.output_shape, np.float32)
-        check(lib.sn_forward_host(self.handle, self._ptr(x), rows, out.ctypes.data_as(C.c_void_p), int(training)))
+        check(lib.sn_forward_host(self.handle, self._ptr(x), rows, out.ctypes.data_as(C.c_void_p), 1 if training else 0))
         return out
 
     def forward_static(self, x, out: "DeviceBuffer", rows: Optional[int] = None) -> None:

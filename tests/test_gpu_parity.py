@@ -775,6 +775,17 @@ def test_batchnorm_pass_of_fewer_rows_than_the_batch(S, ctx):
     h.close()
 
 
+def test_forward_asks_training_for_its_truth(S, ctx):
+    """`training` is any value with a truth: None is the frozen model."""
+    rng = np.random.default_rng(3)
+    h = Harness(S, ctx, [("dense", 4, "tanh"), ("batchnorm", 0.9, 1e-3)], "mse", (3,), 5)
+    h.rep.set_params(glorot_params(h.omodel, (5, 3), rng))
+    xb = ctx.to_device(rng.standard_normal((5, 3)).astype(f32))
+    np.testing.assert_array_equal(h.rep.forward(xb, training=None), h.rep.forward(xb, training=False))
+    np.testing.assert_array_equal(h.rep.forward(xb, training="yes"), h.rep.forward(xb, training=True))
+    h.close()
+
+
 def test_two_layer_pass_of_a_batch_off_the_vectors(S, ctx):
     """The two-launch pass reads whole vectors: a batch 4 bytes off a 16-byte boundary takes the general kernels, to the same gradients."""
     spec, loss, in_shape, batch, kind = MODELS["mlp2_515_rows"]
