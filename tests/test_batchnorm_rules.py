@@ -30,3 +30,11 @@ def test_a_reduction_writes_no_more_slices_than_it_asks_for(ask, cols):
     for rows in (1, 2, 63, 64, 65, 1000, 8192, 8275, 33000, 700001):
         asked, written = ask("written", cols, rows)
         assert 1 <= written <= asked
+
+
+@pytest.mark.parametrize("cols", [4, 12, 100, 132, 256, 260, 388, 516, 600, 1000, 1024])
+def test_whole_vectors_of_channels_fill_the_chip(ask, cols):
+    """Slices are workgroups of the streaming form: some 2 for each of 256 CUs where the rows allow it, whatever the channel count."""
+    for rows in (8192, 40000):
+        _, written = ask("stream", cols, rows)
+        assert written >= min(400, rows // 17, rows * cols // 4 // 4096)
