@@ -263,6 +263,7 @@ template <class F>
 __device__ __forceinline__ void for_slices(int first, int slices, int cols, int c, F f) {
 #pragma unroll
   for (int u = 0; u < FINISH_LOADS; ++u) {
+    if (64 * u >= slices) break;  // (uniform; nearly always all that there are lie before it)
     const int i = first + 64 * u, at = min(i, slices - 1);
     f(u, (int64_t)at * cols + min(c, cols - 1), i < slices);
   }
@@ -495,8 +496,8 @@ unsigned grid_for(const sn_ctx* ctx, int64_t n, int per_block) {
   return blocks < 1 ? 1u : (unsigned)blocks;
 }
 
-bool stream_ok(int64_t rows, int cols, const void* x, const void* dy, const void* part0, int64_t part1_offset) {
-  return bn_stream_form(rows, cols) && part1_offset % 4 == 0 &&
+bool stream_ok(int cols, const void* x, const void* dy, const void* part0, int64_t part1_offset) {
+  return bn_stream_form(cols) && part1_offset % 4 == 0 &&
          ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(dy) | reinterpret_cast<uintptr_t>(part0)) & 15u) == 0;
 }
 
@@ -550,7 +551,7 @@ static int batchnorm_statistics(sn_ctx* ctx, const float* x, int64_t rows, int c
     LaunchScope scope(ctx, "batchnorm_mean_and_variance");
     hipLaunchKernelGGL(bn_moments_kernel, dim3(cb), dim3(256), 0, ctx->stream, (const float*)stats->part_mean, (const float*)stats->part_m2, stats->slices,
                        cols, stats->whole, stats->last, (float)rows, scale);
-  } else if (2 * half <= ws_elems && stream_ok(rows, cols, x, nullptr, ws, half)) {
+  } else if (2 * half <= ws_elems && stream_ok(cols, x, nullptr, ws, half)) {
     const BnStream st = bn_stream_of(ctx->compute_units, rows, cols);
     LaunchScope scope(ctx, "batchnorm_mean_and_variance");
     hipLaunchKernelGGL(bn_stats_v4_kernel, dim3((unsigned)st.slices), dim3(256), 0, ctx->stream, (const bn_f4*)x, ws, ws + half, st.n4, cols, st.active,
@@ -646,7 +647,7 @@ int launch_batchnorm_bwd(sn_ctx* ctx, const float* x, const float* dy, float* dx
   {
     LaunchScope scope(ctx, "batchnorm_gradient_sums");
     int s = 0;
-    if (stream_ok(rows, cols, x, dy, ws, half)) {
+    if (stream_ok(cols, x, dy, ws, half)) {
       const BnStream st = bn_stream_of(ctx->compute_units, rows, cols);
       s = st.slices;
       hipLaunchKernelGGL(bn_grad_sums_v4_kernel, dim3((unsigned)s), dim3(256), 0, ctx->stream, (const bn_f4*)x, (const bn_f4*)dy, mean, ws, part1, st.n4,

@@ -24,7 +24,7 @@ int main(int argc, char** argv) {
   }
   if (!std::strcmp(argv[1], "written")) {
     int most = sn::bn_row_slices(cus, rows, cols);
-    if (sn::bn_stream_form(rows, cols)) most = std::max(most, sn::bn_stream_of(cus, rows, cols).slices);
+    if (sn::bn_stream_form(cols)) most = std::max(most, sn::bn_stream_of(cus, rows, cols).slices);
     std::printf("%d %d\n", sn::bn_max_slices(cus, rows, cols), most);
     return 0;
   }

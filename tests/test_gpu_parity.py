@@ -578,6 +578,11 @@ MODELS = {
     "batchnorm_200_channels": ([("dense", 200, "tanh"), ("batchnorm", 0.9, 1e-3), ("dense", 5, "softmax")], "cce", (31,), 300, "normal_onehot"),
     "batchnorm_256_channels": ([("dense", 256, "relu"), ("batchnorm", 0.9, 1e-3), ("dense", 5, "softmax")], "cce", (31,), 300, "normal_onehot"),
     "batchnorm_50_channels": ([("dense", 50, "tanh"), ("batchnorm", 0.9, 1e-3), ("dense", 5, "softmax")], "cce", (31,), 300, "normal_onehot"),
+    # whole vectors of channels take the streaming form however few rows there are: one row (its own mean), three, and 17 of 1024 channels
+    "batchnorm_8_channels_1_row": ([("dense", 8, "tanh"), ("batchnorm", 0.9, 1e-3), ("dense", 5, "softmax")], "cce", (7,), 1, "normal_onehot"),
+    "batchnorm_20_channels_3_rows": ([("dense", 20, "tanh"), ("batchnorm", 0.9, 1e-3), ("dense", 5, "softmax")], "cce", (7,), 3, "normal_onehot"),
+    "batchnorm_1024_channels_17_rows": ([("dense", 1024, "tanh"), ("batchnorm", 0.9, 1e-3), ("dense", 5, "softmax")], "cce", (7,), 17, "normal_onehot"),
+    "batchnorm_600_channels": ([("dense", 600, "tanh"), ("batchnorm", 0.9, 1e-3), ("dense", 5, "softmax")], "cce", (31,), 700, "normal_onehot"),
     # a 2 x 2 max pooling right above a BatchNorm: overlapping windows that reach into the padding, 12 channels (252 of a block's 256
     # threads); 48 channels with another stride per direction under the plain form; windows that leave a row and a column of the image
     # out, behind a second layer (whose convolution wants its input gradient, so the layers' backward passes stay apart)
