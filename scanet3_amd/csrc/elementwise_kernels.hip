@@ -919,19 +919,18 @@ __global__ __launch_bounds__(256) void pool_bwd_kernel(const float* __restrict__
   }
 }
 
-// The same backward pass for 2x2 max windows, V channels per thread, 32-bit indices.  Along a dimension of stride 1 an input element lies
-// in up to two windows (TWO_H, TWO_W), along another in at most one; their argmax words and gradients are requested together
-// (windows that do not exist re-read the first element and match no place) and added in the order of the general kernel (oh,
-// then ow, ascending).  Bound by requests and index arithmetic: with four windows looked at whatever the stride,
-// [64 x 48 x 48 x 128] took 21.7 us at stride 2 and 28.5 at stride 3, so 18.5 and 16.8; [1000 x 28 x 28 x 33] 75 and 54 at stride 2.
+// The same backward pass for 2x2 max windows, V channels per thread, 32-bit indices: an input element lies in at most 2 x 2
+// windows (oh_hi - a, ow_hi - d for a, d in {0, 1}); their argmax words and gradients are requested together (windows that do
+// not exist re-read the first element and are ignored) and added in the order of the general kernel (oh, then ow, ascending).
+// For windows of stride 1 along a dimension at least; the others have a kernel of their own below.
 template <int V>
 using pool_vec = float __attribute__((ext_vector_type(V)));
-template <int V, bool TWO_H, bool TWO_W>
+template <int V, int S>  // S: 1 when both strides are (no divisions), 0: read sh, sw
 __global__ __launch_bounds__(256) void pool2x2_bwd_kernel(const float* __restrict__ dy, const uint8_t* __restrict__ arg,
-                                                           float* __restrict__ dx, int n, int h, int w, int c, int ho, int wo, int pt, int pl,
-                                                           const float* __restrict__ y_in, int act, float act_param,
-                                                           FastDiv by_cv, FastDiv by_w, FastDiv by_h, FastDiv by_sh, FastDiv by_sw) {
-  constexpr int WH = TWO_H ? 2 : 1, WW = TWO_W ? 2 : 1;
+                                                           float* __restrict__ dx, int n, int h, int w, int c, int ho, int wo, int sh_,
+                                                           int sw_, int pt, int pl, const float* __restrict__ y_in, int act, float act_param,
+                                                           FastDiv by_cv, FastDiv by_w, FastDiv by_h) {
+  const int sh = S ? S : sh_, sw = S ? S : sw_;
   const uint32_t cv = (uint32_t)(c / V);
   const uint32_t total = (uint32_t)n * h * w * cv;
   const uint32_t stride = (uint32_t)gridDim.x * blockDim.x;
@@ -942,30 +941,67 @@ __global__ __launch_bounds__(256) void pool2x2_bwd_kernel(const float* __restric
     const int ix = (int)(t - t2 * (uint32_t)w);
     const uint32_t b = div_by(t2, by_h);
     const int iy = (int)(t2 - b * (uint32_t)h);
-    // the first of the windows along each dimension (it may not exist) and the element's place in it; the second starts one further
-    const int oh0 = TWO_H ? iy + pt - 1 : (int)div_by((uint32_t)(iy + pt), by_sh), ry = iy + pt - oh0 * (int)by_sh.d;
-    const int ow0 = TWO_W ? ix + pl - 1 : (int)div_by((uint32_t)(ix + pl), by_sw), rx = ix + pl - ow0 * (int)by_sw.d;
+    int oh_lo = iy + pt - 1;
+    oh_lo = oh_lo <= 0 ? 0 : (oh_lo + sh - 1) / sh;
+    int oh_hi = (iy + pt) / sh;
+    if (oh_hi > ho - 1) oh_hi = ho - 1;
+    int ow_lo = ix + pl - 1;
+    ow_lo = ow_lo <= 0 ? 0 : (ow_lo + sw - 1) / sw;
+    int ow_hi = (ix + pl) / sw;
+    if (ow_hi > wo - 1) ow_hi = wo - 1;
     pool_vec<V> yv = {};
     if (y_in) yv = *(const pool_vec<V>*)(y_in + i * V);
-    uint32_t at[WH * WW], want[WH * WW];
-    pool_vec<V> g[WH * WW];
+    uint32_t a4[4], want[4];
+    pool_vec<V> g[4];
+    bool on[4];
 #pragma unroll
-    for (int k = 0; k < WH * WW; ++k) {
-      const int oh = oh0 + k / WW, ow = ow0 + k % WW, y = ry - k / WW, x = rx - k % WW;
-      const bool on = (unsigned)oh < (unsigned)ho && (unsigned)ow < (unsigned)wo && (TWO_H || y < 2) && (TWO_W || x < 2);
-      const uint32_t o = on ? ((b * ho + oh) * wo + ow) * c + ch : 0u;
-      want[k] = on ? (uint32_t)(y * 2 + x) : 255u;
-      at[k] = V == 4 ? *(const uint32_t*)(arg + o) : (uint32_t)arg[o];
+    for (int k = 0; k < 4; ++k) {
+      const int oh = oh_lo + (k >> 1), ow = ow_lo + (k & 1);
+      on[k] = oh <= oh_hi && ow <= ow_hi;
+      const uint32_t o = on[k] ? ((b * ho + oh) * wo + ow) * c + ch : 0u;
+      want[k] = (uint32_t)((iy - (oh * sh - pt)) * 2 + (ix - (ow * sw - pl)));
+      a4[k] = V == 4 ? *(const uint32_t*)(arg + o) : (uint32_t)arg[o];
       g[k] = *(const pool_vec<V>*)(dy + o);
     }
     pool_vec<V> s = {};
 #pragma unroll
-    for (int k = 0; k < WH * WW; ++k) {
-      if (want[k] == 255u) continue;
+    for (int k = 0; k < 4; ++k) {
 #pragma unroll
       for (int e = 0; e < V; ++e)
-        if (((at[k] >> (8 * e)) & 255u) == want[k]) s[e] += g[k][e];
+        if (on[k] && ((a4[k] >> (8 * e)) & 255u) == want[k]) s[e] += g[k][e];
     }
+    if (y_in) {
+#pragma unroll
+      for (int e = 0; e < V; ++e) s[e] = act_bwd(act, yv[e], s[e], act_param);
+    }
+    *(pool_vec<V>*)(dx + i * V) = s;
+  }
+}
+
+// Strides of two and more along both dimensions: an element lies in at most one window, found by two multiplications.
+// [64 x 48 x 48 x 128] 18.4 us at stride 2 and 16.7 at stride 3, by the kernel above 22 and 28.8; [1000 x 28 x 28 x 33], stride 2, 53 and 73.
+template <int V>
+__global__ __launch_bounds__(256) void pool2x2_bwd_apart_kernel(const float* __restrict__ dy, const uint8_t* __restrict__ arg,
+                                                                 float* __restrict__ dx, int n, int h, int w, int c, int ho, int wo, int pt, int pl,
+                                                                 const float* __restrict__ y_in, int act, float act_param, FastDiv by_cv,
+                                                                 FastDiv by_w, FastDiv by_h, FastDiv by_sh, FastDiv by_sw) {
+  const uint32_t cv = (uint32_t)(c / V);
+  const uint32_t total = (uint32_t)n * h * w * cv;
+  const uint32_t stride = (uint32_t)gridDim.x * blockDim.x;
+  for (uint32_t i = (uint32_t)xcd_contiguous_block() * blockDim.x + threadIdx.x; i < total; i += stride) {
+    const uint32_t t = div_by(i, by_cv), ch = (i - t * cv) * V;
+    const uint32_t t2 = div_by(t, by_w), b = div_by(t2, by_h);
+    const uint32_t ix = t - t2 * (uint32_t)w + (uint32_t)pl, iy = t2 - b * (uint32_t)h + (uint32_t)pt;
+    const uint32_t oh = div_by(iy, by_sh), ow = div_by(ix, by_sw), y = iy - oh * by_sh.d, x = ix - ow * by_sw.d;
+    const bool on = oh < (uint32_t)ho && ow < (uint32_t)wo && y < 2u && x < 2u;
+    const uint32_t o = on ? ((b * ho + oh) * wo + ow) * c + ch : 0u, want = on ? y * 2u + x : 255u;
+    pool_vec<V> yv = {};
+    if (y_in) yv = *(const pool_vec<V>*)(y_in + i * V);
+    const uint32_t at = V == 4 ? *(const uint32_t*)(arg + o) : (uint32_t)arg[o];
+    const pool_vec<V> g = *(const pool_vec<V>*)(dy + o);
+    pool_vec<V> s = {};
+#pragma unroll
+    for (int e = 0; e < V; ++e) s[e] = ((at >> (8 * e)) & 255u) == want ? s[e] + g[e] : s[e];
     if (y_in) {
 #pragma unroll
       for (int e = 0; e < V; ++e) s[e] = act_bwd(act, yv[e], s[e], act_param);
@@ -978,12 +1014,15 @@ template <int V>
 static void launch_pool2x2_bwd(sn_ctx* ctx, const dim3& grid, const float* dy, const uint8_t* arg, float* dx, int n, int h, int w, int c, int ho, int wo,
                                int sh, int sw, int pt, int pl, const float* y_in, int act, float act_param) {
   const FastDiv by_cv = fast_div((uint32_t)(c / V)), by_w = fast_div((uint32_t)w), by_h = fast_div((uint32_t)h);
-  auto launch = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, ctx->stream, dy, arg, dx, n, h, w, c, ho, wo, pt, pl, y_in, act, act_param, by_cv, by_w, by_h,
-                       fast_div((uint32_t)sh), fast_div((uint32_t)sw));
-  };
-  if (sh == 1) sw == 1 ? launch(pool2x2_bwd_kernel<V, true, true>) : launch(pool2x2_bwd_kernel<V, true, false>);
-  else sw == 1 ? launch(pool2x2_bwd_kernel<V, false, true>) : launch(pool2x2_bwd_kernel<V, false, false>);
+#define SN_POOL2X2_BWD(S)                                                                                                                  \
+  hipLaunchKernelGGL((pool2x2_bwd_kernel<V, S>), grid, dim3(256), 0, ctx->stream, dy, arg, dx, n, h, w, c, ho, wo, sh, sw, pt, pl, y_in, act, \
+                     act_param, by_cv, by_w, by_h)
+  if (sh == 1 && sw == 1) SN_POOL2X2_BWD(1);
+  else if (sh == 1 || sw == 1) SN_POOL2X2_BWD(0);
+  else
+    hipLaunchKernelGGL(pool2x2_bwd_apart_kernel<V>, grid, dim3(256), 0, ctx->stream, dy, arg, dx, n, h, w, c, ho, wo, pt, pl, y_in, act, act_param, by_cv,
+                       by_w, by_h, fast_div((uint32_t)sh), fast_div((uint32_t)sw));
+#undef SN_POOL2X2_BWD
 }
 
 int launch_pool_bwd(sn_ctx* ctx, bool avg, const float* dy, const uint8_t* arg, float* dx, int n, int h, int w, int c, int ho, int wo,
