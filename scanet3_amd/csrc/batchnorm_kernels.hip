@@ -8,7 +8,7 @@
 //
 // All of it is memory bound: every pass reads the activation once with 8 row-loads in flight per
 // lane; the per-channel reductions are cut into row slices so the grid covers the chip, and the
-// slices are added in slice order by one thread per channel (deterministic, no atomics).  So what a pass
+// slices are added by 64 threads a channel whose sums meet in a fixed tree (deterministic, no atomics).  So what a pass
 // can be spared is what counts: mean and variance come out of one read, and where a 2 x 2 max pooling
 // follows, the normalised tensor and its gradient are never in memory (the pooling's windows are normalised as
 // they are compared, and their gradients are looked up where they are needed).
@@ -559,7 +559,7 @@ static int batchnorm_statistics(sn_ctx* ctx, const float* x, int64_t rows, int c
   const BnScale scale = bn_scale_of(a, rows, a.fused_wiring);
   SN_REQUIRE(half <= ws_elems, "batch norm needs %lld workspace elements, %lld given", (long long)half, (long long)ws_elems);
   if (stats && stats->slices > 0) {
-    LaunchScope scope(ctx, "batchnorm_mean_and_variance");
+    LaunchScope scope(ctx, "batchnorm_mean_and_variance_from_convolution");
     hipLaunchKernelGGL(bn_moments_kernel, dim3(cb), dim3(256), 0, ctx->stream, (const float*)stats->part_mean, (const float*)stats->part_m2, stats->slices,
                        cols, stats->whole, stats->last, (float)rows, scale);
   } else if (2 * half <= ws_elems && stream_ok(cols, x, nullptr, ws, half)) {

@@ -574,7 +574,7 @@ MODELS = {
                                      "normal_regression"),
     # an odd feature count (no 8-byte loads in the forward form) and 9 units (three quads, one of them partial)
     "dense_odd_feature_count_9_units": ([("dense", 2049, "sigmoid"), ("dense", 9, "softmax")], "cce", (12,), 33, "normal_onehot"),
-    # BatchNorm reductions: 200 channels take the row-walking form with four column blocks, 256 the float4 stream form
+    # BatchNorm reductions: 200 channels (250 of a workgroup's 256 threads) and 256 take the float4 stream form, 50 the row-walking one
     "batchnorm_200_channels": ([("dense", 200, "tanh"), ("batchnorm", 0.9, 1e-3), ("dense", 5, "softmax")], "cce", (31,), 300, "normal_onehot"),
     "batchnorm_256_channels": ([("dense", 256, "relu"), ("batchnorm", 0.9, 1e-3), ("dense", 5, "softmax")], "cce", (31,), 300, "normal_onehot"),
     "batchnorm_50_channels": ([("dense", 50, "tanh"), ("batchnorm", 0.9, 1e-3), ("dense", 5, "softmax")], "cce", (31,), 300, "normal_onehot"),
@@ -688,6 +688,13 @@ KERNEL_OF_MODEL = {
     "conv_first_layer_one_long_row": "conv2d_filter_gradient_direct",
     "conv_first_layer_segments_of_32": "conv2d_filter_gradient_direct",
     "conv_pool_first_layer_long_rows": "maxpool_backward_and_conv2d_filter_gradient_direct",
+    "conv_first_layer_100_filters_64_taps": "conv2d_forward_direct",
+    "conv_first_layer_96_filters_18_taps": "conv2d_forward_direct",
+    "batchnorm_over_first_layer_100_filters": "batchnorm_mean_and_variance_from_convolution",
+    "batchnorm_over_first_layer_64_filters": "batchnorm_mean_and_variance_from_convolution",
+    "batchnorm_50_channels": "batchnorm_variance",
+    "batchnorm_200_channels": "batchnorm_mean_and_variance",
+    "batchnorm_8_channels_1_row": "batchnorm_mean_and_variance",
     "batchnorm_pool_first_layer_same_s1": "batchnorm_gradient_sums_from_maxpool",
     "batchnorm_pool_48_channels_stride_2_1": "batchnorm_gradient_sums_from_maxpool",
     "batchnorm_pool_second_layer": "batchnorm_apply_and_maxpool",
