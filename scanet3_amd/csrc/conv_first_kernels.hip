@@ -15,8 +15,8 @@
 // act'(y) multiplies.  With a batch normalisation in between (bn_inv) its input gradient is formed on the way as well.
 //
 // Measured, with what the launch takes over: 27 taps x 48 filters over 125 x 32 x 32 positions under a pooling of stride 2, 50.4 -> 14.2 us;
-// 9 x 32 over 1000 x 26 x 26 under a batch normalisation and a pooling 88 -> 36.5 us (it reads 114 MB); 9 x 32 over 100 x 26 x 26
-// under a pooling of stride 1, 11.6 -> 9.7 us.
+// 9 x 32 over 1000 x 26 x 26 under a batch normalisation and a pooling 88 -> 34.9 us (it reads 114 MB); 9 x 32 over 100 x 26 x 26
+// under a pooling of stride 1, 11.1 -> 9.3 us.
 #include "common.hpp"
 #include "conv_first_rules.hpp"
 #include "moments.hpp"
@@ -303,7 +303,7 @@ namespace {
 // time as bn_stats_v4_kernel does eight; lanes and wavefronts join theirs pairwise, and a workgroup leaves one slice of
 // partial statistics: the normalisation need not read the tensor for them.
 // Measured against the kernels this replaces (filters in LDS or registers, vector multiply-adds): 27 taps x 48 filters, 128000 positions
-// 34.4 -> 17.4 us; 9 x 32, 67600 positions 7.3 -> 6.3; 9 x 32, 676000 positions with STATS 26.8, before 22.4 and 17.1 for the statistics.
+// 34.4 -> 17.4 us; 9 x 32, 67600 positions 7.2 -> 6.7; 9 x 32, 676000 positions with STATS 28.0, before 22.4 and 17.1 for the statistics.
 struct FirstForward {
   ConvGeom g;
   const float* x;

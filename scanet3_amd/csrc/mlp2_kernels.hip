@@ -14,8 +14,7 @@
 // products is divided over eight wavefronts that meet in LDS, and the chip is filled (1000 rows are 250 workgroups).  With
 // v_mfma_f32_4x4x1_16b_f32 four rows meet 64 hidden units in one instruction of 8 cycles, its second operand one coalesced row
 // of W1; 16 rows a workgroup on v_mfma_f32_16x16x4_f32 left 63 workgroups with 196 instructions of 32 cycles one after the
-// other.  784 -> 50 -> 10 at batch 1000: 17.1 -> 9.5 us and 14.4 -> 6.5
-// (4.4 of each are what an empty launch takes).
+// other.  784 -> 50 -> 10 at batch 1000, by the profiler: 18.4 -> 10.8 us and 15.2 -> 7.2 (4.4 of each are what an empty launch takes).
 // Every sum has a fixed order, so results do not depend on the launch.
 #include "common.hpp"
 #include "optim_update.hpp"
