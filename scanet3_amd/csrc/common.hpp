@@ -483,6 +483,10 @@ int launch_split_conv_fwd(sn_ctx* ctx, const ConvGeom& g, const float* x, const 
 int launch_split_conv_dgrad(sn_ctx* ctx, const ConvGeom& g, const float* dy, const float* w, float* dx, float* ws, int64_t ws_elems);
 int launch_split_conv_wgrad(sn_ctx* ctx, const ConvGeom& g, const float* x, const float* dy, float* dw, float* ws, int64_t ws_elems);
 
+// forward and input gradient with the filter resident in LDS (conv_resident_kernels.hip; conv_resident_rules.hpp: which)
+int launch_conv_resident_fwd(sn_ctx* ctx, const ConvGeom& g, const float* x, const float* w, const Epilogue& e);
+int launch_conv_resident_dgrad(sn_ctx* ctx, const ConvGeom& g, const float* dy, const float* w, float* dx);
+
 // the same two products with LDS-direct loads into a three-stage ring (conv_ring_kernels.hip), for the shapes *_ok accepts
 bool conv_ring_fwd_ok(const ConvGeom& g, const float* x, const float* w, const Epilogue& e);
 int launch_conv_ring_fwd(sn_ctx* ctx, const ConvGeom& g, const float* x, const float* w, const Epilogue& e);

@@ -1,0 +1,69 @@
+// Which convolutions conv_resident_kernels.hip takes, and how it divides them over workgroups (host only).
+#pragma once
+#include "common.hpp"
+
+#include <algorithm>
+
+namespace sn {
+
+constexpr int RESIDENT_LDS = 160 * 1024 - 64;          // of a CU's 160 KiB (a few words are the kernel's own)
+constexpr int RESIDENT_ELEMENTS = 48;                  // of an image row that the 32 positions of a tile read
+constexpr int RESIDENT_RUN_BYTES = RESIDENT_ELEMENTS * 96;  // ... of a pair of units, as three planes
+
+// 8 bytes for every unit, and for those that are requested but not multiplied
+__host__ __device__ inline constexpr int resident_table_bytes(int pairs) { return (pairs + 4) * 16; }
+
+struct ResidentPlan {
+  int units_per_row = 0, units = 0;  // of 8 channels, of a filter row and of all
+  int pairs = 0, chunk = 0;          // pairs of units, of which LDS holds `chunk` at a time
+  int tn = 0, blocks_n = 0;          // tiles of 32 columns of a workgroup, column blocks
+  int tiles = 0, wvk = 0;            // tiles of 32 positions, wavefronts that share one
+  int per_block = 0, lds = 0;        // workgroups of a column block, bytes of LDS
+};
+inline ResidentPlan resident_plan(int64_t positions, int columns, int channels, int kh, int kw, int cu) {
+  ResidentPlan p;
+  p.units_per_row = (int)ceil_div(channels, 8);
+  p.units = kh * p.units_per_row;
+  p.pairs = (int)ceil_div(p.units, 2);
+  const int column_tiles = (int)ceil_div(columns, 32);
+  p.tn = column_tiles % 2 == 0 ? 2 : 1;
+  p.blocks_n = column_tiles / p.tn;
+  p.tiles = (int)ceil_div(positions, 32);
+  p.wvk = ceil_div(p.tiles, 4) * p.blocks_n <= cu ? 2 : 1;
+  const int fixed = resident_table_bytes(p.pairs) + 8 * RESIDENT_RUN_BYTES, step = p.tn * 3072;
+  const int most = ((RESIDENT_LDS - fixed) / step - 1) / kw;  // (a step more is read than multiplied)
+  p.chunk = (int)ceil_div(p.pairs, ceil_div(p.pairs, most));
+  const int groups = (int)ceil_div(p.tiles, 8 / p.wvk);  // as many workgroups as leave every wavefront a tile (two of them: one tile)
+  p.per_block = p.wvk == 2 ? groups : std::min(groups, std::max(1, cu / p.blocks_n));
+  p.lds = fixed + std::max((p.chunk * kw + 1) * step, p.wvk == 2 ? 4 * (p.tn * 1024 + 64) * 4 : 0);
+  return p;
+}
+
+// 32-bit byte offsets, a bit per filter row, at least one whole unit of channels, and the rows that 32 positions lie in together
+// with what the filter row reaches beyond their ends fit the elements.
+inline bool resident_tensor_ok(const float* p, int64_t elems) { return (reinterpret_cast<uintptr_t>(p) & 3u) == 0 && elems * 4 < ((int64_t)1 << 31); }
+inline bool resident_shape_ok(const ConvGeom& g, int64_t positions, int row, int columns, int channels, int cu) {
+  if (!(g.sh == 1 && g.sw == 1 && (g.kw == 3 || g.kw == 5) && g.kh <= 31 && channels >= 8 && channels <= 4096 && row >= 1 &&
+        32 + (g.kw - 1) * ((row + 30) / row + 1) <= RESIDENT_ELEMENTS))
+    return false;
+  // A workgroup spends some 5 us on taking the filter apart before the first product, so there have to be positions enough to
+  // share it, and a filter of three or more chunks is taken apart again for every eight tiles.  Microseconds, the split or ring
+  // kernels' and here, positions x columns x reduction: 12100 x 64 x 288 15.7 / 17.8, 25600 x 16 x 72 12.1 / 14.8, 25600 x 32 x 576
+  // 20.2 / 24.0, 32000 x 80 x 432 40.8 / 30.0, 39200 x 24 x 144 20.1 / 14.2, 41472 x 9 x 72 23.3 / 13.1, 52900 x 64 x 288 32.8 / 24.6,
+  // 62500 x 32 x 576 32.8 / 32.1, 121000 x 64 x 288 58 / 38, 458643 x 8 x 252 144 / 62; three chunks: 32000 x 48 x 720 45.0 / 45.8,
+  // twelve: 49000 x 64 x 1152 75 / 86; two: 49000 x 128 x 576 81 / 65.
+  const ResidentPlan p = resident_plan(positions, columns, channels, g.kh, g.kw, cu);
+  return positions >= 30000 && p.pairs <= 2 * p.chunk;
+}
+inline bool conv_resident_fwd_ok(const ConvGeom& g, const float* x, const float* w, const Epilogue& e, int cu) {
+  return e.row_index < 0 && e.ldo == g.cout && resident_tensor_ok(x, (int64_t)g.n * g.h * g.w * g.cin) &&
+         resident_tensor_ok(w, (int64_t)g.kh * g.kw * g.cin * g.cout) && resident_tensor_ok(e.out, (int64_t)g.n * g.ho * g.wo * g.cout) &&
+         resident_shape_ok(g, (int64_t)g.n * g.ho * g.wo, g.wo, g.cout, g.cin, cu);
+}
+inline bool conv_resident_dgrad_ok(const ConvGeom& g, const float* dy, const float* w, const float* dx, int cu) {
+  return resident_tensor_ok(dy, (int64_t)g.n * g.ho * g.wo * g.cout) && resident_tensor_ok(w, (int64_t)g.kh * g.kw * g.cin * g.cout) &&
+         resident_tensor_ok(dx, (int64_t)g.n * g.h * g.w * g.cin) &&
+         (g.cout % 32 != 0 || g.cin > 32 || (int64_t)g.n * g.h * g.w >= 80000) && resident_shape_ok(g, (int64_t)g.n * g.h * g.w, g.w, g.cin, g.cout, cu);
+}
+
+}  // namespace sn

@@ -6,6 +6,7 @@
 //     Block = 256 threads = 4 wavefronts in a 2x2 arrangement; block tile BM x BN (64 or 128 each), K step 16.
 //   - small-output products with a long reduction, first-layer convolutions, Dense layers onto a few units.
 #include "conv_first_rules.hpp"
+#include "conv_resident_rules.hpp"
 #include "split_launch.hpp"
 
 namespace sn {
@@ -840,6 +841,7 @@ int launch_conv_fwd(sn_ctx* ctx, const ConvGeom& g, const float* x, const float*
                     ConvStats* stats) {
   const int M = g.n * g.ho * g.wo, N = g.cout, K = g.kh * g.kw * g.cin;
   if (conv_first_fwd_ok(g, e)) return launch_conv_first_fwd(ctx, g, x, w, e, stats);
+  if (conv_resident_fwd_ok(g, x, w, e, ctx->compute_units)) return launch_conv_resident_fwd(ctx, g, x, w, e);
   if (conv_ring_fwd_ok(g, x, w, e)) return launch_conv_ring_fwd(ctx, g, x, w, e);
   StdEpilogue ep{e};
   if (!conv_prefers_float32_tiles(M, N, K, g.cin) && split_conv_fwd_ok(g, x, w)) return launch_split_conv_fwd(ctx, g, x, w, e, ws, ws_elems);
@@ -853,6 +855,7 @@ int launch_conv_dgrad(sn_ctx* ctx, const ConvGeom& g, const float* dy, const flo
   Epilogue e;
   e.out = dx;
   e.ldo = g.cin;
+  if (conv_resident_dgrad_ok(g, dy, w, dx, ctx->compute_units)) return launch_conv_resident_dgrad(ctx, g, dy, w, dx);
   if (conv_ring_dgrad_ok(g, dy, w)) return launch_conv_ring_dgrad(ctx, g, dy, w, dx);
   StdEpilogue ep{e};
   if (!(g.sh == 1 && g.sw == 1 && conv_prefers_float32_tiles(M, N, K, g.cout)) && split_conv_dgrad_ok(g, dy, w)) return launch_split_conv_dgrad(ctx, g, dy, w, dx, ws, ws_elems);

@@ -1,0 +1,54 @@
+"""Which convolutions run with their filter resident in LDS, and how they are divided (csrc/conv_resident_rules.hpp), compiled without
+device code."""
+import itertools
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+@pytest.fixture(scope="module")
+def ask(tmp_path_factory):
+    binary = str(tmp_path_factory.mktemp("host_checks") / "conv_resident_rules")
+    cmd = ["/opt/rocm/bin/hipcc", "-x", "hip", "--offload-arch=gfx950", "--offload-host-only", "-O1", "-std=c++17",
+           os.path.join(ROOT, "tests", "host_checks", "conv_resident_rules.cpp"), "-o", binary]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    assert res.returncode == 0, res.stderr
+    return lambda *q: [int(v) for v in subprocess.run([binary, *map(str, q)], capture_output=True, text=True, check=True).stdout.split()]
+
+
+def test_plans_cover_the_product_and_fit_lds(ask):
+    for positions, columns, channels, kh, kw in itertools.product((30000, 32768, 32801, 529000), (1, 32, 33, 65, 130, 400), (8, 9, 64, 100, 512), (1, 3, 7), (3, 5)):
+        per_row, units, pairs, chunk, tn, blocks_n, tiles, wvk, per_block, lds = ask("plan", positions, columns, channels, kh, kw)
+        assert 8 * per_row >= channels > 8 * (per_row - 1) and units == kh * per_row and 2 * pairs >= units > 2 * (pairs - 1)
+        assert 1 <= chunk <= pairs and tn in (1, 2) and 32 * tn * blocks_n >= columns > 32 * tn * blocks_n - 64
+        assert 32 * tiles >= positions > 32 * (tiles - 1)
+        # table, runs, and a step more of the filter than is multiplied; two wavefronts on a tile hand their sums over where it lay
+        assert (pairs + 4) * 16 + 8 * 48 * 96 + max((chunk * kw + 1) * tn * 3072, 4 * (tn * 1024 + 64) * 4 * (wvk - 1)) <= lds <= 160 * 1024 - 64
+        if wvk == 2:  # one tile for every pair of wavefronts, one round of workgroups
+            assert 4 * per_block >= tiles > 4 * (per_block - 1) and per_block * blocks_n <= 256
+        else:
+            assert 8 * (per_block - 1) < tiles and (per_block == 1 or per_block * blocks_n <= 256)
+
+
+def test_elements_of_a_tile(ask):
+    """32 positions from any place of rows of any length: the rows they touch, with kw - 1 more elements each, fit 48 where the kernel is taken."""
+    for row, kw in itertools.product(range(1, 70), (3, 5)):
+        touched = max((start + 31) // row + 1 for start in range(row))
+        taken = ask("takes", 30000, 3, row, 8, 8, 3, kw, 1)
+        assert taken == [int(32 + (kw - 1) * touched <= 48)] * 2, (row, kw)
+
+
+def test_which_convolutions(ask):
+    for want, *shape in (([1, 0], 100, 25, 25, 32, 64, 3, 3, 0),     # an input gradient onto 32 channels of 62500 positions stays with the ring
+                         ([1, 1], 1000, 13, 13, 32, 64, 3, 3, 0),
+                         ([0, 0], 100, 13, 13, 32, 64, 3, 3, 0),     # too few positions
+                         ([1, 0], 125, 16, 16, 48, 80, 3, 3, 1),     # 80 -> 48 channels: three chunks
+                         ([0, 0], 1000, 13, 13, 4, 7, 3, 3, 0),      # less than a unit of channels
+                         ([0, 0], 1000, 13, 13, 32, 64, 3, 4, 0),
+                         ([0, 0], 1000, 13, 13, 32, 64, 32, 3, 1),
+                         ([0, 1], 60, 24, 24, 7, 50, 3, 3, 1),
+                         ([0, 0], 30000, 60, 60, 8, 8, 3, 3, 1)):    # a tensor beyond 2 GiB
+        assert ask("takes", *shape) == want, shape

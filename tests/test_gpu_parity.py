@@ -2768,3 +2768,76 @@ def test_every_split_tile(S, ctx, tile):
     assert np.all(np.abs(h.rep.forward(xb) - want) <= (6.0 / 16.0 * features + 16.0) * 2.0 ** -24 * size)
     h.close()
     xb.free()
+
+
+# (batch, height, width, channels, filters, kernel, padding): convolutions whose filter is resident in LDS (30000 positions and more), at
+# the edges of their tiles: 5, 0 and 1 channels in the last unit of 8, 1 and 31 columns in the last tile of 32 and one or two tiles a
+# workgroup, 16 and 4 positions in the last tile, two wavefronts a tile, one unit, units without a partner, rows of 5 positions, runs over several
+# images, a filter in two chunks, both kernel widths, a kernel of one row and one of two, uneven padding
+RESIDENT_CONVOLUTIONS = [
+    (100, 18, 18, 13, 33, (3, 3), "same"), (161, 16, 16, 8, 31, (3, 3), "valid"), (61, 23, 23, 16, 64, (5, 5), "same"), (300, 10, 11, 24, 65, (3, 3), "same"),
+    (1000, 7, 5, 9, 8, (1, 3), "same"), (40, 28, 28, 64, 40, (3, 3), "same"), (70, 22, 22, 40, 32, (2, 3), "valid"), (90, 19, 20, 17, 20, (3, 3), (2, 0, 1, 2))]
+
+
+@pytest.mark.parametrize("batch,height,width,channels,filters,kernel,pad", RESIDENT_CONVOLUTIONS)
+def test_convolutions_with_a_resident_filter(S, ctx, batch, height, width, channels, filters, kernel, pad):
+    """Forward, input gradient (behind the first layer's filter gradient) and filter gradient against float64.  One image is of values
+    that are no sums of three bf16 parts."""
+    rng = np.random.default_rng(channels + filters)
+    spec = [("conv", channels, (1, 1), (1, 1), "valid", "identity", False), ("conv", filters, kernel, (1, 1), pad, "identity", False), ("flatten",)]
+    h = Harness(S, ctx, spec, "mse", (height, width, 1), batch)
+    names = [p for p, _, _ in h.cm.params]
+    shapes = {p: s for p, s, _ in h.cm.params}
+    x, w = rng.standard_normal((batch, height, width, 1)).astype(f32), [rng.standard_normal(shapes[n]).astype(f32) for n in names]
+    x[1] = _small(rng, x[1].shape, -128)
+    geometry = {"padding": {"same": O.PAD_SAME, "valid": O.PAD_VALID}.get(pad, O.PAD_EXPLICIT)}
+    if isinstance(pad, tuple):
+        geometry["explicit"] = pad
+    y = rng.standard_normal((batch, h.cm.out_elems)).astype(f32)
+    h.rep.set_params(dict(zip(names, w)))
+    xb, yb = ctx.to_device(x), ctx.to_device(y)
+
+    def run(x, y, w1, w2, sign):
+        a = O.conv2d(x, w1)
+        p = O.conv2d(a, w2, **geometry)
+        dp = 2.0 * (p + sign * y.reshape(p.shape)) / y.size
+        da = O.conv2d_grad_input(a.shape, w2, dp, **geometry)
+        return {"out": p.reshape(y.shape), names[1]: O.conv2d_grad_filter(a, w2.shape, dp, **geometry), names[0]: O.conv2d_grad_filter(x, w1.shape, da)}
+    d = [v.astype(np.float64) for v in (x, y, *w)]
+    want, size = run(*d, -1.0), run(*[np.abs(v) for v in d], 1.0)
+    got = {"out": h.rep.forward(xb)}
+    h.rep.grad(xb, yb)
+    got.update(h.rep.get_grads())
+    # float32 sums of K products round at most K times; the positions' sums are split over at least 32 workgroups
+    taps = kernel[0] * kernel[1]
+    steps = {"out": taps * channels + 16, names[1]: taps * (channels + filters) + got["out"].size / filters / 32 + 64}
+    steps[names[0]] = steps[names[1]]
+    for name in got:
+        bound = steps[name] * 2.0 ** -24 * size[name] + 2.0 ** -149 * (taps * channels + 1) * max(1.0, float(np.abs(w[1]).max()))
+        assert np.all(np.abs(got[name].reshape(want[name].shape) - want[name]) <= bound), name
+    h.close()
+    xb.free()
+    yb.free()
+
+
+@pytest.mark.parametrize("value", [3.4e38, 1e30, np.inf])
+def test_convolutions_with_a_resident_filter_at_the_end_of_the_range(S, ctx, value):
+    """A pixel of the largest values: its outputs are what float64 gives, taken to float32's range; nothing else changes."""
+    rng = np.random.default_rng(5)
+    shape, batch = (18, 18, 11), 100
+    spec = [("conv", 9, (1, 1), (1, 1), "valid", "identity", False), ("conv", 34, (3, 3), (1, 1), "same", "identity", False), ("flatten",)]
+    h = Harness(S, ctx, spec, "mse", shape, batch)
+    x = rng.uniform(0.5, 1.0, (batch,) + shape).astype(f32)
+    params = glorot_params(h.omodel, (batch,) + shape, rng)
+    for p in params:  # positive weights: no Inf - Inf
+        params[p] = np.abs(params[p]) + f32(0.05)
+    if value == 1e30:
+        params[[p for p in params if params[p].ndim == 4][1]][1, 2, 3, 4] = f32(1e10)  # two operands far from the end of the range
+    x[1, 2, 3, 0] = value
+    h.rep.set_params(params)
+    xb = ctx.to_device(x)
+    want = _as_float32_would(h.omodel.forward(np.where(np.isfinite(x), x, 1e300).astype(np.float64), {k: v.astype(np.float64) for k, v in params.items()}))
+    _assert_same_range(h.rep.forward(xb).reshape(want.shape), want, 1e-5)
+    assert np.isinf(want).any() or value == 3.4e38
+    h.close()
+    xb.free()
