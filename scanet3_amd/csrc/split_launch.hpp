@@ -136,16 +136,20 @@ static int launch_split_reduce(sn_ctx* ctx, const float* ws, int splits, int M, 
 // Tile and split count for a product of M x N x K: the cheapest by a model of what a launch costs.  Per tile shape: the time
 // per 32 k-values of a workgroup that has its CU to itself (a chain of load, split, store, read, multiply), and of a CU that
 // is full of workgroups, per workgroup (measured on MI355X: 288 x 64 x 52900 in one split, 8192 x 4096 x 4096; the bf16
-// column is one plane instead of three).  A launch lasts as long as its fullest CU; splitting K costs the partial sums' way
-// through memory and the launch that adds them.
+// column is one plane instead of three, by 1000 x 1500 x 1000, 1000 x 600 x 1500, 700 x 330 x 770 and 2124 x 2820 x 220).  A launch
+// lasts as long as its fullest CU; splitting K costs the partial sums' way through memory and the launch that adds them.
+// One plane has nothing to take apart; where a CU holds several workgroups, what it can fetch bounds them, and larger tiles fetch
+// less: 1000 x 1500 x 1000 25.3 us in tiles of 64 x 32 and 22.8 in 64 x 64, 2124 x 2820 x 220 31.1 in 128 x 64 and 19.4 in 128 x 128.
+// (Three stages of loads in flight instead of one, with every wait counting on the loads behind it, were measured over all tiles: 20 to
+// 60 % slower where a CU holds several workgroups, whose registers they take, and within 5 % of the same where it holds one.)
 struct SplitTile {
   int bm, bn, bk;
   float lone[2], full[2];  // microseconds; [0] three planes (float32), [1] one plane (bf16)
 };
 enum { TILE_128x128, TILE_128x64, TILE_64x64, TILE_64x64_DEEP, TILE_64x32_DEEP, TILE_32x64_DEEP, SPLIT_TILES };
 constexpr SplitTile SPLIT_TILE[SPLIT_TILES] = {
-    {128, 128, 32, {1.45f, 0.75f}, {1.45f, 0.55f}}, {128, 64, 32, {1.14f, 0.70f}, {0.85f, 0.36f}}, {64, 64, 32, {0.83f, 0.56f}, {0.47f, 0.22f}},
-    {64, 64, 64, {0.60f, 0.37f}, {0.52f, 0.27f}},   {64, 32, 64, {0.44f, 0.31f}, {0.31f, 0.17f}},  {32, 64, 64, {0.46f, 0.29f}, {0.34f, 0.21f}}};
+    {128, 128, 32, {1.45f, 0.75f}, {1.45f, 0.72f}}, {128, 64, 32, {1.14f, 1.00f}, {0.85f, 1.00f}}, {64, 64, 32, {0.83f, 0.56f}, {0.47f, 0.39f}},
+    {64, 64, 64, {0.60f, 0.42f}, {0.52f, 0.27f}},   {64, 32, 64, {0.44f, 0.31f}, {0.31f, 0.205f}}, {32, 64, 64, {0.46f, 0.29f}, {0.34f, 0.23f}}};
 struct SplitChoice {
   int tile = 0, splits = 1;
 };
