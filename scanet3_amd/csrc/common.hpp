@@ -453,6 +453,9 @@ int launch_conv_first_wgrad(sn_ctx* ctx, const ConvGeom& g, const float* x, cons
 int launch_conv_wgrad(sn_ctx* ctx, const ConvGeom& g, const float* x, const float* dy, float* dw, float* ws, int64_t ws_elems,
                       const PoolGrad* pool = nullptr);
 
+// Filter gradient with both operands straight from the tensors (conv_wgrad_split_kernels.hip; conv_wgrad_split_rules.hpp: which)
+int launch_conv_wgrad_split(sn_ctx* ctx, const ConvGeom& g, const float* x, const float* dy, float* dw, float* ws, int64_t ws_elems);
+
 // What the split convolutions can read: vectors of four values, clamped to the inside of an image tensor of n * h * w * c
 // values (so it has to hold four of them), and 32-bit byte offsets up to one image behind its end.
 constexpr int64_t SPLIT_SPAN = (int64_t)1 << 31;

@@ -1,0 +1,54 @@
+// Which filter gradients conv_wgrad_split_kernels.hip takes, and how it divides them over workgroups (host only).
+#pragma once
+#include "common.hpp"
+
+#include <algorithm>
+
+namespace sn {
+
+struct WgradSplitPlan {
+  int tm = 0, tn = 0;              // tiles of 32 values of a run, of 32 filters, that a wavefront keeps
+  int groups_m = 0, groups_n = 0;  // workgroups that a filter row's result is divided over
+  int chunks = 0, parts = 0;       // of 16 positions; ranges of them
+  float cost = 0.f;
+  bool padded = false;
+};
+// Up to six tiles a wavefront (96 of its 256 registers).  Which division: what a workgroup's time comes to in cycles, its two
+// wavefronts on a SIMD in turn - a chunk's 6 products a tile of 32 cycles, or taking tm + tn tiles apart where that is more - and 1000
+// for each tile that the wavefronts add and write at the end.
+inline WgradSplitPlan conv_wgrad_split_plan(const ConvGeom& g, int cu, int64_t ws_elems) {
+  WgradSplitPlan p;
+  const int L = g.kw * g.cin, tiles_m = (int)ceil_div(L, 32), tiles_n = (int)ceil_div(g.cout, 32);
+  p.chunks = (int)ceil_div((int64_t)g.n * g.ho * g.wo, 16);
+  const int64_t room = ws_elems / ((int64_t)g.kh * L * g.cout);
+  p.padded = g.pt != 0 || g.pl != 0 || (g.ho - 1) * g.sh + g.kh > g.h || (g.wo - 1) * g.sw + g.kw > g.w;
+  p.cost = 1e30f;
+  for (int tm = 1; tm <= 3; ++tm)
+    for (int tn = 1; tn <= 3; ++tn) {
+      if (tm * tn > (tn == 3 ? 3 : 6)) continue;  // (2 x 3 holds three tiles of dy taken apart twice over and spills: at 28224 x 65 x 108 23 us for 19)
+      const int gm = (int)ceil_div(tiles_m, tm), gn = (int)ceil_div(tiles_n, tn), groups = g.kh * gm * gn;
+      const int parts = (int)std::min<int64_t>({(int64_t)std::max(1, cu / groups), (int64_t)p.chunks, room});
+      if (parts < 1) continue;
+      const float rounds = (float)ceil_div(groups * parts, cu), share = (float)ceil_div(p.chunks, 8 * parts);
+      const float cost = rounds * (share * 2.f * std::max(192.f * (float)(tm * tn), 330.f * (float)(tm + tn)) + 1000.f * (float)(tm * tn));
+      if (cost < p.cost) {
+        p.cost = cost;
+        p.tm = tm; p.tn = tn; p.groups_m = gm; p.groups_n = gn; p.parts = parts;
+      }
+    }
+  return p;
+}
+inline int64_t conv_wgrad_split_workspace(const ConvGeom& g, int cu) {
+  const int64_t size = (int64_t)g.kh * g.kw * g.cin * g.cout;
+  return conv_wgrad_split_plan(g, cu, size * cu).parts * size;
+}
+// 32-bit byte offsets (a tile's values behind a run included), a bit for every row and column of the filter, a run that fills a good part of a tile.  From 4096 positions:
+// at 3136 x 128 x 576 both ways take 15.3 us, at 5760 x 8 x 144 this one 7.9 for 9.8, and below that nothing is left to gain.
+inline bool conv_wgrad_split_ok(const ConvGeom& g, const float* x, const float* dy) {
+  const int64_t positions = (int64_t)g.n * g.ho * g.wo;
+  const auto fits = [](const float* p, int64_t elems) { return (reinterpret_cast<uintptr_t>(p) & 3u) == 0 && elems * 4 < ((int64_t)1 << 31) - 4096; };
+  return g.cin >= 8 && g.cin <= 4096 && g.kh <= 15 && g.kw <= 15 && fits(x, (int64_t)g.n * g.h * g.w * g.cin) && fits(dy, positions * g.cout) &&
+         positions >= 4096;
+}
+
+}  // namespace sn

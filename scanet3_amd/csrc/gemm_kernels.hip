@@ -7,6 +7,7 @@
 //   - small-output products with a long reduction, first-layer convolutions, Dense layers onto a few units.
 #include "conv_first_rules.hpp"
 #include "conv_resident_rules.hpp"
+#include "conv_wgrad_split_rules.hpp"
 #include "split_launch.hpp"
 
 namespace sn {
@@ -891,7 +892,12 @@ int launch_conv_wgrad(sn_ctx* ctx, const ConvGeom& g, const float* x, const floa
     return SN_OK;
   }
   SN_REQUIRE(pool == nullptr, "conv2d_filter_gradient: only the direct kernel takes a pooling's gradient (ask conv_wgrad_is_direct first)");
-  if (ws && aligned16(ws) && conv_wgrad_taps_shape(ctx, g, x, dy) && conv_wgrad_taps_workspace(ctx, g) <= ws_elems) {
+  // A tile per filter tap, for 32 channels onto 32 or 64 filters: level with the split products at 20160 and 24480 x 64 x 288 (18.2 and
+  // 19.0 us), behind them at 28800 (21.1 and 19.2) and 52900 (29.5 and 25.1).
+  const bool taps = ws && aligned16(ws) && conv_wgrad_taps_shape(ctx, g, x, dy) && conv_wgrad_taps_workspace(ctx, g) <= ws_elems;
+  if (ws && (K >= 24576 || !taps) && conv_wgrad_split_ok(g, x, dy) && conv_wgrad_split_plan(g, ctx->compute_units, ws_elems).parts >= 1)
+    return launch_conv_wgrad_split(ctx, g, x, dy, dw, ws, ws_elems);
+  if (taps) {
     // a tile per filter tap: a few dozen partial filters instead of the 64 x 64 tiling's hundreds
     int parts = 0;
     SN_TRY(launch_conv_wgrad_taps(ctx, g, x, dy, ws, ws_elems, &parts));

@@ -1,0 +1,46 @@
+"""Which filter gradients run on split products straight from the tensors, and how they are divided (csrc/conv_wgrad_split_rules.hpp),
+compiled without device code."""
+import itertools
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+@pytest.fixture(scope="module")
+def ask(tmp_path_factory):
+    binary = str(tmp_path_factory.mktemp("host_checks") / "conv_wgrad_split_rules")
+    cmd = ["/opt/rocm/bin/hipcc", "-x", "hip", "--offload-arch=gfx950", "--offload-host-only", "-O1", "-std=c++17",
+           os.path.join(ROOT, "tests", "host_checks", "conv_wgrad_split_rules.cpp"), "-o", binary]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    assert res.returncode == 0, res.stderr
+    return lambda *q: [int(v) for v in subprocess.run([binary, *map(str, q)], capture_output=True, text=True, check=True).stdout.split()]
+
+
+def test_plans_cover_the_product_and_fit_the_workspace(ask):
+    for n, cin, cout, kernel, same in itertools.product((30, 311), (8, 33, 96, 512), (1, 33, 64, 300), ((1, 1), (3, 3), (15, 15)), (0, 1)):
+        shape = (n, 16, 17, cin, cout, *kernel, 1, same)
+        size, length = kernel[0] * kernel[1] * cin * cout, kernel[1] * cin
+        for room in (-1, size, 3 * size):
+            taken, tm, tn, groups_m, groups_n, chunks, parts, padded, workspace = ask(*shape, room)
+            assert (tm, tn) in ((1, 1), (1, 2), (1, 3), (2, 1), (2, 2), (3, 1), (3, 2))
+            assert 32 * tm * groups_m >= length > 32 * tm * (groups_m - 1) and 32 * tn * groups_n >= cout > 32 * tn * (groups_n - 1)
+            assert padded == int(same and kernel != (1, 1))
+            positions = n * (16 * 17 if same else (17 - kernel[0]) * (18 - kernel[1]))
+            assert 16 * chunks >= positions > 16 * (chunks - 1) and 1 <= parts <= chunks and taken == int(positions >= 4096)
+            groups = kernel[0] * groups_m * groups_n
+            assert parts * size <= (workspace if room < 0 else room) and (parts == 1 or groups * parts <= 256)
+        assert ask(*shape, size - 1)[6] == 0  # no room for one partial result: left to the general path
+
+
+def test_which_filter_gradients(ask):
+    for want, *shape in ((1, 100, 25, 25, 32, 64, 3, 3, 1, 0),
+                         (0, 100, 25, 25, 7, 64, 3, 3, 1, 0),       # a run that leaves most of a tile empty
+                         (0, 100, 25, 25, 32, 64, 16, 3, 1, 1),     # a row of the filter for every bit
+                         (1, 100, 25, 25, 32, 64, 15, 15, 1, 1),
+                         (0, 16, 16, 15, 32, 64, 3, 3, 1, 1),       # 3840 positions
+                         (1, 16, 16, 16, 32, 64, 3, 3, 1, 1),
+                         (0, 30000, 60, 60, 8, 8, 3, 3, 1, 1)):     # a tensor beyond 2 GiB
+        assert ask(*shape, -1)[0] == want, shape

@@ -2841,3 +2841,54 @@ def test_convolutions_with_a_resident_filter_at_the_end_of_the_range(S, ctx, val
     assert np.isinf(want).any() or value == 3.4e38
     h.close()
     xb.free()
+
+
+# Every division into tiles, with and without padding: remainders of 16 positions, of 32 values of a run and of 32 filters, a stride
+# down the image, a run that ends in the image's last bytes, and one range of more than the 512 chunks whose table LDS holds.
+SPLIT_FILTER_GRADIENTS = [
+    (64, 9, 9, 8, 31, (1, 1), (1, 1), "valid", 1.0), (37, 13, 11, 9, 40, (3, 3), (1, 1), "same", 1.0), (33, 14, 13, 24, 65, (2, 1), (1, 1), "valid", 1.0),
+    (60, 12, 11, 17, 33, (3, 3), (1, 1), "same", 3.4e38), (130, 14, 9, 21, 96, (3, 3), (2, 1), "same", 1.0), (250, 16, 14, 31, 64, (3, 3), (1, 1), "valid", 3.4e38),
+    (500, 13, 13, 15, 20, (5, 5), (1, 1), (2, 1, 0, 3), 1.0), (300, 16, 15, 32, 64, (3, 3), (1, 1), "valid", 1.0), (150, 8, 8, 64, 300, (15, 2), (1, 1), "same", 1.0)]
+
+
+@pytest.mark.parametrize("batch,height,width,channels,filters,kernel,strides,pad,value", SPLIT_FILTER_GRADIENTS)
+def test_filter_gradients_on_split_products(S, ctx, batch, height, width, channels, filters, kernel, strides, pad, value):
+    """Against float64.  One image holds values that are no sums of three bf16 parts, another one of `value` (3.4e38: its first part is Inf)."""
+    rng = np.random.default_rng(channels + filters)
+    spec = [("conv", channels, (1, 1), (1, 1), "valid", "identity", False), ("conv", filters, kernel, strides, pad, "identity", False), ("flatten",)]
+    h = Harness(S, ctx, spec, "mse", (height, width, 1), batch)
+    names = [p for p, _, _ in h.cm.params]
+    shapes = {p: s for p, s, _ in h.cm.params}
+    x, w = rng.standard_normal((batch, height, width, 1)).astype(f32), [np.ones(shapes[names[0]], f32), rng.standard_normal(shapes[names[1]]).astype(f32)]
+    x[1] = _small(rng, x[1].shape, -128)
+    x[2, height // 2, width // 2, 0] = value
+    w[1] *= f32(1.0 / value)
+    geometry = {"strides": strides, "padding": {"same": O.PAD_SAME, "valid": O.PAD_VALID}.get(pad, O.PAD_EXPLICIT)}
+    if isinstance(pad, tuple):
+        geometry["explicit"] = pad
+    y = rng.standard_normal((batch, h.cm.out_elems)).astype(f32)
+    h.rep.set_params(dict(zip(names, w)))
+    xb, yb = ctx.to_device(x), ctx.to_device(y)
+
+    def run(x, y, w1, w2, sign):
+        a = O.conv2d(x, w1)
+        p = O.conv2d(a, w2, **geometry)
+        return O.conv2d_grad_filter(a, w2.shape, 2.0 * (p + sign * y.reshape(p.shape)) / y.size, **geometry)
+    d = [v.astype(np.float64) for v in (x, y, *w)]
+    want, size = run(*d, -1.0), run(*[np.abs(v) for v in d], 1.0)
+    ctx.profile_reset()
+    ctx.profile(True)
+    h.rep.grad(xb, yb)
+    ctx.sync()
+    ctx.profile(False)
+    assert any(l.startswith("conv2d_filter_gradient_split") for l in ctx.profile_report())
+    got = h.rep.get_grads()[names[1]].reshape(want.shape)
+    # the forward sums round at most taps * channels times; the positions' at most once for two of them over 8 wavefronts, and with
+    # them the sums of the wavefronts and of at most 256 partial results
+    positions = y.size // filters
+    steps = kernel[0] * kernel[1] * channels + positions / 16 + 256 + 64
+    bound = steps * 2.0 ** -24 * size + 2.0 ** -149 * positions
+    assert np.all(np.abs(got - want) <= bound)
+    h.close()
+    xb.free()
+    yb.free()
