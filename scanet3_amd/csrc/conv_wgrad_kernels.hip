@@ -1,7 +1,8 @@
 // Conv2D filter gradient for 32 input channels as fp32 matrix-core tiles per filter tap (gfx950).
 //
 //   dW[r, q, ci, co] = sum over (b, oh, ow) of x[b, oh*sh + r, ow*sw + q, ci] * dy[b, oh, ow, co]
-//   (math/nn/AllKernels.scala:211-261: the filter's side of Conv2D's gradient), no padding.
+//   (math/nn/AllKernels.scala:211-261: the filter's side of Conv2D's gradient), no padding.  From 24576 positions on the
+//   split products of conv_wgrad_split_kernels.hip take its place.
 //
 // As a GEMM the product is [kh*kw*32] x [cout] over tens of thousands of positions: the output is tiny, so filling the
 // chip means many partial results.  Tiled 64 x 64 with a split of the positions, 256 partial filters leave and come back

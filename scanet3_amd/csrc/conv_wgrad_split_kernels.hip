@@ -2,6 +2,7 @@
 // operands loaded straight from the tensors: nothing is staged and no barrier stands in the loop.
 //
 //   dW[r, j, n] = sum over output positions p of x[run of p in filter row r][j] * dy[p][n],   j = q * cin + channel < L = kw * cin
+//   (math/nn/AllKernels.scala:211-261: the filter's side of Conv2D's gradient)
 //
 // For a fixed filter row the taps' channels of a position are one run of L consecutive floats of x, so a tile of 32 values of j x 32
 // filters is one accumulator of v_mfma_f32_32x32x16_bf16: lane l supplies value j = l % 32 (filter n = l % 32) of 8 positions,
