@@ -32,6 +32,7 @@ inline ResidentPlan resident_plan(int64_t positions, int columns, int channels, 
   p.wvk = ceil_div(p.tiles, 4) * p.blocks_n <= cu ? 2 : 1;
   const int fixed = resident_table_bytes(p.pairs) + 8 * RESIDENT_RUN_BYTES, step = p.tn * 3072;
   const int most = ((RESIDENT_LDS - fixed) / step - 1) / kw;  // (a step more is read than multiplied)
+  if (most < 1) return ResidentPlan{};  // the table and the runs leave no room for one pair of units: nothing to divide
   p.chunk = (int)ceil_div(p.pairs, ceil_div(p.pairs, most));
   const int groups = (int)ceil_div(p.tiles, 8 / p.wvk);  // as many workgroups as leave every wavefront a tile (two of them: one tile)
   p.per_block = p.wvk == 2 ? groups : std::min(groups, std::max(1, cu / p.blocks_n));
@@ -43,7 +44,7 @@ inline ResidentPlan resident_plan(int64_t positions, int columns, int channels, 
 // with what the filter row reaches beyond their ends fit the elements.
 inline bool resident_tensor_ok(const float* p, int64_t elems) { return (reinterpret_cast<uintptr_t>(p) & 3u) == 0 && elems * 4 < ((int64_t)1 << 31); }
 inline bool resident_shape_ok(const ConvGeom& g, int64_t positions, int row, int columns, int channels, int cu) {
-  if (!(g.sh == 1 && g.sw == 1 && (g.kw == 3 || g.kw == 5) && g.kh <= 31 && channels >= 8 && channels <= 4096 && row >= 1 &&
+  if (!(positions >= 30000 && g.sh == 1 && g.sw == 1 && (g.kw == 3 || g.kw == 5) && g.kh <= 31 && channels >= 8 && channels <= 4096 && row >= 1 &&
         32 + (g.kw - 1) * ((row + 30) / row + 1) <= RESIDENT_ELEMENTS))
     return false;
   // A workgroup spends some 5 us on taking the filter apart before the first product, so there have to be positions enough to
@@ -53,7 +54,7 @@ inline bool resident_shape_ok(const ConvGeom& g, int64_t positions, int row, int
   // 62500 x 32 x 576 32.8 / 32.1, 121000 x 64 x 288 58 / 38, 458643 x 8 x 252 144 / 62; three chunks: 32000 x 48 x 720 45.0 / 45.8,
   // twelve: 49000 x 64 x 1152 75 / 86; two: 49000 x 128 x 576 81 / 65.
   const ResidentPlan p = resident_plan(positions, columns, channels, g.kh, g.kw, cu);
-  return positions >= 30000 && p.pairs <= 2 * p.chunk;
+  return p.chunk >= 1 && p.pairs <= 2 * p.chunk;
 }
 inline bool conv_resident_fwd_ok(const ConvGeom& g, const float* x, const float* w, const Epilogue& e, int cu) {
   return e.row_index < 0 && e.ldo == g.cout && resident_tensor_ok(x, (int64_t)g.n * g.h * g.w * g.cin) &&

@@ -41,6 +41,27 @@ def test_elements_of_a_tile(ask):
         assert taken == [int(32 + (kw - 1) * touched <= 48)] * 2, (row, kw)
 
 
+def test_filters_beyond_lds(ask):
+    """Filters whose table of units nearly fills LDS by itself are declined in both directions, at any number of positions; the largest
+    that leave room for one pair of units have a plan."""
+    for columns, channels, kh, kw in ((64, 4096, 22, 5), (33, 4096, 23, 5), (65, 4096, 31, 3), (64, 4096, 25, 5), (32, 2904, 31, 5), (64, 4096, 31, 5)):
+        for batch in (1, 16):
+            for same in (0, 1):
+                assert ask("takes", batch, 45, 45, channels, columns, kh, kw, same) == [0, 0]
+                assert ask("takes", batch, 45, 45, columns, channels, kh, kw, same)[1] == 0
+    for columns, kw in itertools.product((32, 64), (3, 5)):
+        step, chunks = (columns // 32) * 3072, {}
+        for pairs in range(5000, 8200):
+            room = 160 * 1024 - 64 - (pairs + 4) * 16 - 8 * 48 * 96
+            if room // step - 1 >= kw:
+                chunks["last"] = pairs
+            else:
+                chunks.setdefault("none", pairs)
+        for pairs, planned in ((chunks["last"], True), (chunks["none"], False)):
+            plan = ask("plan", 529000, columns, 16 * pairs, 1, kw)
+            assert (plan[3] >= 1) == planned and (not planned or plan[2] == pairs and plan[9] <= 160 * 1024 - 64)
+
+
 def test_which_convolutions(ask):
     for want, *shape in (([1, 0], 100, 25, 25, 32, 64, 3, 3, 0),     # an input gradient onto 32 channels of 62500 positions stays with the ring
                          ([1, 1], 1000, 13, 13, 32, 64, 3, 3, 0),
