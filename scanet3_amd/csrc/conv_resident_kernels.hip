@@ -24,7 +24,9 @@
 // a tile's time at the clock that their power leaves (1.75 GHz), the rest is the issue of some 50 other instructions a step, 12
 // of them LDS reads; taking every tap's values apart anew, straight from memory, it was 131, with the loads left to the compiler's
 // order 170.  52900 x 64 x 288: 24.6 us (32.8), of which 5 are the filter's way into LDS.  121000 x 64 x 288 38 (58), 169000 x 32 x
-// 576 59 (73), 409948 x 15 x 522 171 (327), 458643 x 8 x 252 62 (144).
+// 576 59 (73), 409948 x 15 x 522 171 (327), 458643 x 8 x 252 62 (144).  An input gradient reads the filter's channels as vectors of four:
+// value by value, every lane in a cache line of its own, taking the filter apart was as long as the products where it is walked in
+// two chunks (204800 x 64 x 576 175 us, 120 now; 137 to 157 by conv_ring_kernels.hip.  102400 x 64 x 360 69, 47; 63 by split_conv.hip).
 #include "split_launch.hpp"
 
 #include "conv_resident_rules.hpp"
@@ -47,6 +49,7 @@ struct ResidentArgs {
   int H, W, C;             // source image
   int kh;
   const float* w;
+  uint32_t w_bytes;
   int w_tap, w_c, w_n;     // element (tap, channel, n) of the filter at tap * w_tap + channel * w_c + n * w_n
   int N;
   int units_per_row, units, pairs, chunk;  // pairs of units; of which LDS holds `chunk` at a time
@@ -85,7 +88,7 @@ __global__ __launch_bounds__(512) void conv_resident_kernel(ResidentArgs a) {
 
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, lhi = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wk = wave % WVK, wtile = wave / WVK;
-  const __amdgpu_buffer_rsrc_t rs = make_rsrc(a.src, a.src_bytes);
+  const __amdgpu_buffer_rsrc_t rs = make_rsrc(a.src, a.src_bytes), rw = make_rsrc(a.w, a.w_bytes);
 
   if (tid == 0) filter_top = filter_lossy = 0;
   // K runs through the units from the last to the first.  (Either order is as close to float64.  The 100-step LeNet run of the tests is
@@ -122,9 +125,18 @@ __global__ __launch_bounds__(512) void conv_resident_kernel(ResidentArgs a) {
         const int tap = r * KW + (a.reversed ? KW - 1 - q : q), c = min(8 * c8, a.C - 8);
         const bool in = u < a.units;
         skip[e] = in && n < a.N ? 8 * c8 - c : 8;  // channels that the unit before has
-        const float* from = a.w + (in ? tap * a.w_tap + c * a.w_c : 0) + min(n, a.N - 1) * a.w_n;
+        const int from = (in ? tap * a.w_tap + c * a.w_c : 0) + min(n, a.N - 1) * a.w_n;
+        if (a.w_c == 1) {  // (an input gradient: a column's channels lie side by side, the columns themselves a row of filters apart)
+          const f4v first = load16(rw, (uint32_t)from * 4u), second = load16(rw, (uint32_t)from * 4u + 16u);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v[e][j] = from[j * a.w_c];
+          for (int j = 0; j < 4; ++j) {
+            v[e][j] = first[j];
+            v[e][4 + j] = second[j];
+          }
+        } else {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) v[e][j] = a.w[from + j * a.w_c];
+        }
       }
 #pragma unroll
       for (int e = 0; e < AHEAD; ++e) {
@@ -522,7 +534,7 @@ int launch_conv_resident_fwd(sn_ctx* ctx, const ConvGeom& g, const float* x, con
   a.M = g.n * g.ho * g.wo; a.ih = g.ho; a.iw = g.wo;
   a.oy = -g.pt; a.ty = 1; a.ox = -g.pl;
   a.H = g.h; a.W = g.w; a.C = g.cin; a.kh = g.kh;
-  a.w = w; a.w_tap = g.cin * g.cout; a.w_c = g.cout; a.w_n = 1;
+  a.w = w; a.w_bytes = (uint32_t)((int64_t)g.kh * g.kw * g.cin * g.cout * 4); a.w_tap = g.cin * g.cout; a.w_c = g.cout; a.w_n = 1;
   a.N = g.cout;
   a.ep = e;
   return g.kw == 3 ? launch_planned<3>(ctx, "conv2d_forward", a) : launch_planned<5>(ctx, "conv2d_forward", a);
@@ -535,7 +547,7 @@ int launch_conv_resident_dgrad(sn_ctx* ctx, const ConvGeom& g, const float* dy, 
   a.M = g.n * g.h * g.w; a.ih = g.h; a.iw = g.w;
   a.oy = g.pt; a.ty = -1; a.ox = g.pl - (g.kw - 1); a.reversed = 1;
   a.H = g.ho; a.W = g.wo; a.C = g.cout; a.kh = g.kh;
-  a.w = w; a.w_tap = g.cin * g.cout; a.w_c = 1; a.w_n = g.cout;
+  a.w = w; a.w_bytes = (uint32_t)((int64_t)g.kh * g.kw * g.cin * g.cout * 4); a.w_tap = g.cin * g.cout; a.w_c = 1; a.w_n = g.cout;
   a.N = g.cin;
   a.ep.out = dx;
   a.ep.ldo = g.cin;
