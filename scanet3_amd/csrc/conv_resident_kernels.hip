@@ -310,8 +310,8 @@ __global__ __launch_bounds__(512) void conv_resident_kernel(ResidentArgs a) {
   find_run(tile_begin + wtile);
   read_run(0, run_at, af);
   if (resident) read_filter(filter + first_of(0, a.pairs) * KW * STEP + lane * 16, bf);
-  // (all wavefronts go through the same chunks: a tile beyond the workgroup's last is one of zeros, whose stores are dropped)
-  const int rounds_end = resident ? tile_end : tile_begin + (tile_end - tile_begin + TILES - 1) / TILES * TILES;
+  // (all wavefronts go through the same chunks and hand-overs: a tile beyond the workgroup's last is one of zeros, whose stores are dropped)
+  const int rounds_end = resident && WVK == 1 ? tile_end : tile_begin + (tile_end - tile_begin + TILES - 1) / TILES * TILES;
   for (int tile = tile_begin + wtile; tile < rounds_end; tile += TILES) {
     const int m0 = tile < tile_end ? tile * 32 : a.tiles * 32;
     f16v acc[TN], low[TN];  // sums of the hi x hi products, and of the others
