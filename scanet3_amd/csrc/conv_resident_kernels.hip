@@ -45,7 +45,6 @@ struct ResidentArgs {
   FastDiv by_iw, by_ih, by_run;  // by_run: iw + KW - 1
   int oy, ty;              // image row of filter row r: iy + oy + r * ty
   int ox;                  // image column of the first value of a run
-  int reversed;            // a run's values meet the filter row's taps from the last to the first
   int H, W, C;             // source image
   int kh;
   const float* w;
@@ -66,9 +65,10 @@ __device__ __forceinline__ f4v load16(__amdgpu_buffer_rsrc_t rs, uint32_t off) {
   return __builtin_bit_cast(f4v, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)off, 0, 0));
 }
 
-// WVK = 2: two wavefronts share 32 positions and walk half of K each (few positions: twice the workgroups, and still two
-// wavefronts a SIMD); the second hands its sums over through LDS at the end.
-template <int TN, int KW, int WVK>
+// WVK = 2: two wavefronts share 32 positions and walk half of K each (few positions, long reductions: twice the workgroups, and still two
+// wavefronts a SIMD); the second hands its sums over through LDS at the end.  (32512 x 32 x 864 24.1 us for 29.4.)
+// DX: the input gradient, whose runs meet a filter row's taps from the last to the first.
+template <int TN, int KW, int WVK, bool DX>
 __global__ __launch_bounds__(512) void conv_resident_kernel(ResidentArgs a) {
   constexpr int T = 512, TILES = 8 / WVK, STEP = TN * 3 * 1024;  // tiles of a workgroup; bytes of a step of the filter
   constexpr int LOADS = RESIDENT_ELEMENTS / 16, PLANE = RESIDENT_ELEMENTS * 32;
@@ -122,20 +122,22 @@ __global__ __launch_bounds__(512) void conv_resident_kernel(ResidentArgs a) {
         const int u = 2 * (pair0 + pair) + (TN == 1 ? lhi : block % TN);
         int r, c8;
         place_of(u, r, c8);
-        const int tap = r * KW + (a.reversed ? KW - 1 - q : q), c = min(8 * c8, a.C - 8);
+        const int tap = r * KW + (DX ? KW - 1 - q : q), c = min(8 * c8, a.C - 8);
         const bool in = u < a.units;
         skip[e] = in && n < a.N ? 8 * c8 - c : 8;  // channels that the unit before has
-        const int from = (in ? tap * a.w_tap + c * a.w_c : 0) + min(n, a.N - 1) * a.w_n;
-        if (a.w_c == 1) {  // (an input gradient: a column's channels lie side by side, the columns themselves a row of filters apart)
-          const f4v first = load16(rw, (uint32_t)from * 4u), second = load16(rw, (uint32_t)from * 4u + 16u);
+        const int column = min(n, a.N - 1) * a.w_n;
+        if constexpr (DX) {  // (a column's channels lie side by side, the columns themselves a row of filters apart)
+          const uint32_t from = (uint32_t)((in ? tap * a.w_tap + c : 0) + column) * 4u;
+          const f4v first = load16(rw, from), second = load16(rw, from + 16u);
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
             v[e][j] = first[j];
             v[e][4 + j] = second[j];
           }
         } else {
+          const float* from = a.w + (in ? tap * a.w_tap + c * a.w_c : 0) + column;
 #pragma unroll
-          for (int j = 0; j < 8; ++j) v[e][j] = a.w[from + j * a.w_c];
+          for (int j = 0; j < 8; ++j) v[e][j] = from[j * a.w_c];
         }
       }
 #pragma unroll
@@ -469,7 +471,7 @@ __global__ __launch_bounds__(512) void conv_resident_kernel(ResidentArgs a) {
           for (int v = 0; v < 16; ++v) acc[n][v] = 0.f;
         for (int r = 0; r < a.kh; ++r)
           for (int q = 0; q < KW; ++q) {
-            const int tap = r * KW + (a.reversed ? KW - 1 - q : q);
+            const int tap = r * KW + (DX ? KW - 1 - q : q);
             const uint32_t at = value_at(m0 + l32, r, q);
 #pragma unroll 1
             for (int c0 = 0; c0 < a.C; c0 += 8) {
@@ -496,9 +498,9 @@ __global__ __launch_bounds__(512) void conv_resident_kernel(ResidentArgs a) {
   }
 }
 
-template <int TN, int KW, int WVK>
+template <int TN, int KW, int WVK, bool DX>
 int launch_resident(sn_ctx* ctx, const char* name, ResidentArgs& a, const ResidentPlan& p) {
-  auto kernel = conv_resident_kernel<TN, KW, WVK>;
+  auto kernel = conv_resident_kernel<TN, KW, WVK, DX>;
   SN_TRY(allow_dynamic_lds(ctx, reinterpret_cast<const void*>(kernel), RESIDENT_LDS));
   LaunchScope scope(ctx, name, a.M, a.N, a.kh * KW * a.C);
   hipLaunchKernelGGL(kernel, dim3((unsigned)(8 * ceil_div((int64_t)p.blocks_n * p.per_block, 8))), dim3(512), (size_t)p.lds, ctx->stream, a);
@@ -506,7 +508,7 @@ int launch_resident(sn_ctx* ctx, const char* name, ResidentArgs& a, const Reside
   return SN_OK;
 }
 
-template <int KW>
+template <int KW, bool DX>
 int launch_planned(sn_ctx* ctx, const char* name, ResidentArgs& a) {
   const ResidentPlan p = resident_plan(a.M, a.N, a.C, a.kh, KW, ctx->compute_units);
   a.units_per_row = p.units_per_row;
@@ -521,8 +523,8 @@ int launch_planned(sn_ctx* ctx, const char* name, ResidentArgs& a) {
   a.by_run = fast_div((uint32_t)(a.iw + KW - 1));
   a.by_units = fast_div((uint32_t)a.units_per_row);
   a.out_bytes = (uint32_t)((int64_t)a.M * a.N * 4);
-  if (p.wvk == 2) return p.tn == 1 ? launch_resident<1, KW, 2>(ctx, name, a, p) : launch_resident<2, KW, 2>(ctx, name, a, p);
-  return p.tn == 1 ? launch_resident<1, KW, 1>(ctx, name, a, p) : launch_resident<2, KW, 1>(ctx, name, a, p);
+  if (p.wvk == 2) return p.tn == 1 ? launch_resident<1, KW, 2, DX>(ctx, name, a, p) : launch_resident<2, KW, 2, DX>(ctx, name, a, p);
+  return p.tn == 1 ? launch_resident<1, KW, 1, DX>(ctx, name, a, p) : launch_resident<2, KW, 1, DX>(ctx, name, a, p);
 }
 
 }  // namespace
@@ -537,7 +539,7 @@ int launch_conv_resident_fwd(sn_ctx* ctx, const ConvGeom& g, const float* x, con
   a.w = w; a.w_bytes = (uint32_t)((int64_t)g.kh * g.kw * g.cin * g.cout * 4); a.w_tap = g.cin * g.cout; a.w_c = g.cout; a.w_n = 1;
   a.N = g.cout;
   a.ep = e;
-  return g.kw == 3 ? launch_planned<3>(ctx, "conv2d_forward", a) : launch_planned<5>(ctx, "conv2d_forward", a);
+  return g.kw == 3 ? launch_planned<3, false>(ctx, "conv2d_forward", a) : launch_planned<5, false>(ctx, "conv2d_forward", a);
 }
 
 int launch_conv_resident_dgrad(sn_ctx* ctx, const ConvGeom& g, const float* dy, const float* w, float* dx) {
@@ -545,13 +547,13 @@ int launch_conv_resident_dgrad(sn_ctx* ctx, const ConvGeom& g, const float* dy, 
   a.src = dy;
   a.src_bytes = (uint32_t)((int64_t)g.n * g.ho * g.wo * g.cout * 4);
   a.M = g.n * g.h * g.w; a.ih = g.h; a.iw = g.w;
-  a.oy = g.pt; a.ty = -1; a.ox = g.pl - (g.kw - 1); a.reversed = 1;
+  a.oy = g.pt; a.ty = -1; a.ox = g.pl - (g.kw - 1);
   a.H = g.ho; a.W = g.wo; a.C = g.cout; a.kh = g.kh;
   a.w = w; a.w_bytes = (uint32_t)((int64_t)g.kh * g.kw * g.cin * g.cout * 4); a.w_tap = g.cin * g.cout; a.w_c = 1; a.w_n = g.cout;
   a.N = g.cin;
   a.ep.out = dx;
   a.ep.ldo = g.cin;
-  return g.kw == 3 ? launch_planned<3>(ctx, "conv2d_input_gradient", a) : launch_planned<5>(ctx, "conv2d_input_gradient", a);
+  return g.kw == 3 ? launch_planned<3, true>(ctx, "conv2d_input_gradient", a) : launch_planned<5, true>(ctx, "conv2d_input_gradient", a);
 }
 
 }  // namespace sn
