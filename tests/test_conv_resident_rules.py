@@ -27,6 +27,7 @@ def test_plans_cover_the_product_and_fit_lds(ask):
         assert 32 * tiles >= positions > 32 * (tiles - 1)
         # table, runs, and a step more of the filter than is multiplied; two wavefronts on a tile hand their sums over where it lay
         assert (pairs + 4) * 16 + 8 * 48 * 96 + max((chunk * kw + 1) * tn * 3072, 4 * (tn * 1024 + 64) * 4 * (wvk - 1)) <= lds <= 160 * 1024 - 64
+        assert (wvk == 2) == ((tiles + 3) // 4 * blocks_n <= 256 and pairs * kw * tn >= 18)
         if wvk == 2:  # one tile for every pair of wavefronts, one round of workgroups
             assert 4 * per_block >= tiles > 4 * (per_block - 1) and per_block * blocks_n <= 256
         else:
@@ -60,6 +61,15 @@ def test_filters_beyond_lds(ask):
         for pairs, planned in ((chunks["last"], True), (chunks["none"], False)):
             plan = ask("plan", 529000, columns, 16 * pairs, 1, kw)
             assert (plan[3] >= 1) == planned and (not planned or plan[2] == pairs and plan[9] <= 160 * 1024 - 64)
+
+
+def test_which_convolutions_of_one_round(ask):
+    """Up to 128 positions a CU short reductions stay with the tiled kernels, and input gradients from whole 32s of filters with the ring."""
+    for batch, beyond in ((118, 0), (128, 0), (129, 1)):  # 30208, 32768 and 33024 positions
+        for want, *shape in (([beyond, beyond], 8, 16, 1, 5), ([beyond, beyond], 16, 16, 2, 3), ([1, 1], 16, 24, 3, 3), ([1, 1], 24, 40, 3, 3), ([1, 1], 8, 8, 5, 5),
+                             ([1, beyond], 64, 64, 3, 3), ([1, beyond], 64, 64, 1, 3), ([1, 0], 16, 32, 3, 3), ([1, 1], 64, 40, 3, 3)):
+            assert ask("takes", batch, 16, 16, *shape, 1) == want, (batch, shape)
+    assert ask("takes", 117, 16, 16, 24, 40, 3, 3, 1) == [0, 0]
 
 
 def test_which_convolutions(ask):
