@@ -42,13 +42,21 @@ inline int64_t conv_wgrad_split_workspace(const ConvGeom& g, int cu) {
   const int64_t size = (int64_t)g.kh * g.kw * g.cin * g.cout;
   return conv_wgrad_split_plan(g, cu, size * cu).parts * size;
 }
-// 32-bit byte offsets (a tile's values behind a run included), a bit for every row and column of the filter, a run that fills a good part of a tile.  From 4096 positions:
+// 32-bit byte offsets (a tile's values behind a run included), a bit for every row and column of the filter.  From 4096 positions:
 // at 3136 x 128 x 576 both ways take 15.3 us, at 5760 x 8 x 144 this one 7.9 for 9.8, and below that nothing is left to gain.
+// A filter row of a few values leaves most of its tile of 32 empty, once for every row, where the split products' tiles of 64 hold
+// several rows: from half as many rows again on they are ahead, unless the result is small enough (512 values) for the kernel of small
+// outputs, which this one beats at any run.  Positions x filters x values (rows of taps), the kernels before / this one with the sums of
+// the partial results, us: 98000 x 16 x 50 (5) 29.4 / 34.2, 392000 x 64 x 60 (5) 58 / 87, 392000 x 16 x 56 (7) 52 / 94, 98000 x 16 x 252 (7)
+// 46 / 50; 392000 x 16 x 96 (6) 71 / 84; below that 392000 x 16 x 294 (7) 144 / 135, 392000 x 16 x 192 (4) 97 / 84; small results
+// 392000 x 8 x 56 (7) 124 / 93, 392000 x 8 x 60 (3) 128 / 50.
 inline bool conv_wgrad_split_ok(const ConvGeom& g, const float* x, const float* dy) {
-  const int64_t positions = (int64_t)g.n * g.ho * g.wo;
+  const int64_t positions = (int64_t)g.n * g.ho * g.wo, run = (int64_t)g.kw * g.cin, rows = g.kh * run;
   const auto fits = [](const float* p, int64_t elems) { return (reinterpret_cast<uintptr_t>(p) & 3u) == 0 && elems * 4 < ((int64_t)1 << 31) - 4096; };
-  return g.cin >= 8 && g.cin <= 4096 && g.kh <= 15 && g.kw <= 15 && fits(x, (int64_t)g.n * g.h * g.w * g.cin) && fits(dy, positions * g.cout) &&
-         positions >= 4096;
+  if (!(g.cin >= 8 && g.cin <= 4096 && g.kh <= 15 && g.kw <= 15 && fits(x, (int64_t)g.n * g.h * g.w * g.cin) && fits(dy, positions * g.cout) &&
+        positions >= 4096))
+    return false;
+  return 2 * g.kh * 32 * ceil_div(run, 32) < 3 * 64 * ceil_div(rows, 64) || rows * g.cout <= 512;
 }
 
 }  // namespace sn

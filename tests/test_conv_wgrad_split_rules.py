@@ -29,10 +29,20 @@ def test_plans_cover_the_product_and_fit_the_workspace(ask):
             assert 32 * tm * groups_m >= length > 32 * tm * (groups_m - 1) and 32 * tn * groups_n >= cout > 32 * tn * (groups_n - 1)
             assert padded == int(same and kernel != (1, 1))
             positions = n * (16 * 17 if same else (17 - kernel[0]) * (18 - kernel[1]))
-            assert 16 * chunks >= positions > 16 * (chunks - 1) and 1 <= parts <= chunks and taken == int(positions >= 4096)
+            narrow = 2 * kernel[0] * 32 * -(-length // 32) >= 3 * 64 * -(-kernel[0] * length // 64) and kernel[0] * length * cout > 512
+            assert 16 * chunks >= positions > 16 * (chunks - 1) and 1 <= parts <= chunks and taken == int(positions >= 4096 and not narrow)
             groups = kernel[0] * groups_m * groups_n
             assert parts * size <= (workspace if room < 0 else room) and (parts == 1 or groups * parts <= 256)
         assert ask(*shape, size - 1)[6] == 0  # no room for one partial result: left to the general path
+
+
+def test_narrow_runs(ask):
+    """Filter rows of a few values leave their tiles of 32 empty: not where tiles of 64 over all rows multiply two thirds as many or fewer, but
+    for results of at most 512 values."""
+    for want, cin, cout, kh, kw in ((0, 8, 32, 5, 1), (0, 12, 64, 5, 1), (0, 8, 16, 7, 1), (0, 12, 40, 7, 3), (0, 10, 16, 6, 2), (0, 9, 64, 3, 1), (0, 8, 300, 15, 1),
+                                    (1, 8, 8, 5, 1), (1, 8, 8, 7, 1), (1, 10, 16, 3, 1), (0, 12, 16, 3, 1),  # 320, 448 and 480 values; 576
+                                    (1, 8, 64, 1, 1), (1, 16, 16, 5, 1), (1, 14, 16, 7, 3), (1, 8, 16, 3, 3), (1, 8, 16, 5, 3), (1, 32, 64, 7, 1), (1, 10, 64, 4, 4)):
+        assert ask(100, 25, 25, cin, cout, kh, kw, 1, 1, -1)[0] == want, (cin, cout, kh, kw)
 
 
 def test_which_filter_gradients(ask):
