@@ -50,13 +50,24 @@ inline int64_t conv_wgrad_split_workspace(const ConvGeom& g, int cu) {
 // the partial results, us: 98000 x 16 x 50 (5) 29.4 / 34.2, 392000 x 64 x 60 (5) 58 / 87, 392000 x 16 x 56 (7) 52 / 94, 98000 x 16 x 252 (7)
 // 46 / 50; 392000 x 16 x 96 (6) 71 / 84; below that 392000 x 16 x 294 (7) 144 / 135, 392000 x 16 x 192 (4) 97 / 84; small results
 // 392000 x 8 x 56 (7) 124 / 93, 392000 x 8 x 60 (3) 128 / 50.
-inline bool conv_wgrad_split_ok(const ConvGeom& g, const float* x, const float* dy) {
+// Large results: a tile of x is fetched again for every 64 or 96 filters and one of dy for every filter row, and workgroups that leave CUs idle
+// in their last round cost more than the fetches save against split products in tiles of 128 x 128 (more than 64 filters).  So not where
+// a round behind the first is short of full, nor where a fifth of the only round is empty and the product is large enough (some 2e10
+// multiplications) for several of those tiles on a CU.  3 x 3 taps, positions x filters x channels, split products / this one: 39200 x 256 x
+// 256 350 / 399, 196000 x 512 x 128 1497 / 1899, 12544 x 512 x 512 434 / 533, 5 x 5 taps 4312 x 256 x 256 127 / 158, 12544 x 80 x 512
+// 295 / 368, 1 x 1 12544 x 2048 x 2048 743 / 789; full rounds, or smaller: 25088 x 256 x 256 295 / 263, 58800 x 384 x 384 1286 / 1178, 2 x 2
+// 12544 x 1024 x 512 443 / 421, 1 x 1 12544 x 1024 x 2048 402 / 400; at most 64 filters: 5 x 5 12544 x 64 x 1024 428 / 400.
+inline bool conv_wgrad_split_ok(const ConvGeom& g, const float* x, const float* dy, int cu) {
   const int64_t positions = (int64_t)g.n * g.ho * g.wo, run = (int64_t)g.kw * g.cin, rows = g.kh * run;
   const auto fits = [](const float* p, int64_t elems) { return (reinterpret_cast<uintptr_t>(p) & 3u) == 0 && elems * 4 < ((int64_t)1 << 31) - 4096; };
   if (!(g.cin >= 8 && g.cin <= 4096 && g.kh <= 15 && g.kw <= 15 && fits(x, (int64_t)g.n * g.h * g.w * g.cin) && fits(dy, positions * g.cout) &&
         positions >= 4096))
     return false;
-  return 2 * g.kh * 32 * ceil_div(run, 32) < 3 * 64 * ceil_div(rows, 64) || rows * g.cout <= 512;
+  if (2 * g.kh * 32 * ceil_div(run, 32) >= 3 * 64 * ceil_div(rows, 64) && rows * g.cout > 512) return false;
+  if (g.cout <= 64) return true;
+  const WgradSplitPlan p = conv_wgrad_split_plan(g, cu, rows * g.cout * cu);
+  const int64_t items = (int64_t)g.kh * p.groups_m * p.groups_n * p.parts, places = ceil_div(items, cu) * cu, idle = places - items;
+  return places > cu ? 20 * idle <= places : 5 * idle <= places || (double)positions * (double)(rows * g.cout) < 2e10;
 }
 
 }  // namespace sn

@@ -895,7 +895,7 @@ int launch_conv_wgrad(sn_ctx* ctx, const ConvGeom& g, const float* x, const floa
   // A tile per filter tap, for 32 channels onto 32 or 64 filters: level with the split products at 20160 and 24480 x 64 x 288 (18.2 and
   // 19.0 us), behind them at 28800 (21.1 and 19.2) and 52900 (29.5 and 25.1).
   const bool taps = ws && aligned16(ws) && conv_wgrad_taps_shape(ctx, g, x, dy) && conv_wgrad_taps_workspace(ctx, g) <= ws_elems;
-  if (ws && (K >= 24576 || !taps) && conv_wgrad_split_ok(g, x, dy) && conv_wgrad_split_plan(g, ctx->compute_units, ws_elems).parts >= 1)
+  if (ws && (K >= 24576 || !taps) && conv_wgrad_split_ok(g, x, dy, ctx->compute_units) && conv_wgrad_split_plan(g, ctx->compute_units, ws_elems).parts >= 1)
     return launch_conv_wgrad_split(ctx, g, x, dy, dw, ws, ws_elems);
   if (taps) {
     // a tile per filter tap: a few dozen partial filters instead of the 64 x 64 tiling's hundreds

@@ -15,7 +15,7 @@ int main(int argc, char** argv) {
                        same ? (v[5] - 1) / 2 : 0, same ? (v[6] - 1) / 2 : 0};
   const int64_t workspace = sn::conv_wgrad_split_workspace(g, 256), room = std::atoll(argv[10]);
   const sn::WgradSplitPlan p = sn::conv_wgrad_split_plan(g, 256, room < 0 ? workspace : room);
-  std::printf("%d %d %d %d %d %d %d %d %lld\n", sn::conv_wgrad_split_ok(g, at, at), p.tm, p.tn, p.groups_m, p.groups_n, p.chunks, p.parts, p.padded,
+  std::printf("%d %d %d %d %d %d %d %d %lld\n", sn::conv_wgrad_split_ok(g, at, at, 256), p.tm, p.tn, p.groups_m, p.groups_n, p.chunks, p.parts, p.padded,
               (long long)workspace);
   return 0;
 }

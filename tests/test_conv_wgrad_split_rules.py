@@ -30,8 +30,12 @@ def test_plans_cover_the_product_and_fit_the_workspace(ask):
             assert padded == int(same and kernel != (1, 1))
             positions = n * (16 * 17 if same else (17 - kernel[0]) * (18 - kernel[1]))
             narrow = 2 * kernel[0] * 32 * -(-length // 32) >= 3 * 64 * -(-kernel[0] * length // 64) and kernel[0] * length * cout > 512
-            assert 16 * chunks >= positions > 16 * (chunks - 1) and 1 <= parts <= chunks and taken == int(positions >= 4096 and not narrow)
             groups = kernel[0] * groups_m * groups_n
+            if room < 0:
+                places = -(-groups * parts // 256) * 256
+                idle = places - groups * parts
+                short = cout > 64 and (20 * idle > places if places > 256 else 5 * idle > places and positions * kernel[0] * length * cout >= 2e10)
+            assert 16 * chunks >= positions > 16 * (chunks - 1) and 1 <= parts <= chunks and taken == int(positions >= 4096 and not narrow and not short)
             assert parts * size <= (workspace if room < 0 else room) and (parts == 1 or groups * parts <= 256)
         assert ask(*shape, size - 1)[6] == 0  # no room for one partial result: left to the general path
 
@@ -43,6 +47,15 @@ def test_narrow_runs(ask):
                                     (1, 8, 8, 5, 1), (1, 8, 8, 7, 1), (1, 10, 16, 3, 1), (0, 12, 16, 3, 1),  # 320, 448 and 480 values; 576
                                     (1, 8, 64, 1, 1), (1, 16, 16, 5, 1), (1, 14, 16, 7, 3), (1, 8, 16, 3, 3), (1, 8, 16, 5, 3), (1, 32, 64, 7, 1), (1, 10, 64, 4, 4)):
         assert ask(100, 25, 25, cin, cout, kh, kw, 1, 1, -1)[0] == want, (cin, cout, kh, kw)
+
+
+def test_large_results(ask):
+    """More than 64 filters, and a last round of workgroups short of full: not behind a first round, nor in the only one of a large product."""
+    for want, batch, cin, cout, kh, kw in ((1, 128, 256, 256, 3, 3), (0, 200, 256, 256, 3, 3), (0, 1000, 128, 512, 3, 3), (1, 200, 128, 128, 3, 3),
+                                           (0, 22, 512, 512, 3, 3), (1, 64, 256, 512, 3, 3), (0, 128, 256, 512, 3, 3), (1, 300, 384, 384, 3, 3),
+                                           (0, 22, 256, 256, 5, 5), (0, 64, 512, 80, 5, 5), (1, 64, 1024, 64, 5, 5), (1, 150, 512, 64, 5, 5),
+                                           (1, 64, 512, 1024, 2, 2), (1, 64, 2048, 1024, 1, 1), (0, 64, 2048, 2048, 1, 1), (1, 300, 192, 192, 3, 3)):
+        assert ask(batch, 14, 14, cin, cout, kh, kw, 1, 1, -1)[0] == want, (batch, cin, cout, kh, kw)
 
 
 def test_which_filter_gradients(ask):
