@@ -38,10 +38,6 @@ inline WgradSplitPlan conv_wgrad_split_plan(const ConvGeom& g, int cu, int64_t w
     }
   return p;
 }
-inline int64_t conv_wgrad_split_workspace(const ConvGeom& g, int cu) {
-  const int64_t size = (int64_t)g.kh * g.kw * g.cin * g.cout;
-  return conv_wgrad_split_plan(g, cu, size * cu).parts * size;
-}
 // 32-bit byte offsets (a tile's values behind a run included), a bit for every row and column of the filter.  From 4096 positions:
 // at 3136 x 128 x 576 both ways take 15.3 us, at 5760 x 8 x 144 this one 7.9 for 9.8, and below that nothing is left to gain.
 // A filter row of a few values leaves most of its tile of 32 empty, once for every row, where the split products' tiles of 64 hold
@@ -68,6 +64,16 @@ inline bool conv_wgrad_split_ok(const ConvGeom& g, const float* x, const float* 
   const WgradSplitPlan p = conv_wgrad_split_plan(g, cu, rows * g.cout * cu);
   const int64_t items = (int64_t)g.kh * p.groups_m * p.groups_n * p.parts, places = ceil_div(items, cu) * cu, idle = places - items;
   return places > cu ? 20 * idle <= places : 5 * idle <= places || (double)positions * (double)(rows * g.cout) < 2e10;
+}
+
+// Floats of workspace for all parts of the plan, and what a model sets aside for it by its largest batch: nothing where that does not
+// run it (a smaller one that does takes the room there is).
+inline int64_t conv_wgrad_split_workspace(const ConvGeom& g, int cu) {
+  const int64_t size = (int64_t)g.kh * g.kw * g.cin * g.cout;
+  return conv_wgrad_split_plan(g, cu, size * cu).parts * size;
+}
+inline int64_t conv_wgrad_split_reserve(const ConvGeom& g, int cu) {
+  return conv_wgrad_split_ok(g, nullptr, nullptr, cu) ? conv_wgrad_split_workspace(g, cu) : 0;
 }
 
 }  // namespace sn

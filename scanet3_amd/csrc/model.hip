@@ -259,7 +259,7 @@ static int build_plan(sn_model* m, const sn_layer_desc* layers, int n_layers) {
         ws = std::max(ws, gemm_workspace_elems(B * (int)cur[0] * (int)cur[1], (int)cur[2], op.kh * op.kw * L.units, cu));
         {
           const ConvGeom cg{B, (int)cur[0], (int)cur[1], (int)cur[2], (int)ho, (int)wo, L.units, op.kh, op.kw, op.sh, op.sw, op.pt, op.pl};
-          if (cg.cin >= 8) ws = std::max(ws, conv_wgrad_split_workspace(cg, m->ctx->compute_units));
+          ws = std::max(ws, conv_wgrad_split_reserve(cg, m->ctx->compute_units));
           if (cg.cin == 32) ws = std::max(ws, conv_wgrad_taps_workspace(m->ctx, cg));  // the filter gradient's tile-per-tap form
         }
         break;

@@ -1,5 +1,5 @@
 // Which filter gradients conv_wgrad_split_kernels.hip takes and how it divides them, asked on the command line and answered without a GPU:
-//   n h w cin cout kh kw sh same room     taken tm tn groups_m groups_n chunks parts padded workspace (256 compute units; room: workspace floats, -1: its own)
+//   n h w cin cout kh kw sh same room     taken tm tn groups_m groups_n chunks parts padded workspace reserve (256 compute units; room: workspace floats, -1: its own)
 #include "../../scanet3_amd/csrc/conv_wgrad_split_rules.hpp"
 
 #include <cstdio>
@@ -15,7 +15,7 @@ int main(int argc, char** argv) {
                        same ? (v[5] - 1) / 2 : 0, same ? (v[6] - 1) / 2 : 0};
   const int64_t workspace = sn::conv_wgrad_split_workspace(g, 256), room = std::atoll(argv[10]);
   const sn::WgradSplitPlan p = sn::conv_wgrad_split_plan(g, 256, room < 0 ? workspace : room);
-  std::printf("%d %d %d %d %d %d %d %d %lld\n", sn::conv_wgrad_split_ok(g, at, at, 256), p.tm, p.tn, p.groups_m, p.groups_n, p.chunks, p.parts, p.padded,
-              (long long)workspace);
+  std::printf("%d %d %d %d %d %d %d %d %lld %lld\n", sn::conv_wgrad_split_ok(g, at, at, 256), p.tm, p.tn, p.groups_m, p.groups_n, p.chunks, p.parts, p.padded,
+              (long long)workspace, (long long)sn::conv_wgrad_split_reserve(g, 256));
   return 0;
 }

@@ -24,7 +24,7 @@ def test_plans_cover_the_product_and_fit_the_workspace(ask):
         shape = (n, 16, 17, cin, cout, *kernel, 1, same)
         size, length = kernel[0] * kernel[1] * cin * cout, kernel[1] * cin
         for room in (-1, size, 3 * size):
-            taken, tm, tn, groups_m, groups_n, chunks, parts, padded, workspace = ask(*shape, room)
+            taken, tm, tn, groups_m, groups_n, chunks, parts, padded, workspace, reserve = ask(*shape, room)
             assert (tm, tn) in ((1, 1), (1, 2), (1, 3), (2, 1), (2, 2), (3, 1), (3, 2))
             assert 32 * tm * groups_m >= length > 32 * tm * (groups_m - 1) and 32 * tn * groups_n >= cout > 32 * tn * (groups_n - 1)
             assert padded == int(same and kernel != (1, 1))
@@ -36,6 +36,7 @@ def test_plans_cover_the_product_and_fit_the_workspace(ask):
                 idle = places - groups * parts
                 short = cout > 64 and (20 * idle > places if places > 256 else 5 * idle > places and positions * kernel[0] * length * cout >= 2e10)
             assert 16 * chunks >= positions > 16 * (chunks - 1) and 1 <= parts <= chunks and taken == int(positions >= 4096 and not narrow and not short)
+            assert reserve == taken * workspace  # set aside only where it runs
             assert parts * size <= (workspace if room < 0 else room) and (parts == 1 or groups * parts <= 256)
         assert ask(*shape, size - 1)[6] == 0  # no room for one partial result: left to the general path
 
