@@ -539,7 +539,7 @@ int launch_conv_resident_fwd(sn_ctx* ctx, const ConvGeom& g, const float* x, con
   a.w = w; a.w_bytes = (uint32_t)((int64_t)g.kh * g.kw * g.cin * g.cout * 4); a.w_tap = g.cin * g.cout; a.w_c = g.cout; a.w_n = 1;
   a.N = g.cout;
   a.ep = e;
-  return g.kw == 3 ? launch_planned<3, false>(ctx, "conv2d_forward", a) : launch_planned<5, false>(ctx, "conv2d_forward", a);
+  return g.kw == 3 ? launch_planned<3, false>(ctx, "conv2d_forward_resident", a) : launch_planned<5, false>(ctx, "conv2d_forward_resident", a);
 }
 
 int launch_conv_resident_dgrad(sn_ctx* ctx, const ConvGeom& g, const float* dy, const float* w, float* dx) {
@@ -553,7 +553,7 @@ int launch_conv_resident_dgrad(sn_ctx* ctx, const ConvGeom& g, const float* dy, 
   a.N = g.cin;
   a.ep.out = dx;
   a.ep.ldo = g.cin;
-  return g.kw == 3 ? launch_planned<3, true>(ctx, "conv2d_input_gradient", a) : launch_planned<5, true>(ctx, "conv2d_input_gradient", a);
+  return g.kw == 3 ? launch_planned<3, true>(ctx, "conv2d_input_gradient_resident", a) : launch_planned<5, true>(ctx, "conv2d_input_gradient_resident", a);
 }
 
 }  // namespace sn

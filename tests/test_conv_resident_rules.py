@@ -83,3 +83,26 @@ def test_which_convolutions(ask):
                          ([0, 1], 60, 24, 24, 7, 50, 3, 3, 1),
                          ([0, 0], 30000, 60, 60, 8, 8, 3, 3, 1)):    # a tensor beyond 2 GiB
         assert ask("takes", *shape) == want, shape
+
+
+def test_every_variant_has_a_product_in_the_parity_tests(ask):
+    """Tiles of a workgroup x width x wavefronts a tile in both directions, and chunks with one round of tiles and with a second, ragged one; and
+    what those tests say of which products run here is what the rule says."""
+    source = open(os.path.join(ROOT, "tests", "test_gpu_parity.py")).read()
+    at = source.index("RESIDENT_CONVOLUTIONS = [")
+    shapes = eval(source[at + 24:source.index("]\n", at) + 1])
+    variants, rounds = set(), set()
+    for batch, height, width, channels, filters, (kh, kw), pad, taken in shapes:
+        if isinstance(pad, str):
+            assert ask("takes", batch, height, width, channels, filters, kh, kw, int(pad == "same")) == list(taken)
+            oh, ow = (height, width) if pad == "same" else (height - kh + 1, width - kw + 1)
+        else:
+            oh, ow = height + pad[0] + pad[1] - kh + 1, width + pad[2] + pad[3] - kw + 1
+        for direction, positions, columns, k in ((0, batch * oh * ow, filters, channels), (1, batch * height * width, channels, filters)):
+            if taken[direction]:
+                _, _, pairs, chunk, tn, blocks_n, tiles, wvk, per_block, _ = ask("plan", positions, columns, k, kh, kw)
+                variants.add((direction, tn, kw, wvk))
+                if chunk < pairs:
+                    rounds.add((tn, wvk, tiles * wvk > 8 * per_block))
+    assert variants == set(itertools.product((0, 1), (1, 2), (3, 5), (1, 2)))
+    assert rounds >= {(1, 1, True), (2, 1, True), (2, 2, False)}

@@ -2770,17 +2770,32 @@ def test_every_split_tile(S, ctx, tile):
     xb.free()
 
 
-# (batch, height, width, channels, filters, kernel, padding): convolutions whose filter is resident in LDS (30000 positions and more), at
-# the edges of their tiles: 5, 0 and 1 channels in the last unit of 8, 1 and 31 columns in the last tile of 32 and one or two tiles a
-# workgroup, 16 and 4 positions in the last tile, two wavefronts a tile, one unit, units without a partner, rows of 5 positions, runs over several
-# images, a filter in two chunks, both kernel widths, a kernel of one row and one of two, uneven padding
+# (batch, height, width, channels, filters, kernel, padding, which of forward and input gradient): convolutions whose filter is resident in
+# LDS (30000 positions and more), at the edges of their tiles: 5, 0 and 1 channels in the last unit of 8, 1 and 31 columns in the last tile of 32 and
+# one or two tiles a workgroup, 16 and 4 positions in the last tile, two wavefronts a tile, one unit, units without a partner, rows of 5
+# positions, runs over several images, both kernel widths, a kernel of one row and one of two, uneven padding, a filter in two chunks, and such a
+# one with a second, ragged round of tiles; three and more chunks and few positions of whole 32s of filters are left to the other kernels
 RESIDENT_CONVOLUTIONS = [
-    (100, 18, 18, 13, 33, (3, 3), "same"), (161, 16, 16, 8, 31, (3, 3), "valid"), (61, 23, 23, 16, 64, (5, 5), "same"), (300, 10, 11, 24, 65, (3, 3), "same"),
-    (1000, 7, 5, 9, 8, (1, 3), "same"), (40, 28, 28, 64, 40, (3, 3), "same"), (70, 22, 22, 40, 32, (2, 3), "valid"), (90, 19, 20, 17, 20, (3, 3), (2, 0, 1, 2))]
+    (100, 18, 18, 13, 33, (3, 3), "same", (1, 1)), (170, 16, 16, 8, 31, (3, 3), "valid", (1, 1)), (61, 23, 23, 16, 64, (5, 5), "same", (1, 0)),
+    (300, 10, 11, 24, 65, (3, 3), "same", (1, 1)), (1000, 7, 5, 9, 8, (1, 3), "same", (1, 1)), (40, 28, 28, 64, 40, (3, 3), "same", (1, 1)),
+    (80, 22, 22, 40, 32, (2, 3), "valid", (1, 1)), (90, 19, 20, 17, 20, (3, 3), (2, 0, 1, 2), (1, 1)), (75, 21, 22, 10, 20, (5, 5), "same", (1, 1)),
+    (60, 23, 23, 12, 20, (5, 5), "same", (1, 1)), (70, 22, 23, 16, 50, (5, 5), "same", (1, 0)), (70, 22, 23, 34, 14, (5, 5), "same", (1, 1)),
+    (60, 23, 23, 34, 14, (5, 5), "same", (1, 1)), (300, 10, 11, 72, 90, (3, 3), "same", (1, 1)), (330, 10, 11, 40, 127, (3, 3), "same", (1, 0)),
+    (330, 10, 11, 120, 36, (3, 3), "same", (0, 1)), (100, 18, 18, 41, 20, (3, 3), "same", (1, 1))]
 
 
-@pytest.mark.parametrize("batch,height,width,channels,filters,kernel,pad", RESIDENT_CONVOLUTIONS)
-def test_convolutions_with_a_resident_filter(S, ctx, batch, height, width, channels, filters, kernel, pad):
+def _profiled(ctx, call):
+    """What `call` returns, and the labels of the launches it made."""
+    ctx.profile_reset()
+    ctx.profile(True)
+    result = call()
+    ctx.sync()
+    ctx.profile(False)
+    return result, set(ctx.profile_report())
+
+
+@pytest.mark.parametrize("batch,height,width,channels,filters,kernel,pad,taken", RESIDENT_CONVOLUTIONS)
+def test_convolutions_with_a_resident_filter(S, ctx, batch, height, width, channels, filters, kernel, pad, taken):
     """Forward, input gradient (behind the first layer's filter gradient) and filter gradient against float64.  One image is of values
     that are no sums of three bf16 parts."""
     rng = np.random.default_rng(channels + filters)
@@ -2805,9 +2820,12 @@ def test_convolutions_with_a_resident_filter(S, ctx, batch, height, width, chann
         return {"out": p.reshape(y.shape), names[1]: O.conv2d_grad_filter(a, w2.shape, dp, **geometry), names[0]: O.conv2d_grad_filter(x, w1.shape, da)}
     d = [v.astype(np.float64) for v in (x, y, *w)]
     want, size = run(*d, -1.0), run(*[np.abs(v) for v in d], 1.0)
-    got = {"out": h.rep.forward(xb)}
-    h.rep.grad(xb, yb)
+    out, forward = _profiled(ctx, lambda: h.rep.forward(xb))
+    _, backward = _profiled(ctx, lambda: h.rep.grad(xb, yb))
+    got = {"out": out}
     got.update(h.rep.get_grads())
+    assert any(l.startswith("conv2d_forward_resident") for l in forward) == bool(taken[0])
+    assert any(l.startswith("conv2d_input_gradient_resident") for l in backward) == bool(taken[1])
     # float32 sums of K products round at most K times; the positions' sums are split over at least 32 workgroups
     taps = kernel[0] * kernel[1]
     steps = {"out": taps * channels + 16, names[1]: taps * (channels + filters) + got["out"].size / filters / 32 + 64}
@@ -2837,10 +2855,47 @@ def test_convolutions_with_a_resident_filter_at_the_end_of_the_range(S, ctx, val
     h.rep.set_params(params)
     xb = ctx.to_device(x)
     want = _as_float32_would(h.omodel.forward(np.where(np.isfinite(x), x, 1e300).astype(np.float64), {k: v.astype(np.float64) for k, v in params.items()}))
-    _assert_same_range(h.rep.forward(xb).reshape(want.shape), want, 1e-5)
+    got, labels = _profiled(ctx, lambda: h.rep.forward(xb))
+    assert any(l.startswith("conv2d_forward_resident") for l in labels)
+    _assert_same_range(got.reshape(want.shape), want, 1e-5)
     assert np.isinf(want).any() or value == 3.4e38
     h.close()
     xb.free()
+
+
+@pytest.mark.parametrize("batch", [100, 110])  # two wavefronts on a tile, and one
+@pytest.mark.parametrize("case", ["small", "product", "infinite"])
+def test_input_gradients_with_a_resident_filter_at_the_end_of_the_range(S, ctx, batch, case):
+    """Gradients of one image below what three bf16 parts hold, one whose product with a weight leaves the range, and an infinite one: seen
+    through the filter gradient of a 1 x 1 layer below, which only that image's pixels reach.  The outputs are 0, so the targets make dY."""
+    rng = np.random.default_rng(7)
+    side, channels, filters = 18, 11, 34
+    spec = [("conv", channels, (1, 1), (1, 1), "valid", "identity", False), ("conv", filters, (3, 3), (1, 1), "same", "identity", False), ("flatten",)]
+    h = Harness(S, ctx, spec, "mse", (side, side, 1), batch)
+    names = [p for p, _, _ in h.cm.params]
+    shapes = {p: s for p, s, _ in h.cm.params}
+    w = [np.zeros(shapes[names[0]], f32), rng.uniform(0.5, 1.0, shapes[names[1]]).astype(f32)]
+    x, y = np.zeros((batch, side, side, 1), f32), -rng.uniform(0.5, 1.0, (batch, side, side, filters)).astype(f32)
+    x[1] = rng.uniform(0.5, 1.0, x[1].shape)
+    if case == "small":
+        y[1] = -np.abs(_small(rng, y[1].shape, -104))  # (2 / size takes 20 more off)
+    else:
+        y[1, 2, 3, 4] = -1e38 if case == "product" else -np.inf
+        if case == "product":  # one tap of one channel: no other channel's gradient leaves the range
+            w[1][0, 2, 5, 4] = 1e10
+    h.rep.set_params(dict(zip(names, w)))
+    xb, yb = ctx.to_device(x), ctx.to_device(y.reshape(batch, -1))
+    with np.errstate(over="ignore"):
+        da = O.conv2d_grad_input((batch, side, side, channels), w[1].astype(np.float64), -2.0 * np.where(np.isfinite(y), y, -1e300).astype(np.float64) / y.size, padding=O.PAD_SAME)
+        want = _as_float32_would(O.conv2d_grad_filter(x.astype(np.float64), w[0].shape, da))
+    _, labels = _profiled(ctx, lambda: h.rep.grad(xb, yb))
+    assert any(l.startswith("conv2d_input_gradient_resident") for l in labels)
+    # positive terms only: float32 sums of 9 * filters and of side * side products; at 2^-120 a denormal's rounding is below that
+    _assert_same_range(h.rep.get_grads()[names[0]].reshape(want.shape), want, (9 * filters + side * side + 16) * 2.0 ** -24)
+    assert np.isinf(want).sum() == {"small": 0, "product": 1, "infinite": channels}[case]
+    h.close()
+    xb.free()
+    yb.free()
 
 
 # Every division into tiles, with and without padding: remainders of 16 positions, of 32 values of a run and of 32 filters, a stride
