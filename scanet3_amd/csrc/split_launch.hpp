@@ -135,11 +135,14 @@ static int launch_split_reduce(sn_ctx* ctx, const float* ws, int splits, int M, 
 
 // Tile and split count for a product of M x N x K: the cheapest by a model of what a launch costs.  Per tile shape: the time
 // per 32 k-values of a workgroup that has its CU to itself (a chain of load, split, store, read, multiply), and of a CU that
-// is full of workgroups, per workgroup (measured on MI355X: 288 x 64 x 52900 in one split, 8192 x 4096 x 4096; the bf16
-// column is one plane instead of three, by 1000 x 1500 x 1000, 1000 x 600 x 1500, 700 x 330 x 770 and 2124 x 2820 x 220).  A launch
-// lasts as long as its fullest CU; splitting K costs the partial sums' way through memory and the launch that adds them.
+// is full of workgroups, per workgroup (measured on MI355X: 288 x 64 x 52900 in one split, 8192 x 4096 x 4096; the bf16 column, one plane
+// instead of three, by the tiles and splits of 750 products of 16 to 8192 rows, 17 to 4096 columns and as long sums, forward, input and weight
+// gradient: the chosen ones take 1.026 times the fastest on the mean).  A launch lasts as long as its fullest CU; splitting K costs
+// the partial sums' way through memory and the launch that adds them.
 // One plane has nothing to take apart; where a CU holds several workgroups, what it can fetch bounds them, and larger tiles fetch
-// less: 1000 x 1500 x 1000 25.3 us in tiles of 64 x 32 and 22.8 in 64 x 64, 2124 x 2820 x 220 31.1 in 128 x 64 and 19.4 in 128 x 128.
+// less: 2124 x 2820 x 220 19.4 us in tiles of 128 x 128, 1869 x 1496 x 1312 (weight gradient) 35.4 in 64 x 64 and 43.5 in 128 x 128, 1000 x 1500 x
+// 1000 22.8 in 64 x 64 x 64 and 25.3 in 64 x 32.  Tiles of 128 x 64 were the fastest of one product in those 750 (two wavefronts of 64 x 64 each a
+// half of K: three and more of them on a CU take as long each as tiles of 128 x 128, 2124 x 2820 x 220 31.1 us), and are not built for one plane.
 // (Three stages of loads in flight instead of one, with every wait counting on the loads behind it, were measured over all tiles: 20 to
 // 60 % slower where a CU holds several workgroups, whose registers they take, and within 5 % of the same where it holds one.)
 struct SplitTile {
@@ -148,8 +151,8 @@ struct SplitTile {
 };
 enum { TILE_128x128, TILE_128x64, TILE_64x64, TILE_64x64_DEEP, TILE_64x32_DEEP, TILE_32x64_DEEP, SPLIT_TILES };
 constexpr SplitTile SPLIT_TILE[SPLIT_TILES] = {
-    {128, 128, 32, {1.45f, 0.75f}, {1.45f, 0.72f}}, {128, 64, 32, {1.14f, 1.00f}, {0.85f, 1.00f}}, {64, 64, 32, {0.83f, 0.56f}, {0.47f, 0.39f}},
-    {64, 64, 64, {0.60f, 0.42f}, {0.52f, 0.27f}},   {64, 32, 64, {0.44f, 0.31f}, {0.31f, 0.205f}}, {32, 64, 64, {0.46f, 0.29f}, {0.34f, 0.23f}}};
+    {128, 128, 32, {1.45f, 1.00f}, {1.45f, 0.68f}}, {128, 64, 32, {1.14f, 0.f}, {0.85f, 0.f}},  {64, 64, 32, {0.83f, 0.68f}, {0.47f, 0.29f}},
+    {64, 64, 64, {0.60f, 0.46f}, {0.52f, 0.30f}},   {64, 32, 64, {0.44f, 0.31f}, {0.31f, 0.21f}}, {32, 64, 64, {0.46f, 0.29f}, {0.34f, 0.23f}}};
 struct SplitChoice {
   int tile = 0, splits = 1;
 };
@@ -160,6 +163,7 @@ inline SplitChoice split_choose(int M, int N, int K, int cu, int64_t max_parts, 
   const int p = planes == 1 ? 1 : 0;
   for (int t = 0; t < SPLIT_TILES; ++t) {
     const SplitTile& c = SPLIT_TILE[t];
+    if (c.full[p] == 0.f) continue;  // no such tile
     const int64_t tiles = ceil_div(M, c.bm) * ceil_div(N, c.bn);
     const int stages = (int)ceil_div(K, c.bk);
     for (int wanted : counts) {
@@ -219,7 +223,9 @@ static int launch_split(sn_ctx* ctx, const char* name, int M, int N, int K, int 
     int rc = SN_OK;
     switch (c.tile) {
       case TILE_128x128: rc = launch_split_tile<128, 128, 32, 4, 2, 1, PLANES>(ctx, g, c.splits, al, bl, ep); break;
-      case TILE_128x64: rc = launch_split_tile<128, 64, 32, 2, 1, 2, PLANES>(ctx, g, c.splits, al, bl, ep); break;
+      case TILE_128x64:
+        if constexpr (PLANES != 1) rc = launch_split_tile<128, 64, 32, 2, 1, 2, PLANES>(ctx, g, c.splits, al, bl, ep);
+        break;
       case TILE_64x64_DEEP: rc = launch_split_tile<64, 64, 64, 2, 1, 4, PLANES>(ctx, g, c.splits, al, bl, ep); break;
       case TILE_64x32_DEEP: rc = launch_split_tile<64, 32, 64, 2, 1, 4, PLANES>(ctx, g, c.splits, al, bl, ep); break;
       case TILE_32x64_DEEP: rc = launch_split_tile<32, 64, 64, 1, 2, 4, PLANES>(ctx, g, c.splits, al, bl, ep); break;

@@ -2750,19 +2750,24 @@ def test_convolutions_of_many_positions_and_few_columns(S, ctx, channels, filter
     yb.free()
 
 
-# A product for each tile of the split kernels (host_checks' `choose` says which one it takes)
+# A product for each tile of the split kernels (host_checks' `choose` says which one it takes), with three planes and with one
 TILE_SHAPES = {(128, 128, 32): (1000, 4096, 70), (128, 64, 32): (50000, 64, 30), (64, 64, 32): (1030, 2050, 37), (64, 64, 64): (515, 1026, 127),
                (64, 32, 64): (33, 600, 70), (32, 64, 64): (30, 1000, 1000)}
+TILE_SHAPES_BF16 = {(128, 128, 32): (2001, 4097, 70), (64, 64, 32): (1030, 2050, 37), (64, 64, 64): (700, 2050, 37), (64, 32, 64): (515, 1026, 127),
+                    (32, 64, 64): (30, 1000, 1001)}
 
 
-@pytest.mark.parametrize("tile", sorted(TILE_SHAPES))
-def test_every_split_tile(S, ctx, tile):
-    rows, hidden, features = TILE_SHAPES[tile]
+@pytest.mark.parametrize("tile,bf16", [(t, False) for t in sorted(TILE_SHAPES)] + [(t, True) for t in sorted(TILE_SHAPES_BF16)])
+def test_every_split_tile(S, ctx, tile, bf16):
+    from scanet3_amd import _lib as L
+    rows, hidden, features = (TILE_SHAPES_BF16 if bf16 else TILE_SHAPES)[tile]
     rng = np.random.default_rng(sum(tile))
     x, w, b = rng.standard_normal((rows, features)).astype(f32), rng.standard_normal((features, hidden)).astype(f32), rng.standard_normal(hidden).astype(f32)
-    h = Harness(S, ctx, [("dense", hidden, "identity")], "mse", (features,), rows)
+    h = Harness(S, ctx, [("dense", hidden, "identity")], "mse", (features,), rows, flags=L.FLAG_GEMM_BF16 if bf16 else 0)
     h.rep.set_params({p: v for (p, _, _), v in zip(h.cm.params, (w, b))})
     xb = ctx.to_device(x)
+    if bf16:  # the operands are rounded, their products and sums are float32's
+        x, w = O.to_bf16(x), O.to_bf16(w)
     want = x.astype(np.float64) @ w.astype(np.float64) + b
     size = np.abs(x).astype(np.float64) @ np.abs(w).astype(np.float64) + np.abs(b)
     assert np.all(np.abs(h.rep.forward(xb) - want) <= (6.0 / 16.0 * features + 16.0) * 2.0 ** -24 * size)

@@ -70,7 +70,18 @@ def test_the_split_count_is_one_the_stages_reach(ask):
 
 def test_every_tile_has_a_product_in_the_parity_tests(ask):
     source = open(os.path.join(ROOT, "tests", "test_gpu_parity.py")).read()
-    shapes = eval(source[source.index("TILE_SHAPES = ") + 14:source.index("}", source.index("TILE_SHAPES = ")) + 1])
-    assert len(shapes) == 6
-    for tile, (rows, hidden, features) in shapes.items():
-        assert tuple(ask("choose", rows, hidden, features, 3, 0)[:3]) == tile
+    for name, planes, count in (("TILE_SHAPES", 3, 6), ("TILE_SHAPES_BF16", 1, 5)):
+        at = source.index(f"\n{name} = ") + len(name) + 4
+        shapes = eval(source[at:source.index("}", at) + 1])
+        assert len(shapes) == count
+        for tile, (rows, hidden, features) in shapes.items():
+            assert tuple(ask("choose", rows, hidden, features, planes, 0)[:3]) == tile
+
+
+def test_every_tile_of_one_plane_is_some_products(ask):
+    """Products of the sizes classifiers have reach every tile that is built for one plane, and no other."""
+    seen = set()
+    for m, n, k in itertools.product((16, 100, 700, 2001, 8192), (17, 330, 1500, 4097), (33, 600, 1501, 4099)):
+        for deferred in (0, 1):
+            seen.add(tuple(ask("choose", m, n, k, 1, deferred)[:3]))
+    assert seen == {(128, 128, 32), (64, 64, 32), (64, 64, 64), (64, 32, 64), (32, 64, 64)}
