@@ -136,12 +136,12 @@ static int launch_split_reduce(sn_ctx* ctx, const float* ws, int splits, int M, 
 // Tile and split count for a product of M x N x K: the cheapest by a model of what a launch costs.  Per tile shape: the time
 // per 32 k-values of a workgroup that has its CU to itself (a chain of load, split, store, read, multiply), and of a CU that
 // is full of workgroups, per workgroup (measured on MI355X: 288 x 64 x 52900 in one split, 8192 x 4096 x 4096; the bf16 column, one plane
-// instead of three, by the tiles and splits of 750 products of 16 to 8192 rows, 17 to 4096 columns and as long sums, forward, input and weight
+// instead of three, by the tiles and splits of 655 products of 16 to 8192 rows, 17 to 4096 columns and as long sums, forward, input and weight
 // gradient: the chosen ones take 1.026 times the fastest on the mean).  A launch lasts as long as its fullest CU; splitting K costs
 // the partial sums' way through memory and the launch that adds them.
 // One plane has nothing to take apart; where a CU holds several workgroups, what it can fetch bounds them, and larger tiles fetch
 // less: 2124 x 2820 x 220 19.4 us in tiles of 128 x 128, 1869 x 1496 x 1312 (weight gradient) 35.4 in 64 x 64 and 43.5 in 128 x 128, 1000 x 1500 x
-// 1000 22.8 in 64 x 64 x 64 and 25.3 in 64 x 32.  Tiles of 128 x 64 were the fastest of one product in those 750 (two wavefronts of 64 x 64 each a
+// 1000 22.8 in 64 x 64 x 64 and 25.3 in 64 x 32.  Tiles of 128 x 64 were the fastest of one product in those 655 (two wavefronts of 64 x 64 each a
 // half of K: three and more of them on a CU take as long each as tiles of 128 x 128, 2124 x 2820 x 220 31.1 us), and are not built for one plane.
 // (Three stages of loads in flight instead of one, with every wait counting on the loads behind it, were measured over all tiles: 20 to
 // 60 % slower where a CU holds several workgroups, whose registers they take, and within 5 % of the same where it holds one.)
