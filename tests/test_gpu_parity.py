@@ -1015,7 +1015,7 @@ def test_full_config_trajectory_matches_oracle(S, ctx, name):
     back = (lambda p, v: v[np.argsort(perm)] if p == first else v) if twin == "permuted" else (lambda p, v: v)
     xs_elems = batch * int(np.prod(in_shape))
     tol_loss = (TOL_BF16 if bf16 else TOL_TRAJECTORY) if twin else TOL_FULL_LOSS
-    noise = 0.0
+    noise, recent = 0.0, []
     for t in range(1, steps + 1):
         b = (t - 1) % n_batches
         rows = slice(b * batch, (b + 1) * batch)
@@ -1028,10 +1028,14 @@ def test_full_config_trajectory_matches_oracle(S, ctx, name):
             params64, ostate64, oloss2, _ = O.train_step(om, oalg, X64[rows], Y64[rows], params64, ostate64, t)
         gloss = h.rep.step(Xb.offset(b * xs_elems), Yb.offset(b * batch * out_dim), t, want_loss=True)
         assert abs(gloss - float(oloss)) / scale <= max(tol_loss, 3.0 * noise), (t, gloss, float(oloss), noise)
-        # the library is as close to the twin run (float64; for bf16 the permuted reduction) as the oracle itself is,
-        # step by step: at most twice this step's own distance, and never required to be closer than the tolerance
+        # the library is as close to the twin run (float64; for bf16 the permuted reduction) as the oracle itself is:
+        # at most twice its largest distance of the last ten steps, and never required to be closer than the tolerance.
+        # (Not of this step alone: the distances pass through zero.  LeNet's run by eleven float32 oracles that add in other
+        # orders, both layers' filters permuted: at twice the step's own distance ten of them leave the bound, by up to 4.95
+        # times it at step 99; of the ten steps' largest none is beyond 1.72 times.)
         own2 = abs(float(oloss) - float(oloss2)) / scale
-        assert abs(gloss - float(oloss2)) / scale <= max(TOL_BF16 if bf16 else TOL_TRAJECTORY, 2.0 * own2), (t, gloss, float(oloss2), own2)
+        recent = (recent + [own2])[-10:]
+        assert abs(gloss - float(oloss2)) / scale <= max(TOL_BF16 if bf16 else TOL_TRAJECTORY, 2.0 * max(recent)), (t, gloss, float(oloss2), recent)
         record_margin(name, abs(gloss - float(oloss)) / scale, abs(gloss - float(oloss2)) / scale, own2)
     got = [h.rep.get_params(), h.rep.get_opt_state(0), h.rep.get_opt_state(1)]
     measure = norm_err if bf16 else rel_err
