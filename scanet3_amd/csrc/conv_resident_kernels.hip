@@ -91,13 +91,9 @@ __global__ __launch_bounds__(512) void conv_resident_kernel(ResidentArgs a) {
   const __amdgpu_buffer_rsrc_t rs = make_rsrc(a.src, a.src_bytes), rw = make_rsrc(a.w, a.w_bytes);
 
   if (tid == 0) filter_top = filter_lossy = 0;
-  // K runs through the units from the last to the first.  (Either order is as close to float64.  The 100-step LeNet run of the tests is
-  // held to twice the float32 oracle's own distance from it, which at its step 97 depends on which ReLU a rounding flips: this order
-  // stays inside, the other was at 1.46e-3 against 1.09e-3.)
   auto place_of = [&](int u, int& r, int& c8) {
-    const int unit = max(a.units - 1 - u, 0);
-    r = (int)div_by((uint32_t)unit, a.by_units);
-    c8 = unit - r * a.units_per_row;
+    r = (int)div_by((uint32_t)u, a.by_units);
+    c8 = u - r * a.units_per_row;
   };
   for (int u = tid; u < resident_table_bytes(a.pairs) / 8; u += T) {
     int r, c8;
