@@ -27,6 +27,10 @@
 // 576 59 (73), 409948 x 15 x 522 171 (327), 458643 x 8 x 252 62 (144).  An input gradient reads the filter's channels as vectors of four:
 // value by value, every lane in a cache line of its own, taking the filter apart was as long as the products where it is walked in
 // two chunks (204800 x 64 x 576 175 us, 120 now; 137 to 157 by conv_ring_kernels.hip.  102400 x 64 x 360 69, 47; 63 by split_conv.hip).
+// Tiles beyond the ends of the range wait for memory: 32 channels are requested at a time.  One image in twenty of gradients below
+// 2^-110 (a saturated softmax's) takes 40000 x 64 x 576 from 36 to 98 us (241 eight channels at a time, value by value; the ring kernel's
+// float32 products 42 at any values), 64800 x 13 x 360 from 21 to 47 (81), all images 169000 x 32 x 576 from 55 to 189 (401); a single such
+// weight, for which every tile's values are looked at again, 169000 x 64 x 288 from 49 to 65.
 #include "split_launch.hpp"
 
 #include "conv_resident_rules.hpp"
@@ -445,9 +449,13 @@ __global__ __launch_bounds__(512) void conv_resident_kernel(ResidentArgs a) {
         for (int r = 0; r < a.kh; ++r)
           for (int q = 0; q < KW; ++q) {
             const uint32_t from = value_at(m0 + l32, r, q);
-            for (int c = 4 * lhi; c < a.C; c += 8) {
-              const f4v w = load16(rs, from == OOB ? OOB : from + 4u * (uint32_t)min(c, a.C - 4));
-              largest = max_magnitude(max_magnitude(largest, w[0], w[1]), w[2], w[3]);
+#pragma unroll 1
+            for (int c0 = 4 * lhi; c0 < a.C; c0 += 32) {
+              f4v v[4];
+#pragma unroll
+              for (int i = 0; i < 4; ++i) v[i] = load16(rs, from == OOB ? OOB : from + 4u * (uint32_t)min(c0 + 8 * i, a.C - 4));
+#pragma unroll
+              for (int i = 0; i < 4; ++i) largest = max_magnitude(max_magnitude(largest, v[i][0], v[i][1]), v[i][2], v[i][3]);
             }
           }
         for (int o = 32; o > 0; o >>= 1) largest = fmaxf(largest, __shfl_xor(largest, o));
@@ -469,23 +477,36 @@ __global__ __launch_bounds__(512) void conv_resident_kernel(ResidentArgs a) {
           for (int q = 0; q < KW; ++q) {
             const int tap = r * KW + (DX ? KW - 1 - q : q);
             const uint32_t at = value_at(m0 + l32, r, q);
+            // 32 channels requested together, as vectors where they lie side by side: four of a vector are one k of four instructions
 #pragma unroll 1
-            for (int c0 = 0; c0 < a.C; c0 += 8) {
-              float v[4], f[4][TN];
+            for (int c0 = 0; c0 < a.C; c0 += 32) {
+              f4v v[4], f[4][TN];
+              int skip[4];  // channels that the other half of the wavefront, or the vector before, has
 #pragma unroll
-              for (int j = 0; j < 4; ++j) {
-                const int c = c0 + 2 * j + lhi;
-                v[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, (int)(at != OOB && c < a.C ? at + 4u * (uint32_t)c : OOB), 0, 0));
+              for (int i = 0; i < 4; ++i) {
+                const int c = c0 + 8 * i + 4 * lhi, first = min(c, a.C - 4);
+                skip[i] = c - first;
+                v[i] = load16(rs, at == OOB ? OOB : at + 4u * (uint32_t)first);
 #pragma unroll
                 for (int n = 0; n < TN; ++n) {
-                  f[j][n] = a.w[tap * a.w_tap + min(c, a.C - 1) * a.w_c + min(n0 + n * 32 + l32, a.N - 1) * a.w_n];
-                  if (c >= a.C) f[j][n] = 0.f;
+                  const int from = tap * a.w_tap + first * a.w_c + min(n0 + n * 32 + l32, a.N - 1) * a.w_n;
+                  if constexpr (DX) {
+                    f[i][n] = load16(rw, (uint32_t)from * 4u);
+                  } else {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) f[i][n][j] = a.w[from + j * a.w_c];
+                  }
                 }
               }
 #pragma unroll
-              for (int j = 0; j < 4; ++j)
+              for (int i = 0; i < 4; ++i) {
+                if (c0 + 8 * i >= a.C) break;
 #pragma unroll
-                for (int n = 0; n < TN; ++n) acc[n] = __builtin_amdgcn_mfma_f32_32x32x2f32(v[j], f[j][n], acc[n], 0, 0, 0);
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                  for (int n = 0; n < TN; ++n)
+                    acc[n] = __builtin_amdgcn_mfma_f32_32x32x2f32(j < skip[i] ? 0.f : v[i][j], j < skip[i] ? 0.f : f[i][n][j], acc[n], 0, 0, 0);
+              }
             }
           }
       }

@@ -2872,13 +2872,13 @@ def test_convolutions_with_a_resident_filter_at_the_end_of_the_range(S, ctx, val
     xb.free()
 
 
-@pytest.mark.parametrize("batch", [100, 110])  # two wavefronts on a tile, and one
+@pytest.mark.parametrize("batch,channels,filters", [(100, 11, 34), (110, 11, 34), (110, 40, 61)])  # two wavefronts on a tile, and one; two tiles of columns
 @pytest.mark.parametrize("case", ["small", "product", "infinite"])
-def test_input_gradients_with_a_resident_filter_at_the_end_of_the_range(S, ctx, batch, case):
+def test_input_gradients_with_a_resident_filter_at_the_end_of_the_range(S, ctx, batch, channels, filters, case):
     """Gradients of one image below what three bf16 parts hold, one whose product with a weight leaves the range, and an infinite one: seen
     through the filter gradient of a 1 x 1 layer below, which only that image's pixels reach.  The outputs are 0, so the targets make dY."""
     rng = np.random.default_rng(7)
-    side, channels, filters = 18, 11, 34
+    side = 18
     spec = [("conv", channels, (1, 1), (1, 1), "valid", "identity", False), ("conv", filters, (3, 3), (1, 1), "same", "identity", False), ("flatten",)]
     h = Harness(S, ctx, spec, "mse", (side, side, 1), batch)
     names = [p for p, _, _ in h.cm.params]
