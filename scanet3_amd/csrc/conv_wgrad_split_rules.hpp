@@ -40,12 +40,19 @@ inline WgradSplitPlan conv_wgrad_split_plan(const ConvGeom& g, int cu, int64_t w
 }
 // 32-bit byte offsets (a tile's values behind a run included), a bit for every row and column of the filter.  From 4096 positions:
 // at 3136 x 128 x 576 both ways take 15.3 us, at 5760 x 8 x 144 this one 7.9 for 9.8, and below that nothing is left to gain.
-// A filter row of a few values leaves most of its tile of 32 empty, once for every row, where the split products' tiles of 64 hold
-// several rows: from half as many rows again on they are ahead, unless the result is small enough (512 values) for the kernel of small
-// outputs, which this one beats at any run.  Positions x filters x values (rows of taps), the kernels before / this one with the sums of
-// the partial results, us: 98000 x 16 x 50 (5) 29.4 / 34.2, 392000 x 64 x 60 (5) 58 / 87, 392000 x 16 x 56 (7) 52 / 94, 98000 x 16 x 252 (7)
-// 46 / 50; 392000 x 16 x 96 (6) 71 / 84; below that 392000 x 16 x 294 (7) 144 / 135, 392000 x 16 x 192 (4) 97 / 84; small results
-// 392000 x 8 x 56 (7) 124 / 93, 392000 x 8 x 60 (3) 128 / 50.
+// A filter row of a few values leaves most of its tile of 32 empty, once for every row, where the split products' tiles of 64 (32, if
+// that is enough) hold several rows, each made up to whole vectors of four.  How much more is multiplied
+// decides from half as much again on, unless the result is small enough (512 values) for the kernel of small outputs, which this one beats at
+// any run.  Below 32768 positions launches and the sums at the end are most of the time, and either way is within two microseconds up to
+// twice as much.  The kernels before / this one with the sums of the partial results, us, rows x columns x channels of the filter, number
+// of filters, at 31104, 65124 and 250128 positions:
+//   half as much again: 3 x 3 x 11, 64 24.3 / 23.1, 32.4 / 29.8, 70.6 / 63.9   3 x 3 x 12, 64 23.7 / 23.0, 31.4 / 29.3, 70.3 / 64.2
+//     3 x 1 x 12, 64 18.5 / 18.5, 23.1 / 22.8, 45.5 / 46.8   6 x 1 x 20, 64 23.7 / 23.7, 30.6 / 33.2, 70.3 / 80.5 (its rows share tiles of 64 by twos)
+//     tiles of 128 filters: 3 x 3 x 11, 100 31.2 / 30.0, 41.9 / 42.8, 94.6 / 110.4   3 x 1 x 12, 100 21.9 / 22.9, 29.3 / 32.8, 67.8 / 77.9
+//   two thirds: 5 x 3 x 12, 64 28.4 / 28.2, 43.1 / 38.5, 88.2 / 95.7   three quarters: 7 x 3 x 12, 64 31.7 / 32.0, 43.2 / 46.8, 106.6 / 125.7
+//   twice as much: 4 x 1 x 9, 64 19.5 / 20.2, 23.3 / 25.8, 45.7 / 57.7   2.25 times: 9 x 1 x 8, 64 21.9 / 27.3, 28.6 / 40.7, 69.9 / 111.6
+//   a vector more than whole tiles: 3 x 3 x 14, 64 27.1 / 23.2, 44.3 / 30.0, 88.4 / 65.9   3 x 1 x 21, 64 21.7 / 19.0, 28.1 / 23.8, 69.2 / 47.7
+//   small results, 392000 positions: 7 x 1 x 8, 8 124 / 93   3 x 1 x 20, 8 128 / 50
 // Large results: a tile of x is fetched again for every 64 or 96 filters and one of dy for every filter row, and workgroups that leave CUs idle
 // in their last round cost more than the fetches save against split products in tiles of 128 x 128 (more than 64 filters).  So not where
 // a round behind the first is short of full, nor where a fifth of the only round is empty and the product is large enough (some 2e10
@@ -59,21 +66,26 @@ inline bool conv_wgrad_split_ok(const ConvGeom& g, const float* x, const float* 
   if (!(g.cin >= 8 && g.cin <= 4096 && g.kh <= 15 && g.kw <= 15 && fits(x, (int64_t)g.n * g.h * g.w * g.cin) && fits(dy, positions * g.cout) &&
         positions >= 4096))
     return false;
-  if (2 * g.kh * 32 * ceil_div(run, 32) >= 3 * 64 * ceil_div(rows, 64) && rows * g.cout > 512) return false;
+  const int64_t here = g.kh * 32 * ceil_div(run, 32), packed = g.kh * 4 * ceil_div(run, 4), there = packed <= 32 ? 32 : 64 * ceil_div(packed, 64);
+  if (2 * here >= 3 * there && rows * g.cout > 512 &&
+      (4 * here >= 9 * there || (positions >= 32768 && !(g.cout <= 64 && g.kh <= 5 && 3 * here <= 5 * there))))
+    return false;
   if (g.cout <= 64) return true;
   const WgradSplitPlan p = conv_wgrad_split_plan(g, cu, rows * g.cout * cu);
   const int64_t items = (int64_t)g.kh * p.groups_m * p.groups_n * p.parts, places = ceil_div(items, cu) * cu, idle = places - items;
   return places > cu ? 20 * idle <= places : 5 * idle <= places || (double)positions * (double)(rows * g.cout) < 2e10;
 }
 
-// Floats of workspace for all parts of the plan, and what a model sets aside for it by its largest batch: nothing where that does not
-// run it (a smaller one that does takes the room there is).
+// Floats of workspace for all parts of the plan, and what a model sets aside for it: by its largest batch, or by halves of that, the first
+// that runs it (the rule has lines above which it does not), nothing where none does.
 inline int64_t conv_wgrad_split_workspace(const ConvGeom& g, int cu) {
   const int64_t size = (int64_t)g.kh * g.kw * g.cin * g.cout;
   return conv_wgrad_split_plan(g, cu, size * cu).parts * size;
 }
-inline int64_t conv_wgrad_split_reserve(const ConvGeom& g, int cu) {
-  return conv_wgrad_split_ok(g, nullptr, nullptr, cu) ? conv_wgrad_split_workspace(g, cu) : 0;
+inline int64_t conv_wgrad_split_reserve(ConvGeom g, int cu) {
+  for (; g.n > 0; g.n /= 2)
+    if (conv_wgrad_split_ok(g, nullptr, nullptr, cu)) return conv_wgrad_split_workspace(g, cu);
+  return 0;
 }
 
 }  // namespace sn

@@ -19,6 +19,15 @@ def ask(tmp_path_factory):
     return lambda *q: [int(v) for v in subprocess.run([binary, *map(str, q)], capture_output=True, text=True, check=True).stdout.split()]
 
 
+def _narrow(positions, cin, cout, kh, kw):
+    """Tiles of 32 per filter row against tiles of 64 over all rows, each of whole vectors of four."""
+    packed = kh * 4 * -(-kw * cin // 4)
+    ratio = kh * 32 * -(-kw * cin // 32) / (32 if packed <= 32 else 64 * -(-packed // 64))
+    if ratio < 1.5 or kh * kw * cin * cout <= 512:
+        return False
+    return ratio >= 2.25 or positions >= 32768 and not (cout <= 64 and kh <= 5 and 3 * ratio <= 5)
+
+
 def test_plans_cover_the_product_and_fit_the_workspace(ask):
     for n, cin, cout, kernel, same in itertools.product((30, 311), (8, 33, 96, 512), (1, 33, 64, 300), ((1, 1), (3, 3), (15, 15)), (0, 1)):
         shape = (n, 16, 17, cin, cout, *kernel, 1, same)
@@ -29,7 +38,7 @@ def test_plans_cover_the_product_and_fit_the_workspace(ask):
             assert 32 * tm * groups_m >= length > 32 * tm * (groups_m - 1) and 32 * tn * groups_n >= cout > 32 * tn * (groups_n - 1)
             assert padded == int(same and kernel != (1, 1))
             positions = n * (16 * 17 if same else (17 - kernel[0]) * (18 - kernel[1]))
-            narrow = 2 * kernel[0] * 32 * -(-length // 32) >= 3 * 64 * -(-kernel[0] * length // 64) and kernel[0] * length * cout > 512
+            narrow = _narrow(positions, cin, cout, *kernel)
             groups = kernel[0] * groups_m * groups_n
             if room < 0:
                 places = -(-groups * parts // 256) * 256
@@ -42,12 +51,17 @@ def test_plans_cover_the_product_and_fit_the_workspace(ask):
 
 
 def test_narrow_runs(ask):
-    """Filter rows of a few values leave their tiles of 32 empty: not where tiles of 64 over all rows multiply two thirds as many or fewer, but
-    for results of at most 512 values."""
-    for want, cin, cout, kh, kw in ((0, 8, 32, 5, 1), (0, 12, 64, 5, 1), (0, 8, 16, 7, 1), (0, 12, 40, 7, 3), (0, 10, 16, 6, 2), (0, 9, 64, 3, 1), (0, 8, 300, 15, 1),
-                                    (1, 8, 8, 5, 1), (1, 8, 8, 7, 1), (1, 10, 16, 3, 1), (0, 12, 16, 3, 1),  # 320, 448 and 480 values; 576
-                                    (1, 8, 64, 1, 1), (1, 16, 16, 5, 1), (1, 14, 16, 7, 3), (1, 8, 16, 3, 3), (1, 8, 16, 5, 3), (1, 32, 64, 7, 1), (1, 10, 64, 4, 4)):
-        assert ask(100, 25, 25, cin, cout, kh, kw, 1, 1, -1)[0] == want, (cin, cout, kh, kw)
+    """Filter rows of a few values leave their tiles of 32 empty, but for results of at most 512 values: how far, at 22500 and 62500 positions."""
+    for few, many, cin, cout, kh, kw in ((0, 0, 8, 32, 5, 1), (0, 0, 12, 64, 5, 1), (0, 0, 8, 16, 9, 1), (0, 0, 8, 64, 3, 1), (0, 0, 8, 40, 4, 1),
+                                         (1, 1, 8, 8, 5, 1), (1, 1, 8, 8, 7, 1), (1, 1, 10, 16, 3, 1),  # 320, 448 and 480 values
+                                         (1, 0, 12, 40, 7, 3), (1, 0, 10, 16, 6, 2), (1, 0, 9, 64, 4, 1), (1, 0, 8, 64, 2, 1), (1, 0, 11, 65, 3, 3), (1, 0, 17, 100, 5, 2),
+                                         (1, 1, 11, 64, 3, 3), (1, 1, 12, 16, 3, 1), (1, 1, 17, 64, 5, 2),
+                                         (1, 1, 14, 100, 3, 3), (1, 1, 21, 64, 3, 1), (1, 1, 21, 300, 6, 1),  # one vector more than whole tiles of 64
+                                         (1, 1, 8, 64, 1, 1), (1, 1, 16, 16, 5, 1), (1, 1, 14, 16, 7, 3), (1, 1, 8, 16, 3, 3), (1, 1, 32, 64, 7, 1), (1, 1, 10, 64, 4, 4)):
+        for positions, want in ((22500, few), (62500, many)):
+            assert ask(positions // 625, 25, 25, cin, cout, kh, kw, 1, 1, -1)[0] == want == int(not _narrow(positions, cin, cout, kh, kw)), (cin, cout, kh, kw)
+        if few and not many:  # room for the smaller batches that run it
+            assert ask(100, 25, 25, cin, cout, kh, kw, 1, 1, -1)[9] == ask(50, 25, 25, cin, cout, kh, kw, 1, 1, -1)[8] > 0
 
 
 def test_large_results(ask):
