@@ -305,7 +305,7 @@ MEASURED_TRAFFIC = {
     # kernel label (or optimizer name): (bytes per launch, source file, sha1 of the file when measured)
     # rocprofv3 --pmc FETCH_SIZE and --pmc WRITE_SIZE (one run each), KiB per dispatch, scaled by what the same counters read
     # for a plain copy of 400 MB (FETCH_SIZE x 2.0, WRITE_SIZE x 1.0); the summaries are under profiles/
-    "conv2d_forward_resident[52900x64x288]": (22.6e6, "conv_resident_kernels.hip", "3b6871232e8ba95ca20d4b13b2a453e51257462d"),
+    "conv2d_forward_resident[52900x64x288]": (22.6e6, "conv_resident_kernels.hip", "3507d8ad8e7ef39e1da44a5402a994104c0451ff"),
     "conv2d_input_gradient[62500x32x576]": (22.3e6, "conv_ring_kernels.hip", "9ad35c60088e844b2f3f3f3c28cbad9fe520c83f"),
     "conv2d_filter_gradient_split[288x64x52900]": (29.3e6, "conv_wgrad_split_kernels.hip", "5b8cc46b4afd000d33bb69612e6f9a2dc0c5850b"),
     "gemm_bf16_256x256_bf16out[8192x4096x4096]": (474.8e6, "gemm_bf16.hip", "a403cf021cd20e0154725176d99f33018b440f94"),
@@ -318,8 +318,8 @@ MEASURED_TRAFFIC = {
     "lstm_sequence_backward_and_weight_gradient[512x1024x34560]": (520.3e6, "lstm_kernels.hip", "6d2dbe90ac02733993f507dc6304b11f1f3acfbd"),
     "rnn_sequence_forward[32768x256x288]": (74.8e6, "lstm_kernels.hip", "6d2dbe90ac02733993f507dc6304b11f1f3acfbd"),
     "rnn_sequence_backward_and_weight_gradient[512x256x34560]": (116.8e6, "lstm_kernels.hip", "6d2dbe90ac02733993f507dc6304b11f1f3acfbd"),
-    "conv2d_forward_resident[121000x64x288]": (53.7e6, "conv_resident_kernels.hip", "3b6871232e8ba95ca20d4b13b2a453e51257462d"),
-    "conv2d_input_gradient_resident[169000x32x576]": (54.8e6, "conv_resident_kernels.hip", "3b6871232e8ba95ca20d4b13b2a453e51257462d"),
+    "conv2d_forward_resident[121000x64x288]": (53.9e6, "conv_resident_kernels.hip", "3507d8ad8e7ef39e1da44a5402a994104c0451ff"),
+    "conv2d_input_gradient_resident[169000x32x576]": (54.7e6, "conv_resident_kernels.hip", "3507d8ad8e7ef39e1da44a5402a994104c0451ff"),
     "conv2d_filter_gradient_split[288x64x121000]": (62.2e6, "conv_wgrad_split_kernels.hip", "5b8cc46b4afd000d33bb69612e6f9a2dc0c5850b"),
     "mlp2_rows_forward_backward[1000x50x784]": (5.8e6, "mlp2_kernels.hip", "7b5ff003152f3165f7c9972ee5a165131409810f"),
     "mlp2_weight_gradients_and_optimizer[784x50x1000]": (28.9e6, "mlp2_kernels.hip", "7b5ff003152f3165f7c9972ee5a165131409810f"),
